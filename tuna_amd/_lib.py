@@ -15,6 +15,7 @@ import subprocess
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtuna_amd.so")
 BENCH_LIB_PATH = os.path.join(_HERE, "libtuna_amd_bench.so")
+NATIVE_PATH = os.path.join(_HERE, "_native.so")
 CSRC = os.path.join(_HERE, "csrc")
 
 OK = 0
@@ -147,6 +148,10 @@ def build(force: bool = True) -> str:
 
 _libs = {}
 _active = "product"
+_native = None
+# the entry points the extension calls, in the order of its table (EntryPoints in csrc/torch_binding.cpp)
+_NATIVE_ENTRIES = ("tuna_matmul", "tuna_matmul_fused", "tuna_matmul_multi", "tuna_matmul_grouped", "tuna_matmul_blockwise",
+                   "tuna_dequant", "tuna_dequant_blockwise", "tuna_quantize_blockwise")
 
 
 def _load(which: str):
@@ -180,6 +185,32 @@ def lib():
     return _load(_active)
 
 
+def native():
+    """tuna_amd/_native.so, bound to the active library: the ops' calls without a config (csrc/torch_binding.cpp)."""
+    return _native or _bind_native()
+
+
+def _bind_native():
+    global _native
+    import torch  # noqa: F401  (its libraries are what the extension links against)
+
+    if not os.path.exists(NATIVE_PATH):
+        raise RuntimeError(f"{NATIVE_PATH} is missing: build it with `make -C tuna_amd/csrc`")
+    from . import _native as mod
+
+    L = lib()
+    mod.bind(tuple(ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in _NATIVE_ENTRIES))
+    _native = mod
+    return mod
+
+
+def _activate(which: str) -> None:
+    global _active
+    _active = which
+    if _native is not None:
+        _bind_native()
+
+
 def bench_lib():
     """libtuna_amd_bench.so: the product's object files plus timing loops, yardsticks and routing switches."""
     return _load("bench")
@@ -189,18 +220,17 @@ def bench_lib():
 def diagnostic_build():
     """While active, every op of this package runs in libtuna_amd_bench.so, so that its process-wide switches
     (tuna_set_*) and launch counters apply to the calls made.  Yields that library."""
-    global _active
-    prev, _active = _active, "bench"
+    prev = _active
+    _activate("bench")
     try:
         yield bench_lib()
     finally:
-        _active = prev
+        _activate(prev)
 
 
 def use_diagnostic_build() -> None:
     """For a whole process (bench.py, the tuner): route every op through libtuna_amd_bench.so from now on."""
-    global _active
-    _active = "bench"
+    _activate("bench")
     bench_lib()
 
 

@@ -43,6 +43,10 @@ def matmul(x, q, s, c, o, m: int, n: int, k: int, config: GemmConfig = None,
     x fp16 [n, k]; q uint8 [m/8, k/8, 32]; s fp32 [m] (absmax per weight row);
     c fp32 [16] (codebook); o fp16 [n, m], overwritten.
     """
+    if config is None and decode_mode == _lib.DECODE_GEMM:
+        rc = _lib.native().matmul(x, q, s, c, o, m, n, k)
+        if rc is not None:
+            return _lib.check(rc)
     m, n, k = int(m), int(n), int(k)
     if m <= 0 or n <= 0 or k <= 0 or m % 8 or k % 8:
         raise ValueError(f"m and k must be positive multiples of 8 and n positive (m={m}, n={n}, k={k})")
@@ -91,6 +95,10 @@ def matmul_fused(x, q, s, c, o, m: int, n: int, k: int, epilogue: int, residual=
     EPILOGUE_RESIDUAL: o[n, m] = fp16(x @ W^T + residual), residual fp16 [n, m] (may be o).
     EPILOGUE_SILU_MUL: weight rows interleaved (2i: gate_i, 2i+1: up_i); o[n, m/2] =
     fp16(silu(gate) * up)."""
+    if config is None and decode_mode == _lib.DECODE_GEMM:
+        rc = _lib.native().matmul_fused(x, q, s, c, o, m, n, k, epilogue, residual)
+        if rc is not None:
+            return _lib.check(rc)
     m, n, k = int(m), int(n), int(k)
     _require(x, "x", torch.float16, n * k)
     _require(q, "q", torch.uint8, m * k // 2)
@@ -131,6 +139,10 @@ def matmul_multi(problems, block_size: int = None, epilogues=None, residuals=Non
     [m, k / block_size], one scale per block of a row (tuna_matmul_multi_blockwise).  With epilogues (one
     EPILOGUE_* per problem) and residuals (a tensor or None per problem) the stores are fused as in matmul_fused
     (tuna_matmul_multi_fused)."""
+    if block_size is None and epilogues is None:
+        rc = _lib.native().matmul_multi(problems)
+        if rc is not None:
+            return _lib.check(rc)
     if not problems:
         return
     if block_size is not None and (int(block_size) <= 0 or any(int(p[7]) % int(block_size) for p in problems)):
@@ -168,6 +180,10 @@ def matmul_grouped(x, q, s, c, o, m_group: int, n_groups: int, k: int, token_off
     token_offsets: n_groups+1 non-decreasing host ints.  Groups without tokens cost nothing; without a config a
     group of more than 64 tokens runs as a dense GEMM of its own (same bits as `matmul` on its slices).
     """
+    if config is None and decode_mode == _lib.DECODE_GEMM:
+        rc = _lib.native().matmul_grouped(x, q, s, c, o, m_group, n_groups, k, token_offsets)
+        if rc is not None:
+            return _lib.check(rc)
     m_group, n_groups, k = int(m_group), int(n_groups), int(k)
     offs = [int(v) for v in token_offsets]
     if len(offs) != n_groups + 1:
@@ -194,6 +210,10 @@ def dequant(q, absmax, codebook, o, m: int, k: int, decode_mode: int = _lib.DECO
     """o[m, k] = decode(q, codebook, absmax) as fp16  (extension.cpp:40-49).  block_size: weights per
     scale along a row, absmax [m, k/block_size] (the quantizer's layout for block_size < k,
     test.py:15-17); None = one scale per row."""
+    if decode_mode == _lib.DECODE_DEQUANT:
+        rc = _lib.native().dequant(q, absmax, codebook, o, m, k, block_size)
+        if rc is not None:
+            return _lib.check(rc)
     m, k = int(m), int(k)
     if m <= 0 or k <= 0 or m % 8 or k % 8:
         raise ValueError(f"m and k must be positive multiples of 8 (m={m}, k={k})")
@@ -224,6 +244,10 @@ def dequant(q, absmax, codebook, o, m: int, k: int, decode_mode: int = _lib.DECO
 def matmul_blockwise(x, q, s, c, o, m: int, n: int, k: int, block_size: int, config: GemmConfig = None) -> None:
     """matmul with one scale per block_size consecutive weights of a row: s fp32 [m, k/block_size]
     (tuna_matmul_blockwise_ex; config None = the library's choice: its blockwise table, else a derived config)."""
+    if config is None:
+        rc = _lib.native().matmul_blockwise(x, q, s, c, o, m, n, k, block_size)
+        if rc is not None:
+            return _lib.check(rc)
     m, n, k, bs = int(m), int(n), int(k), int(block_size)
     if bs <= 0 or k % bs:
         raise ValueError(f"block_size={bs} must divide k={k}")
@@ -268,6 +292,12 @@ def quantize(w, codebook=None, block_size: int = None):
     the NF4 constants, block_size to k (one scale per row, what the GEMM of the reference runs)."""
     from .quantize import nf4_codebook
 
+    if codebook is not None:
+        done = _lib.native().quantize(w, codebook, block_size)
+        if done is not None:
+            rc, q, absmax = done
+            _lib.check(rc)
+            return q, absmax, codebook
     if w.dim() != 2:
         raise ValueError("w must be [m, k]")
     m, k = w.shape
