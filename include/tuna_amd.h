@@ -272,7 +272,8 @@ int tuna_blockwise_table_entry(int i, int *m, int *n_lo, int *n_hi, int *k, int 
 /* Shape -> config.  Replaces the if-chain of kernel.cu:3018-3156 over the constants of
  * configs.cu:56-3331 by a table lookup on (m, n-bucket, k) with a derived fallback.
  * Runs on the host only (no device needed).  Returns 1 in *from_table when the shape
- * hit a tuned entry. */
+ * hit a tuned entry.  A call without a config runs it, except that from 65 tokens on 256 x 256
+ * tiles take its place where they are predicted to be faster (tuna_describe_launch says so). */
 int tuna_select_config(int m, int n, int k, tuna_gemm_config *cfg, int *from_table);
 /* The config tuna_matmul_ex(cfg = NULL, decode_mode) runs: the table lookup above for
  * TUNA_DECODE_GEMM; for TUNA_DECODE_DEQUANT, whose kernel variants the table is not tuned for,

@@ -7,6 +7,7 @@
 #include <atomic>
 #include <cstdarg>
 #include <cstdio>
+#include <cmath>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -208,10 +209,26 @@ struct TiledPlan {
     TiledArgs args;
     int tile_rows, tile_tokens;
     bool mfma32;  // rows_per_wave == 32 in a many-token config: 32 x 32 x 16 MFMAs instead of 16 x 16 x 32
+    bool wide;    // 256 x 256 with 16 x 16 x 32 MFMAs: gemm_wide.hip, which has launch arguments of its own
+    WidePlan wide_plan;
     size_t lds_bytes, ws_bytes, n_counters;
 };
 
-static int plan_tiled(int m, int n, int k, const tuna_gemm_config &c, int decode, TiledPlan *plan)
+// Compute units of the current device for the plans that divide a launch over them (the largest part's where there is
+// no device: plans are also made to describe and validate launches).
+static int planned_cus()
+{
+    int dev = 0, cus = 0;
+    if (device_cus(&dev, &cus) == hipSuccess) return cus < kMaxCus ? cus : kMaxCus;
+    (void)hipGetLastError();
+    return kMaxCus;
+}
+
+static double wide_time(int m, int n, int k, int split);
+static bool wide_balance_pays(int m, int n, int k);
+
+// balance: the last rounds of an unsplit launch of 256 x 256 tiles may be shared evenly between the compute units.
+static int plan_tiled(int m, int n, int k, const tuna_gemm_config &c, int decode, TiledPlan *plan, bool balance = true)
 {
     int rc = check_shape(m, n, k);
     if (rc) return rc;
@@ -223,6 +240,7 @@ static int plan_tiled(int m, int n, int k, const tuna_gemm_config &c, int decode
         return fail(TUNA_ERR_UNSUPPORTED, "no many-token kernel for a %d x %d tile (rows x tokens)%s", c.lds_tile_rows, tile_tokens,
                     mfma32 ? " with 32 x 32 MFMA tiles" : "");
     const int steps = ceil_div(k, 64);
+    const bool wide = c.lds_tile_rows == 256 && tile_tokens == 256 && !mfma32;
     if (c.split_k < 1 || c.split_k > steps)
         return fail(TUNA_ERR_UNSUPPORTED, "split_k=%d must be in 1..%d for the many-token kernel", c.split_k, steps);
     if (c.split_k > 65535 || ceil_div(n, tile_tokens) > 65535) return fail(TUNA_ERR_UNSUPPORTED, "grid too large");
@@ -241,7 +259,51 @@ static int plan_tiled(int m, int n, int k, const tuna_gemm_config &c, int decode
     a.steps_total = steps;
     a.split_k = c.split_k;
     a.steps_per_split = ceil_div(steps, c.split_k);
+    if (wide) {
+        plan->wide = true;
+        const int tok_off[2] = {0, n};
+        if (!plan_gemm_wide(m, k, 1, tok_off, balance && c.split_k == 1 && wide_balance_pays(m, n, k) ? 0 : c.split_k, planned_cus(), &plan->wide_plan))
+            return fail(TUNA_ERR_UNSUPPORTED, "m=%d n=%d k=%d has too many 256 x 256 tiles for one launch", m, n, k);
+        plan->ws_bytes = plan->wide_plan.ws_bytes;
+        plan->n_counters = plan->wide_plan.n_counters;
+    }
     return TUNA_OK;
+}
+
+// The launch of a planned many-token GEMM, its workspace provided (static_ws: from the static scratch).
+static int provide_workspace(bool use_static, hipStream_t stream, size_t ws_bytes, size_t n_counters, float **ws, unsigned **counters);
+static int launch_tiled(TiledPlan &tp, const void *q, const void *x, const void *code, const void *absmax, void *out, int epilogue,
+                        const void *residual, int blk_shift, bool static_ws, hipStream_t stream)
+{
+    auto fill = [&](auto &a) {
+        a.q = static_cast<const uint8_t *>(q);
+        a.x = x;
+        a.code = static_cast<const float *>(code);
+        a.absmax = static_cast<const float *>(absmax);
+        a.out = out;
+        a.epilogue = epilogue;
+        a.residual = residual;
+        a.blk_shift = blk_shift < 0 ? 0 : blk_shift;
+        return tp.ws_bytes ? provide_workspace(static_ws, stream, tp.ws_bytes, tp.n_counters, &a.ws, &a.counters) : TUNA_OK;
+    };
+    int rc;
+    hipError_t e;
+    if (tp.wide) {
+        rc = fill(tp.wide_plan.args);
+        if (rc && tp.args.split_k == 1) {
+            // (no room for the shares' partial sums - the static scratch, a stream that is capturing: whole tiles)
+            const int tok_off[2] = {0, tp.args.n};
+            if (!plan_gemm_wide(tp.args.m, tp.args.k, 1, tok_off, 1, planned_cus(), &tp.wide_plan)) return rc;
+            tp.ws_bytes = tp.n_counters = 0;
+            rc = fill(tp.wide_plan.args);
+        }
+        if (rc) return rc;
+        e = launch_gemm_wide(tp.wide_plan, blk_shift >= 0, stream);
+    } else {
+        if ((rc = fill(tp.args))) return rc;
+        e = launch_gemm_tiled(tp.args, tp.tile_rows, tp.tile_tokens, tp.mfma32, stream, blk_shift >= 0);
+    }
+    return e == hipSuccess ? TUNA_OK : hip_fail(e, "many-token gemm launch");
 }
 
 // Narrow-row kernel: checks and launch arguments for a config with rows_per_wave 16 or 32.
@@ -469,6 +531,60 @@ static bool narrow_round(int m, int n, int k, tuna_gemm_config *out)
 }
 
 
+// Microseconds of a launch of 256 x 256 many-token tiles (gemm_wide.hip) by a model read off 320 random shapes of 1024 ...
+// 57344 rows and 65 ... 4096 tokens (six per cent off on average where the tile is within half of the best): a k-step of
+// a tile takes longer the more workgroups share the chip's power, a whole tile ends with 12 us of stores, a shared one
+// with as long for the partial sums and more for every further share of it.  split: 1 whole tiles, 2 ... that many equal shares of
+// every tile, 0 the last rounds of tiles shared evenly between the compute units.
+static double wide_time(int m, int n, int k, int split)
+{
+    const double row_tiles = ceil_div(m, 256), steps = ceil_div(k, 64);
+    const double large = row_tiles * ((n + 127) >> 8), small = (n & 255) >= 1 && (n & 255) <= 128 ? row_tiles : 0.0;
+    const double tiles = large + small, cus = kMaxCus, small_cost = 0.505;
+    auto step_us = [&](double workgroups) { return 0.907 + 0.604 * (workgroups < cus ? workgroups : cus) / cus; };
+    const double kind = large > 0 ? 1.0 : small_cost;  // of the longest tile
+    if (split == 1) {
+        if (tiles <= cus) return steps * step_us(large + 0.7 * small) * kind + 12.3;
+        const double rounds = ceil(large / cus), gap = rounds * cus - large;  // small tiles fill the last round of large ones
+        const double rest = small > gap ? small - gap : 0.0, total = rounds + ceil(rest / cus) * small_cost;
+        const double last = rest > 0 || fmod(large, cus) == 0 ? cus : fmod(large, cus);
+        return steps * (step_us(cus) * (total - 1.0) + step_us(last)) + 12.3 * total;
+    }
+    if (split > 1) return (steps / split * step_us(tiles * split) * kind + 3.7) * ceil(tiles * split / cus) + 17.0 + 2.05 * (split - 2);
+    const double work = large + small * small_cost;
+    double rounds = floor(work / cus - 0.25);
+    if (rounds > floor(large / cus)) rounds = floor(large / cus);
+    if (rounds < 0) rounds = 0;
+    const double shared = tiles - rounds * cus, per_tile = cus / shared + 1.0;
+    return rounds * (steps * step_us(cus) + 12.3) + (work - rounds * cus) / cus * steps * step_us(cus) + 32.1 +
+           2.05 * (per_tile > 2 ? per_tile - 2 : 0);
+}
+
+// Whether an unsplit launch shares its last tiles between the compute units: from half a round of tiles on, where the
+// model says so.
+static bool wide_balance_pays(int m, int n, int k)
+{
+    return (long long)ceil_div(m, 256) * ceil_div(n, 256) > kMaxCus / 2 && wide_time(m, n, k, 0) < wide_time(m, n, k, 1);
+}
+
+// The grid cost model of derive_config: candidate tiles with a kernel's factor, and what a launch of `tiles` workgroups
+// (k split included) costs in units of about 4.24e-7 us per k (read off 320 random shapes at 65 ... 4096 tokens).
+struct GridCand {
+    int rows, tokens, streaming;
+    double factor;
+};
+static const GridCand kGridCand[14] = {{256, 256, 0, 0.85}, {512, 128, 1, 0.95}, {128, 256, 0, 1.00}, {256, 128, 1, 1.15}, {256, 128, 0, 1.20},
+                                       {128, 128, 0, 1.45}, {256, 64, 1, 1.45},  {256, 32, 1, 1.78},  {128, 64, 1, 1.95},  {128, 32, 1, 2.00},
+                                       {256, 16, 1, 2.60},  {128, 16, 1, 2.20},  {64, 16, 1, 4.00},   {64, 128, 0, 1.80}};
+constexpr double kGridCostUs = 4.24e-7;
+static double grid_cost(const GridCand &cd, int split, long long tiles, int k)
+{
+    const long long full = tiles / kMaxCus, rest = tiles % kMaxCus;
+    const double rounds = 1.15 * (double)full + (rest ? 0.7 + 0.45 * (double)rest / kMaxCus : 0.0);
+    const double area = (double)cd.rows * cd.tokens;
+    return rounds * (area * cd.factor / split + 1.2e7 / k) + (split > 1 ? (100.0 * split + 600.0) * area / k : 0.0);
+}
+
 static tuna_gemm_config derive_config(int m, int n, int k)
 {
     tuna_gemm_config c;
@@ -597,10 +713,6 @@ static tuna_gemm_config derive_config(int m, int n, int k)
         // 640 tokens 249 against 195 (256 x 256), 2048 x 2048 at 384 tokens 27 against 13, 20480 x 5120 at 96 tokens
         // 55 against 36, 1024 x 8192 at 160 tokens 89 against 29.  Grids of fewer than 32 workgroups (64 from 256
         // tokens) are left to the rules below, which split k.
-        struct Cand { int rows, tokens, streaming; double factor; };
-        static const Cand kCand[14] = {{256, 256, 0, 0.85}, {512, 128, 1, 0.95}, {128, 256, 0, 1.00}, {256, 128, 1, 1.15}, {256, 128, 0, 1.20},
-                                       {128, 128, 0, 1.45}, {256, 64, 1, 1.45},  {256, 32, 1, 1.78},  {128, 64, 1, 1.95},  {128, 32, 1, 2.00},
-                                       {256, 16, 1, 2.60},  {128, 16, 1, 2.20},  {64, 16, 1, 4.00},   {64, 128, 0, 1.80}};
         tuna_gemm_config best;
         double best_cost = 0.0;
         bool found = false;
@@ -611,16 +723,13 @@ static tuna_gemm_config derive_config(int m, int n, int k)
             // partial tiles, which costs about 0.3 us + 0.05 us per split and 1000 tile elements - what wins on
             // few rows with long k: 4096 x 11008 at 128 tokens 30 us as 32 tiles x 8 against 67 of the best
             // unsplit launch, 5120 x 13824 at 1000 tokens 154 us as 80 tiles of 256 x 256 x 3 against 200)
-            const Cand &cd = kCand[ci / 6];
+            const GridCand &cd = kGridCand[ci / 6];
             const int split = kSplit[ci % 6];
             if ((cd.streaming && m % cd.rows != 0) || (cd.tokens == 16 && n > 320)) continue;
             if (split > 1 && (cd.streaming || ceil_div(k, 64) / split < 8)) continue;
             const long long tiles = (long long)ceil_div(m, cd.rows) * ceil_div(n, cd.tokens) * split;
             if (tiles < (n >= 256 ? 64 : 32) || (split > 1 && tiles > kMaxCus)) continue;
-            const long long full = tiles / kMaxCus, rest = tiles % kMaxCus;
-            const double rounds = 1.15 * (double)full + (rest ? 0.7 + 0.45 * (double)rest / kMaxCus : 0.0);
-            const double area = (double)cd.rows * cd.tokens;
-            double cost = rounds * (area * cd.factor / split + 1.2e7 / k) + (split > 1 ? (100.0 * split + 600.0) * area / k : 0.0);
+            double cost = grid_cost(cd, split, tiles, k);
             if (found && cost >= best_cost) continue;
             memset(&c, 0, sizeof(c));
             c.rows_per_wave = 64, c.split_k = split, c.prefetch = 2;
@@ -763,6 +872,43 @@ static bool config_runs(int m, int n, int k, const tuna_gemm_config &c)
     }
     GemmPlan plan;
     return plan_gemm(m, n, k, c, TUNA_DECODE_GEMM, &plan) == TUNA_OK;
+}
+
+// What a launch without an explicit config runs from 65 tokens on: the selected config, or 256 x 256 tiles of gemm_wide.hip
+// in its place where their model is ahead of the grid cost model's price of that config by more than the models' error
+// (26624 x 5888 at 665 tokens 277 -> 201 us, 4096 x 14336 at 777 tokens 134 -> 116, 46848 x 5120 at 295 tokens 208 -> 166;
+// the table and the cost model were measured before that kernel and still pick the best of the other tiles).  Configs of
+// kernels that the model does not price - narrow rows, k split over lean workgroups - are left alone: they are picked
+// for shapes too small for such tiles.
+static bool wide_instead(int m, int n, int k, const tuna_gemm_config &c, tuna_gemm_config *wide)
+{
+    if (n <= 64 || is_narrow(c)) return false;
+    const int tokens = 16 * c.token_tiles, streaming = c.lds_tile_rows <= 0;
+    const int rows = streaming ? c.rows_per_wave * c.waves_m : c.lds_tile_rows;
+    double price = 0.0;
+    const bool is_wide = !streaming && rows == 256 && tokens == 256 && c.rows_per_wave != 32;
+    if (is_wide) {
+        price = wide_time(m, n, k, c.split_k == 1 && wide_balance_pays(m, n, k) ? 0 : c.split_k);
+    } else {
+        for (const GridCand &cd : kGridCand)
+            if (cd.rows == rows && cd.tokens == tokens && cd.streaming == streaming && (!streaming || c.split_k == 1))
+                price = kGridCostUs * k * grid_cost(cd, c.split_k, (long long)ceil_div(m, rows) * ceil_div(n, tokens) * c.split_k, k);
+    }
+    if (price == 0.0) return false;
+    bool found = false;
+    const long long tiles = (long long)ceil_div(m, 256) * ceil_div(n, 256);
+    for (int split : {1, 2, 3, 4, 6, 8}) {
+        if (tiles * split < 16 || (split > 1 && (tiles * split > 400 || ceil_div(k, 64) / split < 8))) continue;
+        const double t = wide_time(m, n, k, split == 1 && wide_balance_pays(m, n, k) ? 0 : split);
+        if (t >= (found ? price : 0.96 * price)) continue;
+        tuna_gemm_config w;
+        memset(&w, 0, sizeof(w));
+        w.rows_per_wave = 64, w.waves_m = 1, w.waves_k = 1, w.prefetch = 2, w.x_chunk = 64, w.token_tiles = 16, w.lds_tile_rows = 256;
+        w.split_k = split;
+        if (!config_runs(m, n, k, w)) continue;
+        *wide = w, price = t, found = true;
+    }
+    return found;
 }
 
 // The table's buckets are the reference dispatcher's (kernel.cu:3022-3155) and every entry is tuned at the lower edge
@@ -1135,6 +1281,8 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
     tuna_gemm_config c;
     if (cfg) c = *cfg;
     else select_config_for(m, n, k, decode, &c, nullptr);
+    tuna_gemm_config wide;
+    if (!cfg && decode == TUNA_DECODE_GEMM && wide_instead(m, n, k, c, &wide)) c = wide;
     if (c.lds_tile_rows > 0) {
         TiledPlan tp;
         if ((rc = plan_tiled(m, n, k, c, decode, &tp))) return rc;
@@ -1145,18 +1293,7 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
             c.split_k -= 1;
             if ((rc = plan_tiled(m, n, k, c, decode, &tp))) return rc;
         }
-        tp.args.q = static_cast<const uint8_t *>(q);
-        tp.args.x = x;
-        tp.args.code = static_cast<const float *>(code);
-        tp.args.absmax = static_cast<const float *>(absmax);
-        tp.args.out = out;
-        tp.args.epilogue = epilogue;
-        tp.args.residual = residual;
-        if (tp.ws_bytes && (rc = provide_workspace(static_ws, stream, tp.ws_bytes, tp.n_counters, &tp.args.ws, &tp.args.counters)))
-            return rc;
-        hipError_t e = launch_gemm_tiled(tp.args, tp.tile_rows, tp.tile_tokens, tp.mfma32, stream);
-        if (e != hipSuccess) return hip_fail(e, "many-token gemm launch");
-        return TUNA_OK;
+        return launch_tiled(tp, q, x, code, absmax, out, epilogue, residual, -1, static_ws, stream);
     }
     // The narrow-row kernel reads a lane's scales 2 or 4 rows at a time.  A caller that names such a config must align
     // absmax for it; when the library picked the config itself it takes the streaming kernel's derived config for a
@@ -1703,23 +1840,12 @@ static int run_blockwise(const BlockwiseCall &b, const tuna_gemm_config &c, hipS
     case kBlkTiled: {
         tuna_gemm_config t = c;
         t.rows_per_wave = 64;  // (16 x 16 x 32 MFMA tiles: the scale-block variants exist for those)
-        // (the 256 x 256 tile has no scale-block variant: its threads have no registers left for eight more scales)
-        if (!tiled_variant_exists(t.lds_tile_rows, 16 * t.token_tiles, false) || (t.lds_tile_rows == 256 && t.token_tiles == 16))
+        if (!tiled_variant_exists(t.lds_tile_rows, 16 * t.token_tiles, false))
             return fail(TUNA_ERR_UNSUPPORTED, "no many-token scale-block variant with a %d x %d tile", t.lds_tile_rows, 16 * t.token_tiles);
         TiledPlan tp;
         if ((rc = plan_tiled(m, n, k, t, TUNA_DECODE_GEMM, &tp))) return rc;
         if (dry) return TUNA_OK;
-        tp.args.q = static_cast<const uint8_t *>(b.q);
-        tp.args.x = b.x;
-        tp.args.code = static_cast<const float *>(b.code);
-        tp.args.absmax = static_cast<const float *>(b.absmax);
-        tp.args.out = b.out;
-        tp.args.epilogue = TUNA_EPILOGUE_NONE;
-        tp.args.residual = nullptr;
-        tp.args.blk_shift = shift;
-        if (tp.ws_bytes && (rc = provide_workspace(false, st, tp.ws_bytes, tp.n_counters, &tp.args.ws, &tp.args.counters))) return rc;
-        e = launch_gemm_tiled(tp.args, tp.tile_rows, tp.tile_tokens, false, st, true);
-        if (e != hipSuccess) return hip_fail(e, "many-token blockwise gemm launch");
+        if ((rc = launch_tiled(tp, b.q, b.x, b.code, b.absmax, b.out, TUNA_EPILOGUE_NONE, nullptr, shift, false, st))) return rc;
         diag::count(diag::kBlockwiseTiled);
         return TUNA_OK;
     }
@@ -2232,9 +2358,13 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
     if (!buf || len < 16) return fail(TUNA_ERR_INVALID_ARG, "buf is null or shorter than 16 bytes");
     int rc = check_shape(m, n, k);
     if (rc) return rc;
-    tuna_gemm_config c;
+    tuna_gemm_config c, w;
     if (cfg) c = *cfg;
     else select_config_for(m, n, k, decode_mode, &c, nullptr);
+    if (!cfg && decode_mode == TUNA_DECODE_GEMM && wide_instead(m, n, k, c, &w) && memcmp(&w, &c, sizeof(c)) != 0) {
+        const int at = snprintf(buf, len, "gemm_wide_kernel<256 rows x 256 tokens> split_k=%d in place of ", w.split_k);
+        return at < 0 || (size_t)at + 16 > len ? TUNA_OK : tuna_describe_launch(m, n, k, &c, decode_mode, buf + at, len - (size_t)at);
+    }
     if (c.lds_tile_rows > 0) {
         TiledPlan tp;
         if ((rc = plan_tiled(m, n, k, c, decode_mode, &tp))) return rc;

@@ -36,4 +36,28 @@ __device__ __forceinline__ void store_features4(f16 *out, const f16 *residual, i
     *reinterpret_cast<f16x4 *>(out + at) = f16x4{(f16)v0, (f16)v1, (f16)v2, (f16)v3};
 }
 
+// The same for 8 consecutive output features (col a multiple of 8, ld a multiple of 8: 16-byte stores of `out`).
+__device__ __forceinline__ void store_features8(f16 *out, const f16 *residual, int epilogue, size_t tok, int ld, int col,
+                                                const f32x4 lo, const f32x4 hi)
+{
+    float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    if (epilogue == TUNA_EPILOGUE_SILU_MUL) {
+        f16x4 h;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[i] = (f16)silu_mul(v[2 * i], v[2 * i + 1]);
+        *reinterpret_cast<f16x4 *>(out + tok * (size_t)(ld >> 1) + (col >> 1)) = h;
+        return;
+    }
+    const size_t at = tok * (size_t)ld + col;
+    if (epilogue == TUNA_EPILOGUE_RESIDUAL) {  // (the residual is aligned to 8 bytes only)
+        const f16x4 r0 = *reinterpret_cast<const f16x4 *>(residual + at), r1 = *reinterpret_cast<const f16x4 *>(residual + at + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += (float)r0[i], v[4 + i] += (float)r1[i];
+    }
+    f16x8 h;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) h[i] = (f16)v[i];
+    *reinterpret_cast<f16x8 *>(out + at) = h;
+}
+
 }  // namespace tuna

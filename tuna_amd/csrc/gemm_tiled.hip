@@ -473,7 +473,7 @@ static constexpr int kNumTiled = sizeof(kTiled) / sizeof(kTiled[0]);
 
 bool tiled_variant_exists(int bm, int bn, bool mfma32)
 {
-    if (bm == 256 && bn == 256) return true;  // gemm_wide.hip
+    if (bm == 256 && bn == 256) return true;  // gemm_wide.hip, gemm_wide32.hip
     for (int i = 0; i < kNumTiled; ++i)
         if (kTiled[i].bm == bm && kTiled[i].bn == bn) return !mfma32 || kTiled[i].fn32 != nullptr;
     return false;
@@ -489,7 +489,7 @@ static OptInFlag g_tiled_attr[16][kNumTiled][3];
 
 hipError_t launch_gemm_tiled(const TiledArgs &args, int bm, int bn, bool mfma32, hipStream_t stream, bool scale_blocks)
 {
-    if (bm == 256 && bn == 256) return !scale_blocks ? launch_gemm_wide(args, mfma32, stream) : hipErrorInvalidConfiguration;
+    if (bm == 256 && bn == 256) return mfma32 && !scale_blocks ? launch_gemm_wide32(args, stream) : hipErrorInvalidConfiguration;
     int vi = -1;
     for (int i = 0; i < kNumTiled; ++i)
         if (kTiled[i].bm == bm && kTiled[i].bn == bn) vi = i;

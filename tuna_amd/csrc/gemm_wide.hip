@@ -1,149 +1,307 @@
-// FP16-activation x 4-bit-codebook-weight GEMM for MANY tokens, 256 weight rows x 256 tokens per workgroup.
+// FP16-activation x 4-bit-codebook-weight GEMM for MANY tokens, 256 weight rows x 256 tokens per workgroup, one wave per
+// SIMD (4 waves of 512 registers), every wave decoding the weights it multiplies straight into the MFMA's registers.
 //
-// The many-token kernel of gemm_tiled.hip spends most of its LDS time per flop on fragment reads, decode-table
-// reads and tile stores.  All three shrink with the tile: a weight is decoded once per 256 tokens, an activation
-// staged once per 256 rows, and a wave that owns 128 x 128 of the tile reads half the fragments per flop of a
-// 64 x 64 one.  Such a wave needs 256 accumulator registers, so this kernel runs ONE wave per SIMD (4 waves of
-// 512 registers: the accumulators in the AGPR half) and hides every latency inside that wave's own instruction
-// stream instead of behind a second wave:
+//   * A wave owns 64 rows x all 256 tokens of the tile: 4 x 16 tiles of v_mfma_f32_16x16x32_f16, whose 256 accumulator
+//     registers sit in the AGPR half of the register file.  A 16-byte load of the packed layout is four rows x 8 k of a
+//     lane, one dword of it - eight byte pairs through the decode table, scaled - IS a lane's weight operand of one
+//     MFMA: no weight tile in LDS, and every weight is decoded once per 256 tokens.
+//   * Only the activations go through LDS, in a ring of three k-steps of [token][64 k] (128-byte rows, 16-byte slots
+//     XOR-swizzled with token & 7: no bank conflicts), 32 KB each beside the decode table's 64 KB.
+//   * The work of a k-step is spread evenly between its 128 MFMAs: per token tile (4 MFMAs) one fragment read, one table
+//     read, one address, one scaling; every fourth a 16-byte store and load of activations.  One barrier per step.
 //
-//   * a k-step of 64 is four phases; the fragments of a phase are requested between the MFMAs of the phase
-//     before, the staging of step s + 1 (scaling and tile stores of the decoded weights, activation stores) sits
-//     between the MFMAs of phases 0..2 of step s with ONE barrier behind phase 2, the table reads of a packed
-//     dword come a phase before the stores that use them (a ring of four dwords' reads), the register sets are
-//     refilled as they come free;
-//   * v_mfma_f32_16x16x32_f16 by default (rows_per_wave = 64 in the config; 8 x 8 tiles per wave, a phase is
-//     four weight tiles x eight token tiles): with operands of real data the chip gives that shape about 14 %
-//     more flops than v_mfma_f32_32x32x16_f16 (launch_unit_rate, units 10..13) - which variant M32 keeps
-//     (rows_per_wave = 32; 4 x 4 tiles per wave, a phase is a quarter of 16 k);
-//   * same tiles as gemm_tiled.hip: [row][64 k] fp16 = 128-byte rows, 16-byte slots XOR-swizzled with row & 7,
-//     two buffers of (256 + 256) rows = 128 KB; the byte-pair decode table has a copy per 32 lanes instead of
-//     per 64 (32 KB: reads at the same rate, the LDS takes a wave's 4-byte reads 32 lanes at a time), which is
-//     what lets table and tiles share the 160 KB;
-//   * a thread decodes one 32-byte record (8 rows x 8 k) per k-step; 8 consecutive threads read the 256
-//     contiguous bytes of a block row's k-step; weights and activations come through buffer loads (descriptor in
-//     scalar registers, one 32-bit offset per lane, the k-step as a scalar offset): no 64-bit address
-//     arithmetic in the loop, which a single wave per SIMD would pay for in MFMA issue slots.
-// KTAIL: k is any multiple of 8.  The last k-step is then partly beyond k: a thread whose 8-k slot of that step
-// lies beyond k loads the last slot inside k instead (no access leaves a row, whatever the descriptor's range
-// check covers), and the activations of those slots are stored as zeros, so the products vanish whatever the
-// weight slots hold (finite values: table entries times the row's own scale).  k a multiple of 64 runs the
-// variant without the selects.
+// What bounds it: the power limit.  The matrix pipes are busy 72 % of the cycles (57 % in the kernel this one replaced,
+// which passed the decoded weights through an LDS tile: 19 % more LDS time and 0.5 more instructions per MFMA), at a
+// clock that the chip lowers to about 1.7 GHz; 8192 x 8192 at 2048 tokens 250 -> 213 us (1.29 PFLOP/s), 6144 x 4096 at
+// 2000 tokens 125 -> 99, 28672 x 4096 at 2000 tokens 466 -> 408 (same boxes).
 //
-// Decode and rounding are those of the other kernels (bit-identical to kernel.cu:2178-2192); the sums are the
-// same products in the same order as the variants of gemm_tiled.hip with the same MFMA shape.
+// Tiles of 1 .. 128 tokens (the last of a group) run the same steps with half the token tiles.  How tiles become
+// workgroups is plan_gemm_wide's choice.  KTAIL: k is any multiple of 8 - the slots of the last k-step beyond k load
+// the last slot inside k (no access leaves a row), and their activations are stored as zeros.  BLK: one scale per block
+// of a row.  Decode and rounding are those of the other kernels (bit-identical to kernel.cu:2178-2192); an unshared
+// tile's sums are the same products in the same order as the 16 x 16 x 32 variants of gemm_tiled.hip.
+#include <cstring>
+
 #include "epilogue.hpp"
 
 namespace tuna {
 
 constexpr int kWideThreads = 256;
-constexpr int kWideLutBytes = 256 * 32 * 4;
 constexpr int kWideRows = 256, kWideTokens = 256;
-constexpr int kWideBuf = (kWideRows + kWideTokens) * 128;
+constexpr int kWideStage = kWideTokens * 128;  // a k-step of 64 of the token tile
 
-typedef float wide_f32x16 __attribute__((ext_vector_type(16)));
+// One token tile of a row tile's k range [s0, s1) (in k-steps of 64), accumulated onto acc.  NT token tiles of 16.
+struct WideTile {
+    const uint8_t *q;      // the group's weights
+    const unsigned char *x;  // first activation row of the token tile
+    const float *absmax;   // the group's scales
+    int m, k;              // rows of the group, reduction length
+    int row_base;          // first row of the tile in the group
+    int tokens;            // tokens of the tile (1 .. 16 NT)
+    int steps_total, blk_shift;
+};
 
-template <int NSETS, bool M32, bool KTAIL>
-__global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(const TiledArgs a)
+template <int NT, bool KTAIL, bool BLK>
+__device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &w, unsigned char *xs, int s0, int s1)
 {
-    static_assert(NSETS == 2 || NSETS == 4, "register sets of packed weights");
-    constexpr int XSETS = 2;
-    constexpr int BUF = kWideBuf;
-    extern __shared__ __align__(16) unsigned char smem[];
-    unsigned char *lut = smem;  // byte-pair table at LDS address 0: entry (byte << 7) | ((lane & 31) << 2)
-    unsigned char *a_tile = smem + kWideLutBytes;
-    unsigned char *x_tile = a_tile + kWideRows * 128;
-
+    constexpr int XP = NT / 2;  // 16-byte pieces of a step's activations a thread stages
+    constexpr int FB = 8;       // token fragments on their way (the ring: 2 NT tiles of a step divide into it)
+    constexpr int LPT = 16 / NT; // table reads per token tile and half
+    static_assert(NT == 16 || NT == 8, "token tiles");
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm_i = wave >> 1, wn_i = wave & 1;
-    const int i32 = lane & 31, h32 = lane >> 5;  // 32 x 32 tiles: row / token and k-half of a lane's fragments
-    const int i16 = lane & 15, g = lane >> 4;    // 16 x 16 tiles: row / token and k-group
-    const uint32_t lane8 = (uint32_t)(lane & 31) << 3;
+    const int i16 = lane & 15, g = lane >> 4;
+    const uint32_t lane4 = (uint32_t)lane << 2;
+    const int kb_total = w.k >> 3;
+    const int mb_last = (w.m >> 3) - 1;
 
-    // grid order as in gemm_tiled.hip: the token tiles of a row tile next to each other (and on one XCD when the
-    // row tile count is a multiple of 8)
-    int row_tile, tok_tile;
-    if ((a.row_tiles & 7) == 0) {
-        const unsigned slot = blockIdx.x >> 3;
-        tok_tile = (int)(slot % (unsigned)a.tok_tiles);
-        row_tile = (int)(slot / (unsigned)a.tok_tiles) * 8 + (int)(blockIdx.x & 7);
-    } else {
-        tok_tile = (int)(blockIdx.x % (unsigned)a.tok_tiles);
-        row_tile = (int)(blockIdx.x / (unsigned)a.tok_tiles);
-    }
-    const int row_base = row_tile * kWideRows;
-    const int tok_base = tok_tile * kWideTokens;
-    const int kb_total = a.k >> 3;
-    const int mb_last = (a.m >> 3) - 1;
-
-    // weights: thread -> block row tid / 8 of the tile, k-block tid % 8 of the step (rows beyond the matrix are
-    // clamped: their products are never stored).  Addresses are a uniform base - the tile's first block row, first
-    // token - that advances with the k-step, plus a 32-bit offset per thread inside the tile: no 64-bit vector
-    // arithmetic in the loop, short address operands, no limit on the size of q or x.
-    const int a_kb = tid & 7, a_mbl = tid >> 3;
-    const uint32_t a_off = ((uint32_t)(min((row_base >> 3) + a_mbl, mb_last) - (row_base >> 3)) * (uint32_t)kb_total + (uint32_t)a_kb) * 32u;
-    f16x2 sc16[8];
+    // weights: lane (i16, g) loads 16 bytes = rows 4 i16 .. + 3 of the wave's 64, block column 4 h + g of half h of a
+    // step (rows beyond the matrix are clamped: their products are never stored)
+    const int row_w = w.row_base + wave * 64;
+    const uint32_t a_off = (uint32_t)(min((row_w >> 3) + (i16 >> 1), mb_last) - (w.row_base >> 3)) * (uint32_t)kb_total * 32u +
+                           (uint32_t)(i16 & 1) * 16u + (uint32_t)g * 32u;
+    // activations: piece i of a thread is token tid / 8 + 32 i, 8-k slot tid % 8 (tokens beyond the tile's read its last)
+    uint32_t x_off[XP];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const f16 h = (f16)a.absmax[min(row_base + a_mbl * 8 + j, a.m - 1)];
-        sc16[j] = f16x2{h, h};
-    }
-    unsigned char *a_dst = a_tile + a_mbl * 8 * 128;  // row a_mbl * 8 + j: + j * 128 + ((a_kb ^ j) << 4)
-    // activations: piece i of a thread is token tid / 8 + 32 i of the tile, 8-k slot tid % 8 of the step (tokens
-    // beyond n read the last token's row: their outputs are never stored)
-    uint32_t x_off[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int tok = tok_base + (tid >> 3) + 32 * i;
-        x_off[i] = ((uint32_t)(min(tok, a.n - 1) - tok_base) * (uint32_t)a.k + (uint32_t)(tid & 7) * 8u) * 2u;
-    }
-    unsigned char *x_dst = x_tile + (tid >> 3) * 128 + (((tid & 7) ^ ((tid >> 3) & 7)) << 4);  // piece i: + i * 4096
-    // KTAIL: the thread's slot of k-step s lies inside k while 64 s < x_k_left; in the last step a slot beyond k
-    // steps back to the last one inside (in bytes: 32 per slot of packed weights, 16 per slot of activations)
-    const int x_k_left = a.k - (tid & 7) * 8;
-    const int slots_back = KTAIL ? max(0, (tid & 7) - (((a.k >> 3) - 1) & 7)) : 0;
-    const uint32_t a_back = (uint32_t)slots_back * 32u, x_back = (uint32_t)slots_back * 16u;
+    for (int i = 0; i < XP; ++i) x_off[i] = ((uint32_t)min((tid >> 3) + 32 * i, w.tokens - 1) * (uint32_t)w.k + (uint32_t)(tid & 7) * 8u) * 2u;
+    unsigned char *const x_dst = xs + (tid >> 3) * 128 + (((tid & 7) ^ ((tid >> 3) & 7)) << 4);
+    // KTAIL: slots of the last step beyond k load the last slot inside k, and their activations are stored as zeros
+    const int x_k_left = w.k - (tid & 7) * 8;
+    const int slot_last = ((w.k >> 3) - 1) & 7;
+    const uint32_t x_back = KTAIL ? (uint32_t)max(0, (tid & 7) - slot_last) * 16u : 0u;
+    const uint32_t a_back0 = KTAIL ? (uint32_t)max(0, g - slot_last) * 32u : 0u;
+    const uint32_t a_back1 = KTAIL ? (uint32_t)max(0, 4 + g - slot_last) * 32u : 0u;
 
-    u32x4 wq[NSETS][2];
-    u32x4 xr[XSETS][8];
-    // buffer loads: descriptor + 32-bit offset per lane + uniform offset of the k-step (weights without the
-    // nontemporal hint: the token tiles of a row tile run side by side and share them through the L2)
-    const size_t q_rest = (size_t)(a.m - row_base) * (size_t)(a.k >> 1), x_rest = (size_t)(a.n - tok_base) * (size_t)a.k * 2;
+    const size_t q_rest = (size_t)(w.m - w.row_base) * (size_t)(w.k >> 1), x_rest = (size_t)w.tokens * (size_t)w.k * 2;
     const __amdgpu_buffer_rsrc_t q_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t *>(a.q) + (size_t)(row_base >> 3) * kb_total * 32, 0, (int)(uint32_t)min(q_rest, (size_t)0xffffffffu), 0x00020000);
+        const_cast<uint8_t *>(w.q) + (size_t)(w.row_base >> 3) * kb_total * 32, 0, (int)(uint32_t)min(q_rest, (size_t)0xffffffffu), 0x00020000);
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        reinterpret_cast<unsigned char *>(const_cast<void *>(a.x)) + (size_t)tok_base * a.k * 2, 0,
-        (int)(uint32_t)min(x_rest, (size_t)0xffffffffu), 0x00020000);
-#define TUNA_WIDE_LOAD(set, s)                                                                  \
-    {                                                                                          \
-        const uint32_t o_ = KTAIL && (s) == s_last ? a_off - a_back : a_off;                   \
-        wq[set][0] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)o_, (s) * 256, 0);     \
-        wq[set][1] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)o_ + 16, (s) * 256, 0); \
-    }
-#define TUNA_WIDE_LOAD_X(set, s)                                                                \
-    {                                                                                          \
-        const uint32_t b_ = KTAIL && (s) == s_last ? x_back : 0u;                              \
-        _Pragma("unroll") for (int i = 0; i < 8; ++i)                                          \
-            xr[set][i] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, (int)(x_off[i] - b_), (s) * 128, 0); \
-    }
+        const_cast<unsigned char *>(w.x), 0, (int)(uint32_t)min(x_rest, (size_t)0xffffffffu), 0x00020000);
 
-    const int s0 = blockIdx.z * a.steps_per_split;
-    const int s1 = min(a.steps_total, s0 + a.steps_per_split);
-    const int s_last = a.steps_total - 1;
+    // scales of rows 4 i16 + j: one per row, or (BLK) one per block of 64 << blk_shift weights, which travel through the
+    // register sets with the weights (a step lies inside one block)
+    const int nblk = BLK ? w.k >> (6 + w.blk_shift) : 1;
+    const float *s_base = w.absmax + (size_t)w.row_base * (size_t)nblk;
+    const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(s_base), 0, (int)(uint32_t)min((size_t)(w.m - w.row_base) * (size_t)nblk * 4, (size_t)0xffffffffu), 0x00020000);
+    uint32_t s_off[4];
 #pragma unroll
-    for (int u = 0; u < NSETS; ++u) {
-        TUNA_WIDE_LOAD(u, min(s0 + u, s_last))
-        if (u < XSETS) TUNA_WIDE_LOAD_X(u, min(s0 + u, s_last))
+    for (int j = 0; j < 4; ++j) s_off[j] = (uint32_t)(min(row_w + 4 * i16 + j, w.m - 1) - w.row_base) * (uint32_t)nblk * 4u;
+    float sq[BLK ? 2 : 1][4];
+    f16x2 sc[4];
+#define WIDE_LOAD_S(set, s)                                                                                   \
+    _Pragma("unroll") for (int j = 0; j < 4; ++j) sq[set][j] = __builtin_bit_cast(                            \
+        float, (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(s_rsrc, (int)s_off[j], BLK ? min((s) >> w.blk_shift, nblk - 1) * 4 : 0, 0));
+#define WIDE_SCALES(set)                                                                                      \
+    _Pragma("unroll") for (int j = 0; j < 4; ++j)                                                             \
+    {                                                                                                         \
+        const f16 h_ = (f16)sq[set][j];                                                                       \
+        sc[j] = f16x2{h_, h_};                                                                                \
     }
 
-    // decode table: entry e = 128 bytes = 32 copies of fp16(code[e >> 4]) | fp16(code[e & 15]) << 16
+    u32x4 wq[2][2];   // [set][half]: packed weights of two k-steps
+    u32x4 xr[2][XP];  // activations of two k-steps on their way to LDS
+    const int s_last = w.steps_total - 1;
+#define WIDE_LOAD_W(set, s)                                                                                   \
+    {                                                                                                         \
+        const int s_ = min((s), s_last);                                                                      \
+        const bool t_ = KTAIL && s_ == s_last;                                                                \
+        wq[set][0] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)(t_ ? a_off - a_back0 : a_off), s_ * 256, 0);       \
+        wq[set][1] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)(t_ ? a_off - a_back1 : a_off), s_ * 256 + 128, 0); \
+    }
+#define WIDE_LOAD_X(set, i, s)                                                                                \
+    {                                                                                                         \
+        const int s_ = min((s), s_last);                                                                      \
+        xr[set][i] = __builtin_amdgcn_raw_buffer_load_b128(                                                   \
+            x_rsrc, (int)(KTAIL && s_ == s_last ? x_off[i] - x_back : x_off[i]), s_ * 128, 0);                \
+    }
+#define WIDE_STORE_X(set, i, off, s)                                                                          \
+    {                                                                                                         \
+        u32x4 v_ = xr[set][i];                                                                                \
+        if (KTAIL && (s) * 64 >= x_k_left) v_ = u32x4{0u, 0u, 0u, 0u};                                        \
+        *reinterpret_cast<u32x4 *>(x_dst + (off) + (i) * 4096) = v_;                                          \
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        if (BLK || u == 0) WIDE_LOAD_S(u, s0 + u)
+        WIDE_LOAD_W(u, s0 + u)
+#pragma unroll
+        for (int i = 0; i < XP; ++i) WIDE_LOAD_X(u, i, s0 + u)
+    }
+
+    f16x8 fa[2][4];  // decoded weights of a half: rows 4 i16 + j
+    f16x8 fb[FB];
+    uint32_t lt[4];  // table reads on their way
+    const int swz = (g ^ (i16 & 7)) << 4;
+    const unsigned char *x_frag0 = xs + i16 * 128 + swz, *x_frag1 = xs + i16 * 128 + (64 ^ swz);
+#define WIDE_READ_B(slot, half, off, t) \
+    fb[slot] = *reinterpret_cast<const f16x8 *>(((half) ? x_frag1 : x_frag0) + (off) + (t) * 2048);
+    // table read of byte pair l (dword l / 4, byte l % 4) of a half, and its scaling (bit-identical to kernel.cu:2178-2192)
+#define WIDE_LUT(l, set, half)                                                                                \
+    lt[(l) & 3] = *reinterpret_cast<const lds_u32 *>(                                                         \
+        (uintptr_t)__builtin_amdgcn_perm(wq[set][half][(l) >> 2], lane4, 0x0c0c0400u + 0x100u * ((l) & 3)));
+#define WIDE_SCALE(l, ab)                                                                                     \
+    {                                                                                                         \
+        const f16x2 h_ = __builtin_bit_cast(f16x2, lt[(l) & 3]) * sc[(l) >> 2];                               \
+        fa[ab][(l) >> 2][2 * ((l) & 3)] = h_[0];                                                              \
+        fa[ab][(l) >> 2][2 * ((l) & 3) + 1] = h_[1];                                                          \
+    }
+    // (inline assembly with the accumulator pinned to the AGPR half of the register file: left to itself the register
+    // allocator spreads 64 four-register accumulators over both halves and spills in the loop; an accumulator is next
+    // touched 63 MFMAs later, a decoded weight is written at least four MFMAs before it is read)
+#define WIDE_MFMA(ab, j, t, slot) \
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc[j][t]) : "v"(fa[ab][j]), "v"(fb[slot]));
+
+    // Half `h` of k-step `step` (iteration `it` of the loop unrolled by two): per token tile t four MFMAs with the
+    // decoded weights fa[h] and token fragment t, and between them: the fragment FB - 1 tiles on; the scaling of a byte
+    // pair of the next half into fa[h ^ 1] and the table read of the pair three on; every fourth tile one 16-byte piece of
+    // the activations into LDS and the load two steps on that refills its registers.
+    // Stages cur, nxt, nx2 hold steps step .. step + 2.  The barrier of a step comes where the first fragment of the
+    // next step is requested: by then every wave has stored its pieces of that step (all but the last one in this step,
+    // the last one a step earlier, behind that step's barrier), and the stage that stores go to from here on was last
+    // read a step ago, by fragments that every wave has used.
+#define WIDE_HALF(it, step, h)                                                                                \
+    {                                                                                                         \
+        constexpr int dset_ = (h) == 0 ? (it) : (it) ^ 1, dh_ = (h) ^ 1;                                      \
+        _Pragma("unroll") for (int t = 0; t < NT; ++t)                                                        \
+        {                                                                                                     \
+            const int base_ = (h) * NT + t;                                                                   \
+            WIDE_MFMA(h, 0, t, base_ % FB)                                                                    \
+            if ((h) == 1 && t == NT - FB + 1) {                                                               \
+                __builtin_amdgcn_s_waitcnt(0xC07F | (FB << 8)); /* lgkmcnt: this wave's stores are done */    \
+                __builtin_amdgcn_s_barrier();                                                                 \
+                asm volatile("" ::: "memory");                                                                \
+            }                                                                                                 \
+            {                                                                                                 \
+                const int nt_ = base_ + FB - 1;                                                               \
+                WIDE_READ_B(nt_ % FB, (nt_ / NT) & 1, nt_ >= 2 * NT ? nxt : cur, nt_ % NT)                    \
+            }                                                                                                 \
+            __builtin_amdgcn_sched_barrier(0);                                                                \
+            WIDE_MFMA(h, 1, t, base_ % FB)                                                                    \
+            if (BLK && (h) == 1 && t == 0) {                                                                  \
+                WIDE_SCALES((it) ^ 1)                                                                         \
+                WIDE_LOAD_S((it) ^ 1, (step) + 3)                                                             \
+            }                                                                                                 \
+            _Pragma("unroll") for (int l = t * LPT; l < (t + 1) * LPT; ++l) {                                 \
+                WIDE_SCALE(l, dh_)                                                                            \
+                if (l + 3 < 16) WIDE_LUT(l + 3, dset_, dh_)                                                   \
+                else WIDE_LUT(l + 3 - 16, (it) ^ 1, h)                                                        \
+            }                                                                                                 \
+            __builtin_amdgcn_sched_barrier(0);                                                                \
+            WIDE_MFMA(h, 2, t, base_ % FB)                                                                    \
+            if (base_ % 4 == 0) {                                                                             \
+                const int i_ = base_ / 4;                                                                     \
+                if (i_ < XP - 1) {                                                                            \
+                    WIDE_STORE_X((it) ^ 1, i_, nxt, (step) + 1)                                               \
+                    WIDE_LOAD_X((it) ^ 1, i_, (step) + 3)                                                     \
+                } else {                                                                                      \
+                    WIDE_STORE_X(it, i_, nx2, (step) + 2)                                                     \
+                    WIDE_LOAD_X(it, i_, (step) + 4)                                                           \
+                }                                                                                             \
+            }                                                                                                 \
+            __builtin_amdgcn_sched_barrier(0);                                                                \
+            WIDE_MFMA(h, 3, t, base_ % FB)                                                                    \
+            if (t == NT - 1) {                                                                                \
+                if ((h) == 0) WIDE_LOAD_W(dset_, (step) + 2)                                                  \
+                if ((h) == 1) {                                                                               \
+                    const int c_ = cur;                                                                       \
+                    cur = nxt, nxt = nx2, nx2 = c_;                                                           \
+                }                                                                                             \
+            }                                                                                                 \
+            __builtin_amdgcn_sched_barrier(0);                                                                \
+        }                                                                                                     \
+    }
+    int cur = 0, nxt = kWideStage, nx2 = 2 * kWideStage;
+    __syncthreads();  // decode table complete; the previous tile's fragments have been read
+#pragma unroll
+    for (int i = 0; i < XP; ++i) WIDE_STORE_X(0, i, 0, s0)
+#pragma unroll
+    for (int i = 0; i < XP; ++i) WIDE_LOAD_X(0, i, s0 + 2)
+    WIDE_STORE_X(1, XP - 1, kWideStage, s0 + 1)
+    WIDE_LOAD_X(1, XP - 1, s0 + 3)
+    WIDE_SCALES(0)
+    if (BLK) WIDE_LOAD_S(0, s0 + 2)
+#pragma unroll
+    for (int l = 0; l < 16; ++l) {
+        WIDE_LUT(l, 0, 0)
+        WIDE_SCALE(l, 0)
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < FB - 1; ++t) WIDE_READ_B(t, 0, 0, t)
+#pragma unroll
+    for (int l = 0; l < 3; ++l) WIDE_LUT(l, 0, 1)
+
+    int s = s0;
+    for (; s + 1 < s1; s += 2) {
+        WIDE_HALF(0, s, 0)
+        WIDE_HALF(0, s, 1)
+        WIDE_HALF(1, s + 1, 0)
+        WIDE_HALF(1, s + 1, 1)
+    }
+    if (s < s1) {
+        WIDE_HALF(0, s, 0)
+        WIDE_HALF(0, s, 1)
+    }
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMAs have written their accumulators
+    // (pinned once more: no copy of an accumulator moves up between the MFMAs, whose latency the compiler does not know)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) asm volatile("" : "+a"(acc[j][t]));
+#undef WIDE_HALF
+#undef WIDE_MFMA
+#undef WIDE_SCALE
+#undef WIDE_LUT
+#undef WIDE_READ_B
+#undef WIDE_STORE_X
+#undef WIDE_LOAD_X
+#undef WIDE_LOAD_W
+#undef WIDE_SCALES
+#undef WIDE_LOAD_S
+}
+
+// Position in the k-steps of the shared tiles laid end to end: tile (counted from `whole`) and step.  A step of a large
+// tile weighs kCostLarge, one of a small tile kCostSmall (half the MFMAs, the same decode).
+// Bytes between the partial-sum slots: a tile's 256 KB and 4352 more.
+constexpr size_t kWideSlot = (size_t)kWideRows * kWideTokens * 4 + 4352;
+constexpr int kCostLarge = 5, kCostSmall = 3;
+struct WidePos {
+    int tile, step;
+};
+__device__ __forceinline__ bool before(const WidePos &a, const WidePos &b) { return a.tile < b.tile || (a.tile == b.tile && a.step < b.step); }
+__device__ __forceinline__ WidePos wide_share_begin(const WideArgs &a, int share)
+{
+    const unsigned large = (unsigned)(a.large - a.whole), span = (unsigned)a.steps_total;
+    const unsigned w_large = large * span * kCostLarge;
+    const unsigned total = w_large + (unsigned)a.small * span * kCostSmall;
+    unsigned p = (unsigned)((unsigned long long)total * (unsigned)share / (unsigned)a.n_shares);
+    if (p < w_large) {
+        p /= kCostLarge;
+        return WidePos{(int)(p / span), (int)(p % span)};
+    }
+    p = (p - w_large) / kCostSmall;
+    return WidePos{(int)(large + p / span), (int)(p % span)};
+}
+
+template <bool KTAIL, bool BLK>
+__global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(const WideArgs a)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    unsigned char *lut = smem;  // byte-pair table at LDS address 0
+    unsigned char *xs = smem + kLutBytes;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i16 = lane & 15, g = lane >> 4;
+
+    // decode table (as in the streaming kernels)
     {
         const int code_bits = (int)(uint32_t)__builtin_bit_cast(uint16_t, (f16)a.code[lane & 15]);
 #pragma unroll 4
-        for (int p = tid; p < kWideLutBytes / 16; p += kWideThreads) {
-            const int e = p >> 3;
+        for (int p = tid; p < kLutBytes / 16; p += kWideThreads) {
+            const int e = p >> 4;
             const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute((e >> 4) << 2, code_bits);
             const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute((e & 15) << 2, code_bits);
             const uint32_t v = hi | (lo << 16);
@@ -151,352 +309,246 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(const TiledA
         }
     }
 
-    // accumulators of the wave's 128 x 128.  32 x 32 tiles (tm, tn): float 4*q + v of lane l is weight row
-    // 32 tm + 8 q + 4 (l / 32) + v, token 32 tn + l % 32.  16 x 16 tiles: element v of lane l is weight row
-    // 16 tm + 4 (l / 16) + v, token 16 tn + l % 16.
-    wide_f32x16 acc[M32 ? 4 : 1][M32 ? 4 : 1];
-    f32x4 acc16[M32 ? 1 : 8][M32 ? 1 : 8];
-    if constexpr (M32) {
-#pragma unroll
-        for (int tm = 0; tm < 4; ++tm)
-#pragma unroll
-            for (int tn = 0; tn < 4; ++tn)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) acc[tm][tn][e] = 0.f;
-    } else {
-#pragma unroll
-        for (int tm = 0; tm < 8; ++tm)
-#pragma unroll
-            for (int tn = 0; tn < 8; ++tn) acc16[tm][tn] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    // Workgroups are dealt to the 8 XCDs in turn (workgroup L sits on XCD L % 8): an XCD takes consecutive tiles - the
+    // token tiles of a few row tiles, which share the weights through its L2 - or consecutive shares.
+    const int grid = (int)gridDim.x, xcd = (int)blockIdx.x & 7;
+    const int place = xcd * (grid >> 3) + min(xcd, grid & 7) + ((int)blockIdx.x >> 3);
 
-    // fragment addresses: row i32 of 32 x 32 tile t, slot (2 quarter + h32) ^ (row & 7)
-    const unsigned char *a_frag = a_tile + (wm_i * 128 + i32) * 128;
-    const unsigned char *x_frag = x_tile + (wn_i * 128 + i32) * 128;
-    const int swz = (h32 ^ (i32 & 7)) << 4;  // slot << 4 = (32 * quarter) ^ swz
-
-    // fragments of a quarter: [0..3] weight tiles, [4..7] token tiles
-    f16x8 fr[2][8];
-#define TUNA_WIDE_READ1(f, kq, buf, t)                                                           \
-    {                                                                                          \
-        const int o_ = ((32 * (kq)) ^ swz) + (buf) * BUF + ((t) & 3) * (32 * 128);             \
-        fr[f][t] = *reinterpret_cast<const f16x8 *>(((t) < 4 ? a_frag : x_frag) + o_);        \
+    int tile = place, s0 = 0, s1 = a.steps_total;  // the segment at hand
+    WidePos at{0, 0}, end{0, 0};
+    bool shared = a.whole <= place;
+    if (a.n_shares) end = wide_share_begin(a, place + 1);
+    if (shared) {
+        if (!a.n_shares) return;
+        at = wide_share_begin(a, place);
     }
-#define TUNA_WIDE_MFMA1(f, i)                                                                    \
-    acc[(i) >> 2][(i) & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[f][(i) >> 2], fr[f][4 + ((i) & 3)], acc[(i) >> 2][(i) & 3], 0, 0, 0);
-    // 16 x 16 tiles: a k-step is two halves of 32 k, a half two phases of 32 MFMAs (weight tiles 0..3, then 4..7,
-    // against all eight token tiles, token tile by token tile): two sets of four weight fragments, and ONE set of
-    // eight token fragments - in the second phase of a half a token fragment is replaced by the next half's right
-    // behind its last MFMA, 29 MFMAs before its first use
-    const unsigned char *a_frag16 = a_tile + (wm_i * 128 + i16) * 128;
-    const unsigned char *x_frag16 = x_tile + (wn_i * 128 + i16) * 128;
-    const int swz16 = (g ^ (i16 & 7)) << 4;  // slot << 4 = (64 * half) ^ swz16
-    f16x8 fa[2][4], fb[8];
-#define TUNA_WIDE_READ_A(ab, h, buf, t)                                                          \
-    fa[ab][(t) & 3] = *reinterpret_cast<const f16x8 *>(a_frag16 + ((64 * (h)) ^ swz16) + (buf) * BUF + (t) * (16 * 128));
-#define TUNA_WIDE_READ_B(h, buf, t)                                                              \
-    fb[t] = *reinterpret_cast<const f16x8 *>(x_frag16 + ((64 * (h)) ^ swz16) + (buf) * BUF + (t) * (16 * 128));
-    // (written out with the accumulator pinned to the AGPR half of the register file: left to itself the
-    // register allocator spreads 64 four-register accumulators over both halves and then spills in the loop;
-    // accumulators are next touched 63 MFMAs later, and the epilogue waits out the last ones before it reads them)
-#define TUNA_WIDE_MFMA16(ab, tm, tn)                                                             \
-    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc16[tm][tn]) : "v"(fa[ab][(tm) & 3]), "v"(fb[tn]));
-
-    // table reads of the four byte pairs of packed dword j of register set `set` ...
-    uint32_t lt[16];  // a ring of four dwords: dword j in entries 4 (j % 4) ..
-#define TUNA_WIDE_LUT(set, j)                                                                    \
-    {                                                                                          \
-        const uint32_t d_ = wq[set][(j) >> 2][(j) & 3];                                        \
-        lt[4 * ((j) & 3) + 0] = *reinterpret_cast<const lds_u32 *>((uintptr_t)(__builtin_amdgcn_perm(d_, lane8, 0x0c0c0400u) >> 1)); \
-        lt[4 * ((j) & 3) + 1] = *reinterpret_cast<const lds_u32 *>((uintptr_t)(__builtin_amdgcn_perm(d_, lane8, 0x0c0c0500u) >> 1)); \
-        lt[4 * ((j) & 3) + 2] = *reinterpret_cast<const lds_u32 *>((uintptr_t)(__builtin_amdgcn_perm(d_, lane8, 0x0c0c0600u) >> 1)); \
-        lt[4 * ((j) & 3) + 3] = *reinterpret_cast<const lds_u32 *>((uintptr_t)(__builtin_amdgcn_perm(d_, lane8, 0x0c0c0700u) >> 1)); \
-    }
-    // ... their scaling (bit-identical to kernel.cu:2178-2192) and the store of the dword's eight weights into
-    // row a_mbl * 8 + j of weight tile `buf` ...
-#define TUNA_WIDE_DECODE(j, buf)                                                                 \
-    {                                                                                          \
-        const f16x2 h0_ = __builtin_bit_cast(f16x2, lt[4 * ((j) & 3) + 0]) * sc16[j];                \
-        const f16x2 h1_ = __builtin_bit_cast(f16x2, lt[4 * ((j) & 3) + 1]) * sc16[j];                \
-        const f16x2 h2_ = __builtin_bit_cast(f16x2, lt[4 * ((j) & 3) + 2]) * sc16[j];                \
-        const f16x2 h3_ = __builtin_bit_cast(f16x2, lt[4 * ((j) & 3) + 3]) * sc16[j];                \
-        const f16x8 w_ = {h0_[0], h0_[1], h1_[0], h1_[1], h2_[0], h2_[1], h3_[0], h3_[1]};     \
-        *reinterpret_cast<f16x8 *>(a_dst + (buf) * BUF + (j) * 128 + ((a_kb ^ (j)) << 4)) = w_; \
-    }
-    // ... and activation piece i into activation tile `buf`.
-#define TUNA_WIDE_XSTAGE(set, i, buf, s)                                                         \
-    {                                                                                          \
-        u32x4 v_ = xr[set][i];                                                                 \
-        if constexpr (KTAIL) {                                                                 \
-            if ((s) * 64 >= x_k_left) v_ = u32x4{0u, 0u, 0u, 0u};                              \
-        }                                                                                      \
-        *reinterpret_cast<u32x4 *>(x_dst + (buf) * BUF + (i) * 4096) = v_;                     \
-    }
-    // Iteration `it` (k-step `step`) of a tile: its tiles are complete in buffer it & 1, the fragments of its
-    // first quarter in fr[0], the table reads of dwords 0..3 of step + 1 in lt.  Side work between the MFMAs:
-    //   quarter 0: fragments of quarter 1; weights 0..3 of step + 1 scaled and stored into the other buffer, each
-    //              followed by the table reads of dword 4..7 into the freed ring entry; refill of that register set
-    //   quarter 1: fragments of quarter 2; weights 4..7; activations 0..1
-    //   quarter 2: fragments of quarter 3; activations 2..7 and the refill of their register set; barrier
-    //   quarter 3: fragments of quarter 0 of step + 1; table reads of dwords 0..3 of step + 2
-#define TUNA_WIDE_ITER(it, step)                                                                 \
-    {                                                                                          \
-        const int cur_ = (it) & 1, nxt_ = cur_ ^ 1, xset_ = ((it) + 1) % XSETS;                \
-        const int set1_ = ((it) + 1) % NSETS, set2_ = ((it) + 2) % NSETS;                      \
-        _Pragma("unroll") for (int i = 0; i < 16; ++i)                                         \
-        {                                                                                      \
-            TUNA_WIDE_MFMA1(0, i)                                                              \
-            if (i < 8) TUNA_WIDE_READ1(1, 1, cur_, i)                                          \
-            if (i >= 8 && (i & 1) == 0) TUNA_WIDE_DECODE((i - 8) >> 1, nxt_)                   \
-            if (i >= 8 && (i & 1) == 1) TUNA_WIDE_LUT(set1_, 4 + ((i - 9) >> 1))               \
-            if (i == 15) TUNA_WIDE_LOAD(set1_, min((step) + 1 + NSETS, s_last))                \
-            __builtin_amdgcn_sched_barrier(0);                                                 \
-        }                                                                                      \
-        _Pragma("unroll") for (int i = 0; i < 16; ++i)                                         \
-        {                                                                                      \
-            TUNA_WIDE_MFMA1(1, i)                                                              \
-            if (i < 8) TUNA_WIDE_READ1(0, 2, cur_, i)                                          \
-            if (i >= 8 && (i & 1) == 0) TUNA_WIDE_DECODE(4 + ((i - 8) >> 1), nxt_)             \
-            if (i == 13 || i == 15) TUNA_WIDE_XSTAGE(xset_, (i - 13) >> 1, nxt_, (step) + 1)   \
-            __builtin_amdgcn_sched_barrier(0);                                                 \
-        }                                                                                      \
-        _Pragma("unroll") for (int i = 0; i < 16; ++i)                                         \
-        {                                                                                      \
-            TUNA_WIDE_MFMA1(0, i)                                                              \
-            if (i < 8) TUNA_WIDE_READ1(1, 3, cur_, i)                                          \
-            if (i >= 8 && i < 14) TUNA_WIDE_XSTAGE(xset_, 2 + (i - 8), nxt_, (step) + 1)       \
-            if (i == 14) TUNA_WIDE_LOAD_X(xset_, min((step) + 1 + XSETS, s_last))              \
-            __builtin_amdgcn_sched_barrier(0);                                                 \
-        }                                                                                      \
-        __syncthreads(); /* the staged tiles are complete; this step's tiles are free once quarter 3 is read */ \
-        _Pragma("unroll") for (int i = 0; i < 16; ++i)                                         \
-        {                                                                                      \
-            TUNA_WIDE_MFMA1(1, i)                                                              \
-            if (i < 8) TUNA_WIDE_READ1(0, 0, nxt_, i)                                          \
-            if (i >= 8 && (i & 1) == 0) TUNA_WIDE_LUT(set2_, (i - 8) >> 1)                     \
-            __builtin_amdgcn_sched_barrier(0);                                                 \
-        }                                                                                      \
-    }
-
-    // The same iteration with 16 x 16 tiles: four phases of 32 MFMAs.  Side work:
-    //   phase 0 (half 0, weight tiles 0..3): weight fragments 4..7 of half 0; weights 0..3 of step + 1 and the
-    //            table reads of dwords 4..7; refill
-    //   phase 1 (half 0, tiles 4..7): weight fragments 0..3 of half 1, token fragments of half 1 as they come
-    //            free; weights 4..7; activations 0..1
-    //   phase 2 (half 1, tiles 0..3): weight fragments 4..7 of half 1; activations 2..7 and their refill; barrier
-    //   phase 3 (half 1, tiles 4..7): weight fragments 0..3 and token fragments of half 0 of step + 1; table reads
-    //            of dwords 0..3 of step + 2
-#define TUNA_WIDE_ITER16(it, step)                                                               \
-    {                                                                                          \
-        const int cur_ = (it) & 1, nxt_ = cur_ ^ 1, xset_ = ((it) + 1) % XSETS;                \
-        const int set1_ = ((it) + 1) % NSETS, set2_ = ((it) + 2) % NSETS;                      \
-        _Pragma("unroll") for (int i = 0; i < 32; ++i)                                         \
-        {                                                                                      \
-            TUNA_WIDE_MFMA16(0, i & 3, i >> 2)                                                 \
-            if (i < 4) TUNA_WIDE_READ_A(1, 0, cur_, 4 + i)                                     \
-            if (i >= 8 && (i - 8) % 6 == 0) TUNA_WIDE_DECODE((i - 8) / 6, nxt_)                \
-            if (i >= 11 && (i - 11) % 6 == 0) TUNA_WIDE_LUT(set1_, 4 + (i - 11) / 6)           \
-            if (i == 31) TUNA_WIDE_LOAD(set1_, min((step) + 1 + NSETS, s_last))                \
-            __builtin_amdgcn_sched_barrier(0);                                                 \
-        }                                                                                      \
-        _Pragma("unroll") for (int i = 0; i < 32; ++i)                                         \
-        {                                                                                      \
-            TUNA_WIDE_MFMA16(1, 4 + (i & 3), i >> 2)                                           \
-            if (i < 4) TUNA_WIDE_READ_A(0, 1, cur_, i)                                         \
-            if ((i & 3) == 3) TUNA_WIDE_READ_B(1, cur_, i >> 2)                                \
-            if (i >= 13 && i < 29 && (i - 13) % 4 == 0) TUNA_WIDE_DECODE(4 + (i - 13) / 4, nxt_) \
-            if (i == 29 || i == 30) TUNA_WIDE_XSTAGE(xset_, i - 29, nxt_, (step) + 1)          \
-            __builtin_amdgcn_sched_barrier(0);                                                 \
-        }                                                                                      \
-        _Pragma("unroll") for (int i = 0; i < 32; ++i)                                         \
-        {                                                                                      \
-            TUNA_WIDE_MFMA16(0, i & 3, i >> 2)                                                 \
-            if (i < 4) TUNA_WIDE_READ_A(1, 1, cur_, 4 + i)                                     \
-            if (i >= 8 && i < 32 && (i - 8) % 4 == 0) TUNA_WIDE_XSTAGE(xset_, 2 + (i - 8) / 4, nxt_, (step) + 1) \
-            if (i == 30) TUNA_WIDE_LOAD_X(xset_, min((step) + 1 + XSETS, s_last))              \
-            __builtin_amdgcn_sched_barrier(0);                                                 \
-        }                                                                                      \
-        __syncthreads(); /* the staged tiles are complete; this step's tiles are free once the last fragments are read */ \
-        _Pragma("unroll") for (int i = 0; i < 32; ++i)                                         \
-        {                                                                                      \
-            TUNA_WIDE_MFMA16(1, 4 + (i & 3), i >> 2)                                           \
-            if (i < 4) TUNA_WIDE_READ_A(0, 0, nxt_, i)                                         \
-            if ((i & 3) == 3) TUNA_WIDE_READ_B(0, nxt_, i >> 2)                                \
-            if (i >= 13 && i < 29 && (i - 13) % 4 == 0) TUNA_WIDE_LUT(set2_, (i - 13) / 4)     \
-            __builtin_amdgcn_sched_barrier(0);                                                 \
-        }                                                                                      \
-    }
-
-    __syncthreads();  // decode table complete
-    // the first step staged with nothing to hide behind, and the table reads of the second step's dwords 0..3
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) TUNA_WIDE_LUT(0, 4 * h + j)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) TUNA_WIDE_DECODE(4 * h + j, 0)
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) TUNA_WIDE_XSTAGE(0, i, 0, s0)
-    TUNA_WIDE_LOAD(0, min(s0 + NSETS, s_last))
-    TUNA_WIDE_LOAD_X(0, min(s0 + XSETS, s_last))
-    __syncthreads();
-    // (fragments first, table reads behind them: the order in which the loop leaves them)
-    if constexpr (M32) {
-#pragma unroll
-        for (int t = 0; t < 8; ++t) TUNA_WIDE_READ1(0, 0, 0, t)
-    } else {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) TUNA_WIDE_READ_A(0, 0, 0, t)
-#pragma unroll
-        for (int t = 0; t < 8; ++t) TUNA_WIDE_READ_B(0, 0, t)
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) TUNA_WIDE_LUT(1 % NSETS, j)
-
-    int s = s0;
-    for (; s + NSETS - 1 < s1; s += NSETS) {
-#pragma unroll
-        for (int it = 0; it < NSETS; ++it) {
-            if constexpr (M32) TUNA_WIDE_ITER(it, s + it)
-            else TUNA_WIDE_ITER16(it, s + it)
+    const WidePos begin = a.n_shares ? wide_share_begin(a, place) : at;
+    for (;;) {
+        if (shared) {
+            if (!before(at, end)) return;
+            tile = a.whole + at.tile;
+            s0 = at.step;
+            s1 = end.tile == at.tile ? end.step : a.steps_total;
         }
-    }
-    // tail: up to NSETS - 1 more steps (the staging of a step past the end is harmless: its loads are clamped
-    // and nothing uses the tiles)
-#pragma unroll
-    for (int it = 0; it < NSETS - 1; ++it)
-        if (s + it < s1) {
-            if constexpr (M32) TUNA_WIDE_ITER(it, s + it)
-            else TUNA_WIDE_ITER16(it, s + it)
-        }
-#undef TUNA_WIDE_ITER16
-#undef TUNA_WIDE_ITER
-#undef TUNA_WIDE_MFMA16
-#undef TUNA_WIDE_READ_B
-#undef TUNA_WIDE_READ_A
-#undef TUNA_WIDE_XSTAGE
-#undef TUNA_WIDE_DECODE
-#undef TUNA_WIDE_LUT
-#undef TUNA_WIDE_MFMA1
-#undef TUNA_WIDE_READ1
-#undef TUNA_WIDE_LOAD_X
-#undef TUNA_WIDE_LOAD
-
-    if constexpr (!M32) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMAs have written their accumulators
-    // ---- epilogue: slot sl (32 x 32 tiles: 4 * tile + q; 16 x 16 tiles: 8 tm + tn) is a float4 of this lane:
-    // 4 consecutive weight rows of one token ------
-    auto slot_value = [&](int sl) {
-        if constexpr (M32) {
-            const wide_f32x16 &t = acc[(sl >> 2) >> 2][(sl >> 2) & 3];
-            const int q = sl & 3;
-            return f32x4{t[4 * q], t[4 * q + 1], t[4 * q + 2], t[4 * q + 3]};
+        // the tile's group, rows and tokens
+        int group = 0, row_tile, tok_tile, index = tile;
+        if (tile < a.large) {
+            for (;; ++group) {
+                const int n = a.tok_off[group + 1] - a.tok_off[group];
+                const int per_row = (n + 127) >> 8, here = per_row * a.row_tiles;
+                if (index < here) {
+                    row_tile = index / per_row, tok_tile = index % per_row;
+                    break;
+                }
+                index -= here;
+            }
         } else {
-            return acc16[sl >> 3][sl & 7];
-        }
-    };
-    auto slot_row = [&](int sl) {
-        if constexpr (M32) return row_base + wm_i * 128 + ((sl >> 2) >> 2) * 32 + (sl & 3) * 8 + h32 * 4;
-        else return row_base + wm_i * 128 + (sl >> 3) * 16 + g * 4;
-    };
-    auto slot_tok = [&](int sl) {
-        if constexpr (M32) return tok_base + wn_i * 128 + ((sl >> 2) & 3) * 32 + i32;
-        else return tok_base + wn_i * 128 + (sl & 7) * 16 + i16;
-    };
-    f16 *outp = reinterpret_cast<f16 *>(a.out);
-    const f16 *resp = reinterpret_cast<const f16 *>(a.residual);
-    if (a.split_k == 1) {
-#pragma unroll
-        for (int sl = 0; sl < 64; ++sl) {
-            const int row = slot_row(sl), tok = slot_tok(sl);
-            if (tok < a.n && row + 4 <= a.m) {
-                const f32x4 v = slot_value(sl);
-                store_features4(outp, resp, a.epilogue, (size_t)tok, a.m, row, v[0], v[1], v[2], v[3]);
+            index -= a.large;
+            for (;; ++group) {
+                const int n = a.tok_off[group + 1] - a.tok_off[group];
+                const int here = (n & 255) >= 1 && (n & 255) <= 128 ? a.row_tiles : 0;
+                if (index < here) {
+                    row_tile = index, tok_tile = n >> 8;
+                    break;
+                }
+                index -= here;
             }
         }
-        return;
-    }
-    // split-K: fp32 partial tiles [split][tile][wave][slot][lane] as float4, the last workgroup of a tile to
-    // arrive adds them in split order (deterministic, no atomics on out)
-    const size_t tile_id = (size_t)tok_tile * a.row_tiles + row_tile;
-    constexpr size_t kTileF4 = (size_t)4 * 64 * 64;  // float4s per partial tile
-    f32x4 *ws4 = reinterpret_cast<f32x4 *>(a.ws);
-    f32x4 *mine = ws4 + (tile_id * a.split_k + blockIdx.z) * kTileF4 + (size_t)wave * (64 * 64) + lane;
+        const int tok0 = a.tok_off[group] + tok_tile * kWideTokens;
+        WideTile w;
+        w.q = a.q + (size_t)group * (size_t)(a.m >> 3) * (size_t)(a.k >> 3) * 32;
+        w.x = reinterpret_cast<const unsigned char *>(a.x) + (size_t)tok0 * (size_t)a.k * 2;
+        w.absmax = a.absmax + (size_t)group * (size_t)a.m * (size_t)(BLK ? a.k >> (6 + a.blk_shift) : 1);
+        w.m = a.m, w.k = a.k, w.row_base = row_tile * kWideRows;
+        w.tokens = min(a.tok_off[group + 1] - tok0, kWideTokens);
+        w.steps_total = a.steps_total, w.blk_shift = a.blk_shift;
+        const bool large = w.tokens > 128;
+
+        // accumulators: [j][t] element v of lane (i16, g) is weight row 16 g + 4 v + j of the wave's 64, token 16 t + i16
+        f32x4 acc[4][16];
 #pragma unroll
-    for (int sl = 0; sl < 64; ++sl) {
-        const f32x4 v = slot_value(sl);
-        asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" : : "v"(mine + sl * 64), "v"(v) : "memory");
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the partial sums have left this CU
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __syncthreads();
-    volatile unsigned *ticket = reinterpret_cast<volatile unsigned *>(a_tile);
-    if (tid == 0) *ticket = __hip_atomic_fetch_add(a.counters + tile_id, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (*ticket != (unsigned)(a.split_k - 1)) return;
-    if (tid == 0) __hip_atomic_store(a.counters + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // (16-byte loads past this CU's and this XCD's caches - the writers sit on any XCD - two slots x two splits
-    // requested before the first is awaited, as in gemm_tiled.hip; a slot's sum adds its splits in ascending order)
-    const f32x4 *src = ws4 + tile_id * a.split_k * kTileF4 + (size_t)wave * (64 * 64) + lane;
-    for (int sl = 0; sl < 64; sl += 2) {
-        f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-        int sp = 0;
-        for (; sp + 1 < a.split_k; sp += 2) {
-            const f32x4 *p = src + (size_t)sp * kTileF4 + sl * 64;
-            f32x4 a0, a1, b0, b1;
-            asm volatile("global_load_dwordx4 %0, %4, off sc1\n\t"
-                         "global_load_dwordx4 %1, %5, off sc1\n\t"
-                         "global_load_dwordx4 %2, %6, off sc1\n\t"
-                         "global_load_dwordx4 %3, %7, off sc1\n\t"
-                         "s_waitcnt vmcnt(0)"
-                         : "=&v"(a0), "=&v"(a1), "=&v"(b0), "=&v"(b1)
-                         : "v"(p), "v"(p + 64), "v"(p + kTileF4), "v"(p + kTileF4 + 64)
-                         : "memory");
-            s0 += a0, s1 += a1;
-            s0 += b0, s1 += b1;
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int t = 0; t < 16; ++t) acc[j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (large) wide_steps<16, KTAIL, BLK>(acc, w, xs, s0, s1);
+        else wide_steps<8, KTAIL, BLK>(acc, w, xs, s0, s1);
+
+        // ---- sums to outputs ----------------------------------------------------------------------------------
+        // Straight-line code for 64 accumulators and every way a tile can end is 60 KB that each workgroup fetches once,
+        // at 30 us a pass.  So the accumulators of four token tiles at a time go through LDS, where a loop can index
+        // them (each lane reads back what it wrote), and one rolled piece of code does the rest.
+        f16 *outp = reinterpret_cast<f16 *>(a.out);
+        const f16 *resp = reinterpret_cast<const f16 *>(a.residual);
+        const int row = w.row_base + wave * 64 + 16 * g;
+        const uint32_t lane_off = (uint32_t)(wave * 64 * 64 + lane) * 16u;  // of the partial sums: [wave][t][j][lane] of 16 bytes
+        int c_lo = 0, c_hi = -1;  // contributors whose partial sums are read
+        bool own = true, store = true;
+        int my_slot = 0, lo = place, lo_slot = 0;
+        // (cache policy 16: sc1, past the XCD's L2 - writer and reader may sit on different XCDs)
+        auto slot = [&](int share) {
+            const int which = share == place ? my_slot : share == lo ? lo_slot : 0;
+            return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char *>(a.ws) + (size_t)(2 * share + which) * kWideSlot, 0,
+                                                     (int)kWideSlot, 0x00020000);
+        };
+        __syncthreads();  // every wave is done with the stages
+        if (s0 != 0 || s1 != a.steps_total) {
+            // A shared tile: its contributors are shares lo .. hi in k order, each with a slot for its partial sums (the
+            // second of a share's two where the share began in an earlier tile).  The last to arrive adds all of them
+            // from memory in that order, so the sums do not depend on who that is.  With two contributors, the usual
+            // number, it adds the other's to its own registers (the same sum), and one that finds the other arrived
+            // does not write its own at all.
+            const WidePos first{at.tile, 0}, past{at.tile + 1, 0};
+            int hi = place;
+            while (before(first, wide_share_begin(a, lo))) --lo;
+            while (before(wide_share_begin(a, hi + 1), past)) ++hi;
+            lo_slot = before(wide_share_begin(a, lo), first) ? 1 : 0;
+            my_slot = before(begin, first) ? 1 : 0;
+            const unsigned others = (unsigned)(hi - lo);
+            unsigned *counter = a.counters + at.tile;
+            volatile unsigned *ticket = reinterpret_cast<volatile unsigned *>(xs);
+            if (tid == 0) *ticket = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            store = others == 1 && *ticket == 1;
+            if (!store) {
+                const auto mine = slot(place);
+#pragma unroll
+                for (int t = 0; t < 16; ++t)
+                    if (t < 8 || large) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[j][t]), mine, (int)lane_off, (4 * t + j) * 1024, 16);
+                    }
+                __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the partial sums have left this CU
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+                __syncthreads();
+                if (tid == 0) *ticket = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __syncthreads();
+                store = *ticket == others;
+            }
+            if (store && tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            own = others == 1;
+            c_lo = lo, c_hi = hi;
+            if (own) c_lo = c_hi = lo == place ? hi : lo;
+            __syncthreads();  // the ticket has been read: its LDS is free
         }
-        if (sp < a.split_k) {
-            const f32x4 *p = src + (size_t)sp * kTileF4 + sl * 64;
-            f32x4 a0, a1;
-            asm volatile("global_load_dwordx4 %0, %2, off sc1\n\t"
-                         "global_load_dwordx4 %1, %3, off sc1\n\t"
-                         "s_waitcnt vmcnt(0)"
-                         : "=&v"(a0), "=&v"(a1)
-                         : "v"(p), "v"(p + 64)
-                         : "memory");
-            s0 += a0, s1 += a1;
+        if (store) {
+            f32x4 *const mine = reinterpret_cast<f32x4 *>(xs) + wave * (16 * 64) + lane;  // [t][j][lane]
+#pragma unroll 1
+            for (int tb = 0; tb < (large ? 16 : 8); tb += 4) {
+                f32x4 sum[4][4];
+                if (own) {
+#pragma unroll
+                    for (int b = 0; b < 16; b += 4)
+                        if (tb == b) {
+#pragma unroll
+                            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) mine[(4 * t + j) * 64] = acc[j][b + t];
+                        }
+                }
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) sum[t][j] = own ? mine[(4 * t + j) * 64] : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+                for (int c = c_lo; c <= c_hi; ++c) {
+                    // (all loads issued before the first is awaited: the pass is a chain of memory round trips)
+                    const auto src = slot(c);
+                    f32x4 v[4][4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            v[t][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(src, (int)lane_off, (4 * (tb + t) + j) * 1024, 16));
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) sum[t][j] += v[t][j];
+                }
+                // a lane's sixteen rows of a token are consecutive: two 16-byte stores
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const int tl = 16 * (tb + t) + i16;
+                    const size_t tok = (size_t)(tok0 + tl);
+                    if (tl < w.tokens && row + 8 <= a.m)
+                        store_features8(outp, resp, a.epilogue, tok, a.m, row, f32x4{sum[t][0][0], sum[t][1][0], sum[t][2][0], sum[t][3][0]},
+                                        f32x4{sum[t][0][1], sum[t][1][1], sum[t][2][1], sum[t][3][1]});
+                    if (tl < w.tokens && row + 16 <= a.m)
+                        store_features8(outp, resp, a.epilogue, tok, a.m, row + 8, f32x4{sum[t][0][2], sum[t][1][2], sum[t][2][2], sum[t][3][2]},
+                                        f32x4{sum[t][0][3], sum[t][1][3], sum[t][2][3], sum[t][3][3]});
+                }
+            }
         }
-        {
-            const int row = slot_row(sl), tok = slot_tok(sl);
-            if (tok < a.n && row + 4 <= a.m) store_features4(outp, resp, a.epilogue, (size_t)tok, a.m, row, s0[0], s0[1], s0[2], s0[3]);
-        }
-        {
-            const int row = slot_row(sl + 1), tok = slot_tok(sl + 1);
-            if (tok < a.n && row + 4 <= a.m) store_features4(outp, resp, a.epilogue, (size_t)tok, a.m, row, s1[0], s1[1], s1[2], s1[3]);
+        if (shared) {
+            at = WidePos{at.tile + 1, 0};
+        } else {
+            tile += grid;
+            if (tile >= a.whole) {
+                if (!a.n_shares) return;
+                shared = true;
+                at = begin;
+            }
         }
     }
 }
 
-size_t wide_lds_bytes() { return (size_t)kWideLutBytes + 2 * (size_t)kWideBuf; }
+size_t wide_lds_bytes() { return (size_t)kLutBytes + 3 * (size_t)kWideStage; }
 
-static OptInFlag g_wide_attr[16][4];
-
-hipError_t launch_gemm_wide(const TiledArgs &args, bool mfma32, hipStream_t stream)
+bool plan_gemm_wide(int m, int k, int n_groups, const int *tok_off, int split, int cus, WidePlan *plan)
 {
-    const bool ktail = args.k % 64 != 0;
-    const auto fn = ktail ? (mfma32 ? gemm_wide_kernel<2, true, true> : gemm_wide_kernel<2, false, true>)
-                          : (mfma32 ? gemm_wide_kernel<2, true, false> : gemm_wide_kernel<2, false, false>);
+    memset(plan, 0, sizeof(*plan));
+    WideArgs &a = plan->args;
+    a.m = m, a.k = k, a.n_groups = n_groups;
+    a.steps_total = ceil_div_i(k, 64);
+    a.row_tiles = ceil_div_i(m, kWideRows);
+    long long large = 0, small = 0;
+    for (int e = 0; e <= n_groups; ++e) a.tok_off[e] = tok_off[e];
+    for (int e = 0; e < n_groups; ++e) {
+        const int n = tok_off[e + 1] - tok_off[e];
+        large += (long long)((n + 127) >> 8) * a.row_tiles;
+        small += (n & 255) >= 1 && (n & 255) <= 128 ? a.row_tiles : 0;
+    }
+    const long long tiles = large + small, weight = (large * kCostLarge + small * kCostSmall) * a.steps_total;
+    if (tiles < 1 || tiles > 0x7fffffff || weight > 0x7fffffff) return false;
+    a.large = (int)large, a.small = (int)small;
+    a.whole = (int)tiles;
+    if (split > 1) {
+        a.whole = 0;
+        a.n_shares = (int)(tiles * split);
+    } else if (split == 0) {
+        // as many rounds of whole large tiles as leave between a quarter and one and a quarter of a tile's work per
+        // compute unit; that is shared
+        const double per_cu = (double)weight / ((double)kCostLarge * a.steps_total * cus);
+        long long rounds = (long long)(per_cu - 0.25);
+        if (rounds > large / cus) rounds = large / cus;
+        a.whole = (int)(rounds * cus);
+        a.n_shares = tiles > a.whole ? cus : 0;
+        // (at most eight shares to a tile, of at least eight steps)
+        const long long rest = weight - (long long)a.whole * kCostLarge * a.steps_total;
+        if (!rounds && a.n_shares > 8 * tiles) a.n_shares = (int)(8 * tiles);
+        if (!rounds && a.n_shares > rest / (8 * kCostLarge)) a.n_shares = (int)(rest / (8 * kCostLarge)) + 1;
+    }
+    // (a share is at least a step of a large tile, so that every share between a tile's first and last has a part of it)
+    if (a.n_shares > weight / kCostLarge) a.n_shares = (int)(weight / kCostLarge) > 0 ? (int)(weight / kCostLarge) : 1;
+    plan->grid = (unsigned)(a.n_shares ? a.n_shares : tiles);
+    plan->ws_bytes = (size_t)a.n_shares * 2 * kWideSlot;
+    plan->n_counters = a.n_shares ? (size_t)(tiles - a.whole) : 0;
+    return true;
+}
+
+hipError_t launch_gemm_wide(const WidePlan &plan, bool scale_blocks, hipStream_t stream)
+{
+    static OptInFlag done[16][3];
+    const bool ktail = plan.args.k % 64 != 0;
+    if (scale_blocks && ktail) return hipErrorInvalidConfiguration;
+    const auto fn = scale_blocks ? gemm_wide_kernel<false, true> : ktail ? gemm_wide_kernel<true, false> : gemm_wide_kernel<false, false>;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev < 0 || dev >= 16) return hipErrorInvalidDevice;
-    if ((e = ensure_lds_opt_in(g_wide_attr[dev][2 * ktail + mfma32], reinterpret_cast<const void *>(fn))) != hipSuccess) return e;
-    TiledArgs a = args;
-    a.row_tiles = ceil_div_i(args.m, kWideRows);
-    a.tok_tiles = ceil_div_i(args.n, kWideTokens);
-    if ((long long)a.row_tiles * a.tok_tiles > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-    const dim3 grid((unsigned)(a.row_tiles * a.tok_tiles), 1, (unsigned)args.split_k);
-    hipLaunchKernelGGL(fn, grid, dim3(kWideThreads), wide_lds_bytes(), stream, a);
+    if ((e = ensure_lds_opt_in(done[dev][scale_blocks ? 2 : ktail], reinterpret_cast<const void *>(fn))) != hipSuccess) return e;
+    hipLaunchKernelGGL(fn, dim3(plan.grid), dim3(kWideThreads), wide_lds_bytes(), stream, plan.args);
     return hipGetLastError();
 }
 

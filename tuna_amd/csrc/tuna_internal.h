@@ -148,6 +148,36 @@ struct TiledArgs {
     int blk_shift;        // scale-block variants: absmax is [m, k / (64 << blk_shift)], one scale per block of a row
 };
 
+// Launch arguments of the 256 x 256 many-token kernel (gemm_wide.hip): n_groups stacked matrices of m rows each, group
+// e multiplying the activation rows tok_off[e] .. tok_off[e + 1] - 1 (a dense GEMM is one group).  A tile is 256 rows x
+// up to 256 tokens of one group; tiles of more than 128 tokens ("large") are numbered first, group by group, row tile by
+// row tile, the token tiles of a row tile next to each other; then the groups' last tiles of 1 .. 128 tokens ("small").
+struct WideArgs {
+    const uint8_t *q;
+    const void *x;
+    const float *code;
+    const float *absmax;
+    void *out;
+    const void *residual;
+    int epilogue;
+    float *ws;           // partial tiles, two slots per share
+    unsigned *counters;  // one arrival counter per shared tile, zero between launches
+    int m, k, n_groups;
+    int steps_total;     // ceil(k / 64)
+    int row_tiles;       // of one group
+    int large, small;    // tiles of either kind
+    int whole;           // tiles 0 .. whole - 1 are computed whole, one workgroup each
+    int n_shares;        // the k-steps of the other tiles, laid end to end, are divided into this many equal shares (0: none)
+    int blk_shift;       // scale-block variants: absmax is [m, k / (64 << blk_shift)]
+    int tok_off[kMaxGroups + 1];
+};
+
+struct WidePlan {
+    WideArgs args;
+    unsigned grid;
+    size_t ws_bytes, n_counters;
+};
+
 inline int ceil_div_i(int a, int b) { return (a + b - 1) / b; }
 
 struct GemmPlan {
@@ -211,9 +241,13 @@ hipError_t device_cus(int *dev, int *cus);
 // gemm_tiled.hip
 hipError_t launch_gemm_tiled(const TiledArgs &args, int tile_rows, int tile_tokens, bool mfma32, hipStream_t stream,
                              bool scale_blocks = false);
-// 256 x 256 tile, one wave per SIMD (gemm_wide.hip): reached through launch_gemm_tiled
+// 256 x 256 tile, one wave per SIMD: gemm_wide.hip, and gemm_wide32.hip with 32 x 32 x 16 MFMAs (reached through
+// launch_gemm_tiled)
 size_t wide_lds_bytes();
-hipError_t launch_gemm_wide(const TiledArgs &args, bool mfma32, hipStream_t stream);
+// split: 0 = balanced over the compute units, 1 = every tile whole, else that many shares per tile.
+bool plan_gemm_wide(int m, int k, int n_groups, const int *tok_off, int split, int cus, WidePlan *plan);
+hipError_t launch_gemm_wide(const WidePlan &plan, bool scale_blocks, hipStream_t stream);
+hipError_t launch_gemm_wide32(const TiledArgs &args, hipStream_t stream);
 bool tiled_variant_exists(int tile_rows, int tile_tokens, bool mfma32);
 size_t tiled_lds_bytes(int tile_rows, int tile_tokens);
 

@@ -274,7 +274,8 @@ def lds_bytes(c: dict) -> int:
 BLOCKWISE_NARROW = ({(16, 4, 2, 1), (16, 8, 4, 1), (16, 16, 2, 1), (32, 8, 2, 1), (32, 8, 4, 1), (32, 16, 2, 1), (64, 4, 4, 1),
                      (64, 8, 2, 1), (64, 8, 4, 1), (64, 16, 2, 1)}
                     | {(16, 4, 2, 2), (16, 8, 4, 2), (32, 8, 2, 2), (32, 8, 4, 2), (64, 8, 2, 2), (64, 8, 4, 2)})
-# many-token tiles with a scale-block variant (16 x 16 x 32 MFMA; not the 256 x 256 tile)
+# many-token tiles with a scale-block variant that entries may name (16 x 16 x 32 MFMA; the 256 x 256 tile's is the
+# derivation's alone)
 BLOCKWISE_TILED = {(64, 128), (64, 256), (128, 64), (128, 128), (128, 256), (256, 64), (256, 128)}
 BLOCKWISE_FAMILIES = ("narrow", "batched", "many-token", "streaming")
 
