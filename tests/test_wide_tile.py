@@ -1,0 +1,138 @@
+"""The 256 x 256 many-token tile (csrc/gemm_wide.hip): tiles whole, split, and shared between workgroups; groups in one
+launch; scale blocks.  Against the oracle on a subset of rows, and deterministic."""
+import numpy as np
+import pytest
+
+from helpers import O, REL_TOL, f16_bits_to_f64, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(m, n, k, seed, block=0):
+    import torch
+
+    from tuna_amd.quantize import nf4_codebook
+    from tuna_amd.synth import make_weights_torch, make_x_torch
+
+    dev = torch.device("cuda")
+    q, s = make_weights_torch(m, k, seed=seed, device=dev)
+    if block:
+        g = torch.Generator(device=dev)
+        g.manual_seed(seed)
+        s = torch.empty((m, k // block), device=dev).uniform_(0.005, 0.02, generator=g)
+    return q, s, make_x_torch(n, k, seed=seed + 1, device=dev), nf4_codebook(dev)
+
+
+def _out(n, m):
+    import torch
+
+    return torch.full((n, m), float("nan"), dtype=torch.float16, device="cuda")
+
+
+def _check(out, q, s, x, code, k, blocks=6, block=0, first_row=0, rows=None):
+    """Rows of `blocks` random block rows (and the last one) of out against the oracle's float64 sums."""
+    import torch
+
+    m = rows or out.shape[1]
+    assert not torch.isnan(out).any()
+    rng = np.random.default_rng(m + out.shape[0])
+    mbs = np.unique(np.append(rng.choice(m // 8, size=min(blocks, m // 8), replace=False), m // 8 - 1))
+    rs = (mbs[:, None] * 8 + np.arange(8)[None, :]).ravel()
+    q_sub = q[torch.from_numpy(mbs + first_row // 8).cuda()].cpu().numpy()
+    s_sub = s[torch.from_numpy(rs + first_row).cuda()].cpu().numpy()
+    xb, cb = x.cpu().numpy().view(np.uint16), code.cpu().numpy()
+    ref = O.gemm_f64(q_sub, xb, cb, s_sub, len(rs), x.shape[0], k, mode=O.D1, block_size=block or None)
+    got = out.cpu().numpy().view(np.uint16)[:, rs]
+    assert rel_err(f16_bits_to_f64(got), ref) <= REL_TOL
+
+
+def _cfg(split):
+    from tuna_amd.ops import GemmConfig
+
+    return GemmConfig.from_dict(dict(rows_per_wave=64, waves_m=1, waves_k=1, split_k=split, prefetch=2, x_chunk=64, token_tiles=16,
+                                     xcd_swizzle=0, lds_tile_rows=256))
+
+
+# whole tiles: 1 .. 128 tokens in the last tile, 129 .. 256, ragged rows; splits with two and more contributors, parts of
+# one step, an odd number of steps; k tails
+@pytest.mark.parametrize("m,n,k,split", [(256, 128, 128, 1), (264, 129, 64, 1), (520, 384, 192, 1), (1024, 257, 320, 2),
+                                         (512, 385, 704, 3), (264, 640, 1088, 5), (256, 100, 512, 8), (512, 129, 1000, 2),
+                                         (768, 300, 4104, 7)])
+@pytest.mark.parametrize("epilogue", [0, 1, 2])
+def test_whole_and_split_tiles(m, n, k, split, epilogue):
+    import torch
+
+    from tuna_amd import _lib, ops
+
+    q, s, x, code = _inputs(m, n, k, seed=m + n)
+    plain, again = _out(n, m), _out(n, m)
+    ops.matmul(x, q, s, code, plain, m, n, k, config=_cfg(split))
+    ops.matmul(x, q, s, code, again, m, n, k, config=_cfg(split))
+    torch.cuda.synchronize()
+    assert torch.equal(plain, again)
+    _check(plain, q, s, x, code, k)
+    if epilogue:
+        res = torch.randn(n, m, device="cuda").half()
+        fused = _out(n, m // epilogue)
+        ops.matmul_fused(x, q, s, code, fused, m, n, k, epilogue, res if epilogue == _lib.EPILOGUE_RESIDUAL else None, config=_cfg(split))
+        torch.cuda.synchronize()
+        p = plain.float()
+        want = p + res.float() if epilogue == _lib.EPILOGUE_RESIDUAL else torch.nn.functional.silu(p[:, 0::2]) * p[:, 1::2]
+        assert (fused.float() - want).abs().max() <= 4e-3 * want.abs().max()
+
+
+# one round of shares (two and three contributors to a tile), one round of whole tiles and shares, with small last tiles
+@pytest.mark.parametrize("m,n,k", [(9728, 1000, 8256), (8448, 1100, 4096), (10240, 2000, 4096)])
+def test_last_tiles_shared_between_the_compute_units(m, n, k):
+    import torch
+
+    from tuna_amd import ops
+
+    assert "last tiles shared" in ops.describe_launch(m, n, k, _cfg(1))
+    q, s, x, code = _inputs(m, n, k, seed=n)
+    outs = [_out(n, m) for _ in range(3)]
+    for o in outs:
+        ops.matmul(x, q, s, code, o, m, n, k, config=_cfg(1))
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    _check(outs[0], q, s, x, code, k)
+
+
+def test_a_capturing_stream_without_workspace_takes_whole_tiles():
+    """Sharing needs room for partial sums, which cannot be allocated during a capture: the launch then runs whole tiles."""
+    import torch
+
+    from tuna_amd import ops
+
+    m, n, k = 9728, 1000, 8256
+    q, s, x, code = _inputs(m, n, k, seed=5)
+    shared, out = _out(n, m), _out(n, m)
+    ops.matmul(x, q, s, code, shared, m, n, k, config=_cfg(1))
+    torch.cuda.synchronize()
+    g, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(g, stream=side):
+        ops.matmul(x, q, s, code, out, m, n, k, config=_cfg(1))
+    for _ in range(3):
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert (out.float() - shared.float()).abs().max() <= 2e-3 * shared.float().abs().max()
+
+
+@pytest.mark.parametrize("m,k,counts", [(512, 512, (200, 65, 0, 128, 129, 256, 257, 70)), (320, 1032, (300, 66, 64, 80, 100, 512)),
+                                        (2048, 1024, (400, 1, 777, 90))])
+def test_groups_of_many_tokens_in_one_launch(m, k, counts):
+    import torch
+
+    from tuna_amd import ops
+
+    offs = np.concatenate([[0], np.cumsum(counts)]).tolist()
+    q, s, x, code = _inputs(m * len(counts), offs[-1], k, seed=k)
+    out, again = _out(offs[-1], m), _out(offs[-1], m)
+    ops.matmul_grouped(x, q, s, code, out, m, len(counts), k, offs)
+    ops.matmul_grouped(x, q, s, code, again, m, len(counts), k, offs)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    for e, (lo, hi) in enumerate(zip(offs, offs[1:])):
+        if hi > lo:
+            _check(out[lo:hi], q, s, x[lo:hi], code, k, first_row=e * m, rows=m)

@@ -224,11 +224,15 @@ static int planned_cus()
     return kMaxCus;
 }
 
-static double wide_time(int m, int n, int k, int split);
 static bool wide_balance_pays(int m, int n, int k);
+static bool plan_wide_dense(int m, int n, int k, int split, WidePlan *plan)
+{
+    memset(plan, 0, sizeof(*plan));
+    plan->args.m = m, plan->args.k = k, plan->args.n_groups = 1, plan->args.tok_count[0] = n;
+    return plan_gemm_wide(split, planned_cus(), plan);
+}
 
-// balance: the last rounds of an unsplit launch of 256 x 256 tiles may be shared evenly between the compute units.
-static int plan_tiled(int m, int n, int k, const tuna_gemm_config &c, int decode, TiledPlan *plan, bool balance = true)
+static int plan_tiled(int m, int n, int k, const tuna_gemm_config &c, int decode, TiledPlan *plan)
 {
     int rc = check_shape(m, n, k);
     if (rc) return rc;
@@ -261,8 +265,7 @@ static int plan_tiled(int m, int n, int k, const tuna_gemm_config &c, int decode
     a.steps_per_split = ceil_div(steps, c.split_k);
     if (wide) {
         plan->wide = true;
-        const int tok_off[2] = {0, n};
-        if (!plan_gemm_wide(m, k, 1, tok_off, balance && c.split_k == 1 && wide_balance_pays(m, n, k) ? 0 : c.split_k, planned_cus(), &plan->wide_plan))
+        if (!plan_wide_dense(m, n, k, c.split_k == 1 && wide_balance_pays(m, n, k) ? 0 : c.split_k, &plan->wide_plan))
             return fail(TUNA_ERR_UNSUPPORTED, "m=%d n=%d k=%d has too many 256 x 256 tiles for one launch", m, n, k);
         plan->ws_bytes = plan->wide_plan.ws_bytes;
         plan->n_counters = plan->wide_plan.n_counters;
@@ -292,8 +295,7 @@ static int launch_tiled(TiledPlan &tp, const void *q, const void *x, const void 
         rc = fill(tp.wide_plan.args);
         if (rc && tp.args.split_k == 1) {
             // (no room for the shares' partial sums - the static scratch, a stream that is capturing: whole tiles)
-            const int tok_off[2] = {0, tp.args.n};
-            if (!plan_gemm_wide(tp.args.m, tp.args.k, 1, tok_off, 1, planned_cus(), &tp.wide_plan)) return rc;
+            if (!plan_wide_dense(tp.args.m, tp.args.n, tp.args.k, 1, &tp.wide_plan)) return rc;
             tp.ws_bytes = tp.n_counters = 0;
             rc = fill(tp.wide_plan.args);
         }
@@ -536,10 +538,8 @@ static bool narrow_round(int m, int n, int k, tuna_gemm_config *out)
 // a tile takes longer the more workgroups share the chip's power, a whole tile ends with 12 us of stores, a shared one
 // with as long for the partial sums and more for every further share of it.  split: 1 whole tiles, 2 ... that many equal shares of
 // every tile, 0 the last rounds of tiles shared evenly between the compute units.
-static double wide_time(int m, int n, int k, int split)
+static double wide_time(double large, double small, double steps, int split)
 {
-    const double row_tiles = ceil_div(m, 256), steps = ceil_div(k, 64);
-    const double large = row_tiles * ((n + 127) >> 8), small = (n & 255) >= 1 && (n & 255) <= 128 ? row_tiles : 0.0;
     const double tiles = large + small, cus = kMaxCus, small_cost = 0.505;
     auto step_us = [&](double workgroups) { return 0.907 + 0.604 * (workgroups < cus ? workgroups : cus) / cus; };
     const double kind = large > 0 ? 1.0 : small_cost;  // of the longest tile
@@ -562,9 +562,37 @@ static double wide_time(int m, int n, int k, int split)
 
 // Whether an unsplit launch shares its last tiles between the compute units: from half a round of tiles on, where the
 // model says so.
+static bool wide_balance_pays(double large, double small, double steps)
+{
+    return large + small > kMaxCus / 2 && wide_time(large, small, steps, 0) < wide_time(large, small, steps, 1);
+}
+
+struct WideTiles {
+    double large, small, steps;
+    WideTiles(int m, int n, int k)
+        : large((double)ceil_div(m, 256) * ((n + 127) >> 8)), small((n & 255) >= 1 && (n & 255) <= 128 ? ceil_div(m, 256) : 0.0), steps(ceil_div(k, 64))
+    {
+    }
+};
+
 static bool wide_balance_pays(int m, int n, int k)
 {
-    return (long long)ceil_div(m, 256) * ceil_div(n, 256) > kMaxCus / 2 && wide_time(m, n, k, 0) < wide_time(m, n, k, 1);
+    const WideTiles t(m, n, k);
+    return wide_balance_pays(t.large, t.small, t.steps);
+}
+
+// The split (as above; 1 where the launch then shares its last tiles by itself) that takes these tiles least time, and
+// that time in *us; 0 if there are too few of them.
+static int wide_best_split(double large, double small, double steps, double *us)
+{
+    int best = 0;
+    for (int split : {1, 2, 3, 4, 6, 8}) {
+        const double wgs = (large + small) * split;
+        if (wgs < 16 || (split > 1 && (wgs > 400 || steps / split < 8))) continue;
+        const double t = wide_time(large, small, steps, split == 1 && wide_balance_pays(large, small, steps) ? 0 : split);
+        if (!best || t < *us) best = split, *us = t;
+    }
+    return best;
 }
 
 // The grid cost model of derive_config: candidate tiles with a kernel's factor, and what a launch of `tiles` workgroups
@@ -885,30 +913,21 @@ static bool wide_instead(int m, int n, int k, const tuna_gemm_config &c, tuna_ge
     if (n <= 64 || is_narrow(c)) return false;
     const int tokens = 16 * c.token_tiles, streaming = c.lds_tile_rows <= 0;
     const int rows = streaming ? c.rows_per_wave * c.waves_m : c.lds_tile_rows;
-    double price = 0.0;
-    const bool is_wide = !streaming && rows == 256 && tokens == 256 && c.rows_per_wave != 32;
-    if (is_wide) {
-        price = wide_time(m, n, k, c.split_k == 1 && wide_balance_pays(m, n, k) ? 0 : c.split_k);
+    const WideTiles t(m, n, k);
+    double price = 0.0, us = 0.0;
+    if (!streaming && rows == 256 && tokens == 256 && c.rows_per_wave != 32) {
+        price = wide_time(t.large, t.small, t.steps, c.split_k == 1 && wide_balance_pays(m, n, k) ? 0 : c.split_k);
     } else {
         for (const GridCand &cd : kGridCand)
             if (cd.rows == rows && cd.tokens == tokens && cd.streaming == streaming && (!streaming || c.split_k == 1))
                 price = kGridCostUs * k * grid_cost(cd, c.split_k, (long long)ceil_div(m, rows) * ceil_div(n, tokens) * c.split_k, k);
     }
-    if (price == 0.0) return false;
-    bool found = false;
-    const long long tiles = (long long)ceil_div(m, 256) * ceil_div(n, 256);
-    for (int split : {1, 2, 3, 4, 6, 8}) {
-        if (tiles * split < 16 || (split > 1 && (tiles * split > 400 || ceil_div(k, 64) / split < 8))) continue;
-        const double t = wide_time(m, n, k, split == 1 && wide_balance_pays(m, n, k) ? 0 : split);
-        if (t >= (found ? price : 0.96 * price)) continue;
-        tuna_gemm_config w;
-        memset(&w, 0, sizeof(w));
-        w.rows_per_wave = 64, w.waves_m = 1, w.waves_k = 1, w.prefetch = 2, w.x_chunk = 64, w.token_tiles = 16, w.lds_tile_rows = 256;
-        w.split_k = split;
-        if (!config_runs(m, n, k, w)) continue;
-        *wide = w, price = t, found = true;
-    }
-    return found;
+    const int split = price == 0.0 ? 0 : wide_best_split(t.large, t.small, t.steps, &us);
+    if (!split || us >= 0.96 * price) return false;
+    memset(wide, 0, sizeof(*wide));
+    wide->rows_per_wave = 64, wide->waves_m = 1, wide->waves_k = 1, wide->prefetch = 2, wide->x_chunk = 64, wide->token_tiles = 16;
+    wide->lds_tile_rows = 256, wide->split_k = split;
+    return config_runs(m, n, k, *wide);
 }
 
 // The table's buckets are the reference dispatcher's (kernel.cu:3022-3155) and every entry is tuned at the lower edge
@@ -1439,9 +1458,50 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
     // tokens) run as dense GEMMs of their own, each with the table's config for its token count - from 128 tokens a
     // group that is the many-token kernel at two to three times the rate, and a launch per group is nothing beside
     // hundreds of microseconds of matrix work.  (With an explicit config every group goes through the grouped kernel.)
+    // Several such groups become ONE launch of 256 x 256 tiles (gemm_wide.hip) where that is predicted to be faster than a
+    // launch each, priced at 6 us and the larger of 0.85 PFLOP/s and 3.5 TB/s: eight experts of 14336 x 4096 on 4096
+    // tokens leave the device half empty at the end of each of eight launches (711 us; 616 with 256 x 256 tiles in each).
     constexpr int kGroupedPassTokens = 64;
     const size_t group_q_bytes = (size_t)m_group * (size_t)k / 2;
-    if (!cfg) {
+    bool many_done = false;
+    if (!cfg && decode == TUNA_DECODE_GEMM && max_tok > kGroupedPassTokens) {
+        WidePlan plan;
+        memset(&plan, 0, sizeof(plan));
+        WideArgs &a = plan.args;
+        a.m = m_group, a.k = k;
+        double apart = 0.0, together = 0.0;
+        for (int e = 0; e < n_groups; ++e) {
+            const int cnt = offsets[e + 1] - offsets[e];
+            if (cnt <= kGroupedPassTokens) continue;
+            const double flops = 2.0 * m_group * cnt * k, bytes = (double)group_q_bytes + 2.0 * cnt * ((double)m_group + k);
+            const double t_flops = flops / 0.85e9, t_bytes = bytes / 3.5e6;
+            apart += 6.0 + (t_flops > t_bytes ? t_flops : t_bytes);
+            a.tok_begin[a.n_groups] = offsets[e], a.tok_count[a.n_groups] = cnt, a.id[a.n_groups] = (unsigned char)e;
+            ++a.n_groups;
+        }
+        long long large, small;
+        count_wide_tiles(a, &large, &small);
+        const double steps = ceil_div(k, 64);
+        const int split = a.n_groups > 1 ? wide_best_split((double)large, (double)small, steps, &together) : 0;
+        if (split && together < apart) {
+            a.q = static_cast<const uint8_t *>(q);
+            a.x = x;
+            a.code = static_cast<const float *>(code);
+            a.absmax = static_cast<const float *>(absmax);
+            a.out = out;
+            const bool balance = split == 1 && wide_balance_pays((double)large, (double)small, steps);
+            rc = plan_gemm_wide(balance ? 0 : split, planned_cus(), &plan) ? TUNA_OK : TUNA_ERR_UNSUPPORTED;
+            if (!rc && plan.ws_bytes) rc = provide_workspace(false, stream, plan.ws_bytes, plan.n_counters, &a.ws, &a.counters);
+            if (rc && balance)  // (a stream that is capturing, with too small a workspace: whole tiles)
+                rc = plan_gemm_wide(1, planned_cus(), &plan) ? TUNA_OK : TUNA_ERR_UNSUPPORTED;
+            if (!rc) {
+                const hipError_t e = launch_gemm_wide(plan, false, stream);
+                if (e != hipSuccess) return hip_fail(e, "grouped many-token gemm launch");
+                many_done = true;
+            }
+        }
+    }
+    if (!cfg && !many_done) {
         // (checked before anything is enqueued: a group that cannot run must not leave the others' rows written)
         for (int e = 0; e < n_groups; ++e) {
             const int cnt = offsets[e + 1] - offsets[e];
@@ -2369,8 +2429,9 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
         TiledPlan tp;
         if ((rc = plan_tiled(m, n, k, c, decode_mode, &tp))) return rc;
         const bool wide = tp.tile_rows == 256 && tp.tile_tokens == 256;  // gemm_wide.hip: one wave per SIMD
-        snprintf(buf, len, "%s<%d rows x %d tokens%s> split_k=%d", wide ? "gemm_wide_kernel" : "gemm_tiled_kernel", tp.tile_rows,
-                 tp.tile_tokens, tp.mfma32 ? ",mfma 32x32x16" : "", c.split_k);
+        snprintf(buf, len, "%s<%d rows x %d tokens%s> split_k=%d%s", wide ? "gemm_wide_kernel" : "gemm_tiled_kernel", tp.tile_rows,
+                 tp.tile_tokens, tp.mfma32 ? ",mfma 32x32x16" : "", c.split_k,
+                 tp.wide && c.split_k == 1 && tp.wide_plan.args.n_shares ? ", last tiles shared" : "");
         return TUNA_OK;
     }
     if (is_narrow(c)) {

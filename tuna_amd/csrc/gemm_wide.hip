@@ -20,8 +20,6 @@
 // the last slot inside k (no access leaves a row), and their activations are stored as zeros.  BLK: one scale per block
 // of a row.  Decode and rounding are those of the other kernels (bit-identical to kernel.cu:2178-2192); an unshared
 // tile's sums are the same products in the same order as the 16 x 16 x 32 variants of gemm_tiled.hip.
-#include <cstring>
-
 #include "epilogue.hpp"
 
 namespace tuna {
@@ -334,8 +332,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(const WideAr
         int group = 0, row_tile, tok_tile, index = tile;
         if (tile < a.large) {
             for (;; ++group) {
-                const int n = a.tok_off[group + 1] - a.tok_off[group];
-                const int per_row = (n + 127) >> 8, here = per_row * a.row_tiles;
+                const int per_row = (a.tok_count[group] + 127) >> 8, here = per_row * a.row_tiles;
                 if (index < here) {
                     row_tile = index / per_row, tok_tile = index % per_row;
                     break;
@@ -345,7 +342,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(const WideAr
         } else {
             index -= a.large;
             for (;; ++group) {
-                const int n = a.tok_off[group + 1] - a.tok_off[group];
+                const int n = a.tok_count[group];
                 const int here = (n & 255) >= 1 && (n & 255) <= 128 ? a.row_tiles : 0;
                 if (index < here) {
                     row_tile = index, tok_tile = n >> 8;
@@ -354,13 +351,13 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(const WideAr
                 index -= here;
             }
         }
-        const int tok0 = a.tok_off[group] + tok_tile * kWideTokens;
+        const int tok0 = a.tok_begin[group] + tok_tile * kWideTokens, id = a.id[group];
         WideTile w;
-        w.q = a.q + (size_t)group * (size_t)(a.m >> 3) * (size_t)(a.k >> 3) * 32;
+        w.q = a.q + (size_t)id * (size_t)(a.m >> 3) * (size_t)(a.k >> 3) * 32;
         w.x = reinterpret_cast<const unsigned char *>(a.x) + (size_t)tok0 * (size_t)a.k * 2;
-        w.absmax = a.absmax + (size_t)group * (size_t)a.m * (size_t)(BLK ? a.k >> (6 + a.blk_shift) : 1);
+        w.absmax = a.absmax + (size_t)id * (size_t)a.m * (size_t)(BLK ? a.k >> (6 + a.blk_shift) : 1);
         w.m = a.m, w.k = a.k, w.row_base = row_tile * kWideRows;
-        w.tokens = min(a.tok_off[group + 1] - tok0, kWideTokens);
+        w.tokens = min(a.tok_count[group] - tok_tile * kWideTokens, kWideTokens);
         w.steps_total = a.steps_total, w.blk_shift = a.blk_shift;
         const bool large = w.tokens > 128;
 
@@ -495,20 +492,25 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(const WideAr
 
 size_t wide_lds_bytes() { return (size_t)kLutBytes + 3 * (size_t)kWideStage; }
 
-bool plan_gemm_wide(int m, int k, int n_groups, const int *tok_off, int split, int cus, WidePlan *plan)
+void count_wide_tiles(const WideArgs &a, long long *large, long long *small)
 {
-    memset(plan, 0, sizeof(*plan));
-    WideArgs &a = plan->args;
-    a.m = m, a.k = k, a.n_groups = n_groups;
-    a.steps_total = ceil_div_i(k, 64);
-    a.row_tiles = ceil_div_i(m, kWideRows);
-    long long large = 0, small = 0;
-    for (int e = 0; e <= n_groups; ++e) a.tok_off[e] = tok_off[e];
-    for (int e = 0; e < n_groups; ++e) {
-        const int n = tok_off[e + 1] - tok_off[e];
-        large += (long long)((n + 127) >> 8) * a.row_tiles;
-        small += (n & 255) >= 1 && (n & 255) <= 128 ? a.row_tiles : 0;
+    const long long row_tiles = ceil_div_i(a.m, kWideRows);
+    *large = *small = 0;
+    for (int e = 0; e < a.n_groups; ++e) {
+        const int n = a.tok_count[e];
+        *large += ((n + 127) >> 8) * row_tiles;
+        *small += (n & 255) >= 1 && (n & 255) <= 128 ? row_tiles : 0;
     }
+}
+
+bool plan_gemm_wide(int split, int cus, WidePlan *plan)
+{
+    WideArgs &a = plan->args;
+    a.steps_total = ceil_div_i(a.k, 64);
+    a.row_tiles = ceil_div_i(a.m, kWideRows);
+    a.n_shares = 0;
+    long long large, small;
+    count_wide_tiles(a, &large, &small);
     const long long tiles = large + small, weight = (large * kCostLarge + small * kCostSmall) * a.steps_total;
     if (tiles < 1 || tiles > 0x7fffffff || weight > 0x7fffffff) return false;
     a.large = (int)large, a.small = (int)small;

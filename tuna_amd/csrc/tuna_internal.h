@@ -148,8 +148,8 @@ struct TiledArgs {
     int blk_shift;        // scale-block variants: absmax is [m, k / (64 << blk_shift)], one scale per block of a row
 };
 
-// Launch arguments of the 256 x 256 many-token kernel (gemm_wide.hip): n_groups stacked matrices of m rows each, group
-// e multiplying the activation rows tok_off[e] .. tok_off[e + 1] - 1 (a dense GEMM is one group).  A tile is 256 rows x
+// Launch arguments of the 256 x 256 many-token kernel (gemm_wide.hip): n_groups of a stack of matrices of m rows each,
+// matrix id[e] multiplying the activation rows tok_begin[e] .. + tok_count[e] - 1 (a dense GEMM is one group).  A tile is 256 rows x
 // up to 256 tokens of one group; tiles of more than 128 tokens ("large") are numbered first, group by group, row tile by
 // row tile, the token tiles of a row tile next to each other; then the groups' last tiles of 1 .. 128 tokens ("small").
 struct WideArgs {
@@ -169,7 +169,8 @@ struct WideArgs {
     int whole;           // tiles 0 .. whole - 1 are computed whole, one workgroup each
     int n_shares;        // the k-steps of the other tiles, laid end to end, are divided into this many equal shares (0: none)
     int blk_shift;       // scale-block variants: absmax is [m, k / (64 << blk_shift)]
-    int tok_off[kMaxGroups + 1];
+    int tok_begin[kMaxGroups], tok_count[kMaxGroups];
+    unsigned char id[kMaxGroups];
 };
 
 struct WidePlan {
@@ -244,8 +245,11 @@ hipError_t launch_gemm_tiled(const TiledArgs &args, int tile_rows, int tile_toke
 // 256 x 256 tile, one wave per SIMD: gemm_wide.hip, and gemm_wide32.hip with 32 x 32 x 16 MFMAs (reached through
 // launch_gemm_tiled)
 size_t wide_lds_bytes();
-// split: 0 = balanced over the compute units, 1 = every tile whole, else that many shares per tile.
-bool plan_gemm_wide(int m, int k, int n_groups, const int *tok_off, int split, int cus, WidePlan *plan);
+// Fills in the launch whose shape and groups plan->args holds (m, k, n_groups, tok_begin, tok_count, id).  split: 0 = the
+// last rounds of tiles balanced over the compute units, 1 = every tile whole, else that many shares per tile.
+bool plan_gemm_wide(int split, int cus, WidePlan *plan);
+// Its tiles of more than 128 tokens and of 1 .. 128.
+void count_wide_tiles(const WideArgs &args, long long *large, long long *small);
 hipError_t launch_gemm_wide(const WidePlan &plan, bool scale_blocks, hipStream_t stream);
 hipError_t launch_gemm_wide32(const TiledArgs &args, hipStream_t stream);
 bool tiled_variant_exists(int tile_rows, int tile_tokens, bool mfma32);

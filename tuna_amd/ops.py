@@ -177,8 +177,9 @@ def matmul_grouped(x, q, s, c, o, m_group: int, n_groups: int, k: int, token_off
 
     x fp16 [n_total, k], rows sorted by group; q uint8 [n_groups*m_group/8, k/8, 32] and s fp32
     [n_groups*m_group]: the groups' weights stacked along m; o fp16 [n_total, m_group];
-    token_offsets: n_groups+1 non-decreasing host ints.  Groups without tokens cost nothing; without a config a
-    group of more than 64 tokens runs as a dense GEMM of its own (same bits as `matmul` on its slices).
+    token_offsets: n_groups+1 non-decreasing host ints.  Groups without tokens cost nothing; without a config
+    groups of more than 64 tokens run as dense GEMMs of their own (same bits as `matmul` on their slices) or, several of
+    them where that is predicted to be faster, as one launch of 256 x 256 tiles.
     """
     if config is None and decode_mode == _lib.DECODE_GEMM:
         rc = _lib.native().matmul_grouped(x, q, s, c, o, m_group, n_groups, k, token_offsets)
