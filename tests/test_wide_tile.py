@@ -136,3 +136,18 @@ def test_groups_of_many_tokens_in_one_launch(m, k, counts):
     for e, (lo, hi) in enumerate(zip(offs, offs[1:])):
         if hi > lo:
             _check(out[lo:hi], q, s, x[lo:hi], code, k, first_row=e * m, rows=m)
+
+
+# scale blocks: one block per step and several steps per block, odd numbers of steps, splits, small last tiles
+@pytest.mark.parametrize("m,n,k,block,split", [(256, 200, 256, 64, 1), (528, 300, 1280, 64, 1), (272, 70, 768, 256, 1), (512, 385, 2048, 128, 3),
+                                               (1024, 129, 1792, 64, 2)])
+def test_scale_blocks(m, n, k, block, split):
+    import torch
+
+    from tuna_amd import ops
+
+    q, s, x, code = _inputs(m, n, k, seed=k + n, block=block)
+    out = _out(n, m)
+    ops.matmul_blockwise(x, q, s, code, out, m, n, k, block, config=_cfg(split))
+    torch.cuda.synchronize()
+    _check(out, q, s, x, code, k, block=block)

@@ -2045,6 +2045,20 @@ static int derive_blockwise(const BlockwiseCall &b, tuna_gemm_config *out)
                 if (run_blockwise(b, c, nullptr, true) != TUNA_OK) continue;
                 best = c, best_cost = cost, found = true;
             }
+        // The 256 x 256 tile by its own model, 1.07 x the time of the per-row kernel (a unit of the costs above is 5.68e-7
+        // us per k, both read off 200 random shapes at 65 ... 4096 tokens with blocks of 64, where this tile is up to
+        // 1.8 x faster than the best of the others: 3584 x 25088 at 2669 tokens 774 us -> 416, 5632 x 16384 at 701 tokens
+        // 236 -> 149, 11136 x 1536 at 2891 tokens 173 -> 118).
+        const WideTiles t(m, n, k);
+        double us = 0.0;
+        const int split = n > 64 ? wide_best_split(t.large, t.small, t.steps, &us) : 0;
+        if (split && (!found || 1.07 * us / 5.68e-7 / k < 0.96 * best_cost)) {
+            tuna_gemm_config c;
+            memset(&c, 0, sizeof(c));
+            c.rows_per_wave = 64, c.waves_m = 1, c.waves_k = 1, c.prefetch = 2, c.x_chunk = 64, c.token_tiles = 16;
+            c.lds_tile_rows = 256, c.split_k = split;
+            if (run_blockwise(b, c, nullptr, true) == TUNA_OK) best = c, found = true;
+        }
         if (found) {
             *out = best;
             return TUNA_OK;
