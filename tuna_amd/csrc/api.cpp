@@ -70,7 +70,7 @@ static int plan_gemm(int m, int n, int k, const tuna_gemm_config &c, int decode,
     if (decode != TUNA_DECODE_GEMM && decode != TUNA_DECODE_DEQUANT)
         return fail(TUNA_ERR_INVALID_ARG, "decode_mode %d is neither TUNA_DECODE_GEMM nor TUNA_DECODE_DEQUANT", decode);
     if (c.lds_tile_rows > 0) return fail(TUNA_ERR_INVALID_ARG, "plan_gemm called with a many-token config");
-    if (c.lds_tile_rows < -1) return fail(TUNA_ERR_INVALID_ARG, "lds_tile_rows=%d (0, -1, 64, 128 or 256)", c.lds_tile_rows);
+    if (c.lds_tile_rows < -1) return fail(TUNA_ERR_INVALID_ARG, "lds_tile_rows=%d (0, -1, -4, 64, 128 or 256)", c.lds_tile_rows);
     if (c.rows_per_wave != 64 && c.rows_per_wave != 128 && c.rows_per_wave != 256)
         return fail(TUNA_ERR_UNSUPPORTED, "rows_per_wave=%d (64, 128 or 256)", c.rows_per_wave);
     if (c.prefetch != 2 && c.prefetch != 4 && c.prefetch != 8)
@@ -225,6 +225,7 @@ static int planned_cus()
 }
 
 static bool wide_balance_pays(int m, int n, int k);
+static bool stream_applies(const tuna_gemm_config &c, int n, int decode, int epilogue);
 static bool plan_wide_dense(int m, int n, int k, int split, WidePlan *plan)
 {
     memset(plan, 0, sizeof(*plan));
@@ -306,6 +307,42 @@ static int launch_tiled(TiledPlan &tp, const void *q, const void *x, const void 
         e = launch_gemm_tiled(tp.args, tp.tile_rows, tp.tile_tokens, tp.mfma32, stream, blk_shift >= 0);
     }
     return e == hipSuccess ? TUNA_OK : hip_fail(e, "many-token gemm launch");
+}
+
+// lds_tile_rows -4: the decode-batch kernel (gemm_flow.hip), its k-steps divided into split_k shares
+static inline bool is_flow(const tuna_gemm_config &c) { return c.lds_tile_rows == -4; }
+
+static int plan_flow(int m, int n, int k, const tuna_gemm_config &c, int decode, FlowPlan *plan)
+{
+    int rc = check_shape(m, n, k);
+    if (rc) return rc;
+    if (decode != TUNA_DECODE_GEMM) return fail(TUNA_ERR_UNSUPPORTED, "the decode-batch kernel implements TUNA_DECODE_GEMM only");
+    if (c.split_k < 1 || c.split_k > 2 * kMaxCus) return fail(TUNA_ERR_UNSUPPORTED, "decode-batch kernel: split_k=%d shares (1..%d)", c.split_k, 2 * kMaxCus);
+    if (n > 16 * c.token_tiles) return fail(TUNA_ERR_UNSUPPORTED, "decode-batch kernel: n=%d tokens in one pass of %d token tiles", n, c.token_tiles);
+    memset(plan, 0, sizeof(*plan));
+    FlowArgs &a = plan->args;
+    a.m = a.m_total = m, a.k = k, a.n_groups = 1, a.tok_count[0] = n;
+    if (!plan_gemm_flow(c.token_tiles, c.split_k, plan))
+        return fail(TUNA_ERR_UNSUPPORTED, "decode-batch kernel: 1 to 4 token tiles (%d), or k=%d too long", c.token_tiles, k);
+    return TUNA_OK;
+}
+
+static int launch_flow(FlowPlan &plan, const void *q, const void *x, const void *code, const void *absmax, void *out, int epilogue,
+                       const void *residual, int blk_shift, bool static_ws, hipStream_t stream)
+{
+    FlowArgs &a = plan.args;
+    a.q = static_cast<const uint8_t *>(q);
+    a.x = x;
+    a.code = static_cast<const float *>(code);
+    a.absmax = static_cast<const float *>(absmax);
+    a.out = out;
+    a.epilogue = epilogue;
+    a.residual = residual;
+    a.blk_shift = blk_shift < 0 ? 0 : blk_shift;
+    int rc = provide_workspace(static_ws, stream, plan.ws_bytes, plan.n_counters, &a.ws, &a.counters);
+    if (rc) return rc;
+    const hipError_t e = launch_gemm_flow(plan, blk_shift >= 0, stream);
+    return e == hipSuccess ? TUNA_OK : hip_fail(e, "decode-batch gemm launch");
 }
 
 // Narrow-row kernel: checks and launch arguments for a config with rows_per_wave 16 or 32.
@@ -894,12 +931,77 @@ static bool config_runs(int m, int n, int k, const tuna_gemm_config &c)
         TiledPlan tp;
         return plan_tiled(m, n, k, c, TUNA_DECODE_GEMM, &tp) == TUNA_OK;
     }
+    if (is_flow(c)) {
+        FlowPlan fp;
+        return plan_flow(m, n, k, c, TUNA_DECODE_GEMM, &fp) == TUNA_OK;
+    }
     if (is_narrow(c)) {
         NarrowPlan np;
         return plan_narrow(m, n, k, c, TUNA_DECODE_GEMM, &np) == TUNA_OK;
     }
     GemmPlan plan;
     return plan_gemm(m, n, k, c, TUNA_DECODE_GEMM, &plan) == TUNA_OK;
+}
+
+// Microseconds of a launch of the decode-batch kernel (gemm_flow.hip) with `tiles` 256-row tiles of `units` units of k in
+// `shares` workgroups, by a model read off 600 random shapes of 6 ... 390 MB of weights at 1 ... 64 tokens, each with up to
+// ten numbers of shares (8 per cent off on average): a k-step takes longer with more token tiles and with two workgroups on
+// a compute unit, a tile that several shares contribute to is handed over, which costs more with every contributor beyond
+// the second.
+static double flow_time(double tiles, int units, int nt, int shares)
+{
+    static const double kTokens[5] = {0, 0.916, 1.0, 1.227, 1.302};
+    const double per_share = ceil(tiles * units / shares) * 4, two = shares <= kMaxCus ? 0.0 : shares / (double)kMaxCus - 1.0;
+    const double step = (0.485 + 0.522 * (two < 1.0 ? two : 1.0)) * kTokens[nt];
+    const long long all = (long long)tiles * units;
+    double contributors = shares / tiles + 1.0;
+    if (all % shares == 0 && (all / shares) % units == 0) contributors = 1.0;
+    else if (shares % (long long)tiles == 0 && units % (shares / (long long)tiles) == 0) contributors = shares / tiles;
+    return 6.1 + per_share * step + (contributors > 1.0 ? 2.7 + (contributors > 2.0 ? 0.3 * nt * (contributors - 2.0) : 0.0) : 0.0);
+}
+
+// The number of shares that takes them least time, and that time in *us: equal parts of every tile, or 64 ... 512 at large.
+static int flow_best_shares(long long tiles, int units, int nt, double *us)
+{
+    int best = 0;
+    auto consider = [&](long long shares) {
+        if (shares < 1 || shares > 2 * kMaxCus || shares > tiles * units) return;
+        const double t = flow_time((double)tiles, units, nt, (int)shares);
+        if (!best || t < *us) best = (int)shares, *us = t;
+    };
+    for (int parts : {1, 2, 3, 4, 6, 8}) consider(parts * tiles);
+    for (int shares : {64, 128, 192, 256, 384, 512}) consider(shares);
+    return best;
+}
+
+// What a launch without an explicit config runs up to 64 tokens: the selected config, or the decode-batch kernel in its place
+// where that is predicted to be faster.  The selected kernels are priced by straight lines over the bytes of the weights,
+// read off the same random shapes; narrow-row, lean and batched launches, which win on the shapes they are picked for, are
+// left alone, and an entry of the table, timed for its shape, has to be beaten by a quarter.
+static bool flow_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, tuna_gemm_config *flow)
+{
+    const double mb = 0.5e-6 * m * k;
+    if (n > 64 || is_narrow(c) || mb < 8) return false;
+    const int nt = ceil_div(n, 16);
+    double price;
+    if (c.lds_tile_rows > 0) {
+        price = nt < 3 ? 0.0 : 14.3 + 0.62 * mb;
+    } else {
+        GemmPlan plan;
+        if (plan_gemm(m, n, k, c, TUNA_DECODE_GEMM, &plan) != TUNA_OK || launch_is_lean(plan, kMaxCus) || stream_applies(c, n, TUNA_DECODE_GEMM, TUNA_EPILOGUE_NONE))
+            return false;
+        const bool mid = mid_applies(plan);
+        static const double kMid[5] = {0, 0, 0.30, 0.40, 0.37}, kGeneral[5] = {0, 0.29, 0.50, 0.55, 0.60};
+        if (mid) price = nt == 1 ? 0.0 : 6.0 + nt + (nt == 2 && c.lds_tile_rows == -1 ? 0.22 : kMid[nt]) * mb;
+        else price = 7.0 + 1.5 * nt + kGeneral[nt] * mb;
+    }
+    double us = 0.0;
+    const int shares = price == 0.0 ? 0 : flow_best_shares(ceil_div(m, 256), ceil_div(ceil_div(k, 64), 4), nt, &us);
+    if (!shares || us >= (from_table ? 0.8 : 0.95) * price) return false;
+    memset(flow, 0, sizeof(*flow));
+    flow->rows_per_wave = 64, flow->waves_m = 4, flow->waves_k = 1, flow->prefetch = 4, flow->x_chunk = 64, flow->token_tiles = nt;
+    flow->lds_tile_rows = -4, flow->split_k = shares;
+    return config_runs(m, n, k, *flow);
 }
 
 // What a launch without an explicit config runs from 65 tokens on: the selected config, or 256 x 256 tiles of gemm_wide.hip
@@ -992,12 +1094,25 @@ static int select_config_for(int m, int n, int k, int decode, tuna_gemm_config *
     return TUNA_OK;
 }
 
+// The config a launch without an explicit one runs: the selected one, or a newer kernel in its place.
+static void select_launch(int m, int n, int k, int decode, tuna_gemm_config *c)
+{
+    int from_table = 0;
+    select_config_for(m, n, k, decode, c, &from_table);
+    tuna_gemm_config other;
+    if (decode == TUNA_DECODE_GEMM && (wide_instead(m, n, k, *c, &other) || flow_instead(m, n, k, *c, from_table != 0, &other))) *c = other;
+}
+
 // The checks of the planner `c` belongs to, for a decode mode.
 static int validate_for(int m, int n, int k, const tuna_gemm_config &c, int decode)
 {
     if (c.lds_tile_rows > 0) {
         TiledPlan tp;
         return plan_tiled(m, n, k, c, decode, &tp);
+    }
+    if (is_flow(c)) {
+        FlowPlan fp;
+        return plan_flow(m, n, k, c, decode, &fp);
     }
     if (is_narrow(c)) {
         NarrowPlan np;
@@ -1299,9 +1414,7 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
         return rc;
     tuna_gemm_config c;
     if (cfg) c = *cfg;
-    else select_config_for(m, n, k, decode, &c, nullptr);
-    tuna_gemm_config wide;
-    if (!cfg && decode == TUNA_DECODE_GEMM && wide_instead(m, n, k, c, &wide)) c = wide;
+    else select_launch(m, n, k, decode, &c);
     if (c.lds_tile_rows > 0) {
         TiledPlan tp;
         if ((rc = plan_tiled(m, n, k, c, decode, &tp))) return rc;
@@ -1313,6 +1426,11 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
             if ((rc = plan_tiled(m, n, k, c, decode, &tp))) return rc;
         }
         return launch_tiled(tp, q, x, code, absmax, out, epilogue, residual, -1, static_ws, stream);
+    }
+    if (is_flow(c)) {
+        FlowPlan fp;
+        if ((rc = plan_flow(m, n, k, c, decode, &fp))) return rc;
+        return launch_flow(fp, q, x, code, absmax, out, epilogue, residual, -1, static_ws, stream);
     }
     // The narrow-row kernel reads a lane's scales 2 or 4 rows at a time.  A caller that names such a config must align
     // absmax for it; when the library picked the config itself it takes the streaming kernel's derived config for a
@@ -1421,6 +1539,17 @@ static int grouped_config(int m_group, int m_active, int max_tok, int k, int dec
     }
     return fail(TUNA_ERR_UNSUPPORTED, "no grouped config for m_group=%d, %d active rows, %d tokens, k=%d: %s", m_group, m_active,
                 max_tok, k, std::string(g_error).c_str());
+}
+
+// Shares of a grouped launch of the decode-batch kernel; 0 for the smallest launches of up to 16 tokens per group, which
+// the general kernel's grouped variants run as fast or faster (2304 x 2432, five groups: 13.3 us against 14.2).  On 90 random
+// launches of 8 ... 64 groups this kernel is 1.4 x faster on average (14336 ... 20096 rows 1.5 ... 3.8 x): it streams
+// whole rounds without a tail per tile and takes 64 tokens in one pass.
+static int grouped_flow_shares(int m_group, int n_active, int nt, int k)
+{
+    double us = 0.0;
+    if (nt == 1 && (double)m_group * n_active * k < 3e7) return 0;
+    return flow_best_shares((long long)ceil_div(m_group, 256) * n_active, ceil_div(ceil_div(k, 64), 4), nt, &us);
 }
 
 // Grouped GEMM: n_groups stacked weight matrices of m_group rows, group e applied to the
@@ -1534,6 +1663,18 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
     }
     if (n_active == 0) return TUNA_OK;  // every group with tokens ran as a dense GEMM
     const int m_active = m_group * n_active;
+    if (!cfg && decode == TUNA_DECODE_GEMM) {
+        FlowPlan fp;
+        memset(&fp, 0, sizeof(fp));
+        FlowArgs &f = fp.args;
+        f.m = m_group, f.m_total = m, f.k = k, f.n_groups = n_active;
+        for (int e = 0; e < n_active; ++e) f.tok_begin[e] = offsets[act[e]], f.tok_count[e] = offsets[act[e] + 1] - offsets[act[e]], f.id[e] = act[e];
+        const int nt = ceil_div(max_tok, 16), shares = grouped_flow_shares(m_group, n_active, nt, k);
+        if (shares && plan_gemm_flow(nt, shares, &fp)) {
+            rc = launch_flow(fp, q, x, code, absmax, out, TUNA_EPILOGUE_NONE, nullptr, -1, false, stream);
+            if (rc != TUNA_ERR_WORKSPACE) return rc;  // (a stream that is capturing, with too small a workspace: the general kernel)
+        }
+    }
     tuna_gemm_config c;
     GemmPlan plan;
     if (cfg) {
@@ -1819,11 +1960,12 @@ TUNA_EXPORT int tuna_quantize_blockwise(const void *w, const void *code, void *q
 // A config comes from the caller (tuna_matmul_blockwise_ex), from the table of tuned entries keyed by (m, token bucket,
 // k, block_size) (config_table.cpp, written by the tuner), or from the rules of derive_blockwise below.
 // ---------------------------------------------------------------------------------------
-enum BlockwiseFamily { kBlkNarrow = 0, kBlkMulti = 1, kBlkTiled = 2, kBlkMid = 3 };
+enum BlockwiseFamily { kBlkNarrow = 0, kBlkMulti = 1, kBlkTiled = 2, kBlkMid = 3, kBlkFlow = 4 };
 
 static BlockwiseFamily blockwise_family(const tuna_gemm_config &c)
 {
     if (c.lds_tile_rows > 0) return kBlkTiled;
+    if (is_flow(c)) return kBlkFlow;
     if (is_narrow(c)) return kBlkNarrow;
     if (c.split_k == 0) return kBlkMulti;
     return kBlkMid;
@@ -1908,6 +2050,11 @@ static int run_blockwise(const BlockwiseCall &b, const tuna_gemm_config &c, hipS
         if ((rc = launch_tiled(tp, b.q, b.x, b.code, b.absmax, b.out, TUNA_EPILOGUE_NONE, nullptr, shift, false, st))) return rc;
         diag::count(diag::kBlockwiseTiled);
         return TUNA_OK;
+    }
+    case kBlkFlow: {
+        FlowPlan fp;
+        if ((rc = plan_flow(m, n, k, c, TUNA_DECODE_GEMM, &fp))) return rc;
+        return dry ? TUNA_OK : launch_flow(fp, b.q, b.x, b.code, b.absmax, b.out, TUNA_EPILOGUE_NONE, nullptr, shift, false, st);
     }
     case kBlkMid: {
         tuna_gemm_config t = c;
@@ -2284,6 +2431,14 @@ TUNA_EXPORT int tuna_config_footprint(int m, int n, int k, const tuna_gemm_confi
         if (workspace_bytes) *workspace_bytes = tp.ws_bytes;
         return TUNA_OK;
     }
+    if (is_flow(*cfg)) {
+        FlowPlan fp;
+        int rc = plan_flow(m, n, k, *cfg, TUNA_DECODE_GEMM, &fp);
+        if (rc) return rc;
+        if (lds_bytes) *lds_bytes = kLutBytes;
+        if (workspace_bytes) *workspace_bytes = fp.ws_bytes;
+        return TUNA_OK;
+    }
     if (is_narrow(*cfg)) {
         NarrowPlan np;
         int rc = plan_narrow(m, n, k, *cfg, TUNA_DECODE_GEMM, &np);
@@ -2435,8 +2590,9 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
     tuna_gemm_config c, w;
     if (cfg) c = *cfg;
     else select_config_for(m, n, k, decode_mode, &c, nullptr);
-    if (!cfg && decode_mode == TUNA_DECODE_GEMM && wide_instead(m, n, k, c, &w) && memcmp(&w, &c, sizeof(c)) != 0) {
-        const int at = snprintf(buf, len, "gemm_wide_kernel<256 rows x 256 tokens> split_k=%d in place of ", w.split_k);
+    if (!cfg && (select_launch(m, n, k, decode_mode, &w), memcmp(&w, &c, sizeof(c)) != 0)) {
+        const int at = is_flow(w) ? snprintf(buf, len, "gemm_flow_kernel<NT=%d> %d shares in place of ", w.token_tiles, w.split_k)
+                                  : snprintf(buf, len, "gemm_wide_kernel<256 rows x 256 tokens> split_k=%d in place of ", w.split_k);
         return at < 0 || (size_t)at + 16 > len ? TUNA_OK : tuna_describe_launch(m, n, k, &c, decode_mode, buf + at, len - (size_t)at);
     }
     if (c.lds_tile_rows > 0) {
@@ -2446,6 +2602,12 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
         snprintf(buf, len, "%s<%d rows x %d tokens%s> split_k=%d%s", wide ? "gemm_wide_kernel" : "gemm_tiled_kernel", tp.tile_rows,
                  tp.tile_tokens, tp.mfma32 ? ",mfma 32x32x16" : "", c.split_k,
                  tp.wide && c.split_k == 1 && tp.wide_plan.args.n_shares ? ", last tiles shared" : "");
+        return TUNA_OK;
+    }
+    if (is_flow(c)) {
+        FlowPlan fp;
+        if ((rc = plan_flow(m, n, k, c, decode_mode, &fp))) return rc;
+        snprintf(buf, len, "gemm_flow_kernel<NT=%d> %d shares", fp.nt, fp.args.n_shares);
         return TUNA_OK;
     }
     if (is_narrow(c)) {

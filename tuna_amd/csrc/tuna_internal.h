@@ -179,6 +179,33 @@ struct WidePlan {
     size_t ws_bytes, n_counters;
 };
 
+// Launch arguments of the decode-batch streaming kernel (gemm_flow.hip): n_groups of a stack of matrices of m rows each,
+// as in WideArgs, every group's tokens in one tile.
+struct FlowArgs {
+    const uint8_t *q;
+    const void *x;
+    const float *code;
+    const float *absmax;
+    void *out;
+    const void *residual;
+    int epilogue;
+    float *ws;           // partial tiles, two slots per share
+    unsigned *counters;  // one arrival counter per tile, zero between launches
+    int m, k, n_groups, m_total;  // rows of a group, reduction length, groups with tokens, rows of all matrices
+    int steps_total, units;       // ceil(k / 64); units of four steps
+    int row_tiles, tiles;         // of a group, of all groups with tokens
+    int n_shares;
+    int blk_shift;
+    int tok_begin[kMaxGroups], tok_count[kMaxGroups];
+    int id[kMaxGroups];  // (an int: read through the scalar cache)
+};
+
+struct FlowPlan {
+    FlowArgs args;
+    int nt;  // token tiles of 16: 1 .. 4
+    size_t ws_bytes, n_counters;
+};
+
 inline int ceil_div_i(int a, int b) { return (a + b - 1) / b; }
 
 struct GemmPlan {
@@ -251,6 +278,9 @@ bool plan_gemm_wide(int split, int cus, WidePlan *plan);
 // Its tiles of more than 128 tokens and of 1 .. 128.
 void count_wide_tiles(const WideArgs &args, long long *large, long long *small);
 hipError_t launch_gemm_wide(const WidePlan &plan, bool scale_blocks, hipStream_t stream);
+// Fills in the launch whose shape and groups plan->args holds (m, k, n_groups, m_total, tok_begin, tok_count, id).
+bool plan_gemm_flow(int nt, int shares, FlowPlan *plan);
+hipError_t launch_gemm_flow(const FlowPlan &plan, bool scale_blocks, hipStream_t stream);
 hipError_t launch_gemm_wide32(const TiledArgs &args, hipStream_t stream);
 bool tiled_variant_exists(int tile_rows, int tile_tokens, bool mfma32);
 size_t tiled_lds_bytes(int tile_rows, int tile_tokens);
