@@ -125,18 +125,23 @@ hipError_t launch_dequant(const uint8_t *q, const float *absmax, const float *co
 // reference divides by zero there, every candidate distance is NaN, and torch.argmin over an all-NaN
 // column returns index 0.
 //
-// One workgroup per block row (8 weight rows), 64 threads per row, 16-byte reads (a row's threads
-// read 1 KB contiguous).  NP > 0: the whole row (k <= 512*NP) is read once into registers, all
-// loads in flight together, so the op streams the weights exactly once; NP == 0: two passes (the
-// second mostly from cache).  Block maxima come from shuffles inside the row's 64 threads.  For a
-// codebook that is sorted with gaps wide enough that fp32 rounding cannot reorder distances, the
-// nearest entry is found by a 4-step binary search over the 15 decision boundaries between
-// neighbouring entries (each the smallest fp32 value the argmin gives to the upper entry, found by
-// bisection with the argmin's own arithmetic once per workgroup) - the argmin's result, since
-// |nv - c| is monotonic in c on either side of nv; any other codebook takes the 16 comparisons.
-// The division by the block maximum is a multiply by its refined reciprocal and one fused correction.  A thread's dword (one row, 8
-// consecutive k) is written through a 2 KB LDS tile so that the stores are 16 bytes per lane and
-// contiguous (the records of 64 block columns), not 4 bytes at a stride of 32.
+// A wave works on 8 weight rows x 256 columns (a "quad": four 16-byte loads per lane, each 128 contiguous bytes of
+// every row).  The eight lanes of a row are neighbours, so the maximum over a block of up to 64 weights is three DPP
+// steps and one over 128 or 256 the maximum over the lane's own registers; with one scale per row the workgroup's eight
+// waves share a block row and exchange their maxima through LDS (one barrier; the row's weights stay in registers up to
+// k = 16384, beyond that a second pass reads them again).  A lane's four dwords (one row each, 8 consecutive k) are
+// turned against the lanes of the other rows with permlane swaps: it then holds 4 rows of one block column, 16 bytes of
+// the packed layout, and the wave stores 1 KB contiguous.  Neither the weights nor the records pass through LDS, so that
+// blocked quantization has no barrier at all.
+// For a codebook that is sorted with gaps wide enough that fp32 rounding cannot reorder distances, the
+// nearest entry is found from the 15 decision boundaries between neighbouring entries (each the smallest fp32 value
+// the argmin gives to the upper entry, found by bisection with the argmin's own arithmetic once per wave) - the
+// argmin's result, since |nv - c| is monotonic in c on either side of nv; any other codebook takes the 16 comparisons.
+// The division by the block maximum is a multiply by its refined reciprocal and one fused correction.
+//
+// What bounds it: at 14336 x 4096 with blocks of 64 (177 MB of traffic) HBM and the vector ALU together, ten instructions a
+// weight: 62 -> 35 us, with one scale per row 54 -> 34; 8192 x 28672 in blocks of 64 238 -> 117 us (4.9 TB/s), 4096 x 14336
+// per row 61 -> 36; 3 us before the first table is complete.
 // Nearest entry of a sorted codebook: bnd[i] (i = 0..14) is the smallest binary32 value that the
 // argmin assigns to entry i + 1 rather than entry i, so the index is the number of boundaries <= nv:
 // a 4-step binary search, as a tree of selects over the 15 values (uniform, held in registers).
@@ -157,8 +162,8 @@ __device__ __forceinline__ uint32_t nearest_sorted(float nv, const float (&b)[16
 
 // The same count of boundaries <= nv without the search: the quotients lie in [-1, 1], cut into 64 buckets
 // of 1/32; when no two boundaries share a bucket, a bucket knows how many boundaries lie below it and the one
-// boundary (if any) inside it, and the index is that count plus one comparison.  bucket_of is monotonic in
-// nv (a fused multiply-add, a clamp, a truncation), so every value of a lower bucket is below the boundary
+// boundary (if any) inside it, and the index is that count plus one comparison.  The bucket is monotonic in
+// nv (a fused multiply-add, a truncation), so every value of a lower bucket is below the boundary
 // of a higher one and vice versa: the result is the binary search's for every nv, NaN included (bucket 0, the
 // comparison false, index 0).  One LDS table of {boundary, count} pairs in the lane-private layout of the
 // GEMM's decode table (entry e of lane l at (e << 9) | (l << 3): one 8-byte read, no bank conflicts whatever
@@ -169,17 +174,16 @@ typedef __attribute__((address_space(3))) unsigned char lds_u8;
 typedef uint32_t quant_u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) quant_u32x2 lds_pair;
 
-__device__ __forceinline__ uint32_t bucket_of(float nv)
+// nv * 16384 + 16384 plus 2^23: the fp32 pattern's low bits are that number as an integer, its multiples of 512 the
+// bucket - which is the entry's offset.  NaN and infinity mask to bucket 0.
+__device__ __forceinline__ uint32_t bucket_bits(float nv)
 {
-    return (uint32_t)__builtin_amdgcn_fmed3f(__builtin_fmaf(nv, 32.0f, 32.0f), 0.0f, 64.0f);
+    return __builtin_bit_cast(uint32_t, __builtin_fmaf(nv, 16384.0f, 8388608.0f + 16384.0f)) & 0xfe00u;
 }
 
-__device__ __forceinline__ uint32_t nearest_bucketed(float nv, uint32_t tab_lane)
+__device__ __forceinline__ quant_u32x2 bucket_entry(float nv, uint32_t tab_lane)
 {
-    const uint32_t e = bucket_of(nv);
-    const quant_u32x2 t = *reinterpret_cast<const lds_pair *>((uintptr_t)((e << 9) + tab_lane));
-    const uint32_t bnd_bits = t[0], below = t[1];
-    return below + (nv >= __builtin_bit_cast(float, bnd_bits) ? 1u : 0u);
+    return *reinterpret_cast<const lds_pair *>((uintptr_t)(bucket_bits(nv) | tab_lane));
 }
 
 __device__ __forceinline__ uint32_t nearest_any(float nv, const float (&c)[16])
@@ -251,190 +255,245 @@ __device__ __forceinline__ quant_f16x2 pk_absmax8(quant_f16x2 acc, f16x8 t)
 }
 __device__ __forceinline__ float pk_absmax_value(quant_f16x2 acc) { return fmaxf((float)acc[0], (float)acc[1]); }
 
-template <int NP>
-__global__ __launch_bounds__(512, NP == 16 ? 2 : 4) void quantize_kernel(const f16 *__restrict__ w, const float *__restrict__ code,
-                                                       uint32_t *__restrict__ q32, float *__restrict__ absmax, int m, int k,
-                                                       int bs)
+// The packed dword of 8 consecutive weights of a row.  MODE 0: bucket table; 1: binary search over the boundaries
+// (c); 2: the 16 comparisons with the codebook (c).  A block of zeros (y is NaN) gets index 0 throughout.
+template <int MODE>
+__device__ __forceinline__ uint32_t quant_dword(f16x8 t, float amax, uint32_t tab_lane, const float (&c)[16])
 {
-    __shared__ float cs[16], bs_[15];
-    __shared__ int fast_s, tab_s, jb_s[15];
-    __shared__ uint32_t pair_s[kQuantBuckets][2];
-    extern __shared__ __align__(16) unsigned char qtab[];  // bucket table
-    constexpr int TPR = 64;  // threads per weight row: a row's threads read 1 KB contiguous
-    // records of the block row being assembled: [step][block column of the step (64)][row (8)] - all NP steps
-    // of a row held in registers (one barrier per block row), or two buffers of one step each (NP == 0)
-    __shared__ __align__(16) uint32_t tile[NP > 0 ? NP : 2][TPR * 8];
-    const int tid = threadIdx.x;
-    if (tid < 16) cs[tid] = code[tid];
-    __syncthreads();
-    if (tid == 0) {
-        // sorted, and every gap far above the rounding of a difference (|nv| <= 1, so a difference is
-        // at most 1 + max|c| and its rounding error below 2^-23 of that)
-        float cmax = fmaxf(fabsf(cs[0]), fabsf(cs[15]));
-        const float thr = (1.0f + cmax) * 9.5367431640625e-7f;  // 2^-20
-        int ok = 1;
-        for (int i = 0; i < 15; ++i) ok &= (cs[i + 1] - cs[i] >= thr) ? 1 : 0;
-        fast_s = ok && cmax < 3.0e38f;
-    }
-    __syncthreads();
-    const bool fast = fast_s != 0;
-    if (fast && tid < 15) bs_[tid] = decision_boundary(cs[tid], cs[tid + 1]);
-    __syncthreads();
-    // bucket tables, if every boundary is finite and has a bucket of its own
-    if (tid == 0) {
-        int ok = fast ? 1 : 0;
-        for (int i = 0; i < 15 && ok; ++i) {
-            jb_s[i] = (int)bucket_of(bs_[i]);
-            ok &= (fabsf(bs_[i]) < 3.0e38f) && (i == 0 || jb_s[i] > jb_s[i - 1]) ? 1 : 0;
-        }
-        tab_s = ok;
-    }
-    __syncthreads();
-    const bool tabled = tab_s != 0;
-    const uint32_t tab0 = (uint32_t)(uintptr_t)(lds_u8 *)qtab;
-    const uint32_t tab_lane = tab0 + ((uint32_t)(tid & 63) << 3);
-    if (tabled) {
-        if (tid < kQuantBuckets) {  // a bucket's pair: its boundary (+inf: none) and the boundaries below it
-            float b = __builtin_inff();
-            uint32_t n = 0;
+    const float y = refined_rcp(amax);
+    const u32x4 w = __builtin_bit_cast(u32x4, t);
+    uint32_t d = 0;
 #pragma unroll
-            for (int i = 0; i < 15; ++i) {
-                b = jb_s[i] == tid ? bs_[i] : b;
-                n += jb_s[i] < tid ? 1u : 0u;
-            }
-            pair_s[tid][0] = __builtin_bit_cast(uint32_t, b);
-            pair_s[tid][1] = n;
-        }
-        __syncthreads();
-        for (int p = tid; p < kQuantTabBytes / 16; p += 512) {  // 32 stores of 16 bytes (two lanes' pairs) per bucket
-            const uint32_t u = pair_s[p >> 5][0], n = pair_s[p >> 5][1];
-            reinterpret_cast<u32x4 *>(qtab)[p] = u32x4{u, n, u, n};
+    for (int p = 3; p >= 0; --p) {  // byte p: columns 2p (high nibble) and 2p + 1
+        const uint32_t pair = w[p];
+        const float n0 = div_by_block_max<0>(pair, amax, y), n1 = div_by_block_max<1>(pair, amax, y);
+        if constexpr (MODE == 0) {
+            const quant_u32x2 e0 = bucket_entry(n0, tab_lane), e1 = bucket_entry(n1, tab_lane);
+            const uint32_t b0 = e0[0], b1 = e1[0];
+            d = (d << 4) + e0[1] + (n0 >= __builtin_bit_cast(float, b0) ? 1u : 0u);
+            d = (d << 4) + e1[1] + (n1 >= __builtin_bit_cast(float, b1) ? 1u : 0u);
+        } else if constexpr (MODE == 1) {
+            d = (d << 4) | nearest_sorted(n0, c);
+            d = (d << 4) | nearest_sorted(n1, c);
+        } else {
+            d = (d << 4) | nearest_any(n0, c);
+            d = (d << 4) | nearest_any(n1, c);
         }
     }
-    __syncthreads();
+    return d;
+}
 
-    // The block rows, with the nearest-entry rule as a compile-time choice (the three loops share nothing
-    // but their registers: the table path must not carry the 15 boundaries of the search).  MODE 0: bucket
-    // tables; 1: binary search over the boundaries; 2: the 16 comparisons.
-    auto run = [&](auto mode_tag) {
-    constexpr int MODE = decltype(mode_tag)::value;
-    float c[16];  // MODE 1: the boundaries; MODE 2: the codebook
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float v)
+{
+    const int i = __builtin_bit_cast(int, v);
+    return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, CTRL, 0xf, 0xf, true)));
+}
+constexpr int kDppXor1 = 0xb1, kDppXor2 = 0x4e, kDppHalfMirror = 0x141;  // (the last: lane i of 8 <-> 7 - i)
+
+// Exchanges register index bits with lane bits 5 and 4: d[i] of lane (b5, b4) <-> d[2 b5 + b4] of lane (i1, i0).
+__device__ __forceinline__ void turn4(uint32_t (&d)[4])
+{
 #pragma unroll
-    for (int i = 0; i < 16; ++i) c[i] = MODE == 1 ? (i < 15 ? bs_[i] : 0.f) : MODE == 2 ? cs[i] : 0.f;
-    constexpr bool AHEAD = NP > 0 && NP <= 8;
-    f16x8 v[NP > 0 ? NP : 1];
-    for (int mb = blockIdx.x; mb < (m >> 3); mb += gridDim.x) {
-    const int r8 = tid / TPR, j = tid % TPR;
-    const int row = mb * 8 + r8;
+    for (int i = 0; i < 2; ++i) {
+        const auto r = __builtin_amdgcn_permlane32_swap(d[i], d[i + 2], false, false);
+        d[i] = r[0];
+        d[i + 2] = r[1];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+        const auto r = __builtin_amdgcn_permlane16_swap(d[i], d[i + 1], false, false);
+        d[i] = r[0];
+        d[i + 1] = r[1];
+    }
+}
+
+constexpr int kQuadCols = 256;  // columns of a quad
+
+// NQ == 0: blocks of up to 256 weights (bs a power of two), the waves walk the quads; NQ > 0: one scale per row, NQ quads
+// per wave in registers (k <= 256 NQ WAVES); NQ < 0: one scale per row, two passes.
+template <int NQ, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, NQ >= 2 ? 4 : 6)
+void quantize_kernel(const f16 *__restrict__ w, const float *__restrict__ code, uint32_t *__restrict__ q32,
+                     float *__restrict__ absmax, int m, int k, int bs)
+{
+    // the bucket table from LDS address 0 on (nothing here is statically allocated: an entry's offset is or-ed to the
+    // lane's address), then the waves' maxima
+    extern __shared__ __align__(16) unsigned char qtab[];
+    float (*wave_max)[WAVES][8] = reinterpret_cast<float (*)[WAVES][8]>(qtab + kQuantTabBytes);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = lane & 7;  // column group of the load
+    const int r8 = ((lane >> 4) & 3) | ((lane >> 1) & 4);  // weight row of the load: lane bits 5, 4 -> row bits 1, 0
     const int kb_total = k >> 3;
-    const int n_steps = (kb_total + TPR - 1) / TPR;  // steps of 64 block columns
-    const f16 *src = w + (size_t)row * k;
-    const bool by_row = bs == k;
-    const int lanes_blk = by_row ? TPR : bs >> 3;  // threads that share a scale (a power of two <= 32)
-    const int nblk = k / bs;
+    const int quads = (k + kQuadCols - 1) / kQuadCols;  // of a block row
+    const int rows8 = m >> 3;
 
-    float row_max = 0.f;
-    if constexpr (NP > 0) {
-        if (!AHEAD || mb == (int)blockIdx.x) {
+    auto load_quad = [&](f16x8 (&v)[4], int mb, int g) {
+        const f16 *src = w + (size_t)(mb * 8 + r8) * k + g * kQuadCols + j * 8;
 #pragma unroll
-            for (int i = 0; i < NP; ++i) {
-                const int kb = i * TPR + j;
-                v[i] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-                if (kb < kb_total) v[i] = *reinterpret_cast<const f16x8 *>(src + (size_t)kb * 8);
-            }
-        }
-    }
-    // the next block row's weights are requested before this one's arithmetic (registers for both up to NP = 8)
-    f16x8 vn[AHEAD ? NP : 1];
-    if constexpr (AHEAD) {
-        if (mb + (int)gridDim.x < (m >> 3)) {
-            const f16 *srcn = src + (size_t)gridDim.x * 8 * k;
-#pragma unroll
-            for (int i = 0; i < NP; ++i) {
-                const int kb = i * TPR + j;
-                vn[i] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-                if (kb < kb_total) vn[i] = *reinterpret_cast<const f16x8 *>(srcn + (size_t)kb * 8);
-            }
-        }
-    }
-    if (by_row) {
-        quant_f16x2 pm = quant_f16x2{(f16)0.f, (f16)0.f};
-        if constexpr (NP > 0) {
-#pragma unroll
-            for (int i = 0; i < NP; ++i) pm = pk_absmax8(pm, v[i]);
-        } else {
-            for (int kb = j; kb < kb_total; kb += TPR) pm = pk_absmax8(pm, *reinterpret_cast<const f16x8 *>(src + (size_t)kb * 8));
-        }
-        row_max = pk_absmax_value(pm);
-#pragma unroll
-        for (int off = TPR / 2; off >= 1; off >>= 1) row_max = fmaxf(row_max, __shfl_xor(row_max, off, TPR));
-        if (j == 0) absmax[row] = row_max;
-    }
-
-    // one step: 64 block columns of the 8 rows -> 2 KB of packed records
-    auto step = [&](int st, f16x8 t) {
-        const int kb = st * TPR + j;
-        float amax = row_max;
-        if (!by_row) {
-            amax = pk_absmax_value(pk_absmax8(quant_f16x2{(f16)0.f, (f16)0.f}, t));
-            for (int off = 1; off < lanes_blk; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, TPR));
-            if (kb < kb_total && (j & (lanes_blk - 1)) == 0) absmax[(size_t)row * nblk + (kb * 8) / bs] = amax;
-        }
-        uint32_t d = 0;
-        if (amax > 0.f) {  // (a block of zeros: every index 0)
-            const float y = refined_rcp(amax);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float nv = div_by_block_max((float)t[e], amax, y);
-                uint32_t best;
-                if constexpr (MODE == 0) best = nearest_bucketed(nv, tab_lane);
-                else if constexpr (MODE == 1) best = nearest_sorted(nv, c);
-                else best = nearest_any(nv, c);
-                d |= best << (8 * (e >> 1) + 4 * (1 - (e & 1)));  // byte e/2 of the dword; even column = high nibble
-            }
-        }
-        if constexpr (NP > 0) {
-            tile[st][j * 8 + r8] = d;  // (stored after the block row's last step)
-        } else {
-            uint32_t *tb = tile[st & 1];
-            tb[j * 8 + r8] = d;
-            __syncthreads();  // (the other buffer was read before the previous step's barrier)
-            if (tid < 2 * TPR) {
-                const int kb0 = st * TPR;
-                const int kbw = kb0 + (tid >> 1);  // block column of the 16 bytes this thread writes
-                if (kbw < kb_total)
-                    *reinterpret_cast<u32x4 *>(q32 + ((size_t)mb * kb_total + kb0) * 8 + tid * 4) = *reinterpret_cast<const u32x4 *>(tb + tid * 4);
-            }
+        for (int i = 0; i < 4; ++i) {
+            v[i] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            if (g * kQuadCols + i * 64 + j * 8 < k) v[i] = __builtin_nontemporal_load(reinterpret_cast<const f16x8 *>(src + i * 64));
         }
     };
-    if constexpr (NP > 0) {
-        // (fully unrolled: an array indexed by a loop counter would live in scratch memory)
+    // the first weights are on their way while the table is built
+    constexpr int NV = NQ > 0 ? NQ : 1;
+    f16x8 v[NV][4];
+    const int n_waves = (int)gridDim.x * WAVES;
+    int item = NQ == 0 ? (int)blockIdx.x * WAVES + wave : (int)blockIdx.x;  // quad, or block row
+    const int items = NQ == 0 ? rows8 * quads : rows8;
+    if constexpr (NQ == 0) {
+        if (item < items) load_quad(v[0], item / quads, item % quads);
+    } else if constexpr (NQ > 0) {
 #pragma unroll
-        for (int st = 0; st < NP; ++st)
-            if (st < n_steps) step(st, v[st]);  // (uniform: every thread of the workgroup takes the same steps)
-        __syncthreads();  // the block row's records are complete
-        // 16 bytes per thread and pass: the records of NP * 64 block columns, contiguous in the packed layout
-#pragma unroll
-        for (int p = tid; p < NP * 2 * TPR; p += 512) {
-            const int kbw = p >> 1;  // block column of the 16 bytes this thread writes
-            if (kbw < kb_total)
-                *reinterpret_cast<u32x4 *>(q32 + (size_t)mb * kb_total * 8 + (size_t)p * 4) =
-                    *reinterpret_cast<const u32x4 *>(&tile[0][0] + p * 4);
-        }
-        if constexpr (AHEAD) {
-#pragma unroll
-            for (int i = 0; i < NP; ++i) v[i] = vn[i];
-        }
-    } else {
-        for (int st = 0; st < n_steps; ++st) {
-            const int kb = st * TPR + j;
-            f16x8 t = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            if (kb < kb_total) t = *reinterpret_cast<const f16x8 *>(src + (size_t)kb * 8);
-            step(st, t);
+        for (int n = 0; n < NQ; ++n) load_quad(v[n], item, wave + n * WAVES);
+    }
+
+    // lane i of every wave: codebook entry i, the boundary above it
+    const float mine = code[lane & 15];
+    const float next = __shfl_down(mine, 1, 64);
+    auto lane_value = [](float x, int i) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), i)); };
+    // sorted, and every gap far above the rounding of a difference (|nv| <= 1, so a difference is
+    // at most 1 + max|c| and its rounding error below 2^-23 of that)
+    const float cmax = fmaxf(fabsf(lane_value(mine, 0)), fabsf(lane_value(mine, 15)));
+    const float thr = (1.0f + cmax) * 9.5367431640625e-7f;  // 2^-20
+    const bool fast = (__ballot(next - mine >= thr) & 0x7fffu) == 0x7fffu && cmax < 3.0e38f;
+    float bnd = 0.f;
+    bool tabled = false;
+    if (fast) {
+        if (lane < 15) bnd = decision_boundary(mine, next);
+        // the bucket table, if every boundary is finite and has a bucket of its own
+        const int bucket = (int)bucket_bits(bnd);
+        const int below = __shfl_up(bucket, 1, 64);
+        const bool ok = fabsf(bnd) < 3.0e38f && (lane == 0 || bucket > below);
+        tabled = (__ballot(ok) & 0x7fffu) == 0x7fffu;
+        // (outside [-1, 1] no quotient lies, and the patterns would wrap)
+        tabled = tabled && (__ballot(fabsf(bnd) <= 1.0f) & 0x7fffu) == 0x7fffu;
+        if (tabled) {
+            for (int e = wave; e < kQuantBuckets; e += WAVES) {
+                const uint64_t at = __ballot(bucket == (e << 9)) & 0x7fffu, under = __ballot(bucket < (e << 9)) & 0x7fffu;
+                const float b = at ? lane_value(bnd, __builtin_ctzll(at | 0x8000u)) : __builtin_inff();
+                const quant_u32x2 pair = {__builtin_bit_cast(uint32_t, b), (uint32_t)__builtin_popcountll(under)};
+                *reinterpret_cast<quant_u32x2 *>(qtab + (e << 9) + (lane << 3)) = pair;
+            }
         }
     }
-    __syncthreads();  // (the next block row writes the tile buffers this one's stores read)
-    }
+    __syncthreads();
+    const uint32_t tab_lane = (uint32_t)(uintptr_t)(lds_u8 *)qtab + ((uint32_t)lane << 3);
+
+    // The nearest-entry rule is a compile-time choice (the loops share nothing but their registers: the table path must
+    // not carry the 15 boundaries of the search).
+    auto run = [&](auto mode_tag) {
+        constexpr int MODE = decltype(mode_tag)::value;
+        float c[16];  // MODE 1: the boundaries; MODE 2: the codebook
+#pragma unroll
+        for (int i = 0; i < 16; ++i) c[i] = MODE == 1 ? lane_value(bnd, i) : MODE == 2 ? lane_value(mine, i) : 0.f;
+        auto pack_quad = [&](const f16x8 (&t)[4], const float (&am)[4], int mb, int g) {
+            uint32_t d[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                d[i] = quant_dword<MODE>(t[i], am[i], tab_lane, c);
+                __builtin_amdgcn_sched_barrier(0);  // (all four at once would not fit in the registers)
+            }
+            turn4(d);  // now rows 4 * (lane bit 3) + 0 .. 3 of block column 8 * (lane bits 5, 4) + j of the quad
+            const int kb = g * (kQuadCols / 8) + (lane >> 4) * 8 + j;
+            if (kb < kb_total)
+                *reinterpret_cast<u32x4 *>(q32 + ((size_t)mb * kb_total + kb) * 8 + ((lane >> 3) & 1) * 4) = u32x4{d[0], d[1], d[2], d[3]};
+        };
+        const quant_f16x2 zero2 = quant_f16x2{(f16)0.f, (f16)0.f};
+        if constexpr (NQ == 0) {
+            const int lanes_blk = bs >> 3;  // 16-byte groups that share a scale: 1, 2, 4 .. 32
+            const int nblk = k / bs;
+            for (; item < items; item += n_waves) {
+                const int mb = item / quads, g = item % quads;
+                f16x8 vn[4];
+                const int after = item + n_waves;
+                if (after < items) load_quad(vn, after / quads, after % quads);
+                float am[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) am[i] = pk_absmax_value(pk_absmax8(zero2, v[0][i]));
+                if (lanes_blk > 1) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) am[i] = dpp_max<kDppXor1>(am[i]);
+                }
+                if (lanes_blk > 2) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) am[i] = dpp_max<kDppXor2>(am[i]);
+                }
+                if (lanes_blk > 4) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) am[i] = dpp_max<kDppHalfMirror>(am[i]);
+                }
+                if (lanes_blk > 8) {
+                    am[0] = am[1] = fmaxf(am[0], am[1]);
+                    am[2] = am[3] = fmaxf(am[2], am[3]);
+                }
+                if (lanes_blk > 16) am[0] = am[1] = am[2] = am[3] = fmaxf(am[0], am[2]);
+                float *scales = absmax + (size_t)(mb * 8 + r8) * nblk;
+                if (lanes_blk == 8) {  // lane i of the row's eight stores the i-th of the four scales
+                    const float s = j & 2 ? (j & 1 ? am[3] : am[2]) : (j & 1 ? am[1] : am[0]);
+                    if (j < 4 && g * 4 + j < nblk) scales[g * 4 + j] = s;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int kb = g * (kQuadCols / 8) + i * 8 + j;
+                        if (kb < kb_total && (kb & (lanes_blk - 1)) == 0) scales[kb / lanes_blk] = am[i];
+                    }
+                }
+                pack_quad(v[0], am, mb, g);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[0][i] = vn[i];
+            }
+        } else {
+            constexpr bool AHEAD = NQ > 0 && NQ <= 2;  // registers for two block rows
+            int flip = 0;
+            for (; item < items; item += (int)gridDim.x) {
+                f16x8 vn[AHEAD ? NQ : 1][4];
+                if constexpr (AHEAD) {
+                    if (item + (int)gridDim.x < items) {
+#pragma unroll
+                        for (int n = 0; n < NQ; ++n) load_quad(vn[n], item + (int)gridDim.x, wave + n * WAVES);
+                    }
+                }
+                quant_f16x2 pm = zero2;
+                if constexpr (NQ < 0) {
+                    for (int g = wave; g < quads; g += WAVES) {
+                        load_quad(v[0], item, g);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) pm = pk_absmax8(pm, v[0][i]);
+                    }
+                }
+#pragma unroll
+                for (int n = 0; n < NQ; ++n)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) pm = pk_absmax8(pm, v[n][i]);
+                float row_max = dpp_max<kDppHalfMirror>(dpp_max<kDppXor2>(dpp_max<kDppXor1>(pk_absmax_value(pm))));
+                if (j == 0) wave_max[flip][wave][r8] = row_max;
+                __syncthreads();  // (two buffers: a wave writes one only after every wave passed the barrier in between)
+#pragma unroll
+                for (int o = 0; o < WAVES; ++o) row_max = fmaxf(row_max, wave_max[flip][o][r8]);
+                flip ^= 1;
+                if (wave == 0 && j == 0) absmax[item * 8 + r8] = row_max;
+                const float am[4] = {row_max, row_max, row_max, row_max};
+#pragma unroll
+                for (int n = 0; n < NQ; ++n) {
+                    if (wave + n * WAVES < quads) pack_quad(v[n], am, item, wave + n * WAVES);
+                    if constexpr (AHEAD) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[n][i] = vn[n][i];
+                    } else if (item + (int)gridDim.x < items) {
+                        load_quad(v[n], item + (int)gridDim.x, wave + n * WAVES);
+                    }
+                }
+                if constexpr (NQ < 0) {
+                    for (int g = wave; g < quads; g += WAVES) {
+                        load_quad(v[0], item, g);
+                        pack_quad(v[0], am, item, g);
+                    }
+                }
+            }
+        }
     };
     if (tabled) run(std::integral_constant<int, 0>{});
     else if (fast) run(std::integral_constant<int, 1>{});
@@ -445,18 +504,24 @@ hipError_t launch_quantize(const void *w, const float *code, void *q, float *abs
 {
     const f16 *wp = static_cast<const f16 *>(w);
     uint32_t *qp = static_cast<uint32_t *>(q);
-    // one workgroup per block row up to three per compute unit (what fits beside the bucket tables), which then
-    // walk the block rows: the tables are built once per workgroup
+    // as many workgroups as fit beside their tables and registers, which then walk the quads or block rows: the
+    // tables are built once per workgroup
     int dev = 0, cus = 0;
     hipError_t e = device_cus(&dev, &cus);
     if (e != hipSuccess) return e;
     const int rows8 = m / 8;
-    const dim3 grid((unsigned)(rows8 < 3 * cus ? rows8 : 3 * cus)), block(512);
-    const size_t lds = (size_t)kQuantTabBytes;
-    if (k <= 512 * 4) hipLaunchKernelGGL(quantize_kernel<4>, grid, block, lds, stream, wp, code, qp, absmax, m, k, bs);
-    else if (k <= 512 * 8) hipLaunchKernelGGL(quantize_kernel<8>, grid, block, lds, stream, wp, code, qp, absmax, m, k, bs);
-    else if (k <= 512 * 16) hipLaunchKernelGGL(quantize_kernel<16>, grid, block, lds, stream, wp, code, qp, absmax, m, k, bs);
-    else hipLaunchKernelGGL(quantize_kernel<0>, grid, block, lds, stream, wp, code, qp, absmax, m, k, bs);
+    const bool blocked = bs <= kQuadCols && (bs & (bs - 1)) == 0;
+    const int waves = blocked || k <= 8192 ? 8 : 16;
+    const int work = blocked ? (int)(((int64_t)rows8 * ((k + kQuadCols - 1) / kQuadCols) + waves - 1) / waves) : rows8;
+    const int per_cu = blocked || k <= 2048 ? 3 : k <= 8192 ? 2 : 1;
+    const dim3 grid((unsigned)(work < per_cu * cus ? work : per_cu * cus)), block((unsigned)waves * 64);
+    const size_t lds = (size_t)kQuantTabBytes + 2 * waves * 8 * sizeof(float);
+    if (blocked) hipLaunchKernelGGL((quantize_kernel<0, 8>), grid, block, lds, stream, wp, code, qp, absmax, m, k, bs);
+    else if (k <= 2048) hipLaunchKernelGGL((quantize_kernel<1, 8>), grid, block, lds, stream, wp, code, qp, absmax, m, k, bs);
+    else if (k <= 4096) hipLaunchKernelGGL((quantize_kernel<2, 8>), grid, block, lds, stream, wp, code, qp, absmax, m, k, bs);
+    else if (k <= 8192) hipLaunchKernelGGL((quantize_kernel<4, 8>), grid, block, lds, stream, wp, code, qp, absmax, m, k, bs);
+    else if (k <= 16384) hipLaunchKernelGGL((quantize_kernel<4, 16>), grid, block, lds, stream, wp, code, qp, absmax, m, k, bs);
+    else hipLaunchKernelGGL((quantize_kernel<-1, 16>), grid, block, lds, stream, wp, code, qp, absmax, m, k, bs);
     return hipGetLastError();
 }
 

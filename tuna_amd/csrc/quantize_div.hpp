@@ -3,6 +3,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
+
 namespace tuna {
 
 // fp32(w) / a, correctly rounded, for the quotients this kernel forms: w an fp16 value, a the
@@ -17,10 +19,29 @@ __device__ __forceinline__ float refined_rcp(float a)
     return __builtin_fmaf(__builtin_fmaf(-a, y, 1.0f), y, y);
 }
 
-__device__ __forceinline__ float div_by_block_max(float w, float a, float y)
+// (float)h * y and w - q * a with the fp16 operand read in place (no conversion instruction).
+template <int HI>
+__device__ __forceinline__ float mix_mul(uint32_t pair, float y)
 {
-    const float q = w * y;
-    return __builtin_fmaf(__builtin_fmaf(-q, a, w), y, q);
+    float q;
+    if constexpr (HI) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(q) : "v"(pair), "v"(y));
+    else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(q) : "v"(pair), "v"(y));
+    return q;
+}
+template <int HI>
+__device__ __forceinline__ float mix_residual(float q, float a, uint32_t pair)
+{
+    float r;
+    if constexpr (HI) asm("v_fma_mix_f32 %0, -%1, %2, %3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r) : "v"(q), "v"(a), "v"(pair));
+    else asm("v_fma_mix_f32 %0, -%1, %2, %3 op_sel:[0,0,0] op_sel_hi:[0,0,1]" : "=v"(r) : "v"(q), "v"(a), "v"(pair));
+    return r;
+}
+
+template <int HI>  // w = the low or high half of `pair`
+__device__ __forceinline__ float div_by_block_max(uint32_t pair, float a, float y)
+{
+    const float q = mix_mul<HI>(pair, y);
+    return __builtin_fmaf(mix_residual<HI>(q, a, pair), y, q);
 }
 
 }  // namespace tuna
