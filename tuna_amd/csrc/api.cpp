@@ -225,7 +225,7 @@ static int planned_cus()
 }
 
 static bool wide_balance_pays(int m, int n, int k);
-static bool stream_applies(const tuna_gemm_config &c, int n, int decode, int epilogue);
+static bool stream_applies(const tuna_gemm_config &c, int n, int decode);
 static bool plan_wide_dense(int m, int n, int k, int split, WidePlan *plan)
 {
     memset(plan, 0, sizeof(*plan));
@@ -988,7 +988,7 @@ static bool flow_instead(int m, int n, int k, const tuna_gemm_config &c, bool fr
         price = nt < 3 ? 0.0 : 14.3 + 0.62 * mb;
     } else {
         GemmPlan plan;
-        if (plan_gemm(m, n, k, c, TUNA_DECODE_GEMM, &plan) != TUNA_OK || launch_is_lean(plan, kMaxCus) || stream_applies(c, n, TUNA_DECODE_GEMM, TUNA_EPILOGUE_NONE))
+        if (plan_gemm(m, n, k, c, TUNA_DECODE_GEMM, &plan) != TUNA_OK || launch_is_lean(plan, kMaxCus) || stream_applies(c, n, TUNA_DECODE_GEMM))
             return false;
         const bool mid = mid_applies(plan);
         static const double kMid[5] = {0, 0, 0.30, 0.40, 0.37}, kGeneral[5] = {0, 0.29, 0.50, 0.55, 0.60};
@@ -1391,12 +1391,12 @@ static bool plan_multi(const tuna_gemm_problem *problems, int count, int cus, Mu
 }
 
 // A dense launch the batched kernel (gemm_multi.hpp) takes as a batch of one: balanced split, 64 rows
-// per wave, 16 waves, one token tile, the GEMM's own decode, no fused epilogue.  (plan_multi checks
-// the shape's alignment.)  A diagnostic build can turn it off together with the other twins (diag.h).
-static bool stream_applies(const tuna_gemm_config &c, int n, int decode, int epilogue)
+// per wave, 16 waves, one token tile, the GEMM's own decode, any epilogue (8192 x 28672 at 16 tokens with a
+// residual: 29 us, 47 in gemm_kernel).  (plan_multi checks the shape's alignment.)  A diagnostic build can turn it off together with the other twins (diag.h).
+static bool stream_applies(const tuna_gemm_config &c, int n, int decode)
 {
     return c.split_k == 0 && !c.lds_tile_rows && c.rows_per_wave == kRowsPerLoad && c.waves_m >= 1 && c.waves_m * c.waves_k == 16 &&
-           c.token_tiles == 1 && n <= 16 && decode == TUNA_DECODE_GEMM && epilogue == TUNA_EPILOGUE_NONE &&
+           c.token_tiles == 1 && n <= 16 && decode == TUNA_DECODE_GEMM &&
            (c.prefetch == 2 || c.prefetch == 4) && diag::lean_kernels() != 0;
 }
 
@@ -1457,7 +1457,7 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
     }
     GemmPlan plan;
     if ((rc = plan_gemm(m, n, k, c, decode, &plan))) return rc;
-    if (stream_applies(c, n, decode, epilogue)) {
+    if (stream_applies(c, n, decode)) {
         // a balanced split over 16-wave workgroups: the batched kernel with a batch of one walks the same
         // segments as gemm_kernel's balanced split and keeps its weight ring full across them
         int dev = 0, cus = 0;
@@ -1465,7 +1465,8 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
         if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
         const tuna_gemm_problem one = {q, x, code, absmax, out, m, n, k};
         MultiPlan mp;
-        if (plan_multi(&one, 1, cus, &mp, c.waves_m, c.prefetch)) {
+        const int32_t ep = epilogue;
+        if (plan_multi(&one, 1, cus, &mp, c.waves_m, c.prefetch, -1, &ep, &residual)) {
             if ((rc = provide_workspace(static_ws, stream, mp.ws_bytes, mp.n_counters, &mp.args.ws, &mp.args.counters))) return rc;
             e = launch_gemm_multi(mp.args, mp.prefetch, dev, stream);
             if (e != hipSuccess) return hip_fail(e, "gemm launch");
@@ -2618,7 +2619,7 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
     }
     GemmPlan plan;
     if ((rc = plan_gemm(m, n, k, c, decode_mode, &plan))) return rc;
-    if (stream_applies(c, n, decode_mode, TUNA_EPILOGUE_NONE)) {
+    if (stream_applies(c, n, decode_mode)) {
         const tuna_gemm_problem one = {buf, buf, buf, nullptr, buf, m, n, k};  // (only sizes and alignment are looked at)
         MultiPlan mp;
         if (plan_multi(&one, 1, kMaxCus, &mp, c.waves_m, c.prefetch)) {
