@@ -98,7 +98,9 @@ typedef struct tuna_gemm_config {
                               wave owns 64 x 256, or 128 x 128 with 32 x 32 MFMA tiles).  -4: the
                               decode-batch kernel - 256 rows x token_tiles (1 .. 4) x 16 tokens per
                               workgroup, the k-steps of all row tiles divided into split_k shares (1 ..
-                              512 workgroups); no other field is read */
+                              512 workgroups); no other field is read.  -5: the narrow-row
+                              kernel's variants for any m and k - rows_per_wave 16, 32 or 64 (waves_m 0)
+                              and the other fields as for that kernel */
 } tuna_gemm_config;
 
 int tuna_version(void);
@@ -275,8 +277,8 @@ int tuna_blockwise_table_entry(int i, int *m, int *n_lo, int *n_hi, int *k, int 
 /* Shape -> config.  Replaces the if-chain of kernel.cu:3018-3156 over the constants of
  * configs.cu:56-3331 by a table lookup on (m, n-bucket, k) with a derived fallback.
  * Runs on the host only (no device needed).  Returns 1 in *from_table when the shape
- * hit a tuned entry.  A call without a config runs it, except that the decode-batch kernel (up to
- * 64 tokens) or 256 x 256 tiles (from 65) take its place where they are predicted to be faster
+ * hit a tuned entry.  A call without a config runs it, except that the decode-batch kernel or the
+ * narrow-row kernel's variants for any k (up to 64 tokens) or 256 x 256 tiles (from 65) take its place where they are predicted to be faster
  * (tuna_describe_launch says so). */
 int tuna_select_config(int m, int n, int k, tuna_gemm_config *cfg, int *from_table);
 /* The config tuna_matmul_ex(cfg = NULL, decode_mode) runs: the table lookup above for

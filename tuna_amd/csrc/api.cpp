@@ -311,6 +311,7 @@ static int launch_tiled(TiledPlan &tp, const void *q, const void *x, const void 
 
 // lds_tile_rows -4: the decode-batch kernel (gemm_flow.hip), its k-steps divided into split_k shares
 static inline bool is_flow(const tuna_gemm_config &c) { return c.lds_tile_rows == -4; }
+static inline bool is_narrow_any(const tuna_gemm_config &c) { return c.lds_tile_rows == -5; }
 
 static int plan_flow(int m, int n, int k, const tuna_gemm_config &c, int decode, FlowPlan *plan)
 {
@@ -396,6 +397,35 @@ static int plan_narrow(int m, int n, int k, const tuna_gemm_config &c, int decod
     plan->args.k = k;
     plan->args.n_it = k / kStepK / c.waves_k;
     return TUNA_OK;
+}
+
+// The narrow-row kernel's variants for any m and k (lds_tile_rows -5; the other fields as for the narrow-row kernel).
+static int plan_narrow_any(int m, int n, int k, const tuna_gemm_config &c, int decode, NarrowPlan *plan)
+{
+    int rc = check_shape(m, n, k);
+    if (rc) return rc;
+    if (decode != TUNA_DECODE_GEMM) return fail(TUNA_ERR_UNSUPPORTED, "the narrow-row kernel implements TUNA_DECODE_GEMM only");
+    // (offsets beyond a buffer's end stay beyond it: both buffers end below 2^31 + a ring turn)
+    if ((unsigned long long)m * (unsigned long long)k / 2 >= (1ull << 31) || (unsigned long long)n * (unsigned long long)k * 2 >= (1ull << 31))
+        return fail(TUNA_ERR_UNSUPPORTED, "operands exceed the kernel's 32-bit offsets");
+    if (c.waves_m != (c.rows_per_wave == 64 ? 0 : 1) || c.split_k != 1 || c.k_stagger != 0 || c.x_chunk != kStepK * c.waves_k * c.prefetch ||
+        !narrow_any_variant_exists(c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles))
+        return fail(TUNA_ERR_UNSUPPORTED, "no narrow-row kernel for any k with rows_per_wave=%d waves_m=%d waves_k=%d prefetch=%d token_tiles=%d "
+                    "split_k=%d x_chunk=%d", c.rows_per_wave, c.waves_m, c.waves_k, c.prefetch, c.token_tiles, c.split_k, c.x_chunk);
+    if (ceil_div(n, 16 * c.token_tiles) > 65535) return fail(TUNA_ERR_UNSUPPORTED, "n=%d needs more than 65535 token chunks", n);
+    memset(plan, 0, sizeof(*plan));
+    plan->token_tiles = c.token_tiles, plan->rows = c.rows_per_wave, plan->waves_k = c.waves_k, plan->prefetch = c.prefetch;
+    plan->lds_bytes = (size_t)kLutBytes + (size_t)c.waves_k * (c.rows_per_wave / 16) * c.token_tiles * 1024;
+    if (plan->lds_bytes > (size_t)kLdsLimit) return fail(TUNA_ERR_UNSUPPORTED, "config needs %zu bytes of LDS, the CU has %d", plan->lds_bytes, kLdsLimit);
+    plan->args.m = m, plan->args.n = n, plan->args.k = k;
+    plan->args.n_it = ceil_div(k, kStepK * c.waves_k * c.prefetch) * c.prefetch;
+    return TUNA_OK;
+}
+
+static int describe_narrow_any(const NarrowPlan &p, int n, char *buf, size_t len, const char *then = "")
+{
+    return snprintf(buf, len, "gemm_narrow_kernel<LW=%d,WK=%d,U=%d,PERM=%d,TT=%d,any k>%s", p.rows / 16, p.waves_k, p.prefetch, n > 4,
+                    p.token_tiles, then);
 }
 
 // The streaming-kernel branch of the derivation: 64 rows per wave, rings of 2 k-steps (those
@@ -935,6 +965,10 @@ static bool config_runs(int m, int n, int k, const tuna_gemm_config &c)
         FlowPlan fp;
         return plan_flow(m, n, k, c, TUNA_DECODE_GEMM, &fp) == TUNA_OK;
     }
+    if (is_narrow_any(c)) {
+        NarrowPlan np;
+        return plan_narrow_any(m, n, k, c, TUNA_DECODE_GEMM, &np) == TUNA_OK;
+    }
     if (is_narrow(c)) {
         NarrowPlan np;
         return plan_narrow(m, n, k, c, TUNA_DECODE_GEMM, &np) == TUNA_OK;
@@ -978,7 +1012,7 @@ static int flow_best_shares(long long tiles, int units, int nt, double *us)
 // where that is predicted to be faster.  The selected kernels are priced by straight lines over the bytes of the weights,
 // read off the same random shapes; narrow-row, lean and batched launches, which win on the shapes they are picked for, are
 // left alone, and an entry of the table, timed for its shape, has to be beaten by a quarter.
-static bool flow_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, tuna_gemm_config *flow)
+static bool flow_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, tuna_gemm_config *flow, double *flow_us)
 {
     const double mb = 0.5e-6 * m * k;
     if (n > 64 || is_narrow(c) || mb < 8) return false;
@@ -1001,7 +1035,63 @@ static bool flow_instead(int m, int n, int k, const tuna_gemm_config &c, bool fr
     memset(flow, 0, sizeof(*flow));
     flow->rows_per_wave = 64, flow->waves_m = 4, flow->waves_k = 1, flow->prefetch = 4, flow->x_chunk = 64, flow->token_tiles = nt;
     flow->lds_tile_rows = -4, flow->split_k = shares;
+    *flow_us = us;
     return config_runs(m, n, k, *flow);
+}
+
+// Microseconds of a launch of the narrow-row kernel, by a model read off 350 random shapes of 0.5 ... 100 MB of weights at
+// 1 ... 64 tokens, each timed with up to 37 variants for any k (6.5 per cent off on average; the variants for whole ring
+// turns are a tenth faster): the busiest compute unit's work, a workgroup's chain of ring turns and the weights' stream -
+// whichever is longest, smoothly - and x, which every workgroup reads.
+static double narrow_time(int m, int n, int k, int rows, int waves_k, int u, int tt)
+{
+    const int lw = ceil_div(rows, 16), n_it = ceil_div(k, kStepK * waves_k * u) * u;
+    const double wgs = (double)ceil_div(m, rows) * ceil_div(n, 16 * tt);
+    const bool two = kLutBytes + waves_k * lw * tt * 1024 <= kLdsLimit / 2;  // workgroups on a compute unit
+    const double rounds = std::ceil(wgs / (two ? 2 * kMaxCus : kMaxCus));
+    const double work = std::ceil(wgs / kMaxCus) * n_it * waves_k * (7.5e-5 + 0.00291 * lw + 0.00252 * tt + 0.00691 * lw * tt);
+    const double chain = rounds * n_it / u * (0.423 + 0.0261 * u);
+    const double stream = 0.075 * 0.5e-6 * m * k;
+    const double x_bytes = wgs * k * (n < 16 * tt ? n : 16 * tt) * 2e-6;
+    return 1.73 + 1.07 * rounds + std::cbrt(work * work * work + chain * chain * chain + stream * stream * stream) + 0.0504 * x_bytes;
+}
+
+// Up to 64 tokens, ahead of the config `c` picked so far (`flow_us`: the decode-batch kernel's predicted time if that is
+// it): the narrow-row kernel's variants for any m and k, where their model is a tenth under that config's price - the
+// narrow-row kernel's own model, or a straight line in the megabytes read off the same shapes (general kernel, many-token
+// tiles).  1192 x 2000 at one token 9.1 -> 3.2 us, 4672 x 1720 14.8 -> 4.3, 8576 x 9856 at 5 tokens 30.5 -> 15.1, 1792 x
+// 4104 at 19 tokens 16.6 -> 6.1, 5824 x 4736 at 34 tokens 24.7 -> 15.0; 1.42 x on average over those shapes.  Streaming and lean
+// launches, and a table's entries that are narrow-row ones, are left alone.
+static bool narrow_any_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, double flow_us, tuna_gemm_config *any)
+{
+    if (n > 64) return false;
+    const double mb = 0.5e-6 * m * k;
+    const int nt = ceil_div(n, 16);
+    double price;
+    if (is_flow(c)) price = flow_us;
+    else if (is_narrow(c)) price = from_table ? 0.0 : 0.9 * narrow_time(m, n, k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles);
+    else if (c.lds_tile_rows > 0) price = nt < 3 ? 0.0 : 11.5 + 0.65 * mb;
+    else {
+        GemmPlan plan;
+        if (plan_gemm(m, n, k, c, TUNA_DECODE_GEMM, &plan) != TUNA_OK || launch_is_lean(plan, kMaxCus) || stream_applies(c, n, TUNA_DECODE_GEMM) ||
+            mid_applies(plan))
+            return false;
+        price = nt == 1 ? 9.4 + 0.286 * mb - 1.2e-4 * m : nt == 2 ? 12.6 + 0.40 * mb - 2e-4 * m : 7.0 + 1.5 * nt + (nt == 3 ? 0.55 : 0.60) * mb;
+    }
+    static const int kTry[11][4] = {{16, 16, 4, 1}, {16, 16, 2, 1}, {32, 8, 4, 1}, {32, 8, 8, 1}, {64, 4, 4, 1}, {64, 8, 4, 1},
+                                    {32, 8, 2, 2}, {32, 8, 4, 2}, {64, 8, 2, 2}, {32, 8, 2, 4}, {64, 4, 2, 4}};  // rows, waves, ring, token tiles
+    double best = (from_table ? 0.8 : 0.9) * price;
+    bool found = false;
+    for (const auto &t : kTry) {
+        if (t[3] > 1 && t[3] >= 2 * nt) continue;
+        const double us = narrow_time(m, n, k, t[0], t[1], t[2], t[3]);
+        if (us >= best) continue;
+        memset(any, 0, sizeof(*any));
+        any->rows_per_wave = t[0], any->waves_m = t[0] == 64 ? 0 : 1, any->waves_k = t[1], any->prefetch = t[2], any->split_k = 1;
+        any->x_chunk = kStepK * t[1] * t[2], any->token_tiles = t[3], any->lds_tile_rows = -5;
+        best = us, found = true;
+    }
+    return found && config_runs(m, n, k, *any);
 }
 
 // What a launch without an explicit config runs from 65 tokens on: the selected config, or 256 x 256 tiles of gemm_wide.hip
@@ -1100,7 +1190,10 @@ static void select_launch(int m, int n, int k, int decode, tuna_gemm_config *c)
     int from_table = 0;
     select_config_for(m, n, k, decode, c, &from_table);
     tuna_gemm_config other;
-    if (decode == TUNA_DECODE_GEMM && (wide_instead(m, n, k, *c, &other) || flow_instead(m, n, k, *c, from_table != 0, &other))) *c = other;
+    double flow_us = 0.0;
+    if (decode != TUNA_DECODE_GEMM) return;
+    if (wide_instead(m, n, k, *c, &other) || flow_instead(m, n, k, *c, from_table != 0, &other, &flow_us)) *c = other;
+    if (narrow_any_instead(m, n, k, *c, from_table != 0, flow_us, &other)) *c = other;
 }
 
 // The checks of the planner `c` belongs to, for a decode mode.
@@ -1113,6 +1206,10 @@ static int validate_for(int m, int n, int k, const tuna_gemm_config &c, int deco
     if (is_flow(c)) {
         FlowPlan fp;
         return plan_flow(m, n, k, c, decode, &fp);
+    }
+    if (is_narrow_any(c)) {
+        NarrowPlan np;
+        return plan_narrow_any(m, n, k, c, decode, &np);
     }
     if (is_narrow(c)) {
         NarrowPlan np;
@@ -1431,6 +1528,23 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
         FlowPlan fp;
         if ((rc = plan_flow(m, n, k, c, decode, &fp))) return rc;
         return launch_flow(fp, q, x, code, absmax, out, epilogue, residual, -1, static_ws, stream);
+    }
+    if (is_narrow_any(c)) {
+        NarrowPlan np;
+        if ((rc = plan_narrow_any(m, n, k, c, decode, &np))) return rc;
+        int dev = 0, cus = 0;
+        hipError_t e = device_cus(&dev, &cus);
+        if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
+        np.args.q = static_cast<const uint8_t *>(q);
+        np.args.x = x;
+        np.args.code = static_cast<const float *>(code);
+        np.args.absmax = static_cast<const float *>(absmax);
+        np.args.out = out;
+        np.args.epilogue = epilogue;
+        np.args.residual = residual;
+        e = launch_gemm_narrow_any(np.args, np.rows, np.waves_k, np.prefetch, np.token_tiles, dev, stream);
+        if (e != hipSuccess) return hip_fail(e, "narrow-row gemm launch");
+        return TUNA_OK;
     }
     // The narrow-row kernel reads a lane's scales 2 or 4 rows at a time.  A caller that names such a config must align
     // absmax for it; when the library picked the config itself it takes the streaming kernel's derived config for a
@@ -2440,6 +2554,14 @@ TUNA_EXPORT int tuna_config_footprint(int m, int n, int k, const tuna_gemm_confi
         if (workspace_bytes) *workspace_bytes = fp.ws_bytes;
         return TUNA_OK;
     }
+    if (is_narrow_any(*cfg)) {
+        NarrowPlan np;
+        int rc = plan_narrow_any(m, n, k, *cfg, TUNA_DECODE_GEMM, &np);
+        if (rc) return rc;
+        if (lds_bytes) *lds_bytes = np.lds_bytes;
+        if (workspace_bytes) *workspace_bytes = 0;
+        return TUNA_OK;
+    }
     if (is_narrow(*cfg)) {
         NarrowPlan np;
         int rc = plan_narrow(m, n, k, *cfg, TUNA_DECODE_GEMM, &np);
@@ -2592,8 +2714,11 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
     if (cfg) c = *cfg;
     else select_config_for(m, n, k, decode_mode, &c, nullptr);
     if (!cfg && (select_launch(m, n, k, decode_mode, &w), memcmp(&w, &c, sizeof(c)) != 0)) {
-        const int at = is_flow(w) ? snprintf(buf, len, "gemm_flow_kernel<NT=%d> %d shares in place of ", w.token_tiles, w.split_k)
-                                  : snprintf(buf, len, "gemm_wide_kernel<256 rows x 256 tokens> split_k=%d in place of ", w.split_k);
+        NarrowPlan np;
+        const int at = is_narrow_any(w) && plan_narrow_any(m, n, k, w, decode_mode, &np) == TUNA_OK
+                           ? describe_narrow_any(np, n, buf, len, " in place of ")
+                       : is_flow(w) ? snprintf(buf, len, "gemm_flow_kernel<NT=%d> %d shares in place of ", w.token_tiles, w.split_k)
+                                    : snprintf(buf, len, "gemm_wide_kernel<256 rows x 256 tokens> split_k=%d in place of ", w.split_k);
         return at < 0 || (size_t)at + 16 > len ? TUNA_OK : tuna_describe_launch(m, n, k, &c, decode_mode, buf + at, len - (size_t)at);
     }
     if (c.lds_tile_rows > 0) {
@@ -2609,6 +2734,12 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
         FlowPlan fp;
         if ((rc = plan_flow(m, n, k, c, decode_mode, &fp))) return rc;
         snprintf(buf, len, "gemm_flow_kernel<NT=%d> %d shares", fp.nt, fp.args.n_shares);
+        return TUNA_OK;
+    }
+    if (is_narrow_any(c)) {
+        NarrowPlan np;
+        if ((rc = plan_narrow_any(m, n, k, c, decode_mode, &np))) return rc;
+        describe_narrow_any(np, n, buf, len);
         return TUNA_OK;
     }
     if (is_narrow(c)) {

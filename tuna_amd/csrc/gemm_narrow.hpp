@@ -31,7 +31,11 @@
 //     there when a ring slot is refilled: a wave's scale load from global memory touches sixteen
 //     cache lines for sixteen values, as much address work as sixteen weight loads.  Without
 //     a_slds (slices that do not fit beside table and reduction planes) they come from memory.
-// Requires k % (32*WK*U) == 0, m % (16*LW) == 0, dense launches; a workgroup takes 16*TT tokens
+//   * ANY variants: any m and k (multiples of 8).  Weights and x come through buffers whose ends return zeros, a
+//     lane's group beyond k included; rows beyond m are computed and not stored.  The general
+//     kernel's staging, split and hand-over cost it 9 us before any work: 1192 x 2000 at one token 9.1 -> 3.2 us, 6264 x
+//     2944 10.6 -> 5.2, 8576 x 9856 at 5 tokens 30.5 -> 15.1, 1792 x 4104 at 19 tokens 16.6 -> 6.1.
+// Otherwise requires k % (32*WK*U) == 0, m % (16*LW) == 0, dense launches; a workgroup takes 16*TT tokens
 // (TT = token_tiles = 1, 2, 4: every decoded weight fragment feeds TT MFMAs), more tokens are
 // gridDim.y chunks.  Selected by rows_per_wave = 16 or 32 in the config,
 // or by rows_per_wave = 64 with waves_m = 0.
@@ -47,7 +51,7 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 // dwords of a kernel's arguments can be preloaded into scalar registers with the wave (built
 // with -amdgpu-kernarg-preload-count=16), which takes the argument fetch - a round trip to
 // memory - off the start of every wave.  A struct passed by value is not preloaded.
-template <int LW, int WK, int U, bool PERM, int TT, bool BLK = false, int ROWS = 16 * LW>
+template <int LW, int WK, int U, bool PERM, int TT, bool BLK = false, int ROWS = 16 * LW, bool ANY = false>
 __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q, const void *a_x, const float *a_code,
                                                               const float *a_absmax, int a_k, int a_n, int a_n_it, int a_m,
                                                               void *a_out, int a_epilogue, const void *a_residual,
@@ -64,6 +68,7 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
     } const a = {a_q, a_x, a_code, a_absmax, a_out, a_residual, a_epilogue, a_m, a_n, a_k, a_n_it};
     extern __shared__ __align__(16) unsigned char smem[];
     static_assert(LW == 1 || LW == 2 || LW == 4, "16, 32 or 64 rows per workgroup");
+    static_assert(!ANY || (!BLK && ROWS == 16 * LW), "ANY: per-row scales, full tiles");
     static_assert(ROWS % 8 == 0 && ROWS % LW == 0 && ROWS <= 16 * LW && ROWS > 8 * LW, "rows of a partly filled tile");
     unsigned char *lut = smem;
     float *red = reinterpret_cast<float *>(smem + kLutBytes);  // [wave][row plane][token tile][lane][4]
@@ -88,6 +93,9 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
     float sc32[LW] = {};
     if constexpr (BLK) {
         // (per block: loaded with the ring below)
+    } else if constexpr (ANY) {
+#pragma unroll
+        for (int j = 0; j < LW; ++j) sc32[j] = a.absmax[min(row0 + LW * ia + j, a.m - 1)];
     } else if constexpr (LW == 1) {
         sc32[0] = a.absmax[row0 + ia];
     } else if constexpr (LW == 2) {
@@ -133,6 +141,37 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
     const float *sp = a.absmax + (size_t)(row0 + LW * ia) * (size_t)(BLK ? a_nblk : 1);
     int dstep = wk;
     static_assert(U % 2 == 0, "whole double steps");
+    // ANY: buffers that end with q and with x's last token; a lane whose 8-k group lies beyond k asks for what lies
+    // beyond the buffer's end and gets zeros (no memory traffic)
+    constexpr uint32_t kBeyond = 0xfffffff0u;
+    __amdgpu_buffer_rsrc_t q_rsrc, x_rsrc;
+    int rem = a.k - wk * 64;  // k values from double step `dstep` on
+    if constexpr (ANY) {
+        q_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(a.q), 0, (int)((uint32_t)(a.m >> 3) * kb_total * 32u), 0x00020000);
+        x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char *>(reinterpret_cast<const unsigned char *>(a.x) + (size_t)tok0 * a.k * 2),
+                                                   0, (int)((uint32_t)(a.n - tok0) * (uint32_t)a.k * 2u), 0x00020000);
+    }
+    uint32_t q_at = lb + (uint32_t)wk * 256u, x_at = (uint32_t)wk * 128u;  // ANY: byte offsets of the turn being loaded
+    const int g8 = g * 8, xg8 = PERM ? (lane & 3) * 8 : g8;
+#define TUNA_NARROW_LOAD_ANY(u)                                                                 \
+    {                                                                                          \
+        const int rem_ = rem - ((u) >> 1) * (WK * 64) - ((u) & 1) * 32;                        \
+        const uint32_t qo_ = g8 < rem_ ? q_at + (uint32_t)(((u) >> 1) * (WK * 256) + ((u) & 1) * 128) : kBeyond; \
+        const uint32_t xo_ = x_at + (uint32_t)(((u) >> 1) * (WK * 128) + ((u) & 1) * 64);      \
+        const bool in_ = xg8 < rem_;                                                           \
+        _Pragma("unroll") for (int tt = 0; tt < TT; ++tt) xq[u][tt] = __builtin_bit_cast(u32x4, \
+            __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, (int)(in_ ? xo_ + xoff[tt] : kBeyond), 0, 0)); \
+        if constexpr (LW == 1) {                                                               \
+            wq[u][0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(q_rsrc, (int)qo_, 0, 2); \
+        } else if constexpr (LW == 2) {                                                        \
+            const u32x2 w2_ = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(q_rsrc, (int)qo_, 0, 2)); \
+            wq[u][0] = w2_[0];                                                                 \
+            wq[u][1] = w2_[1];                                                                 \
+        } else {                                                                               \
+            const u32x4 w4_ = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)qo_, 0, 2)); \
+            _Pragma("unroll") for (int j = 0; j < 4; ++j) wq[u][j] = w4_[j];                   \
+        }                                                                                      \
+    }
 #define TUNA_NARROW_LOAD(u)                                                                     \
     {                                                                                          \
         const size_t xo_ = (size_t)((u) >> 1) * (WK * 128) + ((u) & 1) * 64;               \
@@ -161,11 +200,25 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
             _Pragma("unroll") for (int j = 0; j < 4; ++j) wq[u][j] = w4_[j];                   \
         }                                                                                      \
     }
+#define TUNA_NARROW_REFILL(u)                                                                    \
+    {                                                                                          \
+        if constexpr (ANY) TUNA_NARROW_LOAD_ANY(u)                                             \
+        else TUNA_NARROW_LOAD(u)                                                               \
+    }
+    auto next_turn = [&] {
+        if constexpr (ANY) {
+            rem -= (U / 2) * (WK * 64);
+            q_at += (U / 2) * (WK * 256);
+            x_at += (U / 2) * (WK * 128);
+        } else {
+            qp += (size_t)(U / 2) * (WK * 256);
+            xp += (size_t)(U / 2) * (WK * 128);
+            dstep += (U / 2) * WK;
+        }
+    };
 #pragma unroll
-    for (int u = 0; u < U; ++u) TUNA_NARROW_LOAD(u)
-    qp += (size_t)(U / 2) * (WK * 256);
-    xp += (size_t)(U / 2) * (WK * 128);
-    dstep += (U / 2) * WK;
+    for (int u = 0; u < U; ++u) TUNA_NARROW_REFILL(u)
+    next_turn();
     // BLK, scales through LDS: the first eight scales per thread of the workgroup's slice are requested here and
     // stored behind the table build; longer slices follow in further rounds
     constexpr int SB = 8;
@@ -265,17 +318,17 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             TUNA_NARROW_CONSUME(u)
-            TUNA_NARROW_LOAD(u)
+            TUNA_NARROW_REFILL(u)
             __builtin_amdgcn_sched_barrier(0);  // keep each refill right behind its consume
         }
-        qp += (size_t)(U / 2) * (WK * 256);
-        xp += (size_t)(U / 2) * (WK * 128);
-        dstep += (U / 2) * WK;
+        next_turn();
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) TUNA_NARROW_CONSUME(u)
 #undef TUNA_NARROW_CONSUME
 #undef TUNA_NARROW_LOAD
+#undef TUNA_NARROW_LOAD_ANY
+#undef TUNA_NARROW_REFILL
 
     // ---- reduction over the waves and store -----------------------------------------------------
     // Plane (j, tt) of a wave: lane l, element v is token 16*tt + l % 16, MFMA row 4*(l/16) + v,
@@ -313,7 +366,7 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
             s1 += v1[w];
         }
         const int tok = tok0 + tt * 16 + tk;
-        if (tok >= a.n || (ROWS != 16 * LW && 2 * rp >= ROWS)) continue;
+        if (tok >= a.n || (ROWS != 16 * LW && 2 * rp >= ROWS) || (ANY && row0 + 2 * rp >= a.m)) continue;
         const int col = row0 + 2 * rp;
         if (a.epilogue == TUNA_EPILOGUE_SILU_MUL) {
             outp[(size_t)tok * (size_t)(a.m >> 1) + (col >> 1)] = (f16)silu_mul(s0, s1);
