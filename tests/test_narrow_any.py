@@ -43,3 +43,19 @@ def test_any_shape(m, n, k, rows, wk, u, tt, epilogue):
         p = plain.float()
         want = p + res.float() if epilogue == _lib.EPILOGUE_RESIDUAL else torch.nn.functional.silu(p[:, 0::2]) * p[:, 1::2]
         assert (fused.float() - want).abs().max() <= 4e-3 * want.abs().max() + 6e-8
+
+
+# a scale per block: in LDS and too many for it, double steps beyond the last block, one and two blocks a turn, ragged rows
+@pytest.mark.parametrize("m,n,k,block,rows,wk,u,tt", [(16, 1, 256, 64, 16, 16, 4, 1), (1008, 5, 1280, 64, 32, 8, 4, 1), (64, 16, 14592, 64, 64, 8, 4, 1),
+                                                      (1200, 2, 2304, 128, 64, 4, 4, 1), (272, 17, 4352, 128, 32, 8, 4, 2), (144, 30, 768, 256, 64, 8, 2, 2),
+                                                      (80, 64, 1536, 64, 64, 4, 2, 4), (48, 40, 22784, 64, 16, 16, 2, 1)])
+def test_scale_blocks(m, n, k, block, rows, wk, u, tt):
+    import torch
+
+    from tuna_amd import ops
+
+    q, s, x, code = _inputs(m, n, k, seed=k + n, block=block)
+    out = _out(n, m)
+    ops.matmul_blockwise(x, q, s, code, out, m, n, k, block, config=_cfg(rows, wk, u, tt))
+    torch.cuda.synchronize()
+    _check(out, q, s, x, code, k, block=block)

@@ -422,6 +422,23 @@ static int plan_narrow_any(int m, int n, int k, const tuna_gemm_config &c, int d
     return TUNA_OK;
 }
 
+static int launch_narrow_any(NarrowPlan &np, const void *q, const void *x, const void *code, const void *absmax, void *out, int epilogue,
+                             const void *residual, int blk_shift, hipStream_t stream)
+{
+    int dev = 0, cus = 0;
+    hipError_t e = device_cus(&dev, &cus);
+    if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
+    np.args.q = static_cast<const uint8_t *>(q);
+    np.args.x = x;
+    np.args.code = static_cast<const float *>(code);
+    np.args.absmax = static_cast<const float *>(absmax);
+    np.args.out = out;
+    np.args.epilogue = epilogue;
+    np.args.residual = residual;
+    e = launch_gemm_narrow_any(np.args, blk_shift, np.rows, np.waves_k, np.prefetch, np.token_tiles, dev, stream);
+    return e == hipSuccess ? TUNA_OK : hip_fail(e, "narrow-row gemm launch");
+}
+
 static int describe_narrow_any(const NarrowPlan &p, int n, char *buf, size_t len, const char *then = "")
 {
     return snprintf(buf, len, "gemm_narrow_kernel<LW=%d,WK=%d,U=%d,PERM=%d,TT=%d,any k>%s", p.rows / 16, p.waves_k, p.prefetch, n > 4,
@@ -1043,17 +1060,45 @@ static bool flow_instead(int m, int n, int k, const tuna_gemm_config &c, bool fr
 // 1 ... 64 tokens, each timed with up to 37 variants for any k (6.5 per cent off on average; the variants for whole ring
 // turns are a tenth faster): the busiest compute unit's work, a workgroup's chain of ring turns and the weights' stream -
 // whichever is longest, smoothly - and x, which every workgroup reads.
-static double narrow_time(int m, int n, int k, int rows, int waves_k, int u, int tt)
+// nblk > 0: that many scales per row, kept in LDS where they fit (280 shapes with blocks of 64 and 128, 7 per cent).
+static double narrow_time(int m, int n, int k, int rows, int waves_k, int u, int tt, int nblk = 0)
 {
+    struct Coef { double launch, round, step, rows, tokens, both, turn, ring, stream, x, scale_loads, scale_kb; };
+    static const Coef kPerRow = {1.73, 1.07, 7.5e-5, 0.00291, 0.00252, 0.00691, 0.423, 0.0261, 0.0750, 0.0504, 0.0, 0.0},
+                      kBlocks = {1.98, 2.14, 3.0e-5, 0.00218, 0.00054, 0.00767, 0.0814, 0.190, 0.0355, 0.0461, 0.0220, 0.0642};
+    const Coef &c = nblk ? kBlocks : kPerRow;
     const int lw = ceil_div(rows, 16), n_it = ceil_div(k, kStepK * waves_k * u) * u;
     const double wgs = (double)ceil_div(m, rows) * ceil_div(n, 16 * tt);
-    const bool two = kLutBytes + waves_k * lw * tt * 1024 <= kLdsLimit / 2;  // workgroups on a compute unit
-    const double rounds = std::ceil(wgs / (two ? 2 * kMaxCus : kMaxCus));
-    const double work = std::ceil(wgs / kMaxCus) * n_it * waves_k * (7.5e-5 + 0.00291 * lw + 0.00252 * tt + 0.00691 * lw * tt);
-    const double chain = rounds * n_it / u * (0.423 + 0.0261 * u);
-    const double stream = 0.075 * 0.5e-6 * m * k;
+    int lds = kLutBytes + waves_k * lw * tt * 1024;
+    const int scales = nblk ? rows * (nblk + 1) * 4 : 0;
+    const bool in_lds = lds + scales <= kLdsLimit;
+    if (in_lds) lds += scales;
+    const double rounds = std::ceil(wgs / (lds <= kLdsLimit / 2 ? 2 * kMaxCus : kMaxCus));  // two workgroups on a compute unit
+    const double work = std::ceil(wgs / kMaxCus) * n_it * waves_k * (c.step + c.rows * lw + c.tokens * tt + c.both * lw * tt + (in_lds ? 0.0 : c.scale_loads * lw));
+    const double chain = rounds * n_it / u * (c.turn + c.ring * u);
+    const double stream = c.stream * 0.5e-6 * m * k;
     const double x_bytes = wgs * k * (n < 16 * tt ? n : 16 * tt) * 2e-6;
-    return 1.73 + 1.07 * rounds + std::cbrt(work * work * work + chain * chain * chain + stream * stream * stream) + 0.0504 * x_bytes;
+    return c.launch + (c.round + (in_lds ? c.scale_kb * 1e-3 * scales : 0.0)) * rounds +
+           std::cbrt(work * work * work + chain * chain * chain + stream * stream * stream) + c.x * x_bytes;
+}
+
+// The variant for any m and k with the least predicted time below `limit` us.
+static bool best_narrow_any(int m, int n, int k, int nblk, double limit, tuna_gemm_config *any)
+{
+    static const int kTry[11][4] = {{16, 16, 4, 1}, {16, 16, 2, 1}, {32, 8, 4, 1}, {32, 8, 8, 1}, {64, 4, 4, 1}, {64, 8, 4, 1},
+                                    {32, 8, 2, 2}, {32, 8, 4, 2}, {64, 8, 2, 2}, {32, 8, 2, 4}, {64, 4, 2, 4}};  // rows, waves, ring, token tiles
+    const int nt = ceil_div(n, 16);
+    bool found = false;
+    for (const auto &t : kTry) {
+        if (t[3] > 1 && t[3] >= 2 * nt) continue;
+        const double us = narrow_time(m, n, k, t[0], t[1], t[2], t[3], nblk);
+        if (us >= limit) continue;
+        memset(any, 0, sizeof(*any));
+        any->rows_per_wave = t[0], any->waves_m = t[0] == 64 ? 0 : 1, any->waves_k = t[1], any->prefetch = t[2], any->split_k = 1;
+        any->x_chunk = kStepK * t[1] * t[2], any->token_tiles = t[3], any->lds_tile_rows = -5;
+        limit = us, found = true;
+    }
+    return found;
 }
 
 // Up to 64 tokens, ahead of the config `c` picked so far (`flow_us`: the decode-batch kernel's predicted time if that is
@@ -1078,20 +1123,7 @@ static bool narrow_any_instead(int m, int n, int k, const tuna_gemm_config &c, b
             return false;
         price = nt == 1 ? 9.4 + 0.286 * mb - 1.2e-4 * m : nt == 2 ? 12.6 + 0.40 * mb - 2e-4 * m : 7.0 + 1.5 * nt + (nt == 3 ? 0.55 : 0.60) * mb;
     }
-    static const int kTry[11][4] = {{16, 16, 4, 1}, {16, 16, 2, 1}, {32, 8, 4, 1}, {32, 8, 8, 1}, {64, 4, 4, 1}, {64, 8, 4, 1},
-                                    {32, 8, 2, 2}, {32, 8, 4, 2}, {64, 8, 2, 2}, {32, 8, 2, 4}, {64, 4, 2, 4}};  // rows, waves, ring, token tiles
-    double best = (from_table ? 0.8 : 0.9) * price;
-    bool found = false;
-    for (const auto &t : kTry) {
-        if (t[3] > 1 && t[3] >= 2 * nt) continue;
-        const double us = narrow_time(m, n, k, t[0], t[1], t[2], t[3]);
-        if (us >= best) continue;
-        memset(any, 0, sizeof(*any));
-        any->rows_per_wave = t[0], any->waves_m = t[0] == 64 ? 0 : 1, any->waves_k = t[1], any->prefetch = t[2], any->split_k = 1;
-        any->x_chunk = kStepK * t[1] * t[2], any->token_tiles = t[3], any->lds_tile_rows = -5;
-        best = us, found = true;
-    }
-    return found && config_runs(m, n, k, *any);
+    return best_narrow_any(m, n, k, 0, (from_table ? 0.8 : 0.9) * price, any) && config_runs(m, n, k, *any);
 }
 
 // What a launch without an explicit config runs from 65 tokens on: the selected config, or 256 x 256 tiles of gemm_wide.hip
@@ -1532,19 +1564,7 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
     if (is_narrow_any(c)) {
         NarrowPlan np;
         if ((rc = plan_narrow_any(m, n, k, c, decode, &np))) return rc;
-        int dev = 0, cus = 0;
-        hipError_t e = device_cus(&dev, &cus);
-        if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
-        np.args.q = static_cast<const uint8_t *>(q);
-        np.args.x = x;
-        np.args.code = static_cast<const float *>(code);
-        np.args.absmax = static_cast<const float *>(absmax);
-        np.args.out = out;
-        np.args.epilogue = epilogue;
-        np.args.residual = residual;
-        e = launch_gemm_narrow_any(np.args, np.rows, np.waves_k, np.prefetch, np.token_tiles, dev, stream);
-        if (e != hipSuccess) return hip_fail(e, "narrow-row gemm launch");
-        return TUNA_OK;
+        return launch_narrow_any(np, q, x, code, absmax, out, epilogue, residual, -1, stream);
     }
     // The narrow-row kernel reads a lane's scales 2 or 4 rows at a time.  A caller that names such a config must align
     // absmax for it; when the library picked the config itself it takes the streaming kernel's derived config for a
@@ -2075,12 +2095,13 @@ TUNA_EXPORT int tuna_quantize_blockwise(const void *w, const void *code, void *q
 // A config comes from the caller (tuna_matmul_blockwise_ex), from the table of tuned entries keyed by (m, token bucket,
 // k, block_size) (config_table.cpp, written by the tuner), or from the rules of derive_blockwise below.
 // ---------------------------------------------------------------------------------------
-enum BlockwiseFamily { kBlkNarrow = 0, kBlkMulti = 1, kBlkTiled = 2, kBlkMid = 3, kBlkFlow = 4 };
+enum BlockwiseFamily { kBlkNarrow = 0, kBlkMulti = 1, kBlkTiled = 2, kBlkMid = 3, kBlkFlow = 4, kBlkNarrowAny = 5 };
 
 static BlockwiseFamily blockwise_family(const tuna_gemm_config &c)
 {
     if (c.lds_tile_rows > 0) return kBlkTiled;
     if (is_flow(c)) return kBlkFlow;
+    if (is_narrow_any(c)) return kBlkNarrowAny;
     if (is_narrow(c)) return kBlkNarrow;
     if (c.split_k == 0) return kBlkMulti;
     return kBlkMid;
@@ -2170,6 +2191,11 @@ static int run_blockwise(const BlockwiseCall &b, const tuna_gemm_config &c, hipS
         FlowPlan fp;
         if ((rc = plan_flow(m, n, k, c, TUNA_DECODE_GEMM, &fp))) return rc;
         return dry ? TUNA_OK : launch_flow(fp, b.q, b.x, b.code, b.absmax, b.out, TUNA_EPILOGUE_NONE, nullptr, shift, false, st);
+    }
+    case kBlkNarrowAny: {
+        NarrowPlan np;
+        if ((rc = plan_narrow_any(m, n, k, c, TUNA_DECODE_GEMM, &np))) return rc;
+        return dry ? TUNA_OK : launch_narrow_any(np, b.q, b.x, b.code, b.absmax, b.out, TUNA_EPILOGUE_NONE, nullptr, shift, st);
     }
     case kBlkMid: {
         tuna_gemm_config t = c;
@@ -2417,6 +2443,24 @@ static int check_blockwise_call(const BlockwiseCall &b, bool pointers)
     return TUNA_OK;
 }
 
+// What a call without a config runs: the selected config, or up to 64 tokens the narrow-row kernel's variants for any k in
+// its place where their model is an eighth under the selected config's price - that model for a narrow-row pick, a straight
+// line for many-token tiles (9984 x 7936 at 2 tokens, which no ring turn of more than four waves divides, 38.8 -> 13 us;
+// 2048 x 8960 at 7 tokens 18.9 -> 9.9, 13120 x 23296 at 9 tokens 197 -> 54; 1.30 x on average over 280 random shapes).
+static int select_blockwise_launch(const BlockwiseCall &b, tuna_gemm_config *c)
+{
+    int from_table = 0;
+    const int rc = select_blockwise(b, c, &from_table);
+    if (rc || from_table || b.n > 64) return rc;
+    const int nblk = b.k / b.block_size;
+    double price = 0.0;
+    if (is_narrow(*c)) price = narrow_time(b.m, b.n, b.k, c->rows_per_wave, c->waves_k, c->prefetch, c->token_tiles, nblk);
+    else if (blockwise_family(*c) == kBlkTiled) price = 11.0 + 0.55 * 0.5e-6 * b.m * b.k;
+    tuna_gemm_config any;
+    if (best_narrow_any(b.m, b.n, b.k, nblk, 0.88 * price, &any) && run_blockwise(b, any, nullptr, true) == TUNA_OK) *c = any;
+    return TUNA_OK;
+}
+
 TUNA_EXPORT int tuna_matmul_blockwise_ex(const void *q, const void *x, const void *code, const void *absmax, void *out, int m, int n,
                                          int k, int block_size, const tuna_gemm_config *cfg, void *stream)
 {
@@ -2426,7 +2470,7 @@ TUNA_EXPORT int tuna_matmul_blockwise_ex(const void *q, const void *x, const voi
     if ((rc = check_blockwise_call(b, true))) return rc;
     tuna_gemm_config c;
     if (cfg) c = *cfg;
-    else if ((rc = select_blockwise(b, &c, nullptr))) return rc;
+    else if ((rc = select_blockwise_launch(b, &c))) return rc;
     return run_blockwise(b, c, static_cast<hipStream_t>(stream), false);
 }
 

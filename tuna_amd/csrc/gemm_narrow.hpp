@@ -68,7 +68,7 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
     } const a = {a_q, a_x, a_code, a_absmax, a_out, a_residual, a_epilogue, a_m, a_n, a_k, a_n_it};
     extern __shared__ __align__(16) unsigned char smem[];
     static_assert(LW == 1 || LW == 2 || LW == 4, "16, 32 or 64 rows per workgroup");
-    static_assert(!ANY || (!BLK && ROWS == 16 * LW), "ANY: per-row scales, full tiles");
+    static_assert(!ANY || ROWS == 16 * LW, "ANY: full tiles");
     static_assert(ROWS % 8 == 0 && ROWS % LW == 0 && ROWS <= 16 * LW && ROWS > 8 * LW, "rows of a partly filled tile");
     unsigned char *lut = smem;
     float *red = reinterpret_cast<float *>(smem + kLutBytes);  // [wave][row plane][token tile][lane][4]
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
         return h_ | (h_ << 16);
     };
     // BLK: lane's first scale, and the double step of ring slot 0 in the turn being loaded
-    const float *sp = a.absmax + (size_t)(row0 + LW * ia) * (size_t)(BLK ? a_nblk : 1);
+    const float *sp = a.absmax + (size_t)(ANY ? min(row0 + LW * ia, a.m - LW) : row0 + LW * ia) * (size_t)(BLK ? a_nblk : 1);
     int dstep = wk;
     static_assert(U % 2 == 0, "whole double steps");
     // ANY: buffers that end with q and with x's last token; a lane whose 8-k group lies beyond k asks for what lies
@@ -159,6 +159,7 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
         const uint32_t qo_ = g8 < rem_ ? q_at + (uint32_t)(((u) >> 1) * (WK * 256) + ((u) & 1) * 128) : kBeyond; \
         const uint32_t xo_ = x_at + (uint32_t)(((u) >> 1) * (WK * 128) + ((u) & 1) * 64);      \
         const bool in_ = xg8 < rem_;                                                           \
+        TUNA_NARROW_SCALES(u)                                                                  \
         _Pragma("unroll") for (int tt = 0; tt < TT; ++tt) xq[u][tt] = __builtin_bit_cast(u32x4, \
             __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, (int)(in_ ? xo_ + xoff[tt] : kBeyond), 0, 0)); \
         if constexpr (LW == 1) {                                                               \
@@ -172,12 +173,13 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
             _Pragma("unroll") for (int j = 0; j < 4; ++j) wq[u][j] = w4_[j];                   \
         }                                                                                      \
     }
-#define TUNA_NARROW_LOAD(u)                                                                     \
-    {                                                                                          \
-        const size_t xo_ = (size_t)((u) >> 1) * (WK * 128) + ((u) & 1) * 64;               \
-        const size_t qo_ = (size_t)((u) >> 1) * (WK * 256) + ((u) & 1) * 128;              \
+    const auto block_of = [&](int dstep_) {  // (ANY: double steps beyond k read the last block's scale against zeros of x)
+        const int blk_ = dstep_ >> a_blk_shift;
+        return ANY ? min(blk_, a_nblk - 1) : blk_;
+    };
+#define TUNA_NARROW_SCALES(u)                                                                   \
         if constexpr (BLK) {                                                                   \
-            const int blk_ = (dstep + ((u) >> 1) * WK) >> a_blk_shift;                         \
+            const int blk_ = block_of(dstep + ((u) >> 1) * WK);                                \
             if (a_slds) {                                                                      \
                 /* (the two slots of a double step lie in one block: the second copies the first) */ \
                 if (dstep != wk) {                                                             \
@@ -187,7 +189,12 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
             } else {                                                                           \
                 _Pragma("unroll") for (int j = 0; j < LW; ++j) sq[u][j] = pack_scale(sp[(size_t)j * a_nblk + blk_]); \
             }                                                                                  \
-        }                                                                                      \
+        }
+#define TUNA_NARROW_LOAD(u)                                                                     \
+    {                                                                                          \
+        const size_t xo_ = (size_t)((u) >> 1) * (WK * 128) + ((u) & 1) * 64;               \
+        const size_t qo_ = (size_t)((u) >> 1) * (WK * 256) + ((u) & 1) * 128;              \
+        TUNA_NARROW_SCALES(u)                                                                  \
         _Pragma("unroll") for (int tt = 0; tt < TT; ++tt) xq[u][tt] = *reinterpret_cast<const u32x4 *>(xp + xo_ + xoff[tt]); \
         if constexpr (LW == 1) {                                                               \
             wq[u][0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(qp + qo_ + lb)); \
@@ -210,6 +217,7 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
             rem -= (U / 2) * (WK * 64);
             q_at += (U / 2) * (WK * 256);
             x_at += (U / 2) * (WK * 128);
+            dstep += (U / 2) * WK;
         } else {
             qp += (size_t)(U / 2) * (WK * 256);
             xp += (size_t)(U / 2) * (WK * 128);
@@ -223,7 +231,7 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
     // stored behind the table build; longer slices follow in further rounds
     constexpr int SB = 8;
     float sv[BLK ? SB : 1];
-    const int s_count = BLK ? ROWS * a_nblk : 0;
+    const int s_count = BLK ? (ANY ? min(ROWS, a.m - row0) : ROWS) * a_nblk : 0;
     const float *s_src = a.absmax + (size_t)row0 * (size_t)(BLK ? a_nblk : 1);
     if constexpr (BLK) {
         if (a_slds) {
@@ -281,7 +289,7 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
             const uint32_t *sl = sbuf + LW * ia * (a_nblk + 1);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int blk_ = (wk + (u >> 1) * WK) >> a_blk_shift;
+                const int blk_ = block_of(wk + (u >> 1) * WK);
 #pragma unroll
                 for (int j = 0; j < LW; ++j) sq[u][j] = sl[j * (a_nblk + 1) + blk_];
             }
@@ -329,6 +337,7 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
 #undef TUNA_NARROW_LOAD
 #undef TUNA_NARROW_LOAD_ANY
 #undef TUNA_NARROW_REFILL
+#undef TUNA_NARROW_SCALES
 
     // ---- reduction over the waves and store -----------------------------------------------------
     // Plane (j, tt) of a wave: lane l, element v is token 16*tt + l % 16, MFMA row 4*(l/16) + v,

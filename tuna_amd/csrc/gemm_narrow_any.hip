@@ -5,19 +5,22 @@ namespace tuna {
 
 typedef void (*NarrowKernelFn)(const uint8_t *, const void *, const float *, const float *, int, int, int, int, void *, int,
                                const void *, int, int, int);
-#define ANY1(LW, WK, U) {16 * LW, WK, U, 1, {gemm_narrow_kernel<LW, WK, U, false, 1, false, 16 * LW, true>, gemm_narrow_kernel<LW, WK, U, true, 1, false, 16 * LW, true>}}
-#define ANYT(LW, WK, U, TT) {16 * LW, WK, U, TT, {gemm_narrow_kernel<LW, WK, U, true, TT, false, 16 * LW, true>, gemm_narrow_kernel<LW, WK, U, true, TT, false, 16 * LW, true>}}
+// (fn[2], fn[3]: with a scale per block of a row)
+#define BLKV(LW, WK, U, TT, P) gemm_narrow_kernel<LW, WK, U, P, TT, true, 16 * LW, true>
+#define ANY1(LW, WK, U) {16 * LW, WK, U, 1, {gemm_narrow_kernel<LW, WK, U, false, 1, false, 16 * LW, true>, gemm_narrow_kernel<LW, WK, U, true, 1, false, 16 * LW, true>, BLKV(LW, WK, U, 1, false), BLKV(LW, WK, U, 1, true)}}
+#define ANYT(LW, WK, U, TT) {16 * LW, WK, U, TT, {gemm_narrow_kernel<LW, WK, U, true, TT, false, 16 * LW, true>, gemm_narrow_kernel<LW, WK, U, true, TT, false, 16 * LW, true>, BLKV(LW, WK, U, TT, true), BLKV(LW, WK, U, TT, true)}}
 static const struct {
     int rows, wk, u, tt;
-    NarrowKernelFn fn[2];  // B fragments loaded per lane (up to 4 tokens) / contiguously and permuted
+    NarrowKernelFn fn[4];  // B fragments loaded per lane (up to 4 tokens) / contiguously and permuted
 } kAny[] = {
     ANY1(1, 16, 4), ANY1(1, 16, 2), ANY1(2, 8, 4), ANY1(2, 8, 8), ANY1(4, 4, 4), ANY1(4, 8, 4),
     ANYT(2, 8, 2, 2), ANYT(2, 8, 4, 2), ANYT(4, 8, 2, 2), ANYT(2, 8, 2, 4), ANYT(4, 4, 2, 4),
 };
 #undef ANY1
 #undef ANYT
+#undef BLKV
 static constexpr int kNumAny = sizeof(kAny) / sizeof(kAny[0]);
-static OptInFlag g_any_attr_done[16][kNumAny][2];
+static OptInFlag g_any_attr_done[16][kNumAny][4];
 
 static int find_any(int rows, int wk, int u, int tt)
 {
@@ -31,17 +34,23 @@ bool narrow_any_variant_exists(int rows, int waves_k, int prefetch, int token_ti
     return find_any(rows, waves_k, prefetch, token_tiles) >= 0;
 }
 
-hipError_t launch_gemm_narrow_any(const NarrowArgs &args, int rows, int waves_k, int prefetch, int token_tiles, int dev, hipStream_t stream)
+// blk_shift >= 0: a scale per 64 << blk_shift weights of a row; the workgroup's scales are kept in LDS where they fit.
+hipError_t launch_gemm_narrow_any(const NarrowArgs &args, int blk_shift, int rows, int waves_k, int prefetch, int token_tiles, int dev,
+                                  hipStream_t stream)
 {
-    const int vi = find_any(rows, waves_k, prefetch, token_tiles), perm = args.n > 4;
+    const int vi = find_any(rows, waves_k, prefetch, token_tiles), fi = (args.n > 4 ? 1 : 0) + (blk_shift >= 0 ? 2 : 0);
     if (vi < 0 || dev < 0 || dev >= 16) return hipErrorInvalidConfiguration;
-    const NarrowKernelFn fn = kAny[vi].fn[perm];
-    const hipError_t e = ensure_lds_opt_in(g_any_attr_done[dev][vi][perm], reinterpret_cast<const void *>(fn));
+    const NarrowKernelFn fn = kAny[vi].fn[fi];
+    const hipError_t e = ensure_lds_opt_in(g_any_attr_done[dev][vi][fi], reinterpret_cast<const void *>(fn));
     if (e != hipSuccess) return e;
-    const size_t lds = (size_t)kLutBytes + (size_t)waves_k * (rows / 16) * token_tiles * 1024;
+    size_t lds = (size_t)kLutBytes + (size_t)waves_k * (rows / 16) * token_tiles * 1024;
+    const int nblk = blk_shift >= 0 ? args.k >> (6 + blk_shift) : 1;
+    const size_t scale_bytes = (size_t)rows * (nblk + 1) * 4;
+    const int slds = blk_shift >= 0 && lds + scale_bytes <= (size_t)kLdsLimit;
+    if (slds) lds += scale_bytes;
     const dim3 grid((unsigned)((args.m + rows - 1) / rows), (unsigned)((args.n + 16 * token_tiles - 1) / (16 * token_tiles)), 1);
     hipLaunchKernelGGL(fn, grid, dim3(waves_k * 64), lds, stream, args.q, args.x, args.code, args.absmax, args.k, args.n, args.n_it,
-                       args.m, args.out, args.epilogue, args.residual, 0, 1, 0);
+                       args.m, args.out, args.epilogue, args.residual, blk_shift >= 0 ? blk_shift : 0, nblk, slds);
     return hipGetLastError();
 }
 

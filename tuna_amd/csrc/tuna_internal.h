@@ -251,7 +251,8 @@ bool narrow_variant_exists(int rows, int waves_k, int prefetch, int token_tiles)
 hipError_t launch_gemm_narrow(const NarrowArgs &args, int rows, int waves_k, int prefetch, int token_tiles, hipStream_t stream);
 // its variants for any m and k (multiples of 8); n_it: k-steps per wave in whole ring turns
 bool narrow_any_variant_exists(int rows, int waves_k, int prefetch, int token_tiles);
-hipError_t launch_gemm_narrow_any(const NarrowArgs &args, int rows, int waves_k, int prefetch, int token_tiles, int dev, hipStream_t stream);
+hipError_t launch_gemm_narrow_any(const NarrowArgs &args, int blk_shift, int rows, int waves_k, int prefetch, int token_tiles, int dev,
+                                  hipStream_t stream);
 // the narrow-row kernel's scale-block variants (a scale per 64 << blk_shift weights of a row)
 hipError_t launch_gemm_blockwise(const NarrowArgs &args, int blk_shift, int rows, int waves_k, int prefetch, int token_tiles,
                                  hipStream_t stream);
