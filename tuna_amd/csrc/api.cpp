@@ -1147,7 +1147,8 @@ static bool wide_instead(int m, int n, int k, const tuna_gemm_config &c, tuna_ge
                 price = kGridCostUs * k * grid_cost(cd, c.split_k, (long long)ceil_div(m, rows) * ceil_div(n, tokens) * c.split_k, k);
     }
     const int split = price == 0.0 ? 0 : wide_best_split(t.large, t.small, t.steps, &us);
-    if (!split || us >= 0.96 * price) return false;
+    // (four parts and more: what their hand-over costs beyond the model)
+    if (!split || us * (split >= 4 ? 1.1 : 1.0) >= 0.96 * price) return false;
     memset(wide, 0, sizeof(*wide));
     wide->rows_per_wave = 64, wide->waves_m = 1, wide->waves_k = 1, wide->prefetch = 2, wide->x_chunk = 64, wide->token_tiles = 16;
     wide->lds_tile_rows = 256, wide->split_k = split;
@@ -2340,7 +2341,8 @@ static int derive_blockwise(const BlockwiseCall &b, tuna_gemm_config *out)
         const WideTiles t(m, n, k);
         double us = 0.0;
         const int split = n > 64 ? wide_best_split(t.large, t.small, t.steps, &us) : 0;
-        if (split && (!found || 1.07 * us / 5.68e-7 / k < 0.96 * best_cost)) {
+        // (four parts and more cost a quarter more than the model says: 4032 x 6400 at 580 tokens 73 us, the best other tile 56)
+        if (split && (!found || (1.07 * us * (split >= 4 ? 1.25 : split > 1 ? 1.05 : 1.0) + 2.0) / 5.68e-7 / k < 0.96 * best_cost)) {
             tuna_gemm_config c;
             memset(&c, 0, sizeof(c));
             c.rows_per_wave = 64, c.waves_m = 1, c.waves_k = 1, c.prefetch = 2, c.x_chunk = 64, c.token_tiles = 16;
