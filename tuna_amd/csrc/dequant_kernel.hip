@@ -174,11 +174,13 @@ typedef __attribute__((address_space(3))) unsigned char lds_u8;
 typedef uint32_t quant_u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) quant_u32x2 lds_pair;
 
-// nv * 16384 + 16384 plus 2^23: the fp32 pattern's low bits are that number as an integer, its multiples of 512 the
-// bucket - which is the entry's offset.  NaN and infinity mask to bucket 0.
+// (nv * 16384 + 16384) / 2^24 plus a half: the fp32 pattern's low bits are nv * 16384 + 16384 as an integer, its multiples
+// of 512 the bucket - which is the entry's offset.  Clamped to [0, 1] (an output modifier of the fused multiply-add, no
+// instruction of its own): a NaN becomes 0 whatever its payload - which an fp16 weight's NaN carries through the division
+// and which would otherwise show in those bits - and so goes to bucket 0, as infinities do.
 __device__ __forceinline__ uint32_t bucket_bits(float nv)
 {
-    return __builtin_bit_cast(uint32_t, __builtin_fmaf(nv, 16384.0f, 8388608.0f + 16384.0f)) & 0xfe00u;
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_fmed3f(__builtin_fmaf(nv, 0x1p-10f, 0.5f + 0x1p-10f), 0.0f, 1.0f)) & 0xfe00u;
 }
 
 __device__ __forceinline__ quant_u32x2 bucket_entry(float nv, uint32_t tab_lane)
