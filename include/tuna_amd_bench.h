@@ -123,6 +123,13 @@ int tuna_time_unit_rate(int unit, void *sink, int warmup, int iters, void *strea
  * uint64; counts[0] receives the pairs checked, counts[1] the mismatches. */
 int tuna_selftest_quantizer_division(void *counts, void *stream);
 
+/* Host check of the weight loads of the decode-batch kernel (kernel 0) - for the threads, k-steps and halves of row tile `row_tile` of an m x k matrix, from the functions the kernel
+ * itself takes its offsets from.  out4 receives: loads that reach behind the weights although a descriptor's range
+ * check that subtracts the uniform offset (modulo 2^32) accepts them; the same for a check that ignores the uniform
+ * offset; loads whose uniform offset exceeds the buffer; loads inside the matrix that the first check rejects.  Needs
+ * no device. */
+int tuna_check_weight_reach(int kernel, int m, int k, int row_tile, long long *out4);
+
 /* Diagnostic override of the batched kernel's workgroup shape (tuna_matmul_multi): waves along the
  * rows (1, 2, 4, 8 or 16 of the workgroup's 16 waves; 0 = the library's choice) and ring depth
  * (2 or 4; 0 = the library's choice).  For A/B timing. */

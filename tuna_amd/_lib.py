@@ -124,6 +124,7 @@ BENCH_SIGNATURES = {
     "tuna_time_read": (_i, [_vp, _vp, _sz, _i, _i, _i, _i, _vp, _fp]),
     "tuna_time_unit_rate": (_i, [_i, _vp, _i, _i, _vp, _fp, ctypes.POINTER(ctypes.c_double)]),
     "tuna_selftest_quantizer_division": (_i, [_vp, _vp]),
+    "tuna_check_weight_reach": (_i, [_i, _i, _i, _i, ctypes.POINTER(ctypes.c_longlong)]),
     "tuna_set_multi_shape": (_i, [_i, _i]),
     "tuna_set_multi_min_batch": (_i, [_i]),
     "tuna_time_matmul_blockwise": (_i, [_vpp, _vpp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _cfgp, _i, _i, _i, _vp, _fp]),

@@ -59,7 +59,7 @@ __global__ __launch_bounds__(kFlowThreads, 2) void gemm_flow_kernel(const FlowAr
 
     // per-lane offsets: weights (rows 4 i16 .. + 3 of the wave's 64, block column g of a half), activations (token tid / 8 +
     // 32 i, 8-k slot tid % 8), scales
-    const uint32_t a_off = ((uint32_t)(wave * 8 + (i16 >> 1)) * (uint32_t)kb_total + (uint32_t)g) * 32u + (uint32_t)(i16 & 1) * 16u;
+    const uint32_t a_off = tile_weight_lane(tid, kFlowRows / 8, kb_total);
     uint32_t x_off[XP];
 #pragma unroll
     for (int i = 0; i < XP; ++i) x_off[i] = ((uint32_t)((tid >> 3) + 32 * i) * (uint32_t)a.k + (uint32_t)(tid & 7) * 8u) * 2u;
@@ -87,12 +87,14 @@ __global__ __launch_bounds__(kFlowThreads, 2) void gemm_flow_kernel(const FlowAr
     u32x4 sq[BLK ? kFlowRing : 1];
     // Step `p` of the cursor's unit into register set `p`.  (Steps and slots beyond k: the activations are requested out
     // of range, which gives zeros, so what the weights there hold - of the last step, of the next block row, zeros at the
-    // matrix' end - adds nothing.)
+    // matrix' end - adds nothing.  The weights' offset is all in the vector register: flow_weight_offset says why.  The
+    // uniform offsets of activations and scales stay inside a token's k values and a row's scales, so below the
+    // descriptors' ends.)
 #define FLOW_LOAD(p)                                                                                          \
     {                                                                                                         \
         const int s_ = l_unit * kFlowRing + (p), c_ = min(s_, a.steps_total - 1);                             \
-        wq[p][0] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)a_off, c_ * 256, 2);                    \
-        wq[p][1] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)a_off, c_ * 256 + 128, 2);              \
+        wq[p][0] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)flow_weight_offset(a_off, c_, 0), 0, 2); \
+        wq[p][1] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)flow_weight_offset(a_off, c_, 1), 0, 2); \
         _Pragma("unroll") for (int i = 0; i < XP; ++i) xr[p][i] = __builtin_amdgcn_raw_buffer_load_b128(      \
             x_rsrc, s_ * 64 < x_k_left ? (int)x_off[i] : 0x7fffffff, c_ * 128, 0);                            \
         if constexpr (BLK) {                                                                                  \

@@ -208,6 +208,27 @@ struct FlowPlan {
 
 inline int ceil_div_i(int a, int b) { return (a + b - 1) / b; }
 
+// ---------------------------------------------------------------------------------------
+// Weight loads of the decode-batch kernel (gemm_flow.hip), 16 bytes each through a buffer descriptor that
+// starts at the tile's first row and ends with the weights: thread `tid` takes half h of every k-step of 64.  A descriptor's
+// range check rejects vector offsets from `end - uniform offset` on; it may not be relied on once the uniform offset
+// exceeds `end` (the difference wraps), nor to cover the uniform offset at all.  Shared by the kernel and by the host
+// check of these offsets (tuna_check_weight_reach of the diagnostic build).
+// ---------------------------------------------------------------------------------------
+__host__ __device__ inline uint32_t tile_weight_lane(int tid, int block_row_last, int kb_total)
+{
+    const int lane = tid & 63, wave = tid >> 6;  // rows 4 (lane % 16) .. + 3 of the wave's 64, block column lane / 16 of the half
+    const int mbl = wave * 8 + ((lane & 15) >> 1);
+    return ((uint32_t)(mbl < block_row_last ? mbl : block_row_last) * (uint32_t)kb_total + (uint32_t)(lane >> 4)) * 32u +
+           (uint32_t)(lane & 1) * 16u;
+}
+// Rows beyond the matrix are not clamped and the whole offset is in the vector register, so that the
+// check covers all of it; what lies beyond k is the next block row, or rejected.
+__host__ __device__ inline uint32_t flow_weight_offset(uint32_t lane_offset, int step, int half)
+{
+    return lane_offset + (uint32_t)step * 256u + (uint32_t)half * 128u;
+}
+
 struct GemmPlan {
     GemmArgs args;
     dim3 grid;
