@@ -123,8 +123,9 @@ int tuna_time_unit_rate(int unit, void *sink, int warmup, int iters, void *strea
  * uint64; counts[0] receives the pairs checked, counts[1] the mismatches. */
 int tuna_selftest_quantizer_division(void *counts, void *stream);
 
-/* Host check of the weight loads of the decode-batch kernel (kernel 0) - for the threads, k-steps and halves of row tile `row_tile` of an m x k matrix, from the functions the kernel
- * itself takes its offsets from.  out4 receives: loads that reach behind the weights although a descriptor's range
+/* Host check of the weight loads of the 256-row kernels - kernel 0: the decode-batch kernel, 1: the 256 x 256 many-token
+ * kernel - for the threads, k-steps and halves of row tile `row_tile` of an m x k matrix, from the functions the kernels
+ * themselves take their offsets from.  out4 receives: loads that reach behind the weights although a descriptor's range
  * check that subtracts the uniform offset (modulo 2^32) accepts them; the same for a check that ignores the uniform
  * offset; loads whose uniform offset exceeds the buffer; loads inside the matrix that the first check rejects.  Needs
  * no device. */

@@ -1,4 +1,4 @@
-"""The weight loads of the decode-batch kernel at the edges of the matrix: their offsets, checked on the host for what a buffer
+"""The weight loads of the 256-row kernels at the edges of the matrix: their offsets, checked on the host for what a buffer
 descriptor's range check accepts, and the launches at the shapes where an offset could leave the weights."""
 import ctypes
 
@@ -10,7 +10,7 @@ from tuna_amd import _lib
 EDGES = [(8, 8), (8, 72), (264, 72), (264, 80), (264, 88), (520, 1048), (264, 4104)]
 
 
-@pytest.mark.parametrize("kernel", [0])
+@pytest.mark.parametrize("kernel", [0, 1])
 def test_no_accepted_load_reaches_behind_the_weights(kernel):
     L = _lib.bench_lib()
     out = (ctypes.c_longlong * 4)()
@@ -27,10 +27,10 @@ def test_launches_at_the_edges(m, k):
     import torch
 
     from test_flow_kernel import _cfg as flow
-    from test_wide_tile import _check, _inputs, _out
+    from test_wide_tile import _cfg as wide, _check, _inputs, _out
     from tuna_amd import ops
 
-    for n, cfg in ((5, flow(5, 1)), (40, flow(40, 2))):
+    for n, cfg in ((5, flow(5, 1)), (40, flow(40, 2)), (5, wide(1)), (200, wide(1))):
         q, s, x, code = _inputs(m, n, k, seed=m + k)
         out = _out(n, m)
         ops.matmul(x, q, s, code, out, m, n, k, config=cfg)

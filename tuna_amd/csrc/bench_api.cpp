@@ -343,17 +343,19 @@ TUNA_EXPORT int tuna_selftest_quantizer_division(void *counts, void *stream)
 
 TUNA_EXPORT int tuna_check_weight_reach(int kernel, int m, int k, int row_tile, long long *out4)
 {
-    if (!out4 || kernel != 0 || m < 8 || m % 8 || k < 8 || k % 8 || row_tile < 0 || row_tile >= (m + 255) / 256)
+    if (!out4 || kernel < 0 || kernel > 1 || m < 8 || m % 8 || k < 8 || k % 8 || row_tile < 0 || row_tile >= (m + 255) / 256)
         return fail(TUNA_ERR_INVALID_ARG, "bad arguments");
-    const int rows_left = m - row_tile * 256, steps = ceil_div_i(k, 64);
+    const int rows_left = m - row_tile * 256, steps = ceil_div_i(k, 64), slot_last = (k / 8 - 1) & 7;
     const uint64_t rest = (uint64_t)rows_left * (uint64_t)(k / 2);
     const uint32_t end = rest < 0xffffffffu ? (uint32_t)rest : 0xffffffffu;
     for (int i = 0; i < 4; ++i) out4[i] = 0;
     for (int tid = 0; tid < 256; ++tid) {
-        const uint32_t lane = tile_weight_lane(tid, 32, k / 8);
+        const uint32_t lane = tile_weight_lane(tid, kernel ? rows_left / 8 - 1 : 32, k / 8);
         for (int step = 0; step < steps; ++step)
             for (int half = 0; half < 2; ++half) {
-                const uint32_t vector = flow_weight_offset(lane, step, half), uniform = 0;
+                const bool tail = kernel && k % 64 != 0 && step == steps - 1;
+                const uint32_t vector = kernel ? lane - (tail ? (uint32_t)wide_weight_back(tid, half, slot_last) : 0u) : flow_weight_offset(lane, step, half);
+                const uint32_t uniform = kernel ? (uint32_t)wide_weight_uniform(step, half, tail, slot_last) : 0u;
                 const uint64_t at = (uint64_t)vector + uniform;
                 const bool inside = at + 16 <= rest, accepted = vector < end - uniform;
                 out4[0] += accepted && !inside;

@@ -52,13 +52,11 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
     const int i16 = lane & 15, g = lane >> 4;
     const uint32_t lane4 = (uint32_t)lane << 2;
     const int kb_total = w.k >> 3;
-    const int mb_last = (w.m >> 3) - 1;
 
     // weights: lane (i16, g) loads 16 bytes = rows 4 i16 .. + 3 of the wave's 64, block column 4 h + g of half h of a
     // step (rows beyond the matrix are clamped: their products are never stored)
     const int row_w = w.row_base + wave * 64;
-    const uint32_t a_off = (uint32_t)(min((row_w >> 3) + (i16 >> 1), mb_last) - (w.row_base >> 3)) * (uint32_t)kb_total * 32u +
-                           (uint32_t)(i16 & 1) * 16u + (uint32_t)g * 32u;
+    const uint32_t a_off = tile_weight_lane(tid, ((w.m - w.row_base) >> 3) - 1, kb_total);
     // activations: piece i of a thread is token tid / 8 + 32 i, 8-k slot tid % 8 (tokens beyond the tile's read its last)
     uint32_t x_off[XP];
 #pragma unroll
@@ -68,8 +66,8 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
     const int x_k_left = w.k - (tid & 7) * 8;
     const int slot_last = ((w.k >> 3) - 1) & 7;
     const uint32_t x_back = KTAIL ? (uint32_t)max(0, (tid & 7) - slot_last) * 16u : 0u;
-    const uint32_t a_back0 = KTAIL ? (uint32_t)max(0, g - slot_last) * 32u : 0u;
-    const uint32_t a_back1 = KTAIL ? (uint32_t)max(0, 4 + g - slot_last) * 32u : 0u;
+    const uint32_t a_back0 = KTAIL ? (uint32_t)wide_weight_back(tid, 0, slot_last) : 0u;
+    const uint32_t a_back1 = KTAIL ? (uint32_t)wide_weight_back(tid, 1, slot_last) : 0u;
 
     const size_t q_rest = (size_t)(w.m - w.row_base) * (size_t)(w.k >> 1), x_rest = (size_t)w.tokens * (size_t)w.k * 2;
     const __amdgpu_buffer_rsrc_t q_rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -105,8 +103,10 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
     {                                                                                                         \
         const int s_ = min((s), s_last);                                                                      \
         const bool t_ = KTAIL && s_ == s_last;                                                                \
-        wq[set][0] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)(t_ ? a_off - a_back0 : a_off), s_ * 256, 0);       \
-        wq[set][1] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)(t_ ? a_off - a_back1 : a_off), s_ * 256 + 128, 0); \
+        wq[set][0] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)(t_ ? a_off - a_back0 : a_off),       \
+                                                           wide_weight_uniform(s_, 0, t_, slot_last), 0);     \
+        wq[set][1] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)(t_ ? a_off - a_back1 : a_off),       \
+                                                           wide_weight_uniform(s_, 1, t_, slot_last), 0);     \
     }
 #define WIDE_LOAD_X(set, i, s)                                                                                \
     {                                                                                                         \

@@ -209,10 +209,10 @@ struct FlowPlan {
 inline int ceil_div_i(int a, int b) { return (a + b - 1) / b; }
 
 // ---------------------------------------------------------------------------------------
-// Weight loads of the decode-batch kernel (gemm_flow.hip), 16 bytes each through a buffer descriptor that
+// Weight loads of the 256-row kernels (gemm_flow.hip, gemm_wide.hip), 16 bytes each through a buffer descriptor that
 // starts at the tile's first row and ends with the weights: thread `tid` takes half h of every k-step of 64.  A descriptor's
 // range check rejects vector offsets from `end - uniform offset` on; it may not be relied on once the uniform offset
-// exceeds `end` (the difference wraps), nor to cover the uniform offset at all.  Shared by the kernel and by the host
+// exceeds `end` (the difference wraps), nor to cover the uniform offset at all.  Shared by the kernels and by the host
 // check of these offsets (tuna_check_weight_reach of the diagnostic build).
 // ---------------------------------------------------------------------------------------
 __host__ __device__ inline uint32_t tile_weight_lane(int tid, int block_row_last, int kb_total)
@@ -222,11 +222,23 @@ __host__ __device__ inline uint32_t tile_weight_lane(int tid, int block_row_last
     return ((uint32_t)(mbl < block_row_last ? mbl : block_row_last) * (uint32_t)kb_total + (uint32_t)(lane >> 4)) * 32u +
            (uint32_t)(lane & 1) * 16u;
 }
-// Rows beyond the matrix are not clamped and the whole offset is in the vector register, so that the
+// gemm_flow.hip: rows beyond the matrix are not clamped and the whole offset is in the vector register, so that the
 // check covers all of it; what lies beyond k is the next block row, or rejected.
 __host__ __device__ inline uint32_t flow_weight_offset(uint32_t lane_offset, int step, int half)
 {
     return lane_offset + (uint32_t)step * 256u + (uint32_t)half * 128u;
+}
+// gemm_wide.hip: rows beyond the matrix read the last block row, and with a k tail the slots of the last step beyond k read
+// the last slot inside it: no load leaves its block row, whatever the check covers.  How far a thread steps back there
+// (negative: forward), and the uniform offset: a tail of fewer than five slots has no half 1 to start from.
+__host__ __device__ inline int wide_weight_back(int tid, int half, int slot_last)
+{
+    const int slot = 4 * half + ((tid & 63) >> 4);
+    return (slot > slot_last ? slot - slot_last : 0) * 32 - (half && slot_last < 4 ? 128 : 0);
+}
+__host__ __device__ inline int wide_weight_uniform(int step, int half, bool tail, int slot_last)
+{
+    return step * 256 + (half && !(tail && slot_last < 4) ? 128 : 0);
 }
 
 struct GemmPlan {
