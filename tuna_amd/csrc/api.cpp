@@ -340,7 +340,7 @@ static int launch_flow(FlowPlan &plan, const void *q, const void *x, const void 
     a.epilogue = epilogue;
     a.residual = residual;
     a.blk_shift = blk_shift < 0 ? 0 : blk_shift;
-    int rc = provide_workspace(static_ws, stream, plan.ws_bytes, plan.n_counters, &a.ws, &a.counters);
+    int rc = plan.ws_bytes ? provide_workspace(static_ws, stream, plan.ws_bytes, plan.n_counters, &a.ws, &a.counters) : TUNA_OK;
     if (rc) return rc;
     const hipError_t e = launch_gemm_flow(plan, blk_shift >= 0, stream);
     return e == hipSuccess ? TUNA_OK : hip_fail(e, "decode-batch gemm launch");
@@ -1257,9 +1257,9 @@ static int validate_for(int m, int n, int k, const tuna_gemm_config &c, int deco
 //
 // A buffer that has been handed to a launch is never freed or moved before
 // tuna_release_workspaces: a HIP graph captured on the stream keeps the pointers in its kernel
-// nodes and may be replayed at any later time.  The first request allocates generously (64 MB of
-// partial sums and 64 K counters cover every entry of the tuned table); a larger request adds a
-// new buffer and retires the old one, which stays allocated for the graphs that know it.
+// nodes and may be replayed at any later time.  The first request allocates what it asks for, at
+// least 8 MB of partial sums and 64 K counters; a larger request adds a new buffer, at least twice
+// as large, and retires the old one, which stays allocated for the graphs that know it.
 // ---------------------------------------------------------------------------------------
 
 struct Workspace {
@@ -1271,7 +1271,8 @@ struct Workspace {
 };
 
 // First allocation for a (device, stream) pair: what the launch asks for, but at least this much, so that a process
-// with many streams does not pay for the largest request of the table (48 MB) on each of them.
+// with many streams does not pay for the largest request (136 MB: 256 x 256 tiles whose last ones are shared, two
+// slots of 260 KB for each of 256 shares) on each of them.
 constexpr size_t kWsFirstBytes = (size_t)8 << 20;
 constexpr size_t kWsFirstCounters = (size_t)64 << 10;
 

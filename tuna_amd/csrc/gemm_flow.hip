@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kFlowThreads, 2) void gemm_flow_kernel(const FlowAr
         bool own = true, store = true;
         auto slot = [&](int share) {
             const int which = share == place ? my_slot : share == lo ? lo_slot : 0;
-            return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char *>(a.ws) + (size_t)(2 * share + which) * flow_slot_bytes<NT>(), 0,
+            return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char *>(a.ws) + (size_t)(a.slots * share + which) * flow_slot_bytes<NT>(), 0,
                                                      (int)flow_slot_bytes<NT>(), 0x00020000);
         };
         if (seg0 != 0 || seg1 != a.units) {
@@ -347,8 +347,9 @@ bool plan_gemm_flow(int nt, int shares, FlowPlan *plan)
     a.tiles = (int)tiles;
     plan->nt = nt;
     a.n_shares = shares > units ? (int)units : shares;
-    plan->ws_bytes = (size_t)a.n_shares * 2 * (size_t)kFlowRows * 16 * nt * 4;
-    plan->n_counters = (size_t)tiles;
+    a.slots = a.tiles % a.n_shares == 0 ? 0 : a.n_shares % a.tiles == 0 ? 1 : 2;
+    plan->ws_bytes = (size_t)a.n_shares * a.slots * (size_t)kFlowRows * 16 * nt * 4;
+    plan->n_counters = a.slots ? (size_t)tiles : 0;
     return true;
 }
 

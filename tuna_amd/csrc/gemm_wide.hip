@@ -384,7 +384,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(const WideAr
         // (cache policy 16: sc1, past the XCD's L2 - writer and reader may sit on different XCDs)
         auto slot = [&](int share) {
             const int which = share == place ? my_slot : share == lo ? lo_slot : 0;
-            return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char *>(a.ws) + (size_t)(2 * share + which) * kWideSlot, 0,
+            return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char *>(a.ws) + (size_t)(a.slots * share + which) * kWideSlot, 0,
                                                      (int)kWideSlot, 0x00020000);
         };
         __syncthreads();  // every wave is done with the stages
@@ -534,8 +534,11 @@ bool plan_gemm_wide(int split, int cus, WidePlan *plan)
     // (a share is at least a step of a large tile, so that every share between a tile's first and last has a part of it)
     if (a.n_shares > weight / kCostLarge) a.n_shares = (int)(weight / kCostLarge) > 0 ? (int)(weight / kCostLarge) : 1;
     plan->grid = (unsigned)(a.n_shares ? a.n_shares : tiles);
-    plan->ws_bytes = (size_t)a.n_shares * 2 * kWideSlot;
-    plan->n_counters = a.n_shares ? (size_t)(tiles - a.whole) : 0;
+    const long long divided = tiles - a.whole;
+    const bool alike = a.whole == a.large || !a.small;  // the divided tiles are of one kind: shares are equal parts of them
+    a.slots = !a.n_shares || (alike && divided % a.n_shares == 0) ? 0 : alike && a.n_shares % divided == 0 ? 1 : 2;
+    plan->ws_bytes = (size_t)a.n_shares * a.slots * kWideSlot;
+    plan->n_counters = a.slots ? (size_t)divided : 0;
     return true;
 }
 

@@ -160,7 +160,7 @@ struct WideArgs {
     void *out;
     const void *residual;
     int epilogue;
-    float *ws;           // partial tiles, two slots per share
+    float *ws;           // partial tiles, `slots` per share
     unsigned *counters;  // one arrival counter per shared tile, zero between launches
     int m, k, n_groups;
     int steps_total;     // ceil(k / 64)
@@ -168,6 +168,7 @@ struct WideArgs {
     int large, small;    // tiles of either kind
     int whole;           // tiles 0 .. whole - 1 are computed whole, one workgroup each
     int n_shares;        // the k-steps of the other tiles, laid end to end, are divided into this many equal shares (0: none)
+    int slots;           // 2; 1 where every tile ends with a share, so that no share has parts of two; 0: no tile is divided
     int blk_shift;       // scale-block variants: absmax is [m, k / (64 << blk_shift)]
     int tok_begin[kMaxGroups], tok_count[kMaxGroups];
     unsigned char id[kMaxGroups];
@@ -189,12 +190,12 @@ struct FlowArgs {
     void *out;
     const void *residual;
     int epilogue;
-    float *ws;           // partial tiles, two slots per share
+    float *ws;           // partial tiles, `slots` per share
     unsigned *counters;  // one arrival counter per tile, zero between launches
     int m, k, n_groups, m_total;  // rows of a group, reduction length, groups with tokens, rows of all matrices
     int steps_total, units;       // ceil(k / 64); units of four steps
     int row_tiles, tiles;         // of a group, of all groups with tokens
-    int n_shares;
+    int n_shares, slots;          // (as in WideArgs)
     int blk_shift;
     int tok_begin[kMaxGroups], tok_count[kMaxGroups];
     int id[kMaxGroups];  // (an int: read through the scalar cache)
