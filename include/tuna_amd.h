@@ -138,11 +138,15 @@ int tuna_init(void);
  * fixed array in device memory that is part of the loaded library (16 MB + 256 KB, held on
  * every GPU the library runs on until the process ends) and calls no allocating routine.  A
  * launch that needs more than TUNA_STATIC_WORKSPACE_BYTES of partial sums or more than 65536
- * counters fails with TUNA_ERR_WORKSPACE (where the library picks the config - cfg NULL - and its
- * pick splits k of a many-token tile further than that, it reduces the split until it fits).  All calls on one GPU share that GPU's array: calls
+ * counters fails with TUNA_ERR_WORKSPACE - except where the library picks the config (cfg NULL,
+ * TUNA_DECODE_GEMM): it then picks a launch that fits.  All calls on one GPU share that GPU's array: calls
  * that may overlap (different streams) race; calls on one stream are ordered and safe.  The
  * kernels return the counters they used to zero, so nothing is cleared between calls.  Results
- * are those of tuna_matmul_ex, bit for bit. */
+ * are those of tuna_matmul_ex, bit for bit, where that launch fits; where it does not, they are
+ * another launch's, with the same products summed in another order: cfg NULL and a pick of
+ * tuna_matmul_ex that needs more (another number of shares or parts of k, or another kernel), and
+ * - with or without cfg - unsplit 256 x 256 tiles whose last ones tuna_matmul_ex shares between
+ * the compute units, which run as whole tiles here. */
 int tuna_matmul_static(const void *q, const void *x, const void *code, const void *absmax,
                        void *out, int m, int n, int k, const tuna_gemm_config *cfg,
                        int decode_mode, void *stream);

@@ -214,6 +214,14 @@ struct TiledPlan {
     size_t lds_bytes, ws_bytes, n_counters;
 };
 
+// Workspace that the library's own choice of a launch may count on: what cannot grow - the static scratch - limits
+// which kernels are taken in place of the selected one.
+struct Room {
+    size_t bytes, counters;
+    bool holds(size_t ws_bytes, size_t n_counters) const { return ws_bytes <= bytes && n_counters <= counters; }
+};
+constexpr Room kRoomToGrow = {(size_t)-1, (size_t)-1};
+
 // Compute units of the current device for the plans that divide a launch over them (the largest part's where there is
 // no device: plans are also made to describe and validate launches).
 static int planned_cus()
@@ -665,15 +673,19 @@ static bool wide_balance_pays(int m, int n, int k)
     return wide_balance_pays(t.large, t.small, t.steps);
 }
 
-// The split (as above; 1 where the launch then shares its last tiles by itself) that takes these tiles least time, and
-// that time in *us; 0 if there are too few of them.
-static int wide_best_split(double large, double small, double steps, double *us)
+// The split (as above; 1 where the launch then shares its last tiles by itself) that takes these tiles least time with
+// partial sums that `room` holds, and that time in *us; 0 if there are too few of them.
+static int wide_best_split(double large, double small, double steps, const Room &room, double *us)
 {
     int best = 0;
     for (int split : {1, 2, 3, 4, 6, 8}) {
         const double wgs = (large + small) * split;
         if (wgs < 16 || (split > 1 && (wgs > 400 || steps / split < 8))) continue;
-        const double t = wide_time(large, small, steps, split == 1 && wide_balance_pays(large, small, steps) ? 0 : split);
+        const bool balance = split == 1 && wide_balance_pays(large, small, steps);
+        const size_t slots = split > 1 ? (size_t)wgs * (large > 0 && small > 0 ? 2 : 1) : balance ? (size_t)2 * kMaxCus : 0;
+        const bool holds = !slots || room.holds(slots * kWideSlot, (size_t)(large + small));
+        if (!holds && split > 1) continue;
+        const double t = wide_time(large, small, steps, balance && holds ? 0 : split);
         if (!best || t < *us) best = split, *us = t;
     }
     return best;
@@ -1011,12 +1023,14 @@ static double flow_time(double tiles, int units, int nt, int shares)
     return 6.1 + per_share * step + (contributors > 1.0 ? 2.7 + (contributors > 2.0 ? 0.3 * nt * (contributors - 2.0) : 0.0) : 0.0);
 }
 
-// The number of shares that takes them least time, and that time in *us: equal parts of every tile, or 64 ... 512 at large.
-static int flow_best_shares(long long tiles, int units, int nt, double *us)
+// The number of shares that takes them least time with partial sums that `room` holds, and that time in *us: equal parts of
+// every tile, or 64 ... 512 at large.
+static int flow_best_shares(long long tiles, int units, int nt, const Room &room, double *us)
 {
     int best = 0;
     auto consider = [&](long long shares) {
         if (shares < 1 || shares > 2 * kMaxCus || shares > tiles * units) return;
+        if (!room.holds(flow_ws_bytes(tiles, (int)shares, nt), flow_slots(tiles, shares) ? (size_t)tiles : 0)) return;
         const double t = flow_time((double)tiles, units, nt, (int)shares);
         if (!best || t < *us) best = (int)shares, *us = t;
     };
@@ -1029,7 +1043,8 @@ static int flow_best_shares(long long tiles, int units, int nt, double *us)
 // where that is predicted to be faster.  The selected kernels are priced by straight lines over the bytes of the weights,
 // read off the same random shapes; narrow-row, lean and batched launches, which win on the shapes they are picked for, are
 // left alone, and an entry of the table, timed for its shape, has to be beaten by a quarter.
-static bool flow_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, tuna_gemm_config *flow, double *flow_us)
+static bool flow_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, const Room &room, tuna_gemm_config *flow,
+                         double *flow_us)
 {
     const double mb = 0.5e-6 * m * k;
     if (n > 64 || is_narrow(c) || mb < 8) return false;
@@ -1047,7 +1062,7 @@ static bool flow_instead(int m, int n, int k, const tuna_gemm_config &c, bool fr
         else price = 7.0 + 1.5 * nt + kGeneral[nt] * mb;
     }
     double us = 0.0;
-    const int shares = price == 0.0 ? 0 : flow_best_shares(ceil_div(m, 256), ceil_div(ceil_div(k, 64), 4), nt, &us);
+    const int shares = price == 0.0 ? 0 : flow_best_shares(ceil_div(m, 256), ceil_div(ceil_div(k, 64), 4), nt, room, &us);
     if (!shares || us >= (from_table ? 0.8 : 0.95) * price) return false;
     memset(flow, 0, sizeof(*flow));
     flow->rows_per_wave = 64, flow->waves_m = 4, flow->waves_k = 1, flow->prefetch = 4, flow->x_chunk = 64, flow->token_tiles = nt;
@@ -1132,7 +1147,7 @@ static bool narrow_any_instead(int m, int n, int k, const tuna_gemm_config &c, b
 // the table and the cost model were measured before that kernel and still pick the best of the other tiles).  Configs of
 // kernels that the model does not price - narrow rows, k split over lean workgroups - are left alone: they are picked
 // for shapes too small for such tiles.
-static bool wide_instead(int m, int n, int k, const tuna_gemm_config &c, tuna_gemm_config *wide)
+static bool wide_instead(int m, int n, int k, const tuna_gemm_config &c, const Room &room, tuna_gemm_config *wide)
 {
     if (n <= 64 || is_narrow(c)) return false;
     const int tokens = 16 * c.token_tiles, streaming = c.lds_tile_rows <= 0;
@@ -1146,7 +1161,7 @@ static bool wide_instead(int m, int n, int k, const tuna_gemm_config &c, tuna_ge
             if (cd.rows == rows && cd.tokens == tokens && cd.streaming == streaming && (!streaming || c.split_k == 1))
                 price = kGridCostUs * k * grid_cost(cd, c.split_k, (long long)ceil_div(m, rows) * ceil_div(n, tokens) * c.split_k, k);
     }
-    const int split = price == 0.0 ? 0 : wide_best_split(t.large, t.small, t.steps, &us);
+    const int split = price == 0.0 ? 0 : wide_best_split(t.large, t.small, t.steps, room, &us);
     // (four parts and more: what their hand-over costs beyond the model)
     if (!split || us * (split >= 4 ? 1.1 : 1.0) >= 0.96 * price) return false;
     memset(wide, 0, sizeof(*wide));
@@ -1217,15 +1232,16 @@ static int select_config_for(int m, int n, int k, int decode, tuna_gemm_config *
     return TUNA_OK;
 }
 
-// The config a launch without an explicit one runs: the selected one, or a newer kernel in its place.
-static void select_launch(int m, int n, int k, int decode, tuna_gemm_config *c)
+// The config a launch without an explicit one runs: the selected one, or a newer kernel in its place - one whose partial
+// sums `room` holds.
+static void select_launch(int m, int n, int k, int decode, const Room &room, tuna_gemm_config *c)
 {
     int from_table = 0;
     select_config_for(m, n, k, decode, c, &from_table);
     tuna_gemm_config other;
     double flow_us = 0.0;
     if (decode != TUNA_DECODE_GEMM) return;
-    if (wide_instead(m, n, k, *c, &other) || flow_instead(m, n, k, *c, from_table != 0, &other, &flow_us)) *c = other;
+    if (wide_instead(m, n, k, *c, room, &other) || flow_instead(m, n, k, *c, from_table != 0, room, &other, &flow_us)) *c = other;
     if (narrow_any_instead(m, n, k, *c, from_table != 0, flow_us, &other)) *c = other;
 }
 
@@ -1545,7 +1561,7 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
         return rc;
     tuna_gemm_config c;
     if (cfg) c = *cfg;
-    else select_launch(m, n, k, decode, &c);
+    else select_launch(m, n, k, decode, static_ws ? Room{kStaticWsBytes, kStaticCounters} : kRoomToGrow, &c);
     if (c.lds_tile_rows > 0) {
         TiledPlan tp;
         if ((rc = plan_tiled(m, n, k, c, decode, &tp))) return rc;
@@ -1686,7 +1702,7 @@ static int grouped_flow_shares(int m_group, int n_active, int nt, int k)
 {
     double us = 0.0;
     if (nt == 1 && (double)m_group * n_active * k < 3e7) return 0;
-    return flow_best_shares((long long)ceil_div(m_group, 256) * n_active, ceil_div(ceil_div(k, 64), 4), nt, &us);
+    return flow_best_shares((long long)ceil_div(m_group, 256) * n_active, ceil_div(ceil_div(k, 64), 4), nt, kRoomToGrow, &us);
 }
 
 // Grouped GEMM: n_groups stacked weight matrices of m_group rows, group e applied to the
@@ -1748,7 +1764,7 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
         long long large, small;
         count_wide_tiles(a, &large, &small);
         const double steps = ceil_div(k, 64);
-        const int split = a.n_groups > 1 ? wide_best_split((double)large, (double)small, steps, &together) : 0;
+        const int split = a.n_groups > 1 ? wide_best_split((double)large, (double)small, steps, kRoomToGrow, &together) : 0;
         if (split && together < apart) {
             a.q = static_cast<const uint8_t *>(q);
             a.x = x;
@@ -2341,7 +2357,7 @@ static int derive_blockwise(const BlockwiseCall &b, tuna_gemm_config *out)
         // 236 -> 149, 11136 x 1536 at 2891 tokens 173 -> 118).
         const WideTiles t(m, n, k);
         double us = 0.0;
-        const int split = n > 64 ? wide_best_split(t.large, t.small, t.steps, &us) : 0;
+        const int split = n > 64 ? wide_best_split(t.large, t.small, t.steps, kRoomToGrow, &us) : 0;
         // (four parts and more cost a quarter more than the model says: 4032 x 6400 at 580 tokens 73 us, the best other tile 56)
         if (split && (!found || (1.07 * us * (split >= 4 ? 1.25 : split > 1 ? 1.05 : 1.0) + 2.0) / 5.68e-7 / k < 0.96 * best_cost)) {
             tuna_gemm_config c;
@@ -2760,7 +2776,7 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
     tuna_gemm_config c, w;
     if (cfg) c = *cfg;
     else select_config_for(m, n, k, decode_mode, &c, nullptr);
-    if (!cfg && (select_launch(m, n, k, decode_mode, &w), memcmp(&w, &c, sizeof(c)) != 0)) {
+    if (!cfg && (select_launch(m, n, k, decode_mode, kRoomToGrow, &w), memcmp(&w, &c, sizeof(c)) != 0)) {
         NarrowPlan np;
         const int at = is_narrow_any(w) && plan_narrow_any(m, n, k, w, decode_mode, &np) == TUNA_OK
                            ? describe_narrow_any(np, n, buf, len, " in place of ")

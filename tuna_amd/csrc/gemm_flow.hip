@@ -21,7 +21,7 @@
 namespace tuna {
 
 constexpr int kFlowThreads = 256;
-constexpr int kFlowRows = 256;
+constexpr int kFlowRows = 256;  // (flow_ws_bytes counts on it)
 constexpr int kFlowRing = 4;  // k-steps requested ahead, and the k-steps of a unit
 
 template <int NT>
@@ -347,8 +347,8 @@ bool plan_gemm_flow(int nt, int shares, FlowPlan *plan)
     a.tiles = (int)tiles;
     plan->nt = nt;
     a.n_shares = shares > units ? (int)units : shares;
-    a.slots = a.tiles % a.n_shares == 0 ? 0 : a.n_shares % a.tiles == 0 ? 1 : 2;
-    plan->ws_bytes = (size_t)a.n_shares * a.slots * (size_t)kFlowRows * 16 * nt * 4;
+    a.slots = flow_slots(a.tiles, a.n_shares);
+    plan->ws_bytes = flow_ws_bytes(a.tiles, a.n_shares, nt);
     plan->n_counters = a.slots ? (size_t)tiles : 0;
     return true;
 }

@@ -262,8 +262,6 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
 
 // Position in the k-steps of the shared tiles laid end to end: tile (counted from `whole`) and step.  A step of a large
 // tile weighs kCostLarge, one of a small tile kCostSmall (half the MFMAs, the same decode).
-// Bytes between the partial-sum slots: a tile's 256 KB and 4352 more.
-constexpr size_t kWideSlot = (size_t)kWideRows * kWideTokens * 4 + 4352;
 constexpr int kCostLarge = 5, kCostSmall = 3;
 struct WidePos {
     int tile, step;

@@ -174,6 +174,9 @@ struct WideArgs {
     unsigned char id[kMaxGroups];
 };
 
+// Bytes between the partial-sum slots: a tile's 256 KB and 4352 more.
+constexpr size_t kWideSlot = (size_t)256 * 256 * 4 + 4352;
+
 struct WidePlan {
     WideArgs args;
     unsigned grid;
@@ -200,6 +203,10 @@ struct FlowArgs {
     int tok_begin[kMaxGroups], tok_count[kMaxGroups];
     int id[kMaxGroups];  // (an int: read through the scalar cache)
 };
+
+// Slots of partial sums per share where `shares` shares divide `tiles` equal tiles.
+inline int flow_slots(long long tiles, long long shares) { return tiles % shares == 0 ? 0 : shares % tiles == 0 ? 1 : 2; }
+inline size_t flow_ws_bytes(long long tiles, int shares, int nt) { return (size_t)shares * flow_slots(tiles, shares) * 256 * 16 * nt * 4; }
 
 struct FlowPlan {
     FlowArgs args;

@@ -72,9 +72,10 @@ def matmul(x, q, s, c, o, m: int, n: int, k: int, config: GemmConfig = None,
 
 def matmul_static(x, q, s, c, o, m: int, n: int, k: int, config: GemmConfig = None,
                   decode_mode: int = _lib.DECODE_GEMM) -> None:
-    """matmul through tuna_matmul_static: same result, but the split-K partial sums live in a fixed
-    array of the loaded library instead of an allocated workspace (for callers that cannot
-    allocate).  Raises TunaError (ERR_WORKSPACE) if the launch needs more than that array holds."""
+    """matmul through tuna_matmul_static: the split-K partial sums live in a fixed array of the loaded
+    library instead of an allocated workspace (for callers that cannot allocate).  The same bits where matmul's
+    launch fits that array; without a config a launch that does not is replaced by one that does, and one with
+    `config` raises TunaError (ERR_WORKSPACE) (tuna_amd.h names the exceptions)."""
     m, n, k = int(m), int(n), int(k)
     _require(x, "x", torch.float16, n * k)
     _require(q, "q", torch.uint8, m * k // 2)
