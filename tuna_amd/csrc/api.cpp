@@ -214,8 +214,8 @@ struct TiledPlan {
     size_t lds_bytes, ws_bytes, n_counters;
 };
 
-// Workspace that the library's own choice of a launch may count on: what cannot grow - the static scratch - limits
-// which kernels are taken in place of the selected one.
+// Workspace that the library's own choice of a launch may count on: what cannot grow - the static scratch, what a
+// capturing stream holds - limits which kernels are taken in place of the selected one.
 struct Room {
     size_t bytes, counters;
     bool holds(size_t ws_bytes, size_t n_counters) const { return ws_bytes <= bytes && n_counters <= counters; }
@@ -1321,7 +1321,10 @@ static int get_workspace(hipStream_t stream, size_t ws_bytes, size_t n_counters,
             const size_t want = grown_size(w.ws_bytes, ws_bytes, kWsFirstBytes);
             float *fresh = nullptr;
             e = hipMalloc(reinterpret_cast<void **>(&fresh), want);
-            if (e != hipSuccess) return fail(TUNA_ERR_WORKSPACE, "hipMalloc(%zu) for the split-K workspace: %s", want, hipGetErrorString(e));
+            if (e != hipSuccess) {
+                (void)hipGetLastError();  // (a launch that needs less may follow, which must not find this error)
+                return fail(TUNA_ERR_WORKSPACE, "hipMalloc(%zu) for the split-K workspace: %s", want, hipGetErrorString(e));
+            }
             if (w.ws) w.retired.push_back(w.ws);
             w.ws = fresh;
             w.ws_bytes = want;
@@ -1330,7 +1333,10 @@ static int get_workspace(hipStream_t stream, size_t ws_bytes, size_t n_counters,
             const size_t want = grown_size(w.n_counters, n_counters, kWsFirstCounters);
             unsigned *fresh = nullptr;
             e = hipMalloc(reinterpret_cast<void **>(&fresh), want * sizeof(unsigned));
-            if (e != hipSuccess) return fail(TUNA_ERR_WORKSPACE, "hipMalloc for the split-K counters: %s", hipGetErrorString(e));
+            if (e != hipSuccess) {
+                (void)hipGetLastError();
+                return fail(TUNA_ERR_WORKSPACE, "hipMalloc for the split-K counters: %s", hipGetErrorString(e));
+            }
             // zeroed on the launch stream (it is not capturing: checked above) and waited for there: a device-wide
             // synchronisation would disturb other threads' streams and captures.  Kernels leave the counters at zero.
             e = hipMemsetAsync(fresh, 0, want * sizeof(unsigned), stream);
@@ -1347,6 +1353,16 @@ static int get_workspace(hipStream_t stream, size_t ws_bytes, size_t n_counters,
     *out = w;
     out->retired.clear();
     return TUNA_OK;
+}
+
+// What the stream's workspace holds now.
+static Room workspace_room(hipStream_t stream)
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return Room{0, 0};
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    auto it = g_workspaces.find(std::make_pair(dev, stream));
+    return it == g_workspaces.end() ? Room{0, 0} : Room{it->second.ws_bytes, it->second.n_counters};
 }
 
 static void free_workspace(Workspace &w)
@@ -1549,7 +1565,7 @@ static bool stream_applies(const tuna_gemm_config &c, int n, int decode)
 
 static int matmul_impl(const void *q, const void *x, const void *code, const void *absmax, void *out, int m, int n, int k,
                        const tuna_gemm_config *cfg, int decode, hipStream_t stream, int epilogue = TUNA_EPILOGUE_NONE,
-                       const void *residual = nullptr, bool static_ws = false)
+                       const void *residual = nullptr, bool static_ws = false, const Room *held = nullptr)
 {
     int rc;
     if ((rc = check_shape(m, n, k))) return rc;
@@ -1561,7 +1577,14 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
         return rc;
     tuna_gemm_config c;
     if (cfg) c = *cfg;
-    else select_launch(m, n, k, decode, static_ws ? Room{kStaticWsBytes, kStaticCounters} : kRoomToGrow, &c);
+    else select_launch(m, n, k, decode, held ? *held : static_ws ? Room{kStaticWsBytes, kStaticCounters} : kRoomToGrow, &c);
+    // No room for the partial sums of the library's own pick, and none to be had (the stream is capturing, or the device's
+    // memory is full): once more with what the stream's workspace holds.
+    auto or_with_less = [&](int rc1) {
+        if (rc1 != TUNA_ERR_WORKSPACE || cfg || static_ws || held) return rc1;
+        const Room room = workspace_room(stream);
+        return matmul_impl(q, x, code, absmax, out, m, n, k, cfg, decode, stream, epilogue, residual, false, &room);
+    };
     if (c.lds_tile_rows > 0) {
         TiledPlan tp;
         if ((rc = plan_tiled(m, n, k, c, decode, &tp))) return rc;
@@ -1572,12 +1595,12 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
             c.split_k -= 1;
             if ((rc = plan_tiled(m, n, k, c, decode, &tp))) return rc;
         }
-        return launch_tiled(tp, q, x, code, absmax, out, epilogue, residual, -1, static_ws, stream);
+        return or_with_less(launch_tiled(tp, q, x, code, absmax, out, epilogue, residual, -1, static_ws, stream));
     }
     if (is_flow(c)) {
         FlowPlan fp;
         if ((rc = plan_flow(m, n, k, c, decode, &fp))) return rc;
-        return launch_flow(fp, q, x, code, absmax, out, epilogue, residual, -1, static_ws, stream);
+        return or_with_less(launch_flow(fp, q, x, code, absmax, out, epilogue, residual, -1, static_ws, stream));
     }
     if (is_narrow_any(c)) {
         NarrowPlan np;
@@ -2255,7 +2278,7 @@ static int run_blockwise(const BlockwiseCall &b, const tuna_gemm_config &c, hipS
 // 229376 x 4096 (117 / 102); at 32 tokens 11.9 / 16.9 on 6144 x 4096, 20.3 / 24.6 on 8192 x 8192, 30.9 / 38.7 on
 // 28672 x 4096, but 37.2 / 30.4 on 10240 x 8192, 29.6 / 22.7 on 4096 x 14336, 134 / 106 on 32768 x 14336.  Everything
 // else: the narrow-row kernel, the widest tile that gives nine workgroups per sixteen compute units.
-static int derive_blockwise(const BlockwiseCall &b, tuna_gemm_config *out)
+static int derive_blockwise(const BlockwiseCall &b, const Room &room, tuna_gemm_config *out)
 {
     const int m = b.m, n = b.n, k = b.k, shift = log2i(b.block_size) - 6;
     const long long packed_bytes = (long long)m * k / 2;
@@ -2357,7 +2380,7 @@ static int derive_blockwise(const BlockwiseCall &b, tuna_gemm_config *out)
         // 236 -> 149, 11136 x 1536 at 2891 tokens 173 -> 118).
         const WideTiles t(m, n, k);
         double us = 0.0;
-        const int split = n > 64 ? wide_best_split(t.large, t.small, t.steps, kRoomToGrow, &us) : 0;
+        const int split = n > 64 ? wide_best_split(t.large, t.small, t.steps, room, &us) : 0;
         // (four parts and more cost a quarter more than the model says: 4032 x 6400 at 580 tokens 73 us, the best other tile 56)
         if (split && (!found || (1.07 * us * (split >= 4 ? 1.25 : split > 1 ? 1.05 : 1.0) + 2.0) / 5.68e-7 / k < 0.96 * best_cost)) {
             tuna_gemm_config c;
@@ -2425,7 +2448,7 @@ static int derive_blockwise(const BlockwiseCall &b, tuna_gemm_config *out)
 }
 
 // Tuned entry for (m, n, k, block_size) if the table has one that can run the call, else the derived config.
-static int select_blockwise(const BlockwiseCall &b, tuna_gemm_config *cfg, int *from_table)
+static int select_blockwise(const BlockwiseCall &b, const Room &room, tuna_gemm_config *cfg, int *from_table)
 {
     if (from_table) *from_table = 0;
     for (int i = 0; i < kBlockwiseTableSize; ++i) {
@@ -2441,7 +2464,7 @@ static int select_blockwise(const BlockwiseCall &b, tuna_gemm_config *cfg, int *
             return TUNA_OK;
         }
     }
-    return derive_blockwise(b, cfg);
+    return derive_blockwise(b, room, cfg);
 }
 
 static int check_blockwise_call(const BlockwiseCall &b, bool pointers)
@@ -2466,10 +2489,10 @@ static int check_blockwise_call(const BlockwiseCall &b, bool pointers)
 // its place where their model is an eighth under the selected config's price - that model for a narrow-row pick, a straight
 // line for many-token tiles (9984 x 7936 at 2 tokens, which no ring turn of more than four waves divides, 38.8 -> 13 us;
 // 2048 x 8960 at 7 tokens 18.9 -> 9.9, 13120 x 23296 at 9 tokens 197 -> 54; 1.30 x on average over 280 random shapes).
-static int select_blockwise_launch(const BlockwiseCall &b, tuna_gemm_config *c)
+static int select_blockwise_launch(const BlockwiseCall &b, const Room &room, tuna_gemm_config *c)
 {
     int from_table = 0;
-    const int rc = select_blockwise(b, c, &from_table);
+    const int rc = select_blockwise(b, room, c, &from_table);
     if (rc || from_table || b.n > 64) return rc;
     const int nblk = b.k / b.block_size;
     double price = 0.0;
@@ -2489,8 +2512,14 @@ TUNA_EXPORT int tuna_matmul_blockwise_ex(const void *q, const void *x, const voi
     if ((rc = check_blockwise_call(b, true))) return rc;
     tuna_gemm_config c;
     if (cfg) c = *cfg;
-    else if ((rc = select_blockwise_launch(b, &c))) return rc;
-    return run_blockwise(b, c, static_cast<hipStream_t>(stream), false);
+    else if ((rc = select_blockwise_launch(b, kRoomToGrow, &c))) return rc;
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    rc = run_blockwise(b, c, st, false);
+    if (rc != TUNA_ERR_WORKSPACE || cfg) return rc;
+    // (as in matmul_impl: the library's pick has no room for its partial sums)
+    const Room held = workspace_room(st);
+    if ((rc = select_blockwise_launch(b, held, &c))) return rc;
+    return run_blockwise(b, c, st, false);
 }
 
 TUNA_EXPORT int tuna_matmul_blockwise(const void *q, const void *x, const void *code, const void *absmax, void *out, int m, int n,
@@ -2505,7 +2534,7 @@ TUNA_EXPORT int tuna_select_config_blockwise(int m, int n, int k, int block_size
     const BlockwiseCall b = {nullptr, nullptr, nullptr, nullptr, nullptr, m, n, k, block_size};
     int rc;
     if ((rc = check_blockwise_call(b, false))) return rc;
-    return select_blockwise(b, cfg, from_table);
+    return select_blockwise(b, kRoomToGrow, cfg, from_table);
 }
 
 TUNA_EXPORT int tuna_validate_config_blockwise(int m, int n, int k, int block_size, const tuna_gemm_config *cfg)
