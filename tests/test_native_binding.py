@@ -1,6 +1,8 @@
 """The extension behind the ops (csrc/torch_binding.cpp): what it refuses is left to the Python ops, and what it runs
 gives the bits the same call gives through ctypes."""
 import ctypes
+import sys
+import warnings
 
 import numpy as np
 import pytest
@@ -72,6 +74,42 @@ def test_ops_through_the_extension_equal_the_ctypes_calls(m, n, k):
         torch.cuda.synchronize()
         assert torch.equal(a[0], q2) and torch.equal(a[1], s2) and a[2] is c
         assert b[0].shape == a[0].shape and b[1].shape == a[1].shape
+
+
+@pytest.fixture
+def no_extension(monkeypatch):
+    """As where _native.so was not built: its import fails."""
+    monkeypatch.setitem(sys.modules, "tuna_amd._native", None)
+    monkeypatch.setattr(_lib, "_native", None)
+
+
+def test_without_the_extension_the_ops_take_the_ctypes_path(no_extension):
+    x, q = torch.zeros(16, 64, dtype=torch.float16), torch.zeros(8, 8, 32, dtype=torch.uint8)
+    s, c, o = torch.zeros(64), torch.zeros(16), torch.zeros(16, 64, dtype=torch.float16)
+    with pytest.warns(RuntimeWarning, match="_native.so"):
+        n = _lib.native()
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")  # (once is enough)
+        with _lib.diagnostic_build():
+            assert _lib.native() is n
+        for call in (lambda: ops.matmul(x, q, s, c, o, 64, 16, 64), lambda: ops.matmul_blockwise(x, q, s, c, o, 64, 16, 64, 64),
+                     lambda: ops.matmul_fused(x, q, s, c, o, 64, 16, 64, _lib.EPILOGUE_RESIDUAL, o),
+                     lambda: ops.matmul_multi([(x, q, s, c, o, 64, 16, 64)]), lambda: ops.matmul_grouped(x, q, s, c, o, 64, 1, 64, (0, 16)),
+                     lambda: ops.dequant(q, s, c, o, 64, 64), lambda: ops.quantize(x, c)):
+            with pytest.raises(ValueError, match="HIP device"):  # the Python op's own words for CPU tensors
+                call()
+
+
+@pytest.mark.gpu
+def test_without_the_extension_the_ops_give_the_same_bits(no_extension):
+    q, x, code, absmax = make_inputs_np(512, 16, 1024, seed=9)
+    q, x, c, s = to_dev(q, x, code, absmax)
+    o, o2 = (torch.empty(16, 512, dtype=torch.float16, device="cuda") for _ in range(2))
+    with pytest.warns(RuntimeWarning):
+        ops.matmul(x, q, s, c, o, 512, 16, 1024)
+    assert _lib.lib().tuna_matmul(*[t.data_ptr() for t in (q, x, c, s, o2)], 512, 16, 1024, torch.cuda.current_stream().cuda_stream) == _lib.OK
+    torch.cuda.synchronize()
+    assert torch.equal(o.view(torch.int16), o2.view(torch.int16))
 
 
 @pytest.mark.gpu

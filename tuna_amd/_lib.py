@@ -5,17 +5,19 @@ Both are built in-tree by ``make -C tuna_amd/csrc`` (see build()) from the same 
 diagnostic build adds timing loops, yardstick kernels and process-wide switches between kernels that
 compute identical results.  ``lib()`` is the library the ops call: the product library unless
 ``diagnostic_build()`` is active (bench.py, the tuner, A/B tests).  There is no fallback
-implementation: if a shared object is missing or does not load, every op raises.
+implementation: if one of the two is missing or does not load, every op raises.  Only the extension in front of them
+(_native.so, the same calls without ctypes) may be absent: native().
 """
 import contextlib
 import ctypes
+import importlib
 import os
 import subprocess
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtuna_amd.so")
 BENCH_LIB_PATH = os.path.join(_HERE, "libtuna_amd_bench.so")
-NATIVE_PATH = os.path.join(_HERE, "_native.so")
 CSRC = os.path.join(_HERE, "csrc")
 
 OK = 0
@@ -186,6 +188,18 @@ def lib():
     return _load(_active)
 
 
+class _NoExtension:
+    """What stands in for an extension that is not there: it declines every call, which the Python op then makes
+    through ctypes."""
+
+    @staticmethod
+    def _decline(*args):
+        return None
+
+    matmul = matmul_fused = matmul_blockwise = matmul_multi = matmul_grouped = dequant = quantize = _decline
+    bind = _decline
+
+
 def native():
     """tuna_amd/_native.so, bound to the active library: the ops' calls without a config (csrc/torch_binding.cpp)."""
     return _native or _bind_native()
@@ -195,11 +209,15 @@ def _bind_native():
     global _native
     import torch  # noqa: F401  (its libraries are what the extension links against)
 
-    if not os.path.exists(NATIVE_PATH):
-        raise RuntimeError(f"{NATIVE_PATH} is missing: build it with `make -C tuna_amd/csrc`")
-    from . import _native as mod
-
     L = lib()
+    if isinstance(_native, _NoExtension):
+        return _native
+    try:
+        mod = importlib.import_module(__package__ + "._native")
+    except ImportError as e:  # not built (no torch headers at build time), or built for another torch or Python
+        warnings.warn(f"tuna_amd/_native.so does not load ({e}): the ops take the ctypes path, which costs 5 to 7 us more "
+                      "per call; build it with `make -C tuna_amd/csrc`", RuntimeWarning, stacklevel=3)
+        mod = _NoExtension()
     mod.bind(tuple(ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in _NATIVE_ENTRIES))
     _native = mod
     return mod
