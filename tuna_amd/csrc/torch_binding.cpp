@@ -31,7 +31,7 @@ struct EntryPoints {
     decltype(&tuna_dequant_blockwise) dequant_blockwise;
     decltype(&tuna_quantize_blockwise) quantize_blockwise;
 };
-EntryPoints g_fn;  // written under the GIL only
+EntryPoints g_fn;  // written and read under the GIL only: a call takes its pointer before it lets go of the GIL
 constexpr int kEntryPoints = sizeof(EntryPoints) / sizeof(void *);
 
 // The arguments of one call.  The first tensor names the device; `ok` turns false at the first argument that the
@@ -81,7 +81,7 @@ private:
 
 constexpr at::ScalarType kHalf = at::kHalf, kByte = at::kByte, kFloat = at::kFloat;
 
-// The ABI call runs without the GIL, as it did through ctypes.
+// The ABI call runs without the GIL, as it did through ctypes.  (`call` holds its entry point by value.)
 template <class F>
 PyObject *status_of(F &&call)
 {
@@ -113,7 +113,7 @@ NATIVE_OP(matmul, 8)  // x, q, s, c, o, m, n, k
     void *s = g.tensor(a[2], kFloat, m), *c = g.tensor(a[3], kFloat, 16), *o = g.tensor(a[4], kHalf, (int64_t)n * m);
     if (!g.ok) Py_RETURN_NONE;
     void *st = g.stream();
-    return status_of([&] { return g_fn.matmul(q, x, c, s, o, m, n, k, st); });
+    return status_of([&, fn = g_fn.matmul] { return fn(q, x, c, s, o, m, n, k, st); });
 }
 
 NATIVE_OP(matmul_fused, 10)  // x, q, s, c, o, m, n, k, epilogue, residual or None
@@ -128,7 +128,7 @@ NATIVE_OP(matmul_fused, 10)  // x, q, s, c, o, m, n, k, epilogue, residual or No
     void *r = ep == TUNA_EPILOGUE_RESIDUAL ? g.tensor(a[9], kHalf, (int64_t)n * m) : nullptr;
     if (!g.ok) Py_RETURN_NONE;
     void *st = g.stream();
-    return status_of([&] { return g_fn.matmul_fused(q, x, c, s, o, m, n, k, nullptr, TUNA_DECODE_GEMM, ep, r, st); });
+    return status_of([&, fn = g_fn.matmul_fused] { return fn(q, x, c, s, o, m, n, k, nullptr, TUNA_DECODE_GEMM, ep, r, st); });
 }
 
 NATIVE_OP(matmul_blockwise, 9)  // x, q, s, c, o, m, n, k, block_size
@@ -143,7 +143,7 @@ NATIVE_OP(matmul_blockwise, 9)  // x, q, s, c, o, m, n, k, block_size
     void *o = g.tensor(a[4], kHalf, (int64_t)n * m);
     if (!g.ok) Py_RETURN_NONE;
     void *st = g.stream();
-    return status_of([&] { return g_fn.matmul_blockwise(q, x, c, s, o, m, n, k, bs, st); });
+    return status_of([&, fn = g_fn.matmul_blockwise] { return fn(q, x, c, s, o, m, n, k, bs, st); });
 }
 
 NATIVE_OP(matmul_multi, 1)  // list or tuple of (x, q, s, c, o, m, n, k) tuples
@@ -167,7 +167,7 @@ NATIVE_OP(matmul_multi, 1)  // list or tuple of (x, q, s, c, o, m, n, k) tuples
     }
     if (!g.ok || !count) Py_RETURN_NONE;
     void *st = g.stream();
-    return status_of([&] { return g_fn.matmul_multi(p.data(), (int)count, st); });
+    return status_of([&, fn = g_fn.matmul_multi] { return fn(p.data(), (int)count, st); });
 }
 
 NATIVE_OP(matmul_grouped, 9)  // x, q, s, c, o, m_group, n_groups, k, token_offsets (list or tuple)
@@ -184,7 +184,7 @@ NATIVE_OP(matmul_grouped, 9)  // x, q, s, c, o, m_group, n_groups, k, token_offs
     void *c = g.tensor(a[3], kFloat, 16), *o = g.tensor(a[4], kHalf, n * m);
     if (!g.ok) Py_RETURN_NONE;
     void *st = g.stream();
-    return status_of([&] { return g_fn.matmul_grouped(q, x, c, s, o, m, groups, k, offs.data(), nullptr, TUNA_DECODE_GEMM, st); });
+    return status_of([&, fn = g_fn.matmul_grouped] { return fn(q, x, c, s, o, m, groups, k, offs.data(), nullptr, TUNA_DECODE_GEMM, st); });
 }
 
 NATIVE_OP(dequant, 7)  // q, absmax, codebook, o, m, k, block_size or None
@@ -197,8 +197,8 @@ NATIVE_OP(dequant, 7)  // q, absmax, codebook, o, m, k, block_size or None
     void *c = g.tensor(a[2], kFloat, 16), *o = g.tensor(a[3], kHalf, (int64_t)m * k);
     if (!g.ok) Py_RETURN_NONE;
     void *st = g.stream();
-    return status_of([&] {
-        return bs == k ? g_fn.dequant(q, s, c, o, m, k, st) : g_fn.dequant_blockwise(q, s, c, o, m, k, bs, TUNA_DECODE_DEQUANT, st);
+    return status_of([&, per_row = g_fn.dequant, blockwise = g_fn.dequant_blockwise] {
+        return bs == k ? per_row(q, s, c, o, m, k, st) : blockwise(q, s, c, o, m, k, bs, TUNA_DECODE_DEQUANT, st);
     });
 }
 
@@ -216,8 +216,9 @@ NATIVE_OP(quantize, 3)  // w, codebook, block_size or None -> (status, q, absmax
     at::Tensor q = at::empty({m / 8, k / 8, 32}, wt.options().dtype(kByte));
     at::Tensor absmax = a[2] == Py_None ? at::empty({m}, wt.options().dtype(kFloat)) : at::empty({m, k / bs}, wt.options().dtype(kFloat));
     void *st = g.stream(), *qp = q.data_ptr(), *ap = absmax.data_ptr();
+    const auto fn = g_fn.quantize_blockwise;
     int rc;
-    Py_BEGIN_ALLOW_THREADS rc = g_fn.quantize_blockwise(w, c, qp, ap, m, k, bs, st);
+    Py_BEGIN_ALLOW_THREADS rc = fn(w, c, qp, ap, m, k, bs, st);
     Py_END_ALLOW_THREADS
     return Py_BuildValue("iNN", rc, THPVariable_Wrap(std::move(q)), THPVariable_Wrap(std::move(absmax)));
 }
