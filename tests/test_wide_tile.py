@@ -1,9 +1,9 @@
 """The 256 x 256 many-token tile (csrc/gemm_wide.hip): tiles whole, split, and shared between workgroups; groups in one
-launch; scale blocks.  Against the oracle on a subset of rows, and deterministic."""
+launch; scale blocks.  Whole outputs against float64 sums, a subset of rows against the oracle, and deterministic."""
 import numpy as np
 import pytest
 
-from helpers import O, REL_TOL, f16_bits_to_f64, rel_err
+from helpers import O, REL_FLOOR, REL_TOL, f16_bits_to_f64, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -29,12 +29,27 @@ def _out(n, m):
     return torch.full((n, m), float("nan"), dtype=torch.float16, device="cuda")
 
 
+def _f64_sums(q, s, x, code, k, block):
+    """x @ decode(q, code, s)^T in float64 (weights: an fp16 code times an fp16 scale, rounded to fp16), in plain torch."""
+    import torch
+
+    nib = torch.stack((q >> 4, q & 15), dim=-1).view(-1, k // 8, 8, 8)          # block row, block column, row, column
+    nib = nib.permute(0, 2, 1, 3).reshape(-1, k).long()
+    scale = s.half().view(nib.shape[0], -1).repeat_interleave(block or k, dim=1)
+    return x.double() @ (code.half()[nib] * scale).double().t().contiguous()
+
+
 def _check(out, q, s, x, code, k, blocks=6, block=0, first_row=0, rows=None):
-    """Rows of `blocks` random block rows (and the last one) of out against the oracle's float64 sums."""
+    """All of out against float64 sums in torch; rows of `blocks` random block rows (and the last one) against the oracle's,
+    whose decode is another implementation."""
     import torch
 
     m = rows or out.shape[1]
     assert not torch.isnan(out).any()
+    own = slice(first_row, first_row + m)
+    sums = _f64_sums(q[first_row // 8:(first_row + m) // 8], s[own], x, code, k, block)
+    den = sums.abs().clamp_min(REL_FLOOR * float(sums.abs().max()))
+    assert float(((out.double() - sums).abs() / den).max()) <= REL_TOL
     rng = np.random.default_rng(m + out.shape[0])
     mbs = np.unique(np.append(rng.choice(m // 8, size=min(blocks, m // 8), replace=False), m // 8 - 1))
     rs = (mbs[:, None] * 8 + np.arange(8)[None, :]).ravel()
