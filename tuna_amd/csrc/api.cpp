@@ -70,7 +70,7 @@ static int plan_gemm(int m, int n, int k, const tuna_gemm_config &c, int decode,
     if (decode != TUNA_DECODE_GEMM && decode != TUNA_DECODE_DEQUANT)
         return fail(TUNA_ERR_INVALID_ARG, "decode_mode %d is neither TUNA_DECODE_GEMM nor TUNA_DECODE_DEQUANT", decode);
     if (c.lds_tile_rows > 0) return fail(TUNA_ERR_INVALID_ARG, "plan_gemm called with a many-token config");
-    if (c.lds_tile_rows < -1) return fail(TUNA_ERR_INVALID_ARG, "lds_tile_rows=%d (0, -1, -4, 64, 128 or 256)", c.lds_tile_rows);
+    if (c.lds_tile_rows < -1) return fail(TUNA_ERR_INVALID_ARG, "lds_tile_rows=%d (0, -1, -4, -5, 64, 128 or 256)", c.lds_tile_rows);
     if (c.rows_per_wave != 64 && c.rows_per_wave != 128 && c.rows_per_wave != 256)
         return fail(TUNA_ERR_UNSUPPORTED, "rows_per_wave=%d (64, 128 or 256)", c.rows_per_wave);
     if (c.prefetch != 2 && c.prefetch != 4 && c.prefetch != 8)
