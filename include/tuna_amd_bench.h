@@ -123,6 +123,10 @@ int tuna_time_unit_rate(int unit, void *sink, int warmup, int iters, void *strea
  * uint64; counts[0] receives the pairs checked, counts[1] the mismatches. */
 int tuna_selftest_quantizer_division(void *counts, void *stream);
 
+/* Microseconds that the selection's launch models give `cfg` on the shape (block_size 0: a scale per row), 0 if it names a
+ * kernel they do not price.  Host only; tuna_amd/launch_models.py times launches against it. */
+double tuna_predicted_us(int m, int n, int k, int block_size, const tuna_gemm_config *cfg);
+
 /* Host check of the weight loads of the 256-row kernels - kernel 0: the decode-batch kernel, 1: the 256 x 256 many-token
  * kernel - for the threads, k-steps and halves of row tile `row_tile` of an m x k matrix, from the functions the kernels
  * themselves take their offsets from.  out4 receives: loads that reach behind the weights although a descriptor's range

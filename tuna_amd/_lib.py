@@ -126,6 +126,7 @@ BENCH_SIGNATURES = {
     "tuna_time_read": (_i, [_vp, _vp, _sz, _i, _i, _i, _i, _vp, _fp]),
     "tuna_time_unit_rate": (_i, [_i, _vp, _i, _i, _vp, _fp, ctypes.POINTER(ctypes.c_double)]),
     "tuna_selftest_quantizer_division": (_i, [_vp, _vp]),
+    "tuna_predicted_us": (ctypes.c_double, [_i, _i, _i, _i, _cfgp]),
     "tuna_check_weight_reach": (_i, [_i, _i, _i, _i, ctypes.POINTER(ctypes.c_longlong)]),
     "tuna_set_multi_shape": (_i, [_i, _i]),
     "tuna_set_multi_min_batch": (_i, [_i]),

@@ -628,7 +628,8 @@ static bool narrow_round(int m, int n, int k, tuna_gemm_config *out)
 
 
 // Microseconds of a launch of 256 x 256 many-token tiles (gemm_wide.hip) by a model read off 320 random shapes of 1024 ...
-// 57344 rows and 65 ... 4096 tokens (six per cent off on average where the tile is within half of the best): a k-step of
+// 57344 rows and 65 ... 4096 tokens (14 per cent off on average, and at 0.89 of the measured time, on the 323 launches kept in
+// profiles/launch_model_times.csv, which tuna_amd/launch_models.py times and fits models to, this one and those below): a k-step of
 // a tile takes longer the more workgroups share the chip's power, a whole tile ends with 12 us of stores, a shared one
 // with as long for the partial sums and more for every further share of it.  split: 1 whole tiles, 2 ... that many equal shares of
 // every tile, 0 the last rounds of tiles shared evenly between the compute units.
@@ -1010,7 +1011,7 @@ static bool config_runs(int m, int n, int k, const tuna_gemm_config &c)
 
 // Microseconds of a launch of the decode-batch kernel (gemm_flow.hip) with `tiles` 256-row tiles of `units` units of k in
 // `shares` workgroups, by a model read off 600 random shapes of 6 ... 390 MB of weights at 1 ... 64 tokens, each with up to
-// ten numbers of shares (8 per cent off on average): a k-step takes longer with more token tiles and with two workgroups on
+// ten numbers of shares (9.7 per cent off on average on the 440 launches kept): a k-step takes longer with more token tiles and with two workgroups on
 // a compute unit, a tile that several shares contribute to is handed over, which costs more with every contributor beyond
 // the second.
 static double flow_time(double tiles, int units, int nt, int shares)
@@ -1074,10 +1075,10 @@ static bool flow_instead(int m, int n, int k, const tuna_gemm_config &c, bool fr
 }
 
 // Microseconds of a launch of the narrow-row kernel, by a model read off 350 random shapes of 0.5 ... 100 MB of weights at
-// 1 ... 64 tokens, each timed with up to 37 variants for any k (6.5 per cent off on average; the variants for whole ring
-// turns are a tenth faster): the busiest compute unit's work, a workgroup's chain of ring turns and the weights' stream -
+// 1 ... 64 tokens, each timed with up to 37 variants for any k (10.5 per cent off on average on the 440 launches kept; the
+// variants for whole ring turns are a tenth faster): the busiest compute unit's work, a workgroup's chain of ring turns and the weights' stream -
 // whichever is longest, smoothly - and x, which every workgroup reads.
-// nblk > 0: that many scales per row, kept in LDS where they fit (280 shapes with blocks of 64 and 128, 7 per cent).
+// nblk > 0: that many scales per row, kept in LDS where they fit (280 shapes with blocks of 64 and 128; 7.1 per cent on 440 launches).
 static double narrow_time(int m, int n, int k, int rows, int waves_k, int u, int tt, int nblk = 0)
 {
     struct Coef { double launch, round, step, rows, tokens, both, turn, ring, stream, x, scale_loads, scale_kb; };
@@ -1097,6 +1098,17 @@ static double narrow_time(int m, int n, int k, int rows, int waves_k, int u, int
     const double x_bytes = wgs * k * (n < 16 * tt ? n : 16 * tt) * 2e-6;
     return c.launch + (c.round + (in_lds ? c.scale_kb * 1e-3 * scales : 0.0)) * rounds +
            std::cbrt(work * work * work + chain * chain * chain + stream * stream * stream) + c.x * x_bytes;
+}
+
+double predicted_us(int m, int n, int k, const tuna_gemm_config &c, int nblk)
+{
+    if (is_flow(c)) return flow_time(ceil_div(m, 256), ceil_div(ceil_div(k, 64), 4), c.token_tiles, c.split_k);
+    if (is_narrow_any(c) || is_narrow(c)) return narrow_time(m, n, k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles, nblk);
+    if (c.lds_tile_rows == 256 && c.token_tiles == 16 && c.rows_per_wave != 32) {
+        const WideTiles t(m, n, k);
+        return wide_time(t.large, t.small, t.steps, c.split_k == 1 && wide_balance_pays(m, n, k) ? 0 : c.split_k);
+    }
+    return 0.0;
 }
 
 // The variant for any m and k with the least predicted time below `limit` us.
@@ -1121,8 +1133,8 @@ static bool best_narrow_any(int m, int n, int k, int nblk, double limit, tuna_ge
 // Up to 64 tokens, ahead of the config `c` picked so far (`flow_us`: the decode-batch kernel's predicted time if that is
 // it): the narrow-row kernel's variants for any m and k, where their model is a tenth under that config's price - the
 // narrow-row kernel's own model, or a straight line in the megabytes read off the same shapes (general kernel, many-token
-// tiles).  1192 x 2000 at one token 9.1 -> 3.2 us, 4672 x 1720 14.8 -> 4.3, 8576 x 9856 at 5 tokens 30.5 -> 15.1, 1792 x
-// 4104 at 19 tokens 16.6 -> 6.1, 5824 x 4736 at 34 tokens 24.7 -> 15.0; 1.42 x on average over those shapes.  Streaming and lean
+// tiles).  1192 x 2000 at one token 9.1 -> 3.0 us, 4672 x 1720 14.3 -> 4.2, 8576 x 9856 at 5 tokens 31.0 -> 14.8, 1792 x
+// 4104 at 19 tokens 16.7 -> 6.6, 5824 x 4736 at 34 tokens 23.4 -> 16.5; 1.42 x on average over those shapes.  Streaming and lean
 // launches, and a table's entries that are narrow-row ones, are left alone.
 static bool narrow_any_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, double flow_us, tuna_gemm_config *any)
 {
@@ -1145,7 +1157,7 @@ static bool narrow_any_instead(int m, int n, int k, const tuna_gemm_config &c, b
 
 // What a launch without an explicit config runs from 65 tokens on: the selected config, or 256 x 256 tiles of gemm_wide.hip
 // in its place where their model is ahead of the grid cost model's price of that config by more than the models' error
-// (26624 x 5888 at 665 tokens 277 -> 201 us, 4096 x 14336 at 777 tokens 134 -> 116, 46848 x 5120 at 295 tokens 208 -> 166;
+// (26624 x 5888 at 665 tokens 265 -> 219 us, 4096 x 14336 at 777 tokens 135 -> 117, 46848 x 5120 at 295 tokens 205 -> 175;
 // the table and the cost model were measured before that kernel and still pick the best of the other tiles).  Configs of
 // kernels that the model does not price - narrow rows, k split over lean workgroups - are left alone: they are picked
 // for shapes too small for such tiles.
@@ -1557,7 +1569,7 @@ static bool plan_multi(const tuna_gemm_problem *problems, int count, int cus, Mu
 
 // A dense launch the batched kernel (gemm_multi.hpp) takes as a batch of one: balanced split, 64 rows
 // per wave, 16 waves, one token tile, the GEMM's own decode, any epilogue (8192 x 28672 at 16 tokens with a
-// residual: 29 us, 47 in gemm_kernel).  (plan_multi checks the shape's alignment.)  A diagnostic build can turn it off together with the other twins (diag.h).
+// residual: 29 us, 43 in gemm_kernel).  (plan_multi checks the shape's alignment.)  A diagnostic build can turn it off together with the other twins (diag.h).
 static bool stream_applies(const tuna_gemm_config &c, int n, int decode)
 {
     return c.split_k == 0 && !c.lds_tile_rows && c.rows_per_wave == kRowsPerLoad && c.waves_m >= 1 && c.waves_m * c.waves_k == 16 &&
@@ -1767,7 +1779,7 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
     // hundreds of microseconds of matrix work.  (With an explicit config every group goes through the grouped kernel.)
     // Several such groups become ONE launch of 256 x 256 tiles (gemm_wide.hip) where that is predicted to be faster than a
     // launch each, priced at 6 us and the larger of 0.85 PFLOP/s and 3.5 TB/s: eight experts of 14336 x 4096 on 4096
-    // tokens leave the device half empty at the end of each of eight launches (711 us; 616 with 256 x 256 tiles in each).
+    // tokens leave the device half empty at the end of each of eight launches (706 us; 452 in one).
     constexpr int kGroupedPassTokens = 64;
     const size_t group_q_bytes = (size_t)m_group * (size_t)k / 2;
     bool many_done = false;
@@ -2384,8 +2396,8 @@ static int derive_blockwise(const BlockwiseCall &b, const Room &room, tuna_gemm_
             }
         // The 256 x 256 tile by its own model, 1.07 x the time of the per-row kernel (a unit of the costs above is 5.68e-7
         // us per k, both read off 200 random shapes at 65 ... 4096 tokens with blocks of 64, where this tile is up to
-        // 1.8 x faster than the best of the others: 3584 x 25088 at 2669 tokens 774 us -> 416, 5632 x 16384 at 701 tokens
-        // 236 -> 149, 11136 x 1536 at 2891 tokens 173 -> 118).
+        // 1.6 x faster than the best of the others: 3584 x 25088 at 2669 tokens 756 us -> 462, 5632 x 16384 at 701 tokens
+        // 232 -> 159, 11136 x 1536 at 2891 tokens 158 -> 121).
         const WideTiles t(m, n, k);
         double us = 0.0;
         const int split = n > 64 ? wide_best_split(t.large, t.small, t.steps, room, &us) : 0;
@@ -2495,8 +2507,8 @@ static int check_blockwise_call(const BlockwiseCall &b, bool pointers)
 
 // What a call without a config runs: the selected config, or up to 64 tokens the narrow-row kernel's variants for any k in
 // its place where their model is an eighth under the selected config's price - that model for a narrow-row pick, a straight
-// line for many-token tiles (9984 x 7936 at 2 tokens, which no ring turn of more than four waves divides, 38.8 -> 13 us;
-// 2048 x 8960 at 7 tokens 18.9 -> 9.9, 13120 x 23296 at 9 tokens 197 -> 54; 1.30 x on average over 280 random shapes).
+// line for many-token tiles (9984 x 7936 at 2 tokens, which no ring turn of more than four waves divides, 38.7 -> 15.3 us;
+// 2048 x 8960 at 7 tokens 22.0 -> 10.0, 13120 x 23296 at 9 tokens 197 -> 53; 1.30 x on average over 280 random shapes).
 static int select_blockwise_launch(const BlockwiseCall &b, const Room &room, tuna_gemm_config *c)
 {
     int from_table = 0;

@@ -341,6 +341,11 @@ TUNA_EXPORT int tuna_selftest_quantizer_division(void *counts, void *stream)
     return TUNA_OK;
 }
 
+TUNA_EXPORT double tuna_predicted_us(int m, int n, int k, int block_size, const tuna_gemm_config *cfg)
+{
+    return cfg ? predicted_us(m, n, k, *cfg, block_size && block_size < k ? k / block_size : 0) : 0.0;
+}
+
 TUNA_EXPORT int tuna_check_weight_reach(int kernel, int m, int k, int row_tile, long long *out4)
 {
     if (!out4 || kernel < 0 || kernel > 1 || m < 8 || m % 8 || k < 8 || k % 8 || row_tile < 0 || row_tile >= (m + 255) / 256)

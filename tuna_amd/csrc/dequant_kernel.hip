@@ -139,9 +139,10 @@ hipError_t launch_dequant(const uint8_t *q, const float *absmax, const float *co
 // argmin's result, since |nv - c| is monotonic in c on either side of nv; any other codebook takes the 16 comparisons.
 // The division by the block maximum is a multiply by its refined reciprocal and one fused correction.
 //
-// What bounds it: at 14336 x 4096 with blocks of 64 (177 MB of traffic) HBM and the vector ALU together, ten instructions a
-// weight: 62 -> 35 us, with one scale per row 54 -> 34; 8192 x 28672 in blocks of 64 238 -> 117 us (4.9 TB/s), 4096 x 14336
-// per row 61 -> 36; 3 us before the first table is complete.
+// What bounds it: at 14336 x 4096 with blocks of 64 (151 MB of traffic) the vector ALUs, busy 90 % of the launch at 1.80 GHz
+// with sixteen instructions a weight: 62.5 -> 32.3 us against the version that passed block rows through LDS, with one scale
+// per row 53.1 -> 32.1; 8192 x 28672 in blocks of 64 224 -> 114 us (5.3 TB/s), 4096 x 14336 per row 56 -> 35; 3 us before the
+// first table is complete.
 // Nearest entry of a sorted codebook: bnd[i] (i = 0..14) is the smallest binary32 value that the
 // argmin assigns to entry i + 1 rather than entry i, so the index is the number of boundaries <= nv:
 // a 4-step binary search, as a tree of selects over the 15 values (uniform, held in registers).

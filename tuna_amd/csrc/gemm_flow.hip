@@ -1,7 +1,7 @@
 // FP16-activation x 4-bit-codebook-weight GEMM for a decode batch (up to 64 tokens, or that many per group of a grouped
 // launch) over many rows: the k-steps of all 256-row tiles are laid end to end and divided evenly over the workgroups.
 //
-//   * Four waves of 64 rows x all tokens (1 .. 4 token tiles of 16) per workgroup, two workgroups per compute unit.  As in
+//   * Four waves of 64 rows x all tokens (1 .. 4 token tiles of 16) per workgroup, up to two workgroups per compute unit.  As in
 //     gemm_wide.hip a dword of the packed layout, through the decode table and scaled, is a lane's MFMA operand, and the
 //     work of a k-step is one even sequence: per byte pair one scaling, one address, one table read, the MFMAs and fragment
 //     reads dealt out between them, one barrier.
@@ -11,11 +11,13 @@
 //   * The table (a copy per 32 lanes) takes the lower half of every 256 bytes of LDS and the activations' three stages the
 //     upper halves: 64 KB in all.
 //
-// What bounds it: with two workgroups on a compute unit, HBM and the LDS together (16 tokens, 57344 x 8192: the loop streams
-// 6.7 TB/s; builds without table reads or without MFMAs are no faster), at 64 tokens the LDS; around the loop 3 us until
-// the first steps have arrived and 3 .. 8 us for handing over tiles that several shares contribute to.  Against the kernels
-// the launches took before (general, streaming, many-token): 17920 x 23168 at 30 tokens 155 -> 65 us, 32128 x 13312 at 36
-// tokens 138 -> 65, 28672 x 8192 at 37 tokens 50 -> 41; eight experts of 28672 x 4096 on 128 tokens 142 -> 126.
+// What bounds it: no single unit.  With one workgroup on a compute unit (256 shares: 28672 x 8192 at 37 tokens, eight experts
+// of 28672 x 4096 at 16 each) the LDS is busy 28 .. 31 % of the cycles, the vector ALUs 23 .. 29 %, the matrix pipes 12 .. 21 %,
+// HBM streams 2.8 .. 3.9 TB/s and the waves wait 40 % of their time at a counter or barrier; a second workgroup fills some
+// of that (229376 x 4096 at 16 tokens 107 us on 256 shares, 89 on 512: 5.3 TB/s).  Around the loop 6 us in all, and 3 .. 8
+// for handing over tiles that several shares contribute to.  Against the kernels the launches took before (general, streaming,
+// many-token; one box, launch loop): 17920 x 23168 at 30 tokens 154 -> 60 us, 32128 x 13312 at 36 tokens 129 -> 68, 28672 x
+// 8192 at 37 tokens 51 -> 43; eight experts of 28672 x 4096 on 128 tokens 148 -> 128.
 #include "epilogue.hpp"
 
 namespace tuna {

@@ -10,10 +10,10 @@
 //   * The work of a k-step is spread evenly between its 128 MFMAs: per token tile (4 MFMAs) one fragment read, one table
 //     read, one address, one scaling; every fourth a 16-byte store and load of activations.  One barrier per step.
 //
-// What bounds it: the power limit.  The matrix pipes are busy 72 % of the cycles (57 % in the kernel this one replaced,
-// which passed the decoded weights through an LDS tile: 19 % more LDS time and 0.5 more instructions per MFMA), at a
-// clock that the chip lowers to about 1.7 GHz; 8192 x 8192 at 2048 tokens 250 -> 213 us (1.29 PFLOP/s), 6144 x 4096 at
-// 2000 tokens 125 -> 99, 28672 x 4096 at 2000 tokens 466 -> 408 (same boxes).
+// What bounds it: the power limit.  The matrix pipes are busy 68 % of the cycles (57 % in the kernel this one replaced,
+// which passed the decoded weights through an LDS tile: 22 % more LDS time and 0.3 more instructions per MFMA), at a
+// clock that the chip lowers to 1.72 GHz (1.89); 8192 x 8192 at 2048 tokens 235 -> 216 us (1.27 PFLOP/s), 6144 x 4096 at
+// 2000 tokens 108 -> 100, 28672 x 4096 at 2000 tokens 447 -> 385 (one box, launch loop).
 //
 // Tiles of 1 .. 128 tokens (the last of a group) run the same steps with half the token tiles.  How tiles become
 // workgroups is plan_gemm_wide's choice.  KTAIL: k is any multiple of 8 - the slots of the last k-step beyond k load

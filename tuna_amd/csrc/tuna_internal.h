@@ -343,6 +343,10 @@ int hip_fail(hipError_t e, const char *what);
 int check_ptr(const void *p, const char *name, size_t align);
 void drop_workspace(hipStream_t stream);  // frees the split-K workspace of a stream that is about to be destroyed
 
+// api.cpp: microseconds that the launch models give a config of the kernels they price (nblk: scales per row of a launch
+// with scale blocks, 0 without), 0 for one of another kernel
+double predicted_us(int m, int n, int k, const tuna_gemm_config &c, int nblk);
+
 // config_table.cpp
 struct TableEntry {
     int m, n_lo, n_hi, k;
