@@ -1677,6 +1677,14 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
     return TUNA_OK;
 }
 
+// Whether the general kernel's grouped variants can run a config as it stands.
+static bool grouped_runs(int m_group, int m_active, int max_tok, int k, int decode, const tuna_gemm_config &c, GemmPlan *plan)
+{
+    if (c.lds_tile_rows || is_narrow(c) || c.waves_m < 1 || c.rows_per_wave != kRowsPerLoad) return false;
+    if (m_group % (c.rows_per_wave * c.waves_m)) return false;
+    return plan_gemm(m_active, max_tok, k, c, decode, plan, 1) == TUNA_OK;
+}
+
 // Config of a grouped launch chosen by the library.  Candidates, in order: the tuned entry for the
 // active rows if it is a streaming config the grouped variants can run as it stands; the derived
 // streaming config with its row tile shrunk until it divides m_group; one 64-row group per
@@ -1684,11 +1692,7 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
 // narrow-row, many-token or deep-ring entry has no grouped counterpart.
 static int grouped_config(int m_group, int m_active, int max_tok, int k, int decode, tuna_gemm_config *out, GemmPlan *plan)
 {
-    auto runs = [&](const tuna_gemm_config &c) {
-        if (c.lds_tile_rows || is_narrow(c) || c.waves_m < 1 || c.rows_per_wave != kRowsPerLoad) return false;
-        if (m_group % (c.rows_per_wave * c.waves_m)) return false;
-        return plan_gemm(m_active, max_tok, k, c, decode, plan, 1) == TUNA_OK;
-    };
+    auto runs = [&](const tuna_gemm_config &c) { return grouped_runs(m_group, m_active, max_tok, k, decode, c, plan); };
     tuna_gemm_config c;
     if (decode == TUNA_DECODE_GEMM) {
         select_config(m_active, max_tok, k, &c, nullptr);
@@ -1729,6 +1733,20 @@ static int grouped_config(int m_group, int m_active, int max_tok, int k, int dec
     }
     return fail(TUNA_ERR_UNSUPPORTED, "no grouped config for m_group=%d, %d active rows, %d tokens, k=%d: %s", m_group, m_active,
                 max_tok, k, std::string(g_error).c_str());
+}
+
+// Whether up to 16 tokens per group the table holds an entry for the active rows that the grouped variants can run: tuned
+// for these very rows, it stays ahead of the decode-batch kernel (eight experts of 28672 x 4096 with 4 tokens each 82 us
+// against 112, with 16 each 85 against 115; with 24 each, past that entry, 149 against 127).
+static bool grouped_entry_runs(int m_group, int m_active, int max_tok, int k)
+{
+    bool has = false;
+    for (int i = 0; i < kConfigTableSize && !has; ++i) has = kConfigTable[i].m == m_active && kConfigTable[i].k == k;
+    tuna_gemm_config c;
+    int hit = 0;
+    GemmPlan plan;
+    return has && max_tok <= 16 && select_config(m_active, max_tok, k, &c, &hit) == TUNA_OK && hit &&
+           grouped_runs(m_group, m_active, max_tok, k, TUNA_DECODE_GEMM, c, &plan);
 }
 
 // Shares of a grouped launch of the decode-batch kernel; 0 for the smallest launches of up to 16 tokens per group, which
@@ -1861,7 +1879,7 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
         FlowArgs &f = fp.args;
         f.m = m_group, f.m_total = m, f.k = k, f.n_groups = n_active;
         for (int e = 0; e < n_active; ++e) f.tok_begin[e] = offsets[act[e]], f.tok_count[e] = offsets[act[e] + 1] - offsets[act[e]], f.id[e] = act[e];
-        const int nt = ceil_div(max_tok, 16), shares = grouped_flow_shares(m_group, n_active, nt, k);
+        const int nt = ceil_div(max_tok, 16), shares = grouped_entry_runs(m_group, m_active, max_tok, k) ? 0 : grouped_flow_shares(m_group, n_active, nt, k);
         if (shares && plan_gemm_flow(nt, shares, &fp)) {
             // (partial sums behind those of the launch above, where there is room: a line that a compute unit of another XCD
             // wrote last costs more to write - groups of 52 to 114 tokens, 1920 x 3968: this launch 22.7 us over the other's
