@@ -208,9 +208,10 @@ int tuna_matmul_multi_blockwise(const tuna_gemm_problem *problems, int count, in
  * during the call; n_total = token_offsets[n_groups]).  out [n_total, m_group]:
  *   out[t, r] = x[t, :] . decode(W_e)[r, :]   for t in group e.
  * Groups without tokens are skipped: their weights are not read.  m_group must be a multiple
- * of 64 (of the config's rows per workgroup if cfg is given; NULL = table lookup on
- * (n_groups*m_group, largest group, k)).  With cfg NULL the groups of more than 64 tokens (prefill
- * sizes) leave the grouped launch, which would stream their weights once per 64 tokens: each runs
+ * of 64 (of the config's rows per workgroup if cfg is given).  With cfg NULL groups of up to 64
+ * tokens run in one launch of the decode-batch kernel - or of the general kernel's grouped variants: where the table
+ * has an entry for the active rows and no group more than 16 tokens, for the smallest calls, and where the workspace
+ * cannot grow -, and the groups of more than 64 tokens (prefill sizes) leave the grouped launch, which would stream their weights once per 64 tokens: each runs
  * as a dense GEMM of its own on the same stream - tuna_matmul on its slices of q, absmax, x and
  * out, bit-identical to that call - or, several of them where that is predicted to be faster, all
  * in one launch of 256 x 256 tiles, within the GEMM's tolerance of it.  No counterpart in the reference, whose 8-expert
