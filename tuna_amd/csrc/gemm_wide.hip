@@ -6,21 +6,22 @@
 //     lane, one dword of it - eight byte pairs through the decode table, scaled - IS a lane's weight operand of one
 //     MFMA: no weight tile in LDS, and every weight is decoded once per 256 tokens.
 //   * Only the activations go through LDS, in a ring of three k-steps of [token][64 k] (128-byte rows, 16-byte slots
-//     XOR-swizzled with token & 7: no bank conflicts), 32 KB each beside the decode table's 64 KB.
+//     XOR-swizzled with token & 7: no bank conflicts), 32 KB each beside the decode table's 64 KB.  They are loaded into LDS
+//     directly (lds_dma.hpp): through registers they took the path that LDS reads return their data over.
 //   * The work of a k-step is spread evenly between its 128 MFMAs: per token tile (4 MFMAs) one fragment read, one table
-//     read, one address, one scaling; every fourth a 16-byte store and load of activations.  One barrier per step.
+//     read, one address, one scaling; the loads behind the step's one barrier.
 //
-// What bounds it: the power limit.  The matrix pipes are busy 68 % of the cycles (57 % in the kernel this one replaced,
-// which passed the decoded weights through an LDS tile: 22 % more LDS time and 0.3 more instructions per MFMA), at a
-// clock that the chip lowers to 1.72 GHz (1.89); 8192 x 8192 at 2048 tokens 235 -> 216 us (1.27 PFLOP/s), 6144 x 4096 at
-// 2000 tokens 108 -> 100, 28672 x 4096 at 2000 tokens 447 -> 385 (one box, launch loop).
+// What bounds it: the power limit.  The matrix pipes are busy 75 % of the cycles at a clock that the chip lowers to 1.68 GHz;
+// with the activations loaded into registers and stored to LDS they were busy 68 % at 1.72 GHz.  8192 x 8192 at 2048 tokens
+// 241 -> 224 us, 28672 x 4096 at 2000 tokens 403 -> 381, 4096 x 14336 at 2000 200 -> 190, 6144 x 4096 at 2000 101 -> 93,
+// 8192 x 8200 at 4096 468 -> 420 (one box, launch loop; torch's fp16 product of the first two shapes takes 187 and 367).
 //
 // Tiles of 1 .. 128 tokens (the last of a group) run the same steps with half the token tiles.  How tiles become
 // workgroups is plan_gemm_wide's choice.  KTAIL: k is any multiple of 8 - the slots of the last k-step beyond k load
-// the last slot inside k (no access leaves a row), and their activations are stored as zeros.  BLK: one scale per block
+// the last slot inside k (no access leaves a row), and their activations are zeros.  BLK: one scale per block
 // of a row.  Decode and rounding are those of the other kernels (bit-identical to kernel.cu:2178-2192); an unshared
 // tile's sums are the same products in the same order as the 16 x 16 x 32 variants of gemm_tiled.hip.
-#include "epilogue.hpp"
+#include "lds_dma.hpp"
 
 namespace tuna {
 
@@ -45,6 +46,7 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
     constexpr int XP = NT / 2;  // 16-byte pieces of a step's activations a thread stages
     constexpr int FB = 8;       // token fragments on their way (the ring: 2 NT tiles of a step divide into it)
     constexpr int LPT = 16 / NT; // table reads per token tile and half
+    constexpr int T_NEXT = 13 / LPT; // the token tile from which on the table reads of a half are the one after next's
     static_assert(NT == 16 || NT == 8, "token tiles");
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -57,76 +59,63 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
     // step (rows beyond the matrix are clamped: their products are never stored)
     const int row_w = w.row_base + wave * 64;
     const uint32_t a_off = tile_weight_lane(tid, ((w.m - w.row_base) >> 3) - 1, kb_total);
-    // activations: piece i of a thread is token tid / 8 + 32 i, 8-k slot tid % 8 (tokens beyond the tile's read its last)
+    // activations: piece i of a thread is token tid / 8 + 32 i (tokens beyond the tile's read its last), the 8-k slot that
+    // belongs at place tid % 8 of that token's row of the stage
+    const int x_slot = (tid & 7) ^ ((tid >> 3) & 7);
     uint32_t x_off[XP];
 #pragma unroll
-    for (int i = 0; i < XP; ++i) x_off[i] = ((uint32_t)min((tid >> 3) + 32 * i, w.tokens - 1) * (uint32_t)w.k + (uint32_t)(tid & 7) * 8u) * 2u;
-    unsigned char *const x_dst = xs + (tid >> 3) * 128 + (((tid & 7) ^ ((tid >> 3) & 7)) << 4);
-    // KTAIL: slots of the last step beyond k load the last slot inside k, and their activations are stored as zeros
-    const int x_k_left = w.k - (tid & 7) * 8;
+    for (int i = 0; i < XP; ++i) x_off[i] = ((uint32_t)min((tid >> 3) + 32 * i, w.tokens - 1) * (uint32_t)w.k + (uint32_t)x_slot * 8u) * 2u;
+    const uint32_t xs_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)xs + (uint32_t)wave * 1024u;
+    // KTAIL: slots of the last step beyond k load the last slot inside k, and their activations are requested out of range:
+    // zeros
     const int slot_last = ((w.k >> 3) - 1) & 7;
-    const uint32_t x_back = KTAIL ? (uint32_t)max(0, (tid & 7) - slot_last) * 16u : 0u;
+    const uint32_t x_beyond = KTAIL && x_slot > slot_last ? 0x7fffffffu : 0u;
     const uint32_t a_back0 = KTAIL ? (uint32_t)wide_weight_back(tid, 0, slot_last) : 0u;
     const uint32_t a_back1 = KTAIL ? (uint32_t)wide_weight_back(tid, 1, slot_last) : 0u;
 
-    const size_t q_rest = (size_t)(w.m - w.row_base) * (size_t)(w.k >> 1), x_rest = (size_t)w.tokens * (size_t)w.k * 2;
-    const __amdgpu_buffer_rsrc_t q_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t *>(w.q) + (size_t)(w.row_base >> 3) * kb_total * 32, 0, (int)(uint32_t)min(q_rest, (size_t)0xffffffffu), 0x00020000);
-    const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<unsigned char *>(w.x), 0, (int)(uint32_t)min(x_rest, (size_t)0xffffffffu), 0x00020000);
+    const u32x4 q_rsrc = buffer_at(w.q + (size_t)(w.row_base >> 3) * kb_total * 32, (size_t)(w.m - w.row_base) * (size_t)(w.k >> 1));
+    const u32x4 x_rsrc = buffer_at(w.x, (size_t)w.tokens * (size_t)w.k * 2);
 
     // scales of rows 4 i16 + j: one per row, or (BLK) one per block of 64 << blk_shift weights, which travel through the
     // register sets with the weights (a step lies inside one block)
     const int nblk = BLK ? w.k >> (6 + w.blk_shift) : 1;
     const float *s_base = w.absmax + (size_t)w.row_base * (size_t)nblk;
-    const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float *>(s_base), 0, (int)(uint32_t)min((size_t)(w.m - w.row_base) * (size_t)nblk * 4, (size_t)0xffffffffu), 0x00020000);
+    const u32x4 s_rsrc = buffer_at(s_base, (size_t)(w.m - w.row_base) * (size_t)nblk * 4);
     uint32_t s_off[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) s_off[j] = (uint32_t)(min(row_w + 4 * i16 + j, w.m - 1) - w.row_base) * (uint32_t)nblk * 4u;
-    float sq[BLK ? 2 : 1][4];
+    uint32_t sq[BLK ? 2 : 1][4];
     f16x2 sc[4];
-#define WIDE_LOAD_S(set, s)                                                                                   \
-    _Pragma("unroll") for (int j = 0; j < 4; ++j) sq[set][j] = __builtin_bit_cast(                            \
-        float, (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(s_rsrc, (int)s_off[j], BLK ? min((s) >> w.blk_shift, nblk - 1) * 4 : 0, 0));
 #define WIDE_SCALES(set)                                                                                      \
     _Pragma("unroll") for (int j = 0; j < 4; ++j)                                                             \
     {                                                                                                         \
-        const f16 h_ = (f16)sq[set][j];                                                                       \
+        const f16 h_ = (f16)__builtin_bit_cast(float, sq[set][j]);                                            \
         sc[j] = f16x2{h_, h_};                                                                                \
     }
 
     u32x4 wq[2][2];   // [set][half]: packed weights of two k-steps
-    u32x4 xr[2][XP];  // activations of two k-steps on their way to LDS
     const int s_last = w.steps_total - 1;
+    // Requests, in an order that the waits count on: for a step the weights and scales (WL operations), then the activations
+    // (XP), then the next step's weights ...
+    constexpr int WL = BLK ? 6 : 2;
 #define WIDE_LOAD_W(set, s)                                                                                   \
     {                                                                                                         \
         const int s_ = min((s), s_last);                                                                      \
         const bool t_ = KTAIL && s_ == s_last;                                                                \
-        wq[set][0] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)(t_ ? a_off - a_back0 : a_off),       \
-                                                           wide_weight_uniform(s_, 0, t_, slot_last), 0);     \
-        wq[set][1] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)(t_ ? a_off - a_back1 : a_off),       \
-                                                           wide_weight_uniform(s_, 1, t_, slot_last), 0);     \
+        load_async<false>(wq[set][0], q_rsrc, t_ ? a_off - a_back0 : a_off, (uint32_t)wide_weight_uniform(s_, 0, t_, slot_last)); \
+        load_async<false>(wq[set][1], q_rsrc, t_ ? a_off - a_back1 : a_off, (uint32_t)wide_weight_uniform(s_, 1, t_, slot_last)); \
+        if (BLK)                                                                                              \
+            _Pragma("unroll") for (int j = 0; j < 4; ++j) load_async(sq[set][j], s_rsrc, s_off[j], (uint32_t)min(s_ >> w.blk_shift, nblk - 1) * 4u); \
     }
-#define WIDE_LOAD_X(set, i, s)                                                                                \
+#define WIDE_LOAD_X(i, off, s)                                                                                \
     {                                                                                                         \
         const int s_ = min((s), s_last);                                                                      \
-        xr[set][i] = __builtin_amdgcn_raw_buffer_load_b128(                                                   \
-            x_rsrc, (int)(KTAIL && s_ == s_last ? x_off[i] - x_back : x_off[i]), s_ * 128, 0);                \
+        load_to_lds(x_rsrc, KTAIL && s_ == s_last ? x_off[i] | x_beyond : x_off[i], (uint32_t)s_ * 128u, xs_lds + (off) + (i) * 4096u); \
     }
-#define WIDE_STORE_X(set, i, off, s)                                                                          \
-    {                                                                                                         \
-        u32x4 v_ = xr[set][i];                                                                                \
-        if (KTAIL && (s) * 64 >= x_k_left) v_ = u32x4{0u, 0u, 0u, 0u};                                        \
-        *reinterpret_cast<u32x4 *>(x_dst + (off) + (i) * 4096) = v_;                                          \
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        if (BLK || u == 0) WIDE_LOAD_S(u, s0 + u)
-        WIDE_LOAD_W(u, s0 + u)
-#pragma unroll
-        for (int i = 0; i < XP; ++i) WIDE_LOAD_X(u, i, s0 + u)
-    }
+    // A step's weights (and scales) have arrived: at most N operations behind them are pending.
+#define WIDE_ARRIVED(set, N)                                                                                  \
+    asm volatile("s_waitcnt vmcnt(%2)" : "+v"(wq[set][0]), "+v"(wq[set][1]) : "n"(N));                       \
+    if (BLK) asm volatile("" : "+v"(sq[set][0]), "+v"(sq[set][1]), "+v"(sq[set][2]), "+v"(sq[set][3]));
 
     f16x8 fa[2][4];  // decoded weights of a half: rows 4 i16 + j
     f16x8 fb[FB];
@@ -153,12 +142,10 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
 
     // Half `h` of k-step `step` (iteration `it` of the loop unrolled by two): per token tile t four MFMAs with the
     // decoded weights fa[h] and token fragment t, and between them: the fragment FB - 1 tiles on; the scaling of a byte
-    // pair of the next half into fa[h ^ 1] and the table read of the pair three on; every fourth tile one 16-byte piece of
-    // the activations into LDS and the load two steps on that refills its registers.
+    // pair of the next half into fa[h ^ 1] and the table read of the pair three on.
     // Stages cur, nxt, nx2 hold steps step .. step + 2.  The barrier of a step comes where the first fragment of the
-    // next step is requested: by then every wave has stored its pieces of that step (all but the last one in this step,
-    // the last one a step earlier, behind that step's barrier), and the stage that stores go to from here on was last
-    // read a step ago, by fragments that every wave has used.
+    // next step is requested: every wave has waited for its pieces of that step.  Behind it the pieces of step + 2 are
+    // requested, into the stage of step - 1: its last fragments were used by every wave before that barrier.
 #define WIDE_HALF(it, step, h)                                                                                \
     {                                                                                                         \
         constexpr int dset_ = (h) == 0 ? (it) : (it) ^ 1, dh_ = (h) ^ 1;                                      \
@@ -166,8 +153,9 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
         {                                                                                                     \
             const int base_ = (h) * NT + t;                                                                   \
             WIDE_MFMA(h, 0, t, base_ % FB)                                                                    \
+            if ((h) == 0 && t == T_NEXT) { WIDE_ARRIVED((it) ^ 1, XP) } /* the table reads reach the next step */ \
             if ((h) == 1 && t == NT - FB + 1) {                                                               \
-                __builtin_amdgcn_s_waitcnt(0xC07F | (FB << 8)); /* lgkmcnt: this wave's stores are done */    \
+                wait_loads<WL>(); /* this wave's pieces of the next step are in LDS */                        \
                 __builtin_amdgcn_s_barrier();                                                                 \
                 asm volatile("" ::: "memory");                                                                \
             }                                                                                                 \
@@ -177,10 +165,7 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
             }                                                                                                 \
             __builtin_amdgcn_sched_barrier(0);                                                                \
             WIDE_MFMA(h, 1, t, base_ % FB)                                                                    \
-            if (BLK && (h) == 1 && t == 0) {                                                                  \
-                WIDE_SCALES((it) ^ 1)                                                                         \
-                WIDE_LOAD_S((it) ^ 1, (step) + 3)                                                             \
-            }                                                                                                 \
+            if (BLK && (h) == 1 && t == 0) WIDE_SCALES((it) ^ 1)                                              \
             _Pragma("unroll") for (int l = t * LPT; l < (t + 1) * LPT; ++l) {                                 \
                 WIDE_SCALE(l, dh_)                                                                            \
                 if (l + 3 < 16) WIDE_LUT(l + 3, dset_, dh_)                                                   \
@@ -188,15 +173,9 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
             }                                                                                                 \
             __builtin_amdgcn_sched_barrier(0);                                                                \
             WIDE_MFMA(h, 2, t, base_ % FB)                                                                    \
-            if (base_ % 4 == 0) {                                                                             \
-                const int i_ = base_ / 4;                                                                     \
-                if (i_ < XP - 1) {                                                                            \
-                    WIDE_STORE_X((it) ^ 1, i_, nxt, (step) + 1)                                               \
-                    WIDE_LOAD_X((it) ^ 1, i_, (step) + 3)                                                     \
-                } else {                                                                                      \
-                    WIDE_STORE_X(it, i_, nx2, (step) + 2)                                                     \
-                    WIDE_LOAD_X(it, i_, (step) + 4)                                                           \
-                }                                                                                             \
+            if ((h) == 1 && t > NT - FB + 1 && (t - (NT - FB + 2)) * 2 < XP) {                                \
+                WIDE_LOAD_X((t - (NT - FB + 2)) * 2, (uint32_t)nx2, (step) + 2)                               \
+                WIDE_LOAD_X((t - (NT - FB + 2)) * 2 + 1, (uint32_t)nx2, (step) + 2)                           \
             }                                                                                                 \
             __builtin_amdgcn_sched_barrier(0);                                                                \
             WIDE_MFMA(h, 3, t, base_ % FB)                                                                    \
@@ -211,15 +190,20 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
         }                                                                                                     \
     }
     int cur = 0, nxt = kWideStage, nx2 = 2 * kWideStage;
-    __syncthreads();  // decode table complete; the previous tile's fragments have been read
+    if (!BLK) {
 #pragma unroll
-    for (int i = 0; i < XP; ++i) WIDE_STORE_X(0, i, 0, s0)
+        for (int j = 0; j < 4; ++j) load_async(sq[0][j], s_rsrc, s_off[j], 0u);
+    }
+    WIDE_LOAD_W(0, s0)
+    __syncthreads();  // decode table complete; the previous tile's work area has been read
 #pragma unroll
-    for (int i = 0; i < XP; ++i) WIDE_LOAD_X(0, i, s0 + 2)
-    WIDE_STORE_X(1, XP - 1, kWideStage, s0 + 1)
-    WIDE_LOAD_X(1, XP - 1, s0 + 3)
+    for (int i = 0; i < XP; ++i) WIDE_LOAD_X(i, 0u, s0)
+    WIDE_LOAD_W(1, s0 + 1)
+#pragma unroll
+    for (int i = 0; i < XP; ++i) WIDE_LOAD_X(i, (uint32_t)kWideStage, s0 + 1)
+    WIDE_ARRIVED(0, XP + WL)
+    if (!BLK) asm volatile("" : "+v"(sq[0][0]), "+v"(sq[0][1]), "+v"(sq[0][2]), "+v"(sq[0][3]));
     WIDE_SCALES(0)
-    if (BLK) WIDE_LOAD_S(0, s0 + 2)
 #pragma unroll
     for (int l = 0; l < 16; ++l) {
         WIDE_LUT(l, 0, 0)
@@ -242,6 +226,8 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
         WIDE_HALF(0, s, 0)
         WIDE_HALF(0, s, 1)
     }
+    // (the requests beyond the last step have arrived: their LDS and registers are free)
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(wq[0][0]), "+v"(wq[0][1]), "+v"(wq[1][0]), "+v"(wq[1][1])::"memory");
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMAs have written their accumulators
     // (pinned once more: no copy of an accumulator moves up between the MFMAs, whose latency the compiler does not know)
 #pragma unroll
@@ -253,11 +239,10 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
 #undef WIDE_SCALE
 #undef WIDE_LUT
 #undef WIDE_READ_B
-#undef WIDE_STORE_X
+#undef WIDE_ARRIVED
 #undef WIDE_LOAD_X
 #undef WIDE_LOAD_W
 #undef WIDE_SCALES
-#undef WIDE_LOAD_S
 }
 
 // Position in the k-steps of the shared tiles laid end to end: tile (counted from `whole`) and step.  A step of a large
