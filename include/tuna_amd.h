@@ -100,7 +100,9 @@ typedef struct tuna_gemm_config {
                               workgroup, the k-steps of all row tiles divided into split_k shares (1 ..
                               512 workgroups); no other field is read.  -5: the narrow-row
                               kernel's variants for any m and k - rows_per_wave 16, 32 or 64 (waves_m 0)
-                              and the other fields as for that kernel */
+                              and the other fields as for that kernel.  -6: the tall-tile kernel -
+                              rows_per_wave (32 .. 128 in steps of 16; not 128 with four token tiles) rows
+                              x token_tiles (1 .. 4) x 16 tokens per workgroup, in split_k parts of k */
 } tuna_gemm_config;
 
 int tuna_version(void);

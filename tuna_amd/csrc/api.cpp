@@ -356,6 +356,40 @@ static int launch_flow(FlowPlan &plan, const void *q, const void *x, const void 
     return e == hipSuccess ? TUNA_OK : hip_fail(e, "decode-batch gemm launch");
 }
 
+// The tall-tile kernel (gemm_tall.hip): rows_per_wave rows, a multiple of 16, in split_k parts of k.
+static inline bool is_tall(const tuna_gemm_config &c) { return c.lds_tile_rows == -6; }
+
+static int plan_tall(int m, int n, int k, const tuna_gemm_config &c, int decode, TallPlan *plan)
+{
+    int rc = check_shape(m, n, k);
+    if (rc) return rc;
+    if (decode != TUNA_DECODE_GEMM) return fail(TUNA_ERR_UNSUPPORTED, "the tall-tile kernel implements TUNA_DECODE_GEMM only");
+    if (n > 16 * c.token_tiles) return fail(TUNA_ERR_UNSUPPORTED, "tall-tile kernel: n=%d tokens in one pass of %d token tiles", n, c.token_tiles);
+    memset(plan, 0, sizeof(*plan));
+    TallArgs &a = plan->args;
+    a.m = m, a.n = n, a.k = k;
+    if (c.rows_per_wave % 16 || !plan_gemm_tall(c.rows_per_wave / 16, c.token_tiles, c.split_k, plan))
+        return fail(TUNA_ERR_UNSUPPORTED, "tall-tile kernel: %d rows x %d token tiles, k=%d in %d parts", c.rows_per_wave, c.token_tiles, k, c.split_k);
+    return TUNA_OK;
+}
+
+static int launch_tall(TallPlan &plan, const void *q, const void *x, const void *code, const void *absmax, void *out, int epilogue,
+                       const void *residual, bool static_ws, hipStream_t stream)
+{
+    TallArgs &a = plan.args;
+    a.q = static_cast<const uint8_t *>(q);
+    a.x = x;
+    a.code = static_cast<const float *>(code);
+    a.absmax = static_cast<const float *>(absmax);
+    a.out = out;
+    a.epilogue = epilogue;
+    a.residual = residual;
+    const int rc = plan.ws_bytes ? provide_workspace(static_ws, stream, plan.ws_bytes, plan.n_counters, &a.ws, &a.counters) : TUNA_OK;
+    if (rc) return rc;
+    const hipError_t e = launch_gemm_tall(plan, stream);
+    return e == hipSuccess ? TUNA_OK : hip_fail(e, "tall-tile gemm launch");
+}
+
 // Narrow-row kernel: checks and launch arguments for a config with rows_per_wave 16 or 32.
 struct NarrowPlan {
     NarrowArgs args;
@@ -997,6 +1031,10 @@ static bool config_runs(int m, int n, int k, const tuna_gemm_config &c)
         FlowPlan fp;
         return plan_flow(m, n, k, c, TUNA_DECODE_GEMM, &fp) == TUNA_OK;
     }
+    if (is_tall(c)) {
+        TallPlan tp;
+        return plan_tall(m, n, k, c, TUNA_DECODE_GEMM, &tp) == TUNA_OK;
+    }
     if (is_narrow_any(c)) {
         NarrowPlan np;
         return plan_narrow_any(m, n, k, c, TUNA_DECODE_GEMM, &np) == TUNA_OK;
@@ -1100,8 +1138,47 @@ static double narrow_time(int m, int n, int k, int rows, int waves_k, int u, int
            std::cbrt(work * work * work + chain * chain * chain + stream * stream * stream) + c.x * x_bytes;
 }
 
+// Microseconds of a launch of the tall-tile kernel (gemm_tall.hip) with tiles of `rt` x 16 rows in `split` parts of k, by a model read
+// off 300 random shapes of 0.5 ... 400 MB of weights at 1 ... 64 tokens, each with up to 21 variants (5.1 per cent off on average
+// on the 440 launches kept; the best of a shape's variants by the model takes 1.01 x the time of the best one): rounds of
+// workgroups with a start and the exchange of the waves' sums, the busiest wave's steps and the weights' stream - whichever is
+// longer, smoothly -, the hand-over between parts and the output.
+static double tall_time(int m, int n, int k, int rt, int split)
+{
+    const int nt = ceil_div(n, 16), tiles = ceil_div(m, 16 * rt), steps = ceil_div(k, 64), part = ceil_div(steps, split), parts = ceil_div(steps, part);
+    const double rounds = ceil_div(tiles * parts, kMaxCus);
+    const double work = rounds * ceil_div(part, 8) * (0.2405 + 0.04922 * rt + (k % 64 ? 0.2187 : 0.1367) * nt + 0.0191 * rt * nt);
+    const double stream = 0.1662 * 0.5e-6 * m * k;
+    return 1.519 + rounds * (2.036 + 0.02599 * rt * nt) + std::cbrt(work * work * work + stream * stream * stream) +
+           (parts > 1 ? 2.371 + 0.02158 * parts * nt * rt : 0.0) + 3.18e-6 * n * m;
+}
+
+// The tile height and the number of k parts that take least time with partial sums that `room` holds, and that time in *us.
+static bool best_tall(int m, int n, int k, const Room &room, tuna_gemm_config *tall, double *us)
+{
+    const int nt = ceil_div(n, 16);
+    bool found = false;
+    for (int rt = 2; rt <= 8; ++rt) {
+        const int tiles = ceil_div(m, 16 * rt);
+        if (rt * nt > 28) continue;
+        // (one round of workgroups, each with at least a step per wave)
+        const int most = tiles < kMaxCus ? std::max(1, std::min(kMaxCus / tiles, std::min(16, k / 512))) : 1;
+        for (int split = most; split >= 1; split = split > 2 ? std::max(split / 2, split == most ? split - 1 : 1) : split - 1) {
+            if (split > 1 && !room.holds((size_t)tiles * split * rt * nt * 1024, (size_t)tiles)) continue;
+            const double t = tall_time(m, n, k, rt, split);
+            if (found && t >= *us) continue;
+            memset(tall, 0, sizeof(*tall));
+            tall->rows_per_wave = 16 * rt, tall->waves_m = 1, tall->waves_k = 8, tall->prefetch = 2, tall->x_chunk = 64, tall->token_tiles = nt;
+            tall->split_k = split, tall->lds_tile_rows = -6;
+            *us = t, found = true;
+        }
+    }
+    return found;
+}
+
 double predicted_us(int m, int n, int k, const tuna_gemm_config &c, int nblk)
 {
+    if (is_tall(c)) return tall_time(m, n, k, c.rows_per_wave / 16, c.split_k);
     if (is_flow(c)) return flow_time(ceil_div(m, 256), ceil_div(ceil_div(k, 64), 4), c.token_tiles, c.split_k);
     if (is_narrow_any(c) || is_narrow(c)) return narrow_time(m, n, k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles, nblk);
     if (c.lds_tile_rows == 256 && c.token_tiles == 16 && c.rows_per_wave != 32) {
@@ -1153,6 +1230,37 @@ static bool narrow_any_instead(int m, int n, int k, const tuna_gemm_config &c, b
         price = nt == 1 ? 9.4 + 0.286 * mb - 1.2e-4 * m : nt == 2 ? 12.6 + 0.40 * mb - 2e-4 * m : 7.0 + 1.5 * nt + (nt == 3 ? 0.55 : 0.60) * mb;
     }
     return best_narrow_any(m, n, k, 0, (from_table ? 0.8 : 0.9) * price, any) && config_runs(m, n, k, *any);
+}
+
+// Up to 64 tokens, after all of these: tall tiles where their model is ahead of the price of what is picked so far - that
+// kernel's model, or straight lines in MB of weights.  Against the picks without it on 700 random shapes, as far as they
+// differ: decode-batch picks 1.3 x, many-token tiles 1.9 x, general 1.6 x, narrow rows 1.07 x.  Lean and batched launches are
+// left alone, and so is what the table holds for one token tile a workgroup of narrow rows.
+static bool tall_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, double flow_us, const Room &room, tuna_gemm_config *tall)
+{
+    if (n > 64) return false;
+    const double mb = 0.5e-6 * m * k;
+    const int nt = ceil_div(n, 16);
+    double price;
+    if (is_flow(c)) price = 0.95 * flow_us;
+    else if (is_narrow(c) || is_narrow_any(c)) {
+        if (from_table && c.token_tiles < 2) return false;
+        price = (is_narrow_any(c) ? 0.95 : 0.9) * narrow_time(m, n, k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles);
+    } else if (c.lds_tile_rows > 0) {
+        if (nt < 3) return false;
+        price = 0.95 * (11.5 + 0.65 * mb);
+    } else {
+        GemmPlan plan;
+        if (plan_gemm(m, n, k, c, TUNA_DECODE_GEMM, &plan) != TUNA_OK || launch_is_lean(plan, kMaxCus) || stream_applies(c, n, TUNA_DECODE_GEMM))
+            return false;
+        static const double kMid[5] = {0, 0.172, 0.22, 0.40, 0.37}, kGeneral[5] = {0, 0.286, 0.40, 0.55, 0.60};
+        if (!mid_applies(plan)) price = 0.95 * (7.0 + 1.5 * nt + kGeneral[nt] * mb);
+        else if (plan.ws_bytes) price = 0.88 * (9.0 + (nt > 1 ? nt : 0) + kMid[nt] * mb); // (split: with the hand-over of its sums)
+        else price = 0.85 * (6.0 + (nt > 1 ? nt : 0) + kMid[nt] * mb);
+    }
+    if (4.0 + 0.1662 * mb > price) return false; // (below what the model gives to any launch)
+    double us = 0.0;
+    return best_tall(m, n, k, room, tall, &us) && us < price;
 }
 
 // What a launch without an explicit config runs from 65 tokens on: the selected config, or 256 x 256 tiles of gemm_wide.hip
@@ -1257,6 +1365,7 @@ static void select_launch(int m, int n, int k, int decode, const Room &room, tun
     if (decode != TUNA_DECODE_GEMM) return;
     if (wide_instead(m, n, k, *c, room, &other) || flow_instead(m, n, k, *c, from_table != 0, room, &other, &flow_us)) *c = other;
     if (narrow_any_instead(m, n, k, *c, from_table != 0, flow_us, &other)) *c = other;
+    if (tall_instead(m, n, k, *c, from_table != 0, flow_us, room, &other)) *c = other;
 }
 
 // The checks of the planner `c` belongs to, for a decode mode.
@@ -1269,6 +1378,10 @@ static int validate_for(int m, int n, int k, const tuna_gemm_config &c, int deco
     if (is_flow(c)) {
         FlowPlan fp;
         return plan_flow(m, n, k, c, decode, &fp);
+    }
+    if (is_tall(c)) {
+        TallPlan tp;
+        return plan_tall(m, n, k, c, decode, &tp);
     }
     if (is_narrow_any(c)) {
         NarrowPlan np;
@@ -1615,6 +1728,11 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
         FlowPlan fp;
         if ((rc = plan_flow(m, n, k, c, decode, &fp))) return rc;
         return or_with_less(launch_flow(fp, q, x, code, absmax, out, epilogue, residual, -1, static_ws, stream));
+    }
+    if (is_tall(c)) {
+        TallPlan tp;
+        if ((rc = plan_tall(m, n, k, c, decode, &tp))) return rc;
+        return or_with_less(launch_tall(tp, q, x, code, absmax, out, epilogue, residual, static_ws, stream));
     }
     if (is_narrow_any(c)) {
         NarrowPlan np;
@@ -2684,6 +2802,14 @@ TUNA_EXPORT int tuna_config_footprint(int m, int n, int k, const tuna_gemm_confi
         if (workspace_bytes) *workspace_bytes = fp.ws_bytes;
         return TUNA_OK;
     }
+    if (is_tall(*cfg)) {
+        TallPlan tp;
+        int rc = plan_tall(m, n, k, *cfg, TUNA_DECODE_GEMM, &tp);
+        if (rc) return rc;
+        if (lds_bytes) *lds_bytes = tall_lds_bytes(tp.rt, tp.nt);
+        if (workspace_bytes) *workspace_bytes = tp.ws_bytes;
+        return TUNA_OK;
+    }
     if (is_narrow_any(*cfg)) {
         NarrowPlan np;
         int rc = plan_narrow_any(m, n, k, *cfg, TUNA_DECODE_GEMM, &np);
@@ -2848,6 +2974,7 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
         const int at = is_narrow_any(w) && plan_narrow_any(m, n, k, w, decode_mode, &np) == TUNA_OK
                            ? describe_narrow_any(np, n, buf, len, " in place of ")
                        : is_flow(w) ? snprintf(buf, len, "gemm_flow_kernel<NT=%d> %d shares in place of ", w.token_tiles, w.split_k)
+                       : is_tall(w) ? snprintf(buf, len, "gemm_flow_kernel_tall<%d rows,NT=%d> split_k=%d in place of ", w.rows_per_wave, w.token_tiles, w.split_k)
                                     : snprintf(buf, len, "gemm_wide_kernel<256 rows x 256 tokens> split_k=%d in place of ", w.split_k);
         return at < 0 || (size_t)at + 16 > len ? TUNA_OK : tuna_describe_launch(m, n, k, &c, decode_mode, buf + at, len - (size_t)at);
     }
@@ -2864,6 +2991,12 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
         FlowPlan fp;
         if ((rc = plan_flow(m, n, k, c, decode_mode, &fp))) return rc;
         snprintf(buf, len, "gemm_flow_kernel<NT=%d> %d shares", fp.nt, fp.args.n_shares);
+        return TUNA_OK;
+    }
+    if (is_tall(c)) {
+        TallPlan tp;
+        if ((rc = plan_tall(m, n, k, c, decode_mode, &tp))) return rc;
+        snprintf(buf, len, "gemm_flow_kernel_tall<%d rows,NT=%d> split_k=%d", 16 * tp.rt, tp.nt, tp.split);
         return TUNA_OK;
     }
     if (is_narrow_any(c)) {

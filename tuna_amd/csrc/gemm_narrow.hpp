@@ -44,7 +44,6 @@
 
 namespace tuna {
 
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 // The arguments are separate scalars, the ones the first loads need in front: the first 16

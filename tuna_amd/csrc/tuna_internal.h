@@ -214,6 +214,28 @@ struct FlowPlan {
     size_t ws_bytes, n_counters;
 };
 
+// Launch arguments of the tall-tile kernel (gemm_tall.hip).
+struct TallArgs {
+    const uint8_t *q;
+    const void *x;
+    const float *code;
+    const float *absmax;
+    void *out;
+    const void *residual;
+    int epilogue;
+    float *ws;           // partial sums, a slot per part of a tile, if there are several
+    unsigned *counters;  // one arrival counter per tile, zero between launches
+    int m, n, k;
+};
+
+struct TallPlan {
+    TallArgs args;
+    int rt, nt;             // 16-row tiles and 16-token tiles of a workgroup
+    int tiles, split;       // row tiles; k parts of each
+    int part_steps;         // k-steps of 64 of a part (the last may have fewer)
+    size_t ws_bytes, n_counters;
+};
+
 inline int ceil_div_i(int a, int b) { return (a + b - 1) / b; }
 
 // ---------------------------------------------------------------------------------------
@@ -326,6 +348,10 @@ hipError_t launch_gemm_wide(const WidePlan &plan, bool scale_blocks, hipStream_t
 // Fills in the launch whose shape and groups plan->args holds (m, k, n_groups, m_total, tok_begin, tok_count, id).
 bool plan_gemm_flow(int nt, int shares, FlowPlan *plan);
 hipError_t launch_gemm_flow(const FlowPlan &plan, bool scale_blocks, hipStream_t stream);
+// Fills in the launch whose shape plan->args holds.
+bool plan_gemm_tall(int row_tiles16, int nt, int split, TallPlan *plan);
+hipError_t launch_gemm_tall(const TallPlan &plan, hipStream_t stream);
+size_t tall_lds_bytes(int rt, int nt);
 hipError_t launch_gemm_wide32(const TiledArgs &args, hipStream_t stream);
 bool tiled_variant_exists(int tile_rows, int tile_tokens, bool mfma32);
 size_t tiled_lds_bytes(int tile_rows, int tile_tokens);
