@@ -28,3 +28,18 @@ def test_the_stated_errors_are_those_of_the_kept_launches(kind, launches, off):
     rows = [r for r in lm.read(DATA) if r["kind"] == kind]
     assert len(rows) == launches
     assert 100 * lm.errors(rows, model, coefficients)[0] == pytest.approx(off, abs=0.06)
+
+
+@pytest.mark.parametrize("m,n,k,shares", [(229376, 40, 4096, 512), (120064, 30, 3968, 469), (24576, 20, 3072, 192)])
+def test_long_decode_batches_put_two_workgroups_on_a_compute_unit(m, n, k, shares):
+    """From 14 units of 32 KB per compute unit on; whole tiles where their number is below 512 and near it.  (The last one is
+    short, and what it takes is not a matter of this rule.)"""
+    import re
+
+    from tuna_amd import ops
+
+    got = re.search(r"gemm_flow_kernel<NT=\d> (\d+) shares", ops.describe_launch(m, n, k))
+    if m * k // 2 >= 14 * 256 * 32768:
+        assert got and int(got.group(1)) == shares
+    else:
+        assert got is None or int(got.group(1)) <= 256

@@ -1064,20 +1064,37 @@ static double flow_time(double tiles, int units, int nt, int shares)
     return 6.1 + per_share * step + (contributors > 1.0 ? 2.7 + (contributors > 2.0 ? 0.3 * nt * (contributors - 2.0) : 0.0) : 0.0);
 }
 
+// The same for launches of at least 14 units per compute unit (117 MB) in 257 ... 512 shares: there the second workgroup on a compute
+// unit is worth a fifth and more, and the stream of the weights counts.  Read off 54 random shapes of 134 ... 470 MB at 16, 32,
+// 48 and 64 tokens (98 launches, 4.3 per cent off): the pick takes 1.005 x the time of a shape's best launch (worst 1.09),
+// where flow_time's takes 1.125 x (worst 1.37).  With 14 ... 16 units it is 1.03 x against 1.05 x, with 10 ... 12 1.05 x against 1.02 x.
+static constexpr int kFlowLongUnits = 14;
+static double flow_long_time(double tiles, int units, int nt, int shares)
+{
+    const double work = 4 * ceil(tiles * units / shares) * (0.2536 + 0.1608 * nt), stream = 0.1606 * 0.032768 * tiles * units;
+    const long long whole = (long long)tiles;
+    const double over = whole % shares == 0 ? 0.0 : shares % whole == 0 ? 1.12 * nt : 4.05 + 3.36 * nt;
+    return 9.1 + std::cbrt(work * work * work + stream * stream * stream) + over;
+}
+
 // The number of shares that takes them least time with partial sums that `room` holds, and that time in *us: equal parts of
-// every tile, or 64 ... 512 at large.
+// every tile, or 64 ... 512 at large; of a long launch more than 256, if their sums fit.
 static int flow_best_shares(long long tiles, int units, int nt, const Room &room, double *us)
 {
     int best = 0;
+    bool is_long = tiles * units >= (long long)kFlowLongUnits * kMaxCus;
     auto consider = [&](long long shares) {
-        if (shares < 1 || shares > 2 * kMaxCus || shares > tiles * units) return;
+        if (shares < 1 || shares > 2 * kMaxCus || shares > tiles * units || (is_long && shares <= kMaxCus)) return;
         if (!room.holds(flow_ws_bytes(tiles, (int)shares, nt), flow_slots(tiles, shares) ? (size_t)tiles : 0)) return;
-        const double t = flow_time((double)tiles, units, nt, (int)shares);
+        const double t = is_long ? flow_long_time((double)tiles, units, nt, (int)shares) : flow_time((double)tiles, units, nt, (int)shares);
         if (!best || t < *us) best = (int)shares, *us = t;
     };
-    for (int parts : {1, 2, 3, 4, 6, 8}) consider(parts * tiles);
-    for (int shares : {64, 128, 192, 256, 384, 512}) consider(shares);
-    return best;
+    for (;;) {
+        for (int parts : {1, 2, 3, 4, 6, 8}) consider(parts * tiles);
+        for (int shares : {64, 128, 192, 256, 384, 512}) consider(shares);
+        if (best || !is_long) return best;
+        is_long = false;
+    }
 }
 
 // What a launch without an explicit config runs up to 64 tokens: the selected config, or the decode-batch kernel in its place

@@ -14,10 +14,11 @@
 // What bounds it: no single unit.  With one workgroup on a compute unit (256 shares: 28672 x 8192 at 37 tokens, eight experts
 // of 28672 x 4096 at 16 each) the LDS is busy 28 .. 31 % of the cycles, the vector ALUs 23 .. 29 %, the matrix pipes 12 .. 21 %,
 // HBM streams 2.8 .. 3.9 TB/s and the waves wait 40 % of their time at a counter or barrier; a second workgroup fills some
-// of that (229376 x 4096 at 16 tokens 107 us on 256 shares, 89 on 512: 5.3 TB/s).  Around the loop 6 us in all, and 3 .. 8
-// for handing over tiles that several shares contribute to.  Against the kernels the launches took before (general, streaming,
-// many-token; one box, launch loop): 17920 x 23168 at 30 tokens 154 -> 60 us, 32128 x 13312 at 36 tokens 129 -> 68, 28672 x
-// 8192 at 37 tokens 51 -> 43; eight experts of 28672 x 4096 on 128 tokens 148 -> 128.
+// of that (229376 x 4096 at 32 tokens 132 us on 256 shares, 107 on 512), but costs more for short launches.  Around the loop 6 us
+// in all, and 3 .. 10 for handing over tiles that several shares contribute to (120064 x 3968 at 16 tokens: 46 us on 469 shares of
+// a tile each, 59 on 512; without the hand-over 47).  No gain: each share's part of a tile walked from elsewhere in k on.
+// Against the kernels the launches took before (general, streaming, many-token; one box, launch loop): 17920 x 23168 at 30
+// tokens 154 -> 60 us, 32128 x 13312 at 36 tokens 129 -> 68, 28672 x 8192 at 37 tokens 51 -> 43; eight experts of 28672 x 4096 on 128 tokens 148 -> 128, and 100 on 512 shares (117 on 256 on that box).
 #include "epilogue.hpp"
 
 namespace tuna {
