@@ -64,12 +64,44 @@ def test_nothing_beyond_a_tokens_k_values_or_the_tokens_enters_a_sum(k, rows, sp
     _check(out, q, s, x, code, k)
 
 
+# scales in blocks: every tile height; parts of k that start and end inside a block; a row's blocks no multiple of four; fewer
+# blocks than eight waves or a wave's four; a last tile with rows missing; scales at any multiple of four bytes
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,block,rows,split", [(32, 1, 256, 64, 32, 1), (112, 20, 768, 128, 32, 2), (64, 40, 1280, 64, 48, 3), (1008, 16, 2816, 256, 48, 5),
+                                                    (208, 64, 4096, 64, 64, 8), (80, 33, 1024, 64, 80, 2), (400, 9, 1792, 256, 80, 3), (592, 50, 2304, 128, 96, 7),
+                                                    (112, 16, 5632, 128, 112, 1), (240, 64, 768, 64, 112, 2), (2000, 30, 4096, 64, 112, 1), (128, 48, 1536, 128, 128, 5),
+                                                    (272, 3, 8192, 64, 128, 1)])
+def test_scale_blocks(m, n, k, block, rows, split):
+    import torch
+
+    from tuna_amd import ops
+
+    q, s, x, code = _inputs(m, n, k, seed=m + k, block=block)
+    apart = torch.full((m * (k // block) + 8,), float("nan"), device="cuda")
+    apart[1:1 + s.numel()] = s.reshape(-1)
+    out, again = _out(n, m), _out(n, m)
+    ops.matmul_blockwise(x, q, apart[1:1 + s.numel()].view(m, k // block), code, out, m, n, k, block, config=_cfg(rows, n, split))
+    ops.matmul_blockwise(x, q, s, code, again, m, n, k, block, config=_cfg(rows, n, split))
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    _check(out, q, s, x, code, k, block=block)
+
+
 @pytest.mark.parametrize("rows,n,split", [(16, 8, 1), (144, 8, 1), (40, 8, 1), (128, 64, 1), (64, 8, 0)])
 def test_what_there_is_no_tile_for_is_refused(rows, n, split):
     from tuna_amd import _lib, ops
 
     with pytest.raises(_lib.TunaError):
         ops.validate_config(1024, n, 1024, _cfg(rows, n, split))
+
+
+@pytest.mark.parametrize("k,block,split", [(256, 128, 1), (16384, 64, 1)])
+def test_scale_blocks_it_has_no_room_or_loads_for_are_refused(k, block, split):
+    """Two blocks a row; 256 blocks of 112 rows in LDS beside four token tiles' activations."""
+    from tuna_amd import _lib, ops
+
+    with pytest.raises(_lib.TunaError):
+        ops.validate_config_blockwise(1024, 64, k, block, _cfg(112, 64, split))
 
 
 def test_a_call_without_a_config_takes_it_where_it_is_predicted_to_be_faster():
@@ -81,11 +113,12 @@ def test_a_call_without_a_config_takes_it_where_it_is_predicted_to_be_faster():
         assert "gemm_flow_kernel_tall" not in ops.describe_launch(*shape), shape
 
 
-def test_the_stated_error_is_that_of_the_kept_launches():
+@pytest.mark.parametrize("kind,off", [("tall", 5.1), ("tall blocks", 4.7)])
+def test_the_stated_errors_are_those_of_the_kept_launches(kind, off):
     """(per cent, as stated beside tall_time in csrc/api.cpp)"""
     from test_launch_models import DATA
     from tuna_amd import launch_models as lm
 
-    rows = [r for r in lm.read(DATA) if r["kind"] == "tall"]
+    rows = [r for r in lm.read(DATA) if r["kind"] == kind]
     assert len(rows) == 440
-    assert 100 * lm.errors(rows, lm.tall, lm.TALL)[0] == pytest.approx(5.1, abs=0.06)
+    assert 100 * lm.errors(rows, *lm.MODELS[kind])[0] == pytest.approx(off, abs=0.06)

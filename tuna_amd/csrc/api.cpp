@@ -359,7 +359,8 @@ static int launch_flow(FlowPlan &plan, const void *q, const void *x, const void 
 // The tall-tile kernel (gemm_tall.hip): rows_per_wave rows, a multiple of 16, in split_k parts of k.
 static inline bool is_tall(const tuna_gemm_config &c) { return c.lds_tile_rows == -6; }
 
-static int plan_tall(int m, int n, int k, const tuna_gemm_config &c, int decode, TallPlan *plan)
+// (blk_shift -1: one scale per row, else blocks of 64 << blk_shift weights)
+static int plan_tall(int m, int n, int k, const tuna_gemm_config &c, int decode, TallPlan *plan, int blk_shift = -1)
 {
     int rc = check_shape(m, n, k);
     if (rc) return rc;
@@ -368,7 +369,7 @@ static int plan_tall(int m, int n, int k, const tuna_gemm_config &c, int decode,
     memset(plan, 0, sizeof(*plan));
     TallArgs &a = plan->args;
     a.m = m, a.n = n, a.k = k;
-    if (c.rows_per_wave % 16 || !plan_gemm_tall(c.rows_per_wave / 16, c.token_tiles, c.split_k, plan))
+    if (c.rows_per_wave % 16 || !plan_gemm_tall(c.rows_per_wave / 16, c.token_tiles, c.split_k, blk_shift, plan))
         return fail(TUNA_ERR_UNSUPPORTED, "tall-tile kernel: %d rows x %d token tiles, k=%d in %d parts", c.rows_per_wave, c.token_tiles, k, c.split_k);
     return TUNA_OK;
 }
@@ -1159,21 +1160,25 @@ static double narrow_time(int m, int n, int k, int rows, int waves_k, int u, int
 // off 300 random shapes of 0.5 ... 400 MB of weights at 1 ... 64 tokens, each with up to 21 variants (5.1 per cent off on average
 // on the 440 launches kept; the best of a shape's variants by the model takes 1.01 x the time of the best one): rounds of
 // workgroups with a start and the exchange of the waves' sums, the busiest wave's steps and the weights' stream - whichever is
-// longer, smoothly -, the hand-over between parts and the output.
-static double tall_time(int m, int n, int k, int rt, int split)
+// longer, smoothly -, the hand-over between parts and the output.  With `nblk` scales a row: 1.1 us, a part's scales into
+// LDS, their bytes and a little more per step, read off 260 random shapes with blocks of 64 and 128 (4.7 per cent off
+// on the 440 launches kept; 1.01 x).
+static double tall_time(int m, int n, int k, int rt, int split, int nblk = 0)
 {
     const int nt = ceil_div(n, 16), tiles = ceil_div(m, 16 * rt), steps = ceil_div(k, 64), part = ceil_div(steps, split), parts = ceil_div(steps, part);
     const double rounds = ceil_div(tiles * parts, kMaxCus);
-    const double work = rounds * ceil_div(part, 8) * (0.2405 + 0.04922 * rt + (k % 64 ? 0.2187 : 0.1367) * nt + 0.0191 * rt * nt);
-    const double stream = 0.1662 * 0.5e-6 * m * k;
-    return 1.519 + rounds * (2.036 + 0.02599 * rt * nt) + std::cbrt(work * work * work + stream * stream * stream) +
+    const double step = nblk ? 0.2332 + 0.05657 * rt : 0.2405 + 0.04922 * rt;
+    const double work = rounds * ceil_div(part, 8) * (step + (k % 64 ? 0.2187 : 0.1367) * nt + 0.0191 * rt * nt);
+    const double stream = 0.1662 * (0.5e-6 * m * k + 4e-6 * m * nblk);
+    const double scales = nblk ? 0.0264 * 0.0625 * rt * ceil(part * 64.0 * nblk / k) : 0.0;
+    return (nblk ? 2.622 : 1.519) + rounds * (2.036 + 0.02599 * rt * nt + scales) + std::cbrt(work * work * work + stream * stream * stream) +
            (parts > 1 ? 2.371 + 0.02158 * parts * nt * rt : 0.0) + 3.18e-6 * n * m;
 }
 
 // The tile height and the number of k parts that take least time with partial sums that `room` holds, and that time in *us.
-static bool best_tall(int m, int n, int k, const Room &room, tuna_gemm_config *tall, double *us)
+static bool best_tall(int m, int n, int k, int nblk, const Room &room, tuna_gemm_config *tall, double *us)
 {
-    const int nt = ceil_div(n, 16);
+    const int nt = ceil_div(n, 16), blk_shift = nblk ? log2i(k / nblk) - 6 : -1;
     bool found = false;
     for (int rt = 2; rt <= 8; ++rt) {
         const int tiles = ceil_div(m, 16 * rt);
@@ -1182,12 +1187,15 @@ static bool best_tall(int m, int n, int k, const Room &room, tuna_gemm_config *t
         const int most = tiles < kMaxCus ? std::max(1, std::min(kMaxCus / tiles, std::min(16, k / 512))) : 1;
         for (int split = most; split >= 1; split = split > 2 ? std::max(split / 2, split == most ? split - 1 : 1) : split - 1) {
             if (split > 1 && !room.holds((size_t)tiles * split * rt * nt * 1024, (size_t)tiles)) continue;
-            const double t = tall_time(m, n, k, rt, split);
+            const double t = tall_time(m, n, k, rt, split, nblk);
             if (found && t >= *us) continue;
-            memset(tall, 0, sizeof(*tall));
-            tall->rows_per_wave = 16 * rt, tall->waves_m = 1, tall->waves_k = 8, tall->prefetch = 2, tall->x_chunk = 64, tall->token_tiles = nt;
-            tall->split_k = split, tall->lds_tile_rows = -6;
-            *us = t, found = true;
+            tuna_gemm_config c;
+            memset(&c, 0, sizeof(c));
+            c.rows_per_wave = 16 * rt, c.waves_m = 1, c.waves_k = 8, c.prefetch = 2, c.x_chunk = 64, c.token_tiles = nt;
+            c.split_k = split, c.lds_tile_rows = -6;
+            TallPlan plan;
+            if (plan_tall(m, n, k, c, TUNA_DECODE_GEMM, &plan, blk_shift) != TUNA_OK) continue;
+            *tall = c, *us = t, found = true;
         }
     }
     return found;
@@ -1195,7 +1203,7 @@ static bool best_tall(int m, int n, int k, const Room &room, tuna_gemm_config *t
 
 double predicted_us(int m, int n, int k, const tuna_gemm_config &c, int nblk)
 {
-    if (is_tall(c)) return tall_time(m, n, k, c.rows_per_wave / 16, c.split_k);
+    if (is_tall(c)) return tall_time(m, n, k, c.rows_per_wave / 16, c.split_k, nblk);
     if (is_flow(c)) return flow_time(ceil_div(m, 256), ceil_div(ceil_div(k, 64), 4), c.token_tiles, c.split_k);
     if (is_narrow_any(c) || is_narrow(c)) return narrow_time(m, n, k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles, nblk);
     if (c.lds_tile_rows == 256 && c.token_tiles == 16 && c.rows_per_wave != 32) {
@@ -1277,7 +1285,7 @@ static bool tall_instead(int m, int n, int k, const tuna_gemm_config &c, bool fr
     }
     if (4.0 + 0.1662 * mb > price) return false; // (below what the model gives to any launch)
     double us = 0.0;
-    return best_tall(m, n, k, room, tall, &us) && us < price;
+    return best_tall(m, n, k, 0, room, tall, &us) && us < price;
 }
 
 // What a launch without an explicit config runs from 65 tokens on: the selected config, or 256 x 256 tiles of gemm_wide.hip
@@ -2309,12 +2317,13 @@ TUNA_EXPORT int tuna_quantize_blockwise(const void *w, const void *code, void *q
 // A config comes from the caller (tuna_matmul_blockwise_ex), from the table of tuned entries keyed by (m, token bucket,
 // k, block_size) (config_table.cpp, written by the tuner), or from the rules of derive_blockwise below.
 // ---------------------------------------------------------------------------------------
-enum BlockwiseFamily { kBlkNarrow = 0, kBlkMulti = 1, kBlkTiled = 2, kBlkMid = 3, kBlkFlow = 4, kBlkNarrowAny = 5 };
+enum BlockwiseFamily { kBlkNarrow = 0, kBlkMulti = 1, kBlkTiled = 2, kBlkMid = 3, kBlkFlow = 4, kBlkNarrowAny = 5, kBlkTall = 6 };
 
 static BlockwiseFamily blockwise_family(const tuna_gemm_config &c)
 {
     if (c.lds_tile_rows > 0) return kBlkTiled;
     if (is_flow(c)) return kBlkFlow;
+    if (is_tall(c)) return kBlkTall;
     if (is_narrow_any(c)) return kBlkNarrowAny;
     if (is_narrow(c)) return kBlkNarrow;
     if (c.split_k == 0) return kBlkMulti;
@@ -2405,6 +2414,14 @@ static int run_blockwise(const BlockwiseCall &b, const tuna_gemm_config &c, hipS
         FlowPlan fp;
         if ((rc = plan_flow(m, n, k, c, TUNA_DECODE_GEMM, &fp))) return rc;
         return dry ? TUNA_OK : launch_flow(fp, b.q, b.x, b.code, b.absmax, b.out, TUNA_EPILOGUE_NONE, nullptr, shift, false, st);
+    }
+    case kBlkTall: {
+        TallPlan tp;
+        if ((rc = plan_tall(m, n, k, c, TUNA_DECODE_GEMM, &tp, shift))) return rc;
+        if (dry) return TUNA_OK;
+        if ((rc = launch_tall(tp, b.q, b.x, b.code, b.absmax, b.out, TUNA_EPILOGUE_NONE, nullptr, false, st))) return rc;
+        diag::count(diag::kBlockwiseTall);
+        return TUNA_OK;
     }
     case kBlkNarrowAny: {
         NarrowPlan np;
@@ -2620,24 +2637,53 @@ static int derive_blockwise(const BlockwiseCall &b, const Room &room, tuna_gemm_
     return TUNA_OK;
 }
 
+// Up to 64 tokens: tall tiles (gemm_tall.hip) where their model is ahead of `c`'s price - the narrow-row kernel's model, of
+// its variants for any k too, or straight lines over the bytes of the weights (28672 x 4096 with blocks of 64: at 16 tokens
+// 20.2 -> 18.2 us, at 64 37.1 -> 27.6; 5440 x 21760 at 46 tokens 53.9 -> 26.8, 4224 x 21248 at 16 31.4 -> 17.1; 220 random
+// shapes 1.26 x, 1.4 x where the choice changes).
+static bool blockwise_tall_instead(const BlockwiseCall &b, const tuna_gemm_config &c, const Room &room, tuna_gemm_config *tall)
+{
+    if (b.n > 64) return false;
+    const int nblk = b.k / b.block_size, nt = ceil_div(b.n, 16);
+    const double mb = 0.5e-6 * b.m * b.k;
+    static const double kBatched[5] = {0, 0.19, 0.45, 0.45, 0.45}, kStreaming[5] = {0, 0.27, 0.39, 0.40, 0.40};
+    double price;
+    switch (blockwise_family(c)) {
+    case kBlkNarrow: price = narrow_time(b.m, b.n, b.k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles, nblk); break;
+    case kBlkTiled: price = 11.0 + 0.55 * mb; break;
+    case kBlkMulti: price = (nt == 1 ? 4.5 : 9.5) + kBatched[nt] * mb; break;
+    case kBlkMid: price = (nt == 1 ? 4.5 : 9.5) + kStreaming[nt] * mb; break;
+    default: return false;
+    }
+    price *= 0.95;
+    double us = 0.0;
+    if (4.0 + 0.1662 * mb > price || !best_tall(b.m, b.n, b.k, nblk, room, tall, &us) || us >= price) return false;
+    tuna_gemm_config any;
+    return !best_narrow_any(b.m, b.n, b.k, nblk, us, &any);
+}
+
 // Tuned entry for (m, n, k, block_size) if the table has one that can run the call, else the derived config.
 static int select_blockwise(const BlockwiseCall &b, const Room &room, tuna_gemm_config *cfg, int *from_table)
 {
     if (from_table) *from_table = 0;
+    tuna_gemm_config tall;
     for (int i = 0; i < kBlockwiseTableSize; ++i) {
         const BlockwiseTableEntry &e = kBlockwiseTable[i];
         // (from 33 tokens an entry holds at the count it was tuned at, its bucket's lower edge: further into the bucket
         // the derivation knows the token tiles that n has gained - 8192 x 8192 at 100 tokens with blocks of 64 runs
         // 68 us with the entry of the bucket 64..127 and 41 with the model's pick, 8192 x 28672 at 56 tokens 115 us
-        // with the entry of the bucket 32..63 and 69 derived)
+        // with the entry of the bucket 32..63 and 69 derived; up to 32 it gives way to tall tiles)
         if (e.m == b.m && e.k == b.k && e.block_size == b.block_size && b.n >= e.n_lo && b.n <= e.n_hi &&
             (b.n <= 32 || b.n == e.n_lo) && run_blockwise(b, e.cfg, nullptr, true) == TUNA_OK) {
             *cfg = e.cfg;
-            if (from_table) *from_table = 1;
+            if (b.n != e.n_lo && blockwise_tall_instead(b, e.cfg, room, &tall)) *cfg = tall;
+            else if (from_table) *from_table = 1;
             return TUNA_OK;
         }
     }
-    return derive_blockwise(b, room, cfg);
+    const int rc = derive_blockwise(b, room, cfg);
+    if (!rc && blockwise_tall_instead(b, *cfg, room, &tall)) *cfg = tall;
+    return rc;
 }
 
 static int check_blockwise_call(const BlockwiseCall &b, bool pointers)
@@ -2669,7 +2715,7 @@ static int select_blockwise_launch(const BlockwiseCall &b, const Room &room, tun
     if (rc || from_table || b.n > 64) return rc;
     const int nblk = b.k / b.block_size;
     double price = 0.0;
-    if (is_narrow(*c)) price = narrow_time(b.m, b.n, b.k, c->rows_per_wave, c->waves_k, c->prefetch, c->token_tiles, nblk);
+    if (blockwise_family(*c) == kBlkNarrow) price = narrow_time(b.m, b.n, b.k, c->rows_per_wave, c->waves_k, c->prefetch, c->token_tiles, nblk);
     else if (blockwise_family(*c) == kBlkTiled) price = 11.0 + 0.55 * 0.5e-6 * b.m * b.k;
     tuna_gemm_config any;
     if (best_narrow_any(b.m, b.n, b.k, nblk, 0.88 * price, &any) && run_blockwise(b, any, nullptr, true) == TUNA_OK) *c = any;
@@ -2823,7 +2869,7 @@ TUNA_EXPORT int tuna_config_footprint(int m, int n, int k, const tuna_gemm_confi
         TallPlan tp;
         int rc = plan_tall(m, n, k, *cfg, TUNA_DECODE_GEMM, &tp);
         if (rc) return rc;
-        if (lds_bytes) *lds_bytes = tall_lds_bytes(tp.rt, tp.nt);
+        if (lds_bytes) *lds_bytes = tall_lds_bytes(tp);
         if (workspace_bytes) *workspace_bytes = tp.ws_bytes;
         return TUNA_OK;
     }

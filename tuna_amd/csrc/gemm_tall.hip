@@ -21,6 +21,10 @@
 // 7, 23, 12 and 6.  Compute alone (table, scaling, MFMA) runs at 29 .. 36 ns per KB and CU, which is what is left.  Not better,
 // and not kept: activations straight into LDS (pieces of 64 bytes 28.4 for 24.9 us at NT 4, of 128 equal), four steps ahead, a
 // deeper ring of table reads, part of the decode on the VALU (5 .. 14 per cent slower).
+//
+// Scales finer than a row (BLK): a part's scales go to LDS once, two bytes each and a lane's of a block together, and a step's
+// are read half a step ahead.  28672 x 4096 with blocks of 64: 20.2 -> 18.2 us at 16 tokens, 37 -> 27.6 at 64; 8192 x 28672 at 32
+// tokens 58 -> 39.
 #include "epilogue.hpp"
 
 namespace tuna {
@@ -51,13 +55,21 @@ constexpr size_t work_bytes(int rt, int nt)  // x of the waves; the waves' sums;
     const size_t a = x > red ? x : red;
     return a > out ? a : out;
 }
-constexpr size_t lds_bytes(int rt, int nt) { return (size_t)kLutBytes + work_bytes(rt, nt) + 16; }
+// Scales in blocks of 64 << blk_shift weights: those of a tile's part of k lie behind the activations, two bytes each and a
+// lane's of a block together: [block][16 lanes][scale_dwords], where the waves' sums go in the end.
+constexpr int scale_dwords(int rt) { return rt <= 2 ? 1 : rt <= 4 ? 2 : 4; }
+constexpr size_t lds_bytes(int rt, int nt, int blocks)
+{
+    const size_t with_scales = (size_t)kWaves * nt * 2048 + (size_t)blocks * 64 * scale_dwords(rt);
+    const size_t work = work_bytes(rt, nt);
+    return (size_t)kLutBytes + (with_scales > work ? with_scales : work) + 16;
+}
 
 // (separate scalars, the ones the first loads need in front: the first sixteen dwords arrive in scalar registers with the wave)
-template <int RT, int NT>
+template <int RT, int NT, bool BLK>
 __global__ __launch_bounds__(kThreads, 2) void gemm_flow_kernel_tall(const uint8_t *a_q, const void *a_x, const float *a_code, const float *a_absmax,
                                                                      int a_k, int a_n, int a_m, int a_part_steps, void *a_out, int a_epilogue,
-                                                                     const void *a_residual, float *a_ws, unsigned *a_counters)
+                                                                     const void *a_residual, float *a_ws, unsigned *a_counters, int a_blk_shift, int a_ticket)
 {
     using P = Pieces<RT>;
     constexpr int NS = 2;      // steps whose weights are on their way
@@ -73,7 +85,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_flow_kernel_tall(const uint8
     const int kb_total = a_k >> 3, steps_total = (a_k + 63) >> 6;
 
     unsigned char *const work = smem + kLutBytes;
-    volatile unsigned *const ticket = reinterpret_cast<volatile unsigned *>(work + work_bytes(RT, NT));
+    volatile unsigned *const ticket = reinterpret_cast<volatile unsigned *>(smem + a_ticket);
     const float code_lane = a_code[lane & 15];
     auto build_table = [&]() {  // as in the streaming kernels
         const int code_bits = (int)(uint32_t)__builtin_bit_cast(uint16_t, (f16)code_lane);
@@ -113,8 +125,9 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_flow_kernel_tall(const uint8
         (int)(uint32_t)min(rows_left * (size_t)(a_k >> 1), (size_t)0xffffffffu), 0x00020000);
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         reinterpret_cast<unsigned char *>(const_cast<void *>(a_x)), 0, (int)((uint32_t)a_n * (uint32_t)a_k * 2u), 0x00020000);
+    const int nblk = BLK ? a_k >> (6 + a_blk_shift) : 1;
     const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float *>(a_absmax) + row_base, 0, (int)(uint32_t)min(rows_left * 4, (size_t)0xffffffffu), 0x00020000);
+        const_cast<float *>(a_absmax) + (size_t)row_base * (size_t)nblk, 0, (int)(uint32_t)min(rows_left * (size_t)nblk * 4, (size_t)0xffffffffu), 0x00020000);
 
     f32x4 acc[RT][NT];
 #pragma unroll
@@ -161,14 +174,16 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_flow_kernel_tall(const uint8
     for (int i = 0; i < 2 * NT; ++i) TALL_LOAD_X(i)
     TALL_LOAD_W(0, 0)
     float sc32[RT];
+    if constexpr (!BLK) {
 #pragma unroll
-    for (int r = 0; r < RT; ++r) {
-        const int p = P::of(r);
-        sc32[r] = __builtin_bit_cast(float, (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(
-                                                s_rsrc, (16 * P::first(p) + P::width(p) * i16 + r - P::first(p)) * 4, 0, 0));
+        for (int r = 0; r < RT; ++r) {
+            const int p = P::of(r);
+            sc32[r] = __builtin_bit_cast(float, (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(
+                                                    s_rsrc, (16 * P::first(p) + P::width(p) * i16 + r - P::first(p)) * 4, 0, 0));
+        }
     }
     TALL_LOAD_W(0, 1)
-    f16x2 sc[(RT + 1) / 2];
+    f16x2 sc[BLK ? 2 : 1][(RT + 1) / 2];  // of the step at hand and of the next one
     f16x8 fa[2], fb[2][NT];
     uint32_t lt[LR][4];
     // (turn tau of step u: row tile tau % RT of half tau / RT; u and tau may run over into the next step)
@@ -181,12 +196,12 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_flow_kernel_tall(const uint8
     }
 #define TALL_SCALE(u, tau)                                                                                    \
     {                                                                                                         \
-        const int r_ = (tau) % RT, l_ = ((u) * T + (tau)) % LR, f_ = (tau) & 1;                               \
+        const int r_ = (tau) % RT, l_ = ((u) * T + (tau)) % LR, f_ = (tau) & 1; /* (as for TALL_LUT) */       \
         _Pragma("unroll") for (int b = 0; b < 4; ++b)                                                         \
         {                                                                                                     \
             f16x2 v_;                                                                                         \
-            if (r_ & 1) asm volatile("v_pk_mul_f16 %0, %1, %2 op_sel:[0,1] op_sel_hi:[1,1]" : "=v"(v_) : "v"(lt[l_][b]), "v"(sc[r_ / 2])); \
-            else asm volatile("v_pk_mul_f16 %0, %1, %2 op_sel:[0,0] op_sel_hi:[1,0]" : "=v"(v_) : "v"(lt[l_][b]), "v"(sc[r_ / 2])); \
+            if (r_ & 1) asm volatile("v_pk_mul_f16 %0, %1, %2 op_sel:[0,1] op_sel_hi:[1,1]" : "=v"(v_) : "v"(lt[l_][b]), "v"(sc[BLK ? ((u) + (tau) / T) % NS : 0][r_ / 2])); \
+            else asm volatile("v_pk_mul_f16 %0, %1, %2 op_sel:[0,0] op_sel_hi:[1,0]" : "=v"(v_) : "v"(lt[l_][b]), "v"(sc[BLK ? ((u) + (tau) / T) % NS : 0][r_ / 2])); \
             fa[f_][2 * b] = v_[0];                                                                            \
             fa[f_][2 * b + 1] = v_[1];                                                                        \
         }                                                                                                     \
@@ -208,7 +223,50 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_flow_kernel_tall(const uint8
             TALL_LOAD_X(i)                                                                                    \
         }                                                                                                     \
         _Pragma("unroll") for (int t = 0; t < NT; ++t) if (tau == 3 * RT / 2 + t * RT / (2 * NT)) TALL_READ_B(0, t) \
+        if (BLK && tau == RT) TALL_READ_SCALES(((u) + 1) % NS)                                                \
         __builtin_amdgcn_sched_barrier(0);                                                                    \
+    }
+    // (the scales of the step after the one at hand)
+#define TALL_READ_SCALES(set)                                                                                 \
+    {                                                                                                         \
+        s_sc = next(s_sc);                                                                                    \
+        const lds_u32 *const from_ = sc_lane + ((s_sc >> a_blk_shift) - b0) * (16 * SD);                      \
+        _Pragma("unroll") for (int j = 0; j < (RT + 1) / 2; ++j) sc[BLK ? (set) : 0][j] = __builtin_bit_cast(f16x2, from_[j]); \
+    }
+    constexpr int SD = scale_dwords(RT);
+    const int b0 = BLK ? s0 >> a_blk_shift : 0;
+    int s_sc = s_first + 8 * (int)turn;
+    unsigned char *const scales = work + (size_t)kWaves * NT * 2048;
+    const lds_u32 *const sc_lane = reinterpret_cast<const lds_u32 *>((uintptr_t)(uint32_t)(kLutBytes + kWaves * NT * 2048 + i16 * (SD * 4)));
+    if constexpr (BLK) {
+        // Four blocks of a row a lane, 64 rows a wave: the LDS banks of a store are those of 16 lanes and two or four pairs of
+        // row tiles.  (The last four of a row where four from here on would go beyond it: what is in front of the part or
+        // behind it isn't stored.)
+        const int nb = ((s1 - 1) >> a_blk_shift) + 1 - b0, quads = (nb + 3) >> 2;
+        constexpr int RG = (ROWS + 63) / 64, PIECES = 4;  // groups of 64 rows; loads on their way
+        for (int j0 = wave; j0 < RG * quads; j0 += kWaves * PIECES) {
+            u32x4 v[PIECES];
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i) {
+                const int j = min(j0 + kWaves * i, RG * quads - 1), rg = RG == 1 ? 0 : j & 1, c = min(b0 + 4 * (RG == 1 ? j : j >> 1), nblk - 4);
+                v[i] = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, ((64 * rg + lane) * nblk + c) * 4, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i) {
+                const int j = min(j0 + kWaves * i, RG * quads - 1), rg = RG == 1 ? 0 : j & 1, c = min(b0 + 4 * (RG == 1 ? j : j >> 1), nblk - 4) - b0;
+                const int row = 64 * rg + lane, r16 = row >> 4;
+                const int width = r16 < 4 * P::fours ? 4 : r16 < 4 * P::fours + 2 * P::twos ? 2 : 1;
+                const int first = width == 4 ? r16 & ~3 : width == 2 ? 4 * P::fours : RT - 1;
+                const int in = row - 16 * first, lane16 = in / width, r = first + in % width;
+                if (row < ROWS)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const uint32_t bits = v[i][e];  // (a copy: a bit cast of a vector's element would take the first)
+                        if (c + e >= 0 && c + e < nb)
+                            *reinterpret_cast<f16 *>(scales + ((c + e) * 16 + lane16) * (SD * 4) + r * 2) = (f16)__builtin_bit_cast(float, bits);
+                    }
+            }
+        }
     }
     build_table();
     TALL_LOAD_W(1, 0)
@@ -219,8 +277,14 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_flow_kernel_tall(const uint8
         *reinterpret_cast<u32x4 *>(x_dst + i * 1024) = xr[i];
         TALL_LOAD_X(i)
     }
+    if constexpr (BLK) {
+        const lds_u32 *const from = sc_lane + ((s_sc >> a_blk_shift) - b0) * (16 * SD);
 #pragma unroll
-    for (int r = 0; r < RT; ++r) sc[r / 2][r & 1] = (f16)sc32[r];
+        for (int j = 0; j < (RT + 1) / 2; ++j) sc[0][j] = __builtin_bit_cast(f16x2, from[j]);
+    } else {
+#pragma unroll
+        for (int r = 0; r < RT; ++r) sc[0][r / 2][r & 1] = (f16)sc32[r];
+    }
     TALL_LUT(0, 0)
     TALL_SCALE(0, 0)
     TALL_LUT(0, 1)
@@ -239,6 +303,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_flow_kernel_tall(const uint8
         } while (left > 0);
     }
 #undef TALL_STEP
+#undef TALL_READ_SCALES
 #undef TALL_READ_B
 #undef TALL_SCALE
 #undef TALL_LUT
@@ -340,38 +405,40 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_flow_kernel_tall(const uint8
     }
 }
 
-template <int RT, int NT>
+template <int RT, int NT, bool BLK>
 hipError_t launch(const TallPlan &plan, hipStream_t stream)
 {
     static OptInFlag done[16];
-    const auto fn = gemm_flow_kernel_tall<RT, NT>;
+    const auto fn = gemm_flow_kernel_tall<RT, NT, BLK>;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev < 0 || dev >= 16) return hipErrorInvalidDevice;
     if ((e = ensure_lds_opt_in(done[dev], reinterpret_cast<const void *>(fn))) != hipSuccess) return e;
     const TallArgs &a = plan.args;
-    hipLaunchKernelGGL(fn, dim3((unsigned)plan.tiles, (unsigned)plan.split), dim3(kThreads), lds_bytes(RT, NT), stream, a.q, a.x, a.code, a.absmax,
-                       a.k, a.n, a.m, plan.part_steps, a.out, a.epilogue, a.residual, a.ws, a.counters);
+    const size_t lds = lds_bytes(RT, NT, plan.part_blocks);
+    hipLaunchKernelGGL(fn, dim3((unsigned)plan.tiles, (unsigned)plan.split), dim3(kThreads), lds, stream, a.q, a.x, a.code, a.absmax, a.k, a.n, a.m,
+                       plan.part_steps, a.out, a.epilogue, a.residual, a.ws, a.counters, a.blk_shift, (int)lds - 16);
     return hipGetLastError();
 }
 template <int RT>
 hipError_t launch(const TallPlan &plan, hipStream_t stream)
 {
+    const bool blk = plan.part_blocks != 0;
     switch (plan.nt) {
-    case 1: return launch<RT, 1>(plan, stream);
-    case 2: return launch<RT, 2>(plan, stream);
-    case 3: return launch<RT, 3>(plan, stream);
+    case 1: return blk ? launch<RT, 1, true>(plan, stream) : launch<RT, 1, false>(plan, stream);
+    case 2: return blk ? launch<RT, 2, true>(plan, stream) : launch<RT, 2, false>(plan, stream);
+    case 3: return blk ? launch<RT, 3, true>(plan, stream) : launch<RT, 3, false>(plan, stream);
     default:
-        if constexpr (RT <= 7) return launch<RT, 4>(plan, stream);
+        if constexpr (RT <= 7) return blk ? launch<RT, 4, true>(plan, stream) : launch<RT, 4, false>(plan, stream);
         else return hipErrorInvalidConfiguration;
     }
 }
 }  // namespace
 
-bool plan_gemm_tall(int row_tiles16, int nt, int split, TallPlan *plan)
+bool plan_gemm_tall(int row_tiles16, int nt, int split, int blk_shift, TallPlan *plan)
 {
-    const TallArgs &a = plan->args;
+    TallArgs &a = plan->args;
     if (row_tiles16 < 2 || row_tiles16 > 8 || nt < 1 || nt > 4 || (row_tiles16 == 8 && nt == 4) || split < 1 || split > 65535) return false;
     const int rows = 16 * row_tiles16, steps = ceil_div_i(a.k, 64);
     if (16ll * nt * a.k * 2 > 0x7fffffff || (long long)rows * a.k / 2 > 0x7fffffff) return false;  // 32-bit offsets inside a tile
@@ -380,10 +447,19 @@ bool plan_gemm_tall(int row_tiles16, int nt, int split, TallPlan *plan)
     plan->split = ceil_div_i(steps, plan->part_steps);  // (every part has steps)
     plan->ws_bytes = plan->split > 1 ? (size_t)plan->tiles * plan->split * row_tiles16 * nt * 1024 : 0;
     plan->n_counters = plan->split > 1 ? (size_t)plan->tiles : 0;
+    plan->part_blocks = 0;
+    if (blk_shift >= 0) {
+        // the blocks that a part touches: one more than it fills where it starts inside one
+        const int size = 1 << blk_shift, nblk = a.k >> (6 + blk_shift);
+        if (a.k % (64 << blk_shift) || nblk < 4) return false;
+        plan->part_blocks = ceil_div_i(plan->part_steps, size) + (plan->split > 1 && plan->part_steps % size ? 1 : 0);
+        a.blk_shift = blk_shift;
+        if (lds_bytes(row_tiles16, nt, plan->part_blocks) > (size_t)kLdsLimit) return false;
+    }
     return true;
 }
 
-size_t tall_lds_bytes(int rt, int nt) { return lds_bytes(rt, nt); }
+size_t tall_lds_bytes(const TallPlan &plan) { return lds_bytes(plan.rt, plan.nt, plan.part_blocks); }
 
 hipError_t launch_gemm_tall(const TallPlan &plan, hipStream_t stream)
 {

@@ -226,6 +226,7 @@ struct TallArgs {
     float *ws;           // partial sums, a slot per part of a tile, if there are several
     unsigned *counters;  // one arrival counter per tile, zero between launches
     int m, n, k;
+    int blk_shift;       // a scale block is 64 << blk_shift weights, if the plan has part_blocks
 };
 
 struct TallPlan {
@@ -233,6 +234,7 @@ struct TallPlan {
     int rt, nt;             // 16-row tiles and 16-token tiles of a workgroup
     int tiles, split;       // row tiles; k parts of each
     int part_steps;         // k-steps of 64 of a part (the last may have fewer)
+    int part_blocks;        // scale blocks that a part touches at most; 0: one scale per row
     size_t ws_bytes, n_counters;
 };
 
@@ -349,9 +351,10 @@ hipError_t launch_gemm_wide(const WidePlan &plan, bool scale_blocks, hipStream_t
 bool plan_gemm_flow(int nt, int shares, FlowPlan *plan);
 hipError_t launch_gemm_flow(const FlowPlan &plan, bool scale_blocks, hipStream_t stream);
 // Fills in the launch whose shape plan->args holds.
-bool plan_gemm_tall(int row_tiles16, int nt, int split, TallPlan *plan);
+// (blk_shift -1: one scale per row)
+bool plan_gemm_tall(int row_tiles16, int nt, int split, int blk_shift, TallPlan *plan);
 hipError_t launch_gemm_tall(const TallPlan &plan, hipStream_t stream);
-size_t tall_lds_bytes(int rt, int nt);
+size_t tall_lds_bytes(const TallPlan &plan);
 hipError_t launch_gemm_wide32(const TiledArgs &args, hipStream_t stream);
 bool tiled_variant_exists(int tile_rows, int tile_tokens, bool mfma32);
 size_t tiled_lds_bytes(int tile_rows, int tile_tokens);

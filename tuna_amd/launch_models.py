@@ -98,24 +98,27 @@ def wide(r, c):
     return _wide(large, small, steps, split, c)
 
 
-# launch, round, step, rows, tokens, both, tokens where rows of x start inside a cache line, stream, hand-over, its parts, sums, output
-TALL = (1.519, 2.036, 0.2405, 0.04922, 0.1367, 0.0191, 0.2187, 0.1662, 2.371, 0.02158, 0.02599, 3.18)
+# launch, round, step, rows, tokens, both, tokens where rows of x start inside a cache line, stream, hand-over, its parts, sums, output,
+# KB of a workgroup's scales
+TALL = (1.519, 2.036, 0.2405, 0.04922, 0.1367, 0.0191, 0.2187, 0.1662, 2.371, 0.02158, 0.02599, 3.18, 0.0)
+TALL_BLOCKS = (2.622, 2.036, 0.2332, 0.05657, 0.1367, 0.0191, 0.2187, 0.1662, 2.371, 0.02158, 0.02599, 3.18, 0.0264)
 
 
 def tall(r, c):
     m, n, k, split = r["m"], r["n"], r["k"], r["split"]
-    rt, nt, steps = r["rows"] // 16, r["token_tiles"], _cd(k, 64)
+    rt, nt, steps, nblk = r["rows"] // 16, r["token_tiles"], _cd(k, 64), k // r["block"] if r["block"] else 0
     part = _cd(steps, split)
     parts = _cd(steps, part)
     rounds = _cd(_cd(m, 16 * rt) * parts, CUS)
     work = rounds * _cd(part, 8) * (c[2] + c[3] * rt + (c[6] if k % 64 else c[4]) * nt + c[5] * rt * nt)
-    stream = c[7] * 0.5e-6 * m * k
+    stream = c[7] * (0.5e-6 * m * k + 4e-6 * m * nblk)
+    scales = c[12] * 0.0625 * rt * math.ceil(part * 64.0 * nblk / k) if nblk else 0.0
     over = c[8] + c[9] * parts * nt * rt if parts > 1 else 0.0
-    return c[0] + rounds * (c[1] + c[10] * rt * nt) + (abs(work) ** 3 + abs(stream) ** 3) ** (1 / 3) + over + c[11] * 1e-6 * n * m
+    return c[0] + rounds * (c[1] + c[10] * rt * nt + scales) + (abs(work) ** 3 + abs(stream) ** 3) ** (1 / 3) + over + c[11] * 1e-6 * n * m
 
 
 MODELS = {"flow": (flow, FLOW), "narrow": (narrow, NARROW), "narrow blocks": (narrow, NARROW_BLOCKS), "wide": (wide, WIDE),
-          "tall": (tall, TALL)}
+          "tall": (tall, TALL), "tall blocks": (tall, TALL_BLOCKS)}
 
 
 def config_of(r):
@@ -124,7 +127,7 @@ def config_of(r):
 
     if r["kind"] == "flow":
         d = dict(rows_per_wave=64, waves_m=4, waves_k=1, split_k=r["split"], prefetch=4, x_chunk=64, lds_tile_rows=-4)
-    elif r["kind"] == "tall":
+    elif r["kind"] in ("tall", "tall blocks"):
         d = dict(rows_per_wave=r["rows"], waves_m=1, waves_k=8, split_k=r["split"], prefetch=2, x_chunk=64, lds_tile_rows=-6)
     elif r["kind"] == "wide":
         d = dict(rows_per_wave=64, waves_m=1, waves_k=1, split_k=r["split"], prefetch=2, x_chunk=64, lds_tile_rows=256)
@@ -158,8 +161,8 @@ def launches(kind, rng, per_shape):
         tiles = _cd(m, 256) * _cd(n, 256)
         splits = [s for s in (1, 2, 3, 4, 6, 8) if s == 1 or (tiles * s <= 400 and _cd(k, 64) / s >= 8)]
         return [row(m, n, k, token_tiles=16, split=s) for s in rng.sample(splits, min(per_shape, len(splits)))]
-    lo, hi = (6, 390) if kind == "flow" else (0.5, 400) if kind == "tall" else (0.5, 100)
-    unit = 256 if kind == "narrow blocks" else 8
+    lo, hi = (6, 390) if kind == "flow" else (0.5, 400) if kind in ("tall", "tall blocks") else (0.5, 100)
+    unit = 256 if kind in ("narrow blocks", "tall blocks") else 8
     while True:
         m, k = 16 * round(_log_uniform(rng, 64, 3584)), unit * round(_log_uniform(rng, 1024 / unit, 28672 / unit))
         if lo <= m * k / 2e6 <= hi:
@@ -171,13 +174,13 @@ def launches(kind, rng, per_shape):
         shares = {p * tiles for p in (1, 2, 3, 4, 6, 8)} | {64, 128, 192, 256, 384, 512}
         shares = sorted(s for s in shares if s <= 2 * CUS and s <= tiles * units)
         return [row(m, n, k, token_tiles=nt, split=s) for s in rng.sample(shares, min(per_shape, len(shares)))]
-    if kind == "tall":
-        fit = []
+    if kind in ("tall", "tall blocks"):
+        block, fit = rng.choice((64, 128)) if kind == "tall blocks" else 0, []
         for rt in range(2, 8 if nt == 4 else 9):
             tiles = _cd(m, 16 * rt)
             most = max(1, min(CUS // tiles, 16, k // 512))
             fit += [(16 * rt, split) for split in sorted({most, max(1, most - 1), max(1, most // 2)})]
-        return [row(m, n, k, rows=rows, token_tiles=nt, split=split) for rows, split in rng.sample(fit, min(per_shape, len(fit)))]
+        return [row(m, n, k, block, rows=rows, token_tiles=nt, split=split) for rows, split in rng.sample(fit, min(per_shape, len(fit)))]
     block = rng.choice((64, 128)) if kind == "narrow blocks" else 0
     fit = [v for v in VARIANTS if v[3] == 1 or v[3] < 2 * nt]
     return [row(m, n, k, block, *v, split=1) for v in rng.sample(fit, min(per_shape, len(fit)))]
