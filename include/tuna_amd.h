@@ -102,7 +102,10 @@ typedef struct tuna_gemm_config {
                               kernel's variants for any m and k - rows_per_wave 16, 32 or 64 (waves_m 0)
                               and the other fields as for that kernel.  -6: the tall-tile kernel -
                               rows_per_wave (32 .. 128 in steps of 16; not 128 with four token tiles) rows
-                              x token_tiles (1 .. 4) x 16 tokens per workgroup, in split_k parts of k */
+                              x token_tiles (1 .. 4) x 16 tokens per workgroup, in split_k parts of k.
+                              -7: the broad-tile kernel - rows_per_wave (64, 96, 128, 160, 192 or 256; times
+                              token_tiles at most 1024) rows x token_tiles (4 .. 6) x 16 tokens per
+                              workgroup, in split_k parts of k */
 } tuna_gemm_config;
 
 int tuna_version(void);

@@ -145,7 +145,8 @@ int tuna_set_multi_shape(int waves_m, int prefetch);
 int tuna_set_multi_weight_path(int through_lds);
 /* Diagnostic: tuna_matmul_blockwise calls so far in this process that ran the narrow-row kernel (kernel 0), launches of
  * the batched streaming kernel (1), calls that ran the many-token kernel (2), calls that ran the streaming kernel's
- * scale-block twin (3) and calls that ran the tall-tile kernel (4) on their behalf. */
+ * scale-block twin (3) and calls that ran the tall-tile kernel (4)
+ * or the broad-tile kernel (5) on their behalf. */
 unsigned long long tuna_blockwise_launches(int kernel);
 /* A/B switch of the narrow-row blockwise GEMM, process-wide: 1 (default) copies a workgroup's scales into LDS once and
  * reads them from there (when they fit beside the decode table), 0 reads them from memory with every ring slot.

@@ -391,6 +391,39 @@ static int launch_tall(TallPlan &plan, const void *q, const void *x, const void 
     return e == hipSuccess ? TUNA_OK : hip_fail(e, "tall-tile gemm launch");
 }
 
+// The broad-tile kernel (gemm_broad.hip): rows_per_wave rows per tile, token_tiles x 16 tokens, split_k parts of k.
+static inline bool is_broad(const tuna_gemm_config &c) { return c.lds_tile_rows == -7; }
+
+static int plan_broad(int m, int n, int k, const tuna_gemm_config &c, int decode, BroadPlan *plan, int blk_shift = -1)
+{
+    int rc = check_shape(m, n, k);
+    if (rc) return rc;
+    if (decode != TUNA_DECODE_GEMM) return fail(TUNA_ERR_UNSUPPORTED, "the broad-tile kernel implements TUNA_DECODE_GEMM only");
+    memset(plan, 0, sizeof(*plan));
+    BroadArgs &a = plan->args;
+    a.m = m, a.n = n, a.k = k;
+    if (!plan_gemm_broad(c.rows_per_wave, c.token_tiles, c.split_k, blk_shift, plan))
+        return fail(TUNA_ERR_UNSUPPORTED, "broad-tile kernel: %d rows x %d token tiles, k=%d in %d parts", c.rows_per_wave, c.token_tiles, k, c.split_k);
+    return TUNA_OK;
+}
+
+static int launch_broad(BroadPlan &plan, const void *q, const void *x, const void *code, const void *absmax, void *out, int epilogue,
+                        const void *residual, bool static_ws, hipStream_t stream)
+{
+    BroadArgs &a = plan.args;
+    a.q = static_cast<const uint8_t *>(q);
+    a.x = x;
+    a.code = static_cast<const float *>(code);
+    a.absmax = static_cast<const float *>(absmax);
+    a.out = out;
+    a.epilogue = epilogue;
+    a.residual = residual;
+    const int rc = plan.ws_bytes ? provide_workspace(static_ws, stream, plan.ws_bytes, plan.n_counters, &a.ws, &a.counters) : TUNA_OK;
+    if (rc) return rc;
+    const hipError_t e = launch_gemm_broad(plan, stream);
+    return e == hipSuccess ? TUNA_OK : hip_fail(e, "broad-tile gemm launch");
+}
+
 // Narrow-row kernel: checks and launch arguments for a config with rows_per_wave 16 or 32.
 struct NarrowPlan {
     NarrowArgs args;
@@ -1036,6 +1069,10 @@ static bool config_runs(int m, int n, int k, const tuna_gemm_config &c)
         TallPlan tp;
         return plan_tall(m, n, k, c, TUNA_DECODE_GEMM, &tp) == TUNA_OK;
     }
+    if (is_broad(c)) {
+        BroadPlan bp;
+        return plan_broad(m, n, k, c, TUNA_DECODE_GEMM, &bp) == TUNA_OK;
+    }
     if (is_narrow_any(c)) {
         NarrowPlan np;
         return plan_narrow_any(m, n, k, c, TUNA_DECODE_GEMM, &np) == TUNA_OK;
@@ -1065,7 +1102,8 @@ static double flow_time(double tiles, int units, int nt, int shares)
     return 6.1 + per_share * step + (contributors > 1.0 ? 2.7 + (contributors > 2.0 ? 0.3 * nt * (contributors - 2.0) : 0.0) : 0.0);
 }
 
-// The same for launches of at least 14 units per compute unit (117 MB) in 257 ... 512 shares: there the second workgroup on a compute
+// The same for launches of at least 14 units per compute unit (117 MB) and 64 tiles (with fewer, tiles with more contributors than
+// any it was read off: 8192 x 28672 at 54 tokens 56 us on 256 shares, 70 on 512) in 257 ... 512 shares: there the second workgroup on a compute
 // unit is worth a fifth and more, and the stream of the weights counts.  Read off 54 random shapes of 134 ... 470 MB at 16, 32,
 // 48 and 64 tokens (98 launches, 4.3 per cent off): the pick takes 1.005 x the time of a shape's best launch (worst 1.09),
 // where flow_time's takes 1.125 x (worst 1.37).  With 14 ... 16 units it is 1.03 x against 1.05 x, with 10 ... 12 1.05 x against 1.02 x.
@@ -1083,7 +1121,7 @@ static double flow_long_time(double tiles, int units, int nt, int shares)
 static int flow_best_shares(long long tiles, int units, int nt, const Room &room, double *us)
 {
     int best = 0;
-    bool is_long = tiles * units >= (long long)kFlowLongUnits * kMaxCus;
+    bool is_long = tiles >= kMaxCus / 4 && tiles * units >= (long long)kFlowLongUnits * kMaxCus;
     auto consider = [&](long long shares) {
         if (shares < 1 || shares > 2 * kMaxCus || shares > tiles * units || (is_long && shares <= kMaxCus)) return;
         if (!room.holds(flow_ws_bytes(tiles, (int)shares, nt), flow_slots(tiles, shares) ? (size_t)tiles : 0)) return;
@@ -1201,9 +1239,52 @@ static bool best_tall(int m, int n, int k, int nblk, const Room &room, tuna_gemm
     return found;
 }
 
+// Microseconds of a launch of the broad-tile kernel (gemm_broad.hip): tiles of `rows` rows and 16 `nt` tokens in `split` parts of k,
+// by a model read off 300 random shapes of 0.5 ... 400 MB of weights at 49 ... 640 tokens, each with up to 14 variants (4.9 per cent
+// off on average on the 440 launches kept; the pick takes 1.01 x the time of a shape's best): units of four k-steps whose time
+// is a row tile's decode and a token tile's way through LDS, more where all compute units have a workgroup; with `nblk` scales
+// a row 200 shapes with blocks of 64 and 128 (5.1 per cent; 1.01 x).
+static double broad_time(int m, int n, int k, int rows, int nt, int split, int nblk = 0)
+{
+    const int rt = rows / 32, units = ceil_div(ceil_div(k, 64), 4), part = ceil_div(units, split), parts = ceil_div(units, part);
+    const long long items = (long long)ceil_div(m, rows) * ceil_div(n, 16 * nt) * parts, full = items / kMaxCus, rest = items % kMaxCus;
+    const double unit = 0.1557 + (nblk ? 0.1365 : 0.13) * rt + (k % 64 ? 0.1034 : 0.0865) * nt + 0.00105 * rt * nt;
+    const double work = part * ((double)full * (unit + 0.0496 * nt) + (rest ? unit + 0.0496 * nt * rest / kMaxCus : 0.0));
+    const double scales = nblk ? 0.0298 * 0.125 * rt * ceil(part * 256.0 * nblk / k) : 0.0;
+    return (nblk ? 4.096 : 3.015) + (double)(full + (rest ? 1 : 0)) * (1.578 + 0.0809 * rt * nt + scales) + work +
+           (parts > 1 ? 1.831 + 0.0343 * parts * nt * rt : 0.0) + 0.8826e-6 * n * m;
+}
+
+// The tile and the number of k parts that take least time with partial sums that `room` holds, and that time in *us.
+static bool best_broad(int m, int n, int k, int nblk, const Room &room, tuna_gemm_config *broad, double *us)
+{
+    static const int kRows[6] = {64, 96, 128, 160, 192, 256};
+    const int blk_shift = nblk ? log2i(k / nblk) - 6 : -1;
+    bool found = false;
+    for (int nt = 4; nt <= 6; ++nt)
+        for (const int rows : kRows) {
+            if (rows * nt > 1024) continue;
+            const long long items = (long long)ceil_div(m, rows) * ceil_div(n, 16 * nt);
+            const int most = items < kMaxCus ? std::max(1, std::min((int)(kMaxCus / items), std::min(16, k / 1024))) : 1;
+            for (int split = most; split >= 1; split = split > 2 ? std::max(split / 2, split == most ? split - 1 : 1) : split - 1) {
+                const double t = broad_time(m, n, k, rows, nt, split, nblk);
+                if (found && t >= *us) continue;
+                tuna_gemm_config c;
+                memset(&c, 0, sizeof(c));
+                c.rows_per_wave = rows, c.waves_m = 2, c.waves_k = 4, c.prefetch = 2, c.x_chunk = 256, c.token_tiles = nt;
+                c.split_k = split, c.lds_tile_rows = -7;
+                BroadPlan plan;
+                if (plan_broad(m, n, k, c, TUNA_DECODE_GEMM, &plan, blk_shift) != TUNA_OK || !room.holds(plan.ws_bytes, plan.n_counters)) continue;
+                *broad = c, *us = t, found = true;
+            }
+        }
+    return found;
+}
+
 double predicted_us(int m, int n, int k, const tuna_gemm_config &c, int nblk)
 {
     if (is_tall(c)) return tall_time(m, n, k, c.rows_per_wave / 16, c.split_k, nblk);
+    if (is_broad(c)) return broad_time(m, n, k, c.rows_per_wave, c.token_tiles, c.split_k, nblk);
     if (is_flow(c)) return flow_time(ceil_div(m, 256), ceil_div(ceil_div(k, 64), 4), c.token_tiles, c.split_k);
     if (is_narrow_any(c) || is_narrow(c)) return narrow_time(m, n, k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles, nblk);
     if (c.lds_tile_rows == 256 && c.token_tiles == 16 && c.rows_per_wave != 32) {
@@ -1288,6 +1369,22 @@ static bool tall_instead(int m, int n, int k, const tuna_gemm_config &c, bool fr
     return best_tall(m, n, k, 0, room, tall, &us) && us < price;
 }
 
+// What a config for more than 64 tokens takes by its kernel's model, in microseconds: 256 x 256 tiles by theirs, many-token and
+// streaming tiles by the grid cost model; 0 where there is none.
+static double many_token_price(int m, int n, int k, const tuna_gemm_config &c)
+{
+    const int tokens = 16 * c.token_tiles, streaming = c.lds_tile_rows <= 0;
+    const int rows = streaming ? c.rows_per_wave * c.waves_m : c.lds_tile_rows;
+    if (!streaming && rows == 256 && tokens == 256 && c.rows_per_wave != 32) {
+        const WideTiles t(m, n, k);
+        return wide_time(t.large, t.small, t.steps, c.split_k == 1 && wide_balance_pays(m, n, k) ? 0 : c.split_k);
+    }
+    for (const GridCand &cd : kGridCand)
+        if (cd.rows == rows && cd.tokens == tokens && cd.streaming == streaming && (!streaming || c.split_k == 1))
+            return kGridCostUs * k * grid_cost(cd, c.split_k, (long long)ceil_div(m, rows) * ceil_div(n, tokens) * c.split_k, k);
+    return 0.0;
+}
+
 // What a launch without an explicit config runs from 65 tokens on: the selected config, or 256 x 256 tiles of gemm_wide.hip
 // in its place where their model is ahead of the grid cost model's price of that config by more than the models' error
 // (26624 x 5888 at 665 tokens 265 -> 219 us, 4096 x 14336 at 777 tokens 135 -> 117, 46848 x 5120 at 295 tokens 205 -> 175;
@@ -1297,17 +1394,9 @@ static bool tall_instead(int m, int n, int k, const tuna_gemm_config &c, bool fr
 static bool wide_instead(int m, int n, int k, const tuna_gemm_config &c, const Room &room, tuna_gemm_config *wide)
 {
     if (n <= 64 || is_narrow(c)) return false;
-    const int tokens = 16 * c.token_tiles, streaming = c.lds_tile_rows <= 0;
-    const int rows = streaming ? c.rows_per_wave * c.waves_m : c.lds_tile_rows;
     const WideTiles t(m, n, k);
-    double price = 0.0, us = 0.0;
-    if (!streaming && rows == 256 && tokens == 256 && c.rows_per_wave != 32) {
-        price = wide_time(t.large, t.small, t.steps, c.split_k == 1 && wide_balance_pays(m, n, k) ? 0 : c.split_k);
-    } else {
-        for (const GridCand &cd : kGridCand)
-            if (cd.rows == rows && cd.tokens == tokens && cd.streaming == streaming && (!streaming || c.split_k == 1))
-                price = kGridCostUs * k * grid_cost(cd, c.split_k, (long long)ceil_div(m, rows) * ceil_div(n, tokens) * c.split_k, k);
-    }
+    const double price = many_token_price(m, n, k, c);
+    double us = 0.0;
     const int split = price == 0.0 ? 0 : wide_best_split(t.large, t.small, t.steps, room, &us);
     // (four parts and more: what their hand-over costs beyond the model)
     if (!split || us * (split >= 4 ? 1.1 : 1.0) >= 0.96 * price) return false;
@@ -1379,6 +1468,23 @@ static int select_config_for(int m, int n, int k, int decode, tuna_gemm_config *
     return TUNA_OK;
 }
 
+// From 49 to 512 tokens, last: broad tiles where their model is ahead of the pick's.  On 249 random shapes of 65 ... 640 tokens
+// it takes 152, 1.28 x faster (many-token tiles 1.26 x, streaming ones 1.2 x, 256 x 256 tiles split over k 1.2 x; worst 0.84:
+// 8192 x 28672 at 303 tokens in three rounds, hence less trust in those).  What the table holds of narrow rows stays.
+static bool broad_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, double flow_us, const Room &room, tuna_gemm_config *broad)
+{
+    if (n < 49 || n > 512) return false;
+    double price;
+    if (is_flow(c)) price = flow_us;
+    else if (is_tall(c)) price = tall_time(m, n, k, c.rows_per_wave / 16, c.split_k);
+    else if (is_narrow(c) || is_narrow_any(c)) price = n > 64 && !from_table ? narrow_time(m, n, k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles) : 0.0;
+    else price = n > 64 ? many_token_price(m, n, k, c) : 0.0;
+    double us = 0.0;
+    if (price == 0.0 || !best_broad(m, n, k, 0, room, broad, &us)) return false;
+    const double rounds = ceil((double)ceil_div(m, broad->rows_per_wave) * ceil_div(n, 16 * broad->token_tiles) / kMaxCus);
+    return us < (rounds > 2 ? 0.88 : 0.95) * price;
+}
+
 // The config a launch without an explicit one runs: the selected one, or a newer kernel in its place - one whose partial
 // sums `room` holds.
 static void select_launch(int m, int n, int k, int decode, const Room &room, tuna_gemm_config *c)
@@ -1391,6 +1497,7 @@ static void select_launch(int m, int n, int k, int decode, const Room &room, tun
     if (wide_instead(m, n, k, *c, room, &other) || flow_instead(m, n, k, *c, from_table != 0, room, &other, &flow_us)) *c = other;
     if (narrow_any_instead(m, n, k, *c, from_table != 0, flow_us, &other)) *c = other;
     if (tall_instead(m, n, k, *c, from_table != 0, flow_us, room, &other)) *c = other;
+    if (broad_instead(m, n, k, *c, from_table != 0, flow_us, room, &other)) *c = other;
 }
 
 // The checks of the planner `c` belongs to, for a decode mode.
@@ -1407,6 +1514,10 @@ static int validate_for(int m, int n, int k, const tuna_gemm_config &c, int deco
     if (is_tall(c)) {
         TallPlan tp;
         return plan_tall(m, n, k, c, decode, &tp);
+    }
+    if (is_broad(c)) {
+        BroadPlan bp;
+        return plan_broad(m, n, k, c, decode, &bp);
     }
     if (is_narrow_any(c)) {
         NarrowPlan np;
@@ -1758,6 +1869,11 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
         TallPlan tp;
         if ((rc = plan_tall(m, n, k, c, decode, &tp))) return rc;
         return or_with_less(launch_tall(tp, q, x, code, absmax, out, epilogue, residual, static_ws, stream));
+    }
+    if (is_broad(c)) {
+        BroadPlan bp;
+        if ((rc = plan_broad(m, n, k, c, decode, &bp))) return rc;
+        return or_with_less(launch_broad(bp, q, x, code, absmax, out, epilogue, residual, static_ws, stream));
     }
     if (is_narrow_any(c)) {
         NarrowPlan np;
@@ -2317,13 +2433,14 @@ TUNA_EXPORT int tuna_quantize_blockwise(const void *w, const void *code, void *q
 // A config comes from the caller (tuna_matmul_blockwise_ex), from the table of tuned entries keyed by (m, token bucket,
 // k, block_size) (config_table.cpp, written by the tuner), or from the rules of derive_blockwise below.
 // ---------------------------------------------------------------------------------------
-enum BlockwiseFamily { kBlkNarrow = 0, kBlkMulti = 1, kBlkTiled = 2, kBlkMid = 3, kBlkFlow = 4, kBlkNarrowAny = 5, kBlkTall = 6 };
+enum BlockwiseFamily { kBlkNarrow = 0, kBlkMulti = 1, kBlkTiled = 2, kBlkMid = 3, kBlkFlow = 4, kBlkNarrowAny = 5, kBlkTall = 6, kBlkBroad = 7 };
 
 static BlockwiseFamily blockwise_family(const tuna_gemm_config &c)
 {
     if (c.lds_tile_rows > 0) return kBlkTiled;
     if (is_flow(c)) return kBlkFlow;
     if (is_tall(c)) return kBlkTall;
+    if (is_broad(c)) return kBlkBroad;
     if (is_narrow_any(c)) return kBlkNarrowAny;
     if (is_narrow(c)) return kBlkNarrow;
     if (c.split_k == 0) return kBlkMulti;
@@ -2423,6 +2540,14 @@ static int run_blockwise(const BlockwiseCall &b, const tuna_gemm_config &c, hipS
         diag::count(diag::kBlockwiseTall);
         return TUNA_OK;
     }
+    case kBlkBroad: {
+        BroadPlan bp;
+        if ((rc = plan_broad(m, n, k, c, TUNA_DECODE_GEMM, &bp, shift))) return rc;
+        if (dry) return TUNA_OK;
+        if ((rc = launch_broad(bp, b.q, b.x, b.code, b.absmax, b.out, TUNA_EPILOGUE_NONE, nullptr, false, st))) return rc;
+        diag::count(diag::kBlockwiseBroad);
+        return TUNA_OK;
+    }
     case kBlkNarrowAny: {
         NarrowPlan np;
         if ((rc = plan_narrow_any(m, n, k, c, TUNA_DECODE_GEMM, &np))) return rc;
@@ -2453,6 +2578,24 @@ static int run_blockwise(const BlockwiseCall &b, const tuna_gemm_config &c, hipS
     }
     return fail(TUNA_ERR_UNSUPPORTED, "unknown blockwise kernel family");
 }
+
+// Many-token tiles with scale blocks and their factors in the model of derive_config, what a launch of `tiles` workgroups costs
+// in units of 5.68e-7 us per k, and the 256 x 256 tile by its per-row time: 1.07 x, more where k is split (four parts and more
+// cost a quarter more than the model says: 4032 x 6400 at 580 tokens 73 us, the best other tile 56).
+struct BlockwiseTile {
+    int rows, tokens;
+    double factor;
+};
+static const BlockwiseTile kBlockwiseTiles[6] = {{128, 256, 1.0}, {256, 128, 1.2}, {128, 128, 1.2}, {64, 256, 1.2}, {256, 64, 1.6}, {64, 128, 1.6}};
+constexpr double kBlockwiseCostUs = 5.68e-7;
+static double blockwise_tile_cost(const BlockwiseTile &t, int split, long long tiles, int k)
+{
+    const long long full = tiles / kMaxCus, rest = tiles % kMaxCus;
+    const double rounds = 1.15 * (double)full + (rest ? 0.7 + 0.45 * (double)rest / kMaxCus : 0.0);
+    const double area = (double)t.rows * t.tokens;
+    return rounds * (area * t.factor / split + 0.6e7 / k) + (split > 1 ? (100.0 * split + 300.0) * area / k : 0.0);
+}
+static double blockwise_wide_time(double per_row_us, int split) { return 1.07 * per_row_us * (split >= 4 ? 1.25 : split > 1 ? 1.05 : 1.0) + 2.0; }
 
 // The config for a shape that has no tuned entry, from what the tuner found on the benchmark shapes (a scale per 64
 // weights, us).  The streaming kernel's twin where the per-row table has an unsplit streaming entry for the shape and
@@ -2541,21 +2684,16 @@ static int derive_blockwise(const BlockwiseCall &b, const Room &room, tuna_gemm_
         // shapes x ten counts from 72 to 2048 tokens with blocks of 64, each timed with every tile and split: the
         // model's pick is within 7 % of the best on all 160 cases (the rule below, which this one precedes: 1.23 x
         // on average, up to 2.8 x where it split k by 8 or 10 - 4096 x 4096 at 200 tokens 74 us against 26).
-        struct Tile { int rows, tokens; double factor; };
-        static const Tile kTiles[6] = {{128, 256, 1.0}, {256, 128, 1.2}, {128, 128, 1.2}, {64, 256, 1.2}, {256, 64, 1.6}, {64, 128, 1.6}};
         static const int kSplits[6] = {1, 2, 3, 4, 6, 8};
         tuna_gemm_config best;
         double best_cost = 0.0;
         bool found = false;
-        for (const Tile &t : kTiles)
+        for (const BlockwiseTile &t : kBlockwiseTiles)
             for (int split : kSplits) {
                 const long long tiles = (long long)ceil_div(m, t.rows) * ceil_div(n, t.tokens) * split;
                 if (split > 1 && (tiles > 300 || ceil_div(k, 64) / split < 8)) continue;
                 if (tiles < 32) continue;
-                const long long full = tiles / kMaxCus, rest = tiles % kMaxCus;
-                const double rounds = 1.15 * (double)full + (rest ? 0.7 + 0.45 * (double)rest / kMaxCus : 0.0);
-                const double area = (double)t.rows * t.tokens;
-                const double cost = rounds * (area * t.factor / split + 0.6e7 / k) + (split > 1 ? (100.0 * split + 300.0) * area / k : 0.0);
+                const double cost = blockwise_tile_cost(t, split, tiles, k);
                 if (found && cost >= best_cost) continue;
                 tuna_gemm_config c;
                 memset(&c, 0, sizeof(c));
@@ -2564,15 +2702,13 @@ static int derive_blockwise(const BlockwiseCall &b, const Room &room, tuna_gemm_
                 if (run_blockwise(b, c, nullptr, true) != TUNA_OK) continue;
                 best = c, best_cost = cost, found = true;
             }
-        // The 256 x 256 tile by its own model, 1.07 x the time of the per-row kernel (a unit of the costs above is 5.68e-7
-        // us per k, both read off 200 random shapes at 65 ... 4096 tokens with blocks of 64, where this tile is up to
+        // The 256 x 256 tile by its own model (blockwise_wide_time), read off 200 random shapes at 65 ... 4096 tokens with blocks of 64, where this tile is up to
         // 1.6 x faster than the best of the others: 3584 x 25088 at 2669 tokens 756 us -> 462, 5632 x 16384 at 701 tokens
         // 232 -> 159, 11136 x 1536 at 2891 tokens 158 -> 121).
         const WideTiles t(m, n, k);
         double us = 0.0;
         const int split = n > 64 ? wide_best_split(t.large, t.small, t.steps, room, &us) : 0;
-        // (four parts and more cost a quarter more than the model says: 4032 x 6400 at 580 tokens 73 us, the best other tile 56)
-        if (split && (!found || (1.07 * us * (split >= 4 ? 1.25 : split > 1 ? 1.05 : 1.0) + 2.0) / 5.68e-7 / k < 0.96 * best_cost)) {
+        if (split && (!found || blockwise_wide_time(us, split) / kBlockwiseCostUs / k < 0.96 * best_cost)) {
             tuna_gemm_config c;
             memset(&c, 0, sizeof(c));
             c.rows_per_wave = 64, c.waves_m = 1, c.waves_k = 1, c.prefetch = 2, c.x_chunk = 64, c.token_tiles = 16;
@@ -2662,6 +2798,31 @@ static bool blockwise_tall_instead(const BlockwiseCall &b, const tuna_gemm_confi
     return !best_narrow_any(b.m, b.n, b.k, nblk, us, &any);
 }
 
+// From 65 to 384 tokens: broad tiles (gemm_broad.hip) where their model is ahead of the derived config's.  Of 180
+// random shapes of 49 ... 640 tokens with blocks of 64 and 128 it takes 64, 1.23 x faster (worst 0.87: 24384 x 3584 at
+// 217 tokens, which puts 508 tiles on 256 compute units; above 384 tokens it loses as often as it gains).
+static bool blockwise_broad_instead(const BlockwiseCall &b, const tuna_gemm_config &c, const Room &room, tuna_gemm_config *broad)
+{
+    if (b.n <= 64 || b.n > 384) return false;
+    const int nblk = b.k / b.block_size, tokens = 16 * c.token_tiles;
+    double price = 0.0;
+    if (blockwise_family(c) == kBlkNarrow) {
+        price = narrow_time(b.m, b.n, b.k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles, nblk);
+    } else if (blockwise_family(c) == kBlkTiled) {
+        if (c.lds_tile_rows == 256 && tokens == 256) {
+            const WideTiles t(b.m, b.n, b.k);
+            price = blockwise_wide_time(wide_time(t.large, t.small, t.steps, c.split_k == 1 && wide_balance_pays(b.m, b.n, b.k) ? 0 : c.split_k), c.split_k);
+        }
+        for (const BlockwiseTile &t : kBlockwiseTiles)
+            if (t.rows == c.lds_tile_rows && t.tokens == tokens)
+                price = kBlockwiseCostUs * b.k * blockwise_tile_cost(t, c.split_k, (long long)ceil_div(b.m, t.rows) * ceil_div(b.n, tokens) * c.split_k, b.k);
+    }
+    double us = 0.0;
+    if (price == 0.0 || !best_broad(b.m, b.n, b.k, nblk, room, broad, &us)) return false;
+    const double rounds = ceil((double)ceil_div(b.m, broad->rows_per_wave) * ceil_div(b.n, 16 * broad->token_tiles) / kMaxCus);
+    return us < (rounds > 2 ? 0.88 : 0.95) * price;
+}
+
 // Tuned entry for (m, n, k, block_size) if the table has one that can run the call, else the derived config.
 static int select_blockwise(const BlockwiseCall &b, const Room &room, tuna_gemm_config *cfg, int *from_table)
 {
@@ -2682,7 +2843,7 @@ static int select_blockwise(const BlockwiseCall &b, const Room &room, tuna_gemm_
         }
     }
     const int rc = derive_blockwise(b, room, cfg);
-    if (!rc && blockwise_tall_instead(b, *cfg, room, &tall)) *cfg = tall;
+    if (!rc && (blockwise_tall_instead(b, *cfg, room, &tall) || blockwise_broad_instead(b, *cfg, room, &tall))) *cfg = tall;
     return rc;
 }
 
@@ -2873,6 +3034,14 @@ TUNA_EXPORT int tuna_config_footprint(int m, int n, int k, const tuna_gemm_confi
         if (workspace_bytes) *workspace_bytes = tp.ws_bytes;
         return TUNA_OK;
     }
+    if (is_broad(*cfg)) {
+        BroadPlan bp;
+        int rc = plan_broad(m, n, k, *cfg, TUNA_DECODE_GEMM, &bp);
+        if (rc) return rc;
+        if (lds_bytes) *lds_bytes = broad_lds_bytes(bp);
+        if (workspace_bytes) *workspace_bytes = bp.ws_bytes;
+        return TUNA_OK;
+    }
     if (is_narrow_any(*cfg)) {
         NarrowPlan np;
         int rc = plan_narrow_any(m, n, k, *cfg, TUNA_DECODE_GEMM, &np);
@@ -3037,6 +3206,7 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
         const int at = is_narrow_any(w) && plan_narrow_any(m, n, k, w, decode_mode, &np) == TUNA_OK
                            ? describe_narrow_any(np, n, buf, len, " in place of ")
                        : is_flow(w) ? snprintf(buf, len, "gemm_flow_kernel<NT=%d> %d shares in place of ", w.token_tiles, w.split_k)
+                       : is_broad(w) ? snprintf(buf, len, "gemm_broad_kernel<%d rows x %d tokens> split_k=%d in place of ", w.rows_per_wave, 16 * w.token_tiles, w.split_k)
                        : is_tall(w) ? snprintf(buf, len, "gemm_flow_kernel_tall<%d rows,NT=%d> split_k=%d in place of ", w.rows_per_wave, w.token_tiles, w.split_k)
                                     : snprintf(buf, len, "gemm_wide_kernel<256 rows x 256 tokens> split_k=%d in place of ", w.split_k);
         return at < 0 || (size_t)at + 16 > len ? TUNA_OK : tuna_describe_launch(m, n, k, &c, decode_mode, buf + at, len - (size_t)at);
@@ -3060,6 +3230,12 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
         TallPlan tp;
         if ((rc = plan_tall(m, n, k, c, decode_mode, &tp))) return rc;
         snprintf(buf, len, "gemm_flow_kernel_tall<%d rows,NT=%d> split_k=%d", 16 * tp.rt, tp.nt, tp.split);
+        return TUNA_OK;
+    }
+    if (is_broad(c)) {
+        BroadPlan bp;
+        if ((rc = plan_broad(m, n, k, c, decode_mode, &bp))) return rc;
+        snprintf(buf, len, "gemm_broad_kernel<%d rows x %d tokens> split_k=%d", c.rows_per_wave, 16 * bp.nt, bp.split);
         return TUNA_OK;
     }
     if (is_narrow_any(c)) {

@@ -19,7 +19,7 @@ int multi_lds();             // 1: batches with a ring of two stage weights and 
 int multi_min_batch();       // batches shorter than this are launched problem by problem (2)
 int blockwise_scales_lds();  // 1: the narrow-row blockwise kernel keeps a workgroup's scales in LDS
 
-enum Counter { kLeanLaunches, kMultiLaunches, kBlockwiseNarrow, kBlockwiseMulti, kBlockwiseTiled, kBlockwiseMid, kBlockwiseTall, kNumCounters };
+enum Counter { kLeanLaunches, kMultiLaunches, kBlockwiseNarrow, kBlockwiseMulti, kBlockwiseTiled, kBlockwiseMid, kBlockwiseTall, kBlockwiseBroad, kNumCounters };
 void count(Counter c);
 
 }  // namespace diag

@@ -48,7 +48,7 @@ TUNA_EXPORT unsigned long long tuna_multi_launches(void) { return g_counters[kMu
 
 TUNA_EXPORT unsigned long long tuna_blockwise_launches(int kernel)
 {
-    return kernel >= 0 && kernel < 5 ? g_counters[kBlockwiseNarrow + kernel].load(std::memory_order_relaxed) : 0ull;
+    return kernel >= 0 && kernel < 6 ? g_counters[kBlockwiseNarrow + kernel].load(std::memory_order_relaxed) : 0ull;
 }
 TUNA_EXPORT int tuna_set_blockwise_scales_lds(int enabled) { return g_blockwise_scales_lds.exchange(enabled ? 1 : 0); }
 }  // extern "C"

@@ -26,20 +26,12 @@
 // are read half a step ahead.  28672 x 4096 with blocks of 64: 20.2 -> 18.2 us at 16 tokens, 37 -> 27.6 at 64; 8192 x 28672 at 32
 // tokens 58 -> 39.
 #include "epilogue.hpp"
+#include "row_pieces.hpp"
 
 namespace tuna {
 
 namespace {
 constexpr int kWaves = 8, kThreads = 64 * kWaves;
-
-// Pieces of a lane's weights of a k-step's half: row tiles of 16 in loads of four, two and one dwords.
-template <int RT>
-struct Pieces {
-    static constexpr int fours = RT / 4, twos = (RT & 2) / 2, ones = RT & 1, count = fours + twos + ones;
-    static constexpr int width(int p) { return p < fours ? 4 : p < fours + twos ? 2 : 1; }
-    static constexpr int first(int p) { return p <= fours ? 4 * p : p <= fours + twos ? 4 * fours + 2 * (p - fours) : RT - 1; }  // row tile
-    static constexpr int of(int r) { return r < 4 * fours ? r / 4 : r < 4 * fours + 2 * twos ? fours : count - 1; }
-};
 
 template <int RT, int NT>
 constexpr size_t slot_bytes() { return (size_t)RT * NT * 1024; }

@@ -229,12 +229,23 @@ struct TallArgs {
     int blk_shift;       // a scale block is 64 << blk_shift weights, if the plan has part_blocks
 };
 
+typedef TallArgs BroadArgs;  // of gemm_broad.hip too
+
 struct TallPlan {
     TallArgs args;
     int rt, nt;             // 16-row tiles and 16-token tiles of a workgroup
     int tiles, split;       // row tiles; k parts of each
     int part_steps;         // k-steps of 64 of a part (the last may have fewer)
     int part_blocks;        // scale blocks that a part touches at most; 0: one scale per row
+    size_t ws_bytes, n_counters;
+};
+
+struct BroadPlan {
+    BroadArgs args;
+    int rt, nt;                   // 16-row tiles of a row group and 16-token tiles of a workgroup
+    int tiles, tok_tiles, split;  // row tiles and token tiles; k parts of each
+    int part_steps;               // k-steps of 64 of a part, whole units of four (the last may have fewer)
+    int part_blocks;              // as of TallPlan
     size_t ws_bytes, n_counters;
 };
 
@@ -355,6 +366,9 @@ hipError_t launch_gemm_flow(const FlowPlan &plan, bool scale_blocks, hipStream_t
 bool plan_gemm_tall(int row_tiles16, int nt, int split, int blk_shift, TallPlan *plan);
 hipError_t launch_gemm_tall(const TallPlan &plan, hipStream_t stream);
 size_t tall_lds_bytes(const TallPlan &plan);
+bool plan_gemm_broad(int rows, int nt, int split, int blk_shift, BroadPlan *plan);
+hipError_t launch_gemm_broad(const BroadPlan &plan, hipStream_t stream);
+size_t broad_lds_bytes(const BroadPlan &plan);
 hipError_t launch_gemm_wide32(const TiledArgs &args, hipStream_t stream);
 bool tiled_variant_exists(int tile_rows, int tile_tokens, bool mfma32);
 size_t tiled_lds_bytes(int tile_rows, int tile_tokens);

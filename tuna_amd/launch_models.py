@@ -1,4 +1,4 @@
-"""The time models behind the choice between kernels (flow_time, narrow_time, tall_time and wide_time of csrc/api.cpp): the launches
+"""The time models behind the choice between kernels (flow_time, narrow_time, tall_time, broad_time and wide_time of csrc/api.cpp): the launches
 they are read off, how far they are from them, and the fit of their coefficients.
 
     python -m tuna_amd.launch_models --measure times.csv    # on a GPU: random shapes, several launches each
@@ -117,8 +117,27 @@ def tall(r, c):
     return c[0] + rounds * (c[1] + c[10] * rt * nt + scales) + (abs(work) ** 3 + abs(stream) ** 3) ** (1 / 3) + over + c[11] * 1e-6 * n * m
 
 
+# launch, round, unit, rows, tokens, both, tokens where rows of x start inside a cache line, with every compute unit at work,
+# hand-over, its parts, sums, output, KB of a workgroup's scales
+BROAD = (3.015, 1.578, 0.1557, 0.13, 0.0865, 0.00105, 0.1034, 0.0496, 1.831, 0.0343, 0.0809, 0.8826, 0.0)
+BROAD_BLOCKS = (4.096, 1.578, 0.1557, 0.1365, 0.0865, 0.00105, 0.1034, 0.0496, 1.831, 0.0343, 0.0809, 0.8826, 0.0298)
+
+
+def broad(r, c):
+    m, n, k, nt, split = r["m"], r["n"], r["k"], r["token_tiles"], r["split"]
+    rt, units, nblk = r["rows"] // 32, _cd(_cd(k, 64), 4), k // r["block"] if r["block"] else 0
+    part = _cd(units, split)
+    parts = _cd(units, part)
+    full, rest = divmod(_cd(m, r["rows"]) * _cd(n, 16 * nt) * parts, CUS)
+    unit = c[2] + c[3] * rt + (c[6] if k % 64 else c[4]) * nt + c[5] * rt * nt
+    work = part * (full * (unit + c[7] * nt) + (unit + c[7] * nt * rest / CUS if rest else 0.0))
+    scales = c[12] * 0.125 * rt * math.ceil(part * 256.0 * nblk / k) if nblk else 0.0
+    over = c[8] + c[9] * parts * nt * rt if parts > 1 else 0.0
+    return c[0] + (full + (1 if rest else 0)) * (c[1] + c[10] * rt * nt + scales) + work + over + c[11] * 1e-6 * n * m
+
+
 MODELS = {"flow": (flow, FLOW), "narrow": (narrow, NARROW), "narrow blocks": (narrow, NARROW_BLOCKS), "wide": (wide, WIDE),
-          "tall": (tall, TALL), "tall blocks": (tall, TALL_BLOCKS)}
+          "tall": (tall, TALL), "tall blocks": (tall, TALL_BLOCKS), "broad": (broad, BROAD), "broad blocks": (broad, BROAD_BLOCKS)}
 
 
 def config_of(r):
@@ -129,6 +148,8 @@ def config_of(r):
         d = dict(rows_per_wave=64, waves_m=4, waves_k=1, split_k=r["split"], prefetch=4, x_chunk=64, lds_tile_rows=-4)
     elif r["kind"] in ("tall", "tall blocks"):
         d = dict(rows_per_wave=r["rows"], waves_m=1, waves_k=8, split_k=r["split"], prefetch=2, x_chunk=64, lds_tile_rows=-6)
+    elif r["kind"] in ("broad", "broad blocks"):
+        d = dict(rows_per_wave=r["rows"], waves_m=2, waves_k=4, split_k=r["split"], prefetch=2, x_chunk=256, lds_tile_rows=-7)
     elif r["kind"] == "wide":
         d = dict(rows_per_wave=64, waves_m=1, waves_k=1, split_k=r["split"], prefetch=2, x_chunk=64, lds_tile_rows=256)
     else:
@@ -161,19 +182,28 @@ def launches(kind, rng, per_shape):
         tiles = _cd(m, 256) * _cd(n, 256)
         splits = [s for s in (1, 2, 3, 4, 6, 8) if s == 1 or (tiles * s <= 400 and _cd(k, 64) / s >= 8)]
         return [row(m, n, k, token_tiles=16, split=s) for s in rng.sample(splits, min(per_shape, len(splits)))]
-    lo, hi = (6, 390) if kind == "flow" else (0.5, 400) if kind in ("tall", "tall blocks") else (0.5, 100)
-    unit = 256 if kind in ("narrow blocks", "tall blocks") else 8
+    lo, hi = (6, 390) if kind == "flow" else (0.5, 400) if kind.startswith(("tall", "broad")) else (0.5, 100)
+    unit = 256 if kind.endswith("blocks") else 8
     while True:
         m, k = 16 * round(_log_uniform(rng, 64, 3584)), unit * round(_log_uniform(rng, 1024 / unit, 28672 / unit))
         if lo <= m * k / 2e6 <= hi:
             break
-    n = round(_log_uniform(rng, 1, 64))
+    n = round(_log_uniform(rng, 49, 640) if kind.startswith("broad") else _log_uniform(rng, 1, 64))
     nt = _cd(n, 16)
     if kind == "flow":
         tiles, units = _cd(m, 256), _cd(_cd(k, 64), 4)
         shares = {p * tiles for p in (1, 2, 3, 4, 6, 8)} | {64, 128, 192, 256, 384, 512}
         shares = sorted(s for s in shares if s <= 2 * CUS and s <= tiles * units)
         return [row(m, n, k, token_tiles=nt, split=s) for s in rng.sample(shares, min(per_shape, len(shares)))]
+    if kind.startswith("broad"):
+        block, fit = rng.choice((64, 128)) if kind == "broad blocks" else 0, []
+        for nt in (4, 5, 6):
+            for rows in (64, 96, 128, 160, 192, 256):
+                items = _cd(m, rows) * _cd(n, 16 * nt)
+                most = max(1, min(CUS // items, 16, k // 1024))
+                if rows * nt <= 1024 and items * most <= 1200:
+                    fit += [(rows, nt, split) for split in sorted({most, max(1, most - 1), max(1, most // 2)})]
+        return [row(m, n, k, block, rows=rows, token_tiles=nt, split=split) for rows, nt, split in rng.sample(fit, min(per_shape, len(fit)))]
     if kind in ("tall", "tall blocks"):
         block, fit = rng.choice((64, 128)) if kind == "tall blocks" else 0, []
         for rt in range(2, 8 if nt == 4 else 9):

@@ -277,15 +277,15 @@ BLOCKWISE_NARROW = ({(16, 4, 2, 1), (16, 8, 4, 1), (16, 16, 2, 1), (32, 8, 2, 1)
 # many-token tiles with a scale-block variant that entries may name (16 x 16 x 32 MFMA; the 256 x 256 tile's is the
 # derivation's alone)
 BLOCKWISE_TILED = {(64, 128), (64, 256), (128, 64), (128, 128), (128, 256), (256, 64), (256, 128)}
-BLOCKWISE_FAMILIES = ("narrow", "batched", "many-token", "streaming", "tall")
+BLOCKWISE_FAMILIES = ("narrow", "batched", "many-token", "streaming", "tall", "broad")
 
 
 def blockwise_family(c: dict) -> str:
     """Which kernel a blockwise config names (mirrors blockwise_family in csrc/api.cpp)."""
     if c.get("lds_tile_rows", 0) > 0:
         return "many-token"
-    if c.get("lds_tile_rows", 0) == -6:
-        return "tall"
+    if c.get("lds_tile_rows", 0) in (-6, -7):
+        return "tall" if c["lds_tile_rows"] == -6 else "broad"
     if is_narrow(c):
         return "narrow"
     if c["split_k"] == 0:

@@ -277,7 +277,7 @@ def validate_config_blockwise(m: int, n: int, k: int, block_size: int, config: G
     _lib.check(_lib.lib().tuna_validate_config_blockwise(int(m), int(n), int(k), int(block_size), ctypes.byref(config)))
 
 
-BLOCKWISE_FAMILIES = ("narrow", "batched", "many-token", "streaming", "tall")
+BLOCKWISE_FAMILIES = ("narrow", "batched", "many-token", "streaming", "tall", "broad")
 
 
 def blockwise_family(config: GemmConfig) -> str:
