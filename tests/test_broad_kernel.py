@@ -95,6 +95,30 @@ def test_what_there_is_no_tile_for_is_refused(rows, tokens, split):
         ops.validate_config(1024, 100, 1024, _cfg(rows, tokens, split))
 
 
+# groups of one to several token tiles, empty ones among them, one token more or less than a tile's; rows no multiple of any
+# tile's; k no multiple of a unit or of 64
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,counts", [(2048, 1408, (65, 64, 96, 97, 33, 0, 80, 81, 70, 1, 128, 66, 90, 72, 0, 100)), (1088, 4096, (70, 90, 40, 88, 96, 66, 71, 80)),
+                                        (4992, 1000, (64, 0, 0, 161, 5, 76, 95, 77)), (4096, 2056, (33, 48, 64, 60, 50, 41, 64, 63, 59, 37, 62, 64)),
+                                        (14336, 512, (0, 66, 79, 0))])
+def test_groups(m, k, counts):
+    import numpy as np
+    import torch
+
+    from tuna_amd import ops
+
+    offs = np.concatenate([[0], np.cumsum(counts)]).tolist()
+    q, s, x, code = _inputs(m * len(counts), offs[-1], k, seed=k)
+    out, again = _out(offs[-1], m), _out(offs[-1], m)
+    ops.matmul_grouped(x, q, s, code, out, m, len(counts), k, offs)
+    ops.matmul_grouped(x, q, s, code, again, m, len(counts), k, offs)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    for e, (lo, hi) in enumerate(zip(offs, offs[1:])):
+        if hi > lo:
+            _check(out[lo:hi], q, s, x[lo:hi], code, k, first_row=e * m, rows=m)
+
+
 def test_a_call_without_a_config_takes_it_where_it_is_predicted_to_be_faster():
     from tuna_amd import ops
 

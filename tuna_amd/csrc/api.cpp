@@ -420,7 +420,7 @@ static int launch_broad(BroadPlan &plan, const void *q, const void *x, const voi
     a.residual = residual;
     const int rc = plan.ws_bytes ? provide_workspace(static_ws, stream, plan.ws_bytes, plan.n_counters, &a.ws, &a.counters) : TUNA_OK;
     if (rc) return rc;
-    const hipError_t e = launch_gemm_broad(plan, stream);
+    const hipError_t e = launch_gemm_broad(plan, nullptr, stream);
     return e == hipSuccess ? TUNA_OK : hip_fail(e, "broad-tile gemm launch");
 }
 
@@ -1244,15 +1244,19 @@ static bool best_tall(int m, int n, int k, int nblk, const Room &room, tuna_gemm
 // off on average on the 440 launches kept; the pick takes 1.01 x the time of a shape's best): units of four k-steps whose time
 // is a row tile's decode and a token tile's way through LDS, more where all compute units have a workgroup; with `nblk` scales
 // a row 200 shapes with blocks of 64 and 128 (5.1 per cent; 1.01 x).
-static double broad_time(int m, int n, int k, int rows, int nt, int split, int nblk = 0)
+static double broad_items_time(long long items, int k, int rt, int nt, int part, int parts, int nblk)
 {
-    const int rt = rows / 32, units = ceil_div(ceil_div(k, 64), 4), part = ceil_div(units, split), parts = ceil_div(units, part);
-    const long long items = (long long)ceil_div(m, rows) * ceil_div(n, 16 * nt) * parts, full = items / kMaxCus, rest = items % kMaxCus;
+    const long long full = items / kMaxCus, rest = items % kMaxCus;
     const double unit = 0.1557 + (nblk ? 0.1365 : 0.13) * rt + (k % 64 ? 0.1034 : 0.0865) * nt + 0.00105 * rt * nt;
     const double work = part * ((double)full * (unit + 0.0496 * nt) + (rest ? unit + 0.0496 * nt * rest / kMaxCus : 0.0));
     const double scales = nblk ? 0.0298 * 0.125 * rt * ceil(part * 256.0 * nblk / k) : 0.0;
     return (nblk ? 4.096 : 3.015) + (double)(full + (rest ? 1 : 0)) * (1.578 + 0.0809 * rt * nt + scales) + work +
-           (parts > 1 ? 1.831 + 0.0343 * parts * nt * rt : 0.0) + 0.8826e-6 * n * m;
+           (parts > 1 ? 1.831 + 0.0343 * parts * nt * rt : 0.0);
+}
+static double broad_time(int m, int n, int k, int rows, int nt, int split, int nblk = 0)
+{
+    const int units = ceil_div(ceil_div(k, 64), 4), part = ceil_div(units, split), parts = ceil_div(units, part);
+    return broad_items_time((long long)ceil_div(m, rows) * ceil_div(n, 16 * nt) * parts, k, rows / 32, nt, part, parts, nblk) + 0.8826e-6 * n * m;
 }
 
 // The tile and the number of k parts that take least time with partial sums that `room` holds, and that time in *us.
@@ -2019,6 +2023,76 @@ static int grouped_flow_shares(int m_group, int n_active, int nt, int k)
     return flow_best_shares((long long)ceil_div(m_group, 256) * n_active, ceil_div(ceil_div(k, 64), 4), nt, kRoomToGrow, &us);
 }
 
+// What the groups with more than `pass` tokens take as a launch each, or in one of 256 x 256 tiles (its split in *split, 0 if
+// that is no option or slower; its tiles in a): 6 us and the larger of 0.85 PFLOP/s and 3.5 TB/s apart, wide_time together.
+static double grouped_many_time(int m_group, int n_groups, int k, const int32_t *offsets, int pass, WideArgs *a, int *split, long long *large, long long *small)
+{
+    a->m = m_group, a->k = k, a->n_groups = 0;
+    double apart = 0.0, together = 0.0;
+    for (int e = 0; e < n_groups; ++e) {
+        const int cnt = offsets[e + 1] - offsets[e];
+        if (cnt <= pass) continue;
+        const double flops = 2.0 * m_group * cnt * k, bytes = 0.5 * m_group * k + 2.0 * cnt * ((double)m_group + k);
+        const double t_flops = flops / 0.85e9, t_bytes = bytes / 3.5e6;
+        apart += 6.0 + (t_flops > t_bytes ? t_flops : t_bytes);
+        a->tok_begin[a->n_groups] = offsets[e], a->tok_count[a->n_groups] = cnt, a->id[a->n_groups] = (unsigned char)e;
+        ++a->n_groups;
+    }
+    count_wide_tiles(*a, large, small);
+    *split = a->n_groups > 1 ? wide_best_split((double)*large, (double)*small, ceil_div(k, 64), kRoomToGrow, &together) : 0;
+    if (*split && together < apart) return together;
+    *split = 0;
+    return apart;
+}
+
+// One launch of broad tiles for all groups with tokens, where broad_time of its workgroups - a row tile and up to 96 tokens of a
+// group each, k unsplit - is ahead of the launches below: eight experts of 14336 x 4096 on 512 tokens, some of them with more than
+// 64, 147 -> 98 us, of 4096 x 14336 131 -> 84; 64 experts of 1536 x 4096 on 6144 tokens 135 -> 120.  On 120 random launches of 16 to
+// 400 tokens per group 1.18 x, up to 3.3 x for small experts, which launched one by one before; worst 0.92.
+static bool grouped_broad_pays(int m_group, int n_groups, int k, const int32_t *offsets, int max_tok, BroadPlan *plan, BroadGroups *groups)
+{
+    if (max_tok <= 32) return false;
+    memset(groups, 0, sizeof(*groups));
+    int few = 0, few_tok = 0, n_total = 0;  // groups of up to 64 tokens, which take one pass of the decode-batch kernel
+    for (int e = 0; e < n_groups; ++e) {
+        const int cnt = offsets[e + 1] - offsets[e];
+        if (cnt <= 0) continue;
+        groups->tok_begin[groups->n] = offsets[e], groups->tok_count[groups->n] = cnt, groups->id[groups->n] = e;
+        ++groups->n;
+        n_total += cnt;
+        if (cnt <= 64) ++few, few_tok = cnt > few_tok ? cnt : few_tok;
+    }
+    // (less than 4 MB of weights: as before, a large group by the launch that a dense call takes; none of the measured ones is
+    // that small)
+    if (groups->n < 2 || 0.5 * m_group * groups->n * k < 4e6) return false;
+    double price = 0.0, us = 0.0;
+    if (groups->n > few) {
+        WideArgs wide;
+        int split;
+        long long large, small;
+        price += grouped_many_time(m_group, n_groups, k, offsets, 64, &wide, &split, &large, &small);
+    }
+    if (few) {
+        if (!flow_best_shares((long long)ceil_div(m_group, 256) * few, ceil_div(ceil_div(k, 64), 4), ceil_div(few_tok, 16), kRoomToGrow, &us)) return false;
+        price += us;
+    }
+    static const int kRows[6] = {64, 96, 128, 160, 192, 256};
+    int best_rows = 0, best_nt = 0;
+    for (int nt = 4; nt <= 6; ++nt) {
+        long long tok_tiles = 0;
+        for (int e = 0; e < groups->n; ++e) tok_tiles += ceil_div(groups->tok_count[e], 16 * nt);
+        for (const int rows : kRows) {
+            if (rows * nt > 1024) continue;
+            const double t = broad_items_time(ceil_div(m_group, rows) * tok_tiles, k, rows / 32, nt, ceil_div(ceil_div(k, 64), 4), 1, 0) + 0.8826e-6 * n_total * m_group;
+            if (!best_rows || t < us) best_rows = rows, best_nt = nt, us = t;
+        }
+    }
+    if (us > 0.93 * price) return false;
+    memset(plan, 0, sizeof(*plan));
+    plan->args.m = m_group, plan->args.n = max_tok, plan->args.k = k;
+    return plan_gemm_broad_groups(best_rows, best_nt, plan, groups);
+}
+
 // Grouped GEMM: n_groups stacked weight matrices of m_group rows, group e applied to the
 // activation rows offsets[e] .. offsets[e+1]-1 only.  The offsets are a host array: they are
 // validated here and travel to the kernel as launch arguments (no device buffer, no copy).
@@ -2057,7 +2131,23 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
     // Several such groups become ONE launch of 256 x 256 tiles (gemm_wide.hip) where that is predicted to be faster than a
     // launch each, priced at 6 us and the larger of 0.85 PFLOP/s and 3.5 TB/s: eight experts of 14336 x 4096 on 4096
     // tokens leave the device half empty at the end of each of eight launches (706 us; 452 in one).
+    // Before either: one launch of broad tiles over all groups where its model is ahead of these two and of the decode-batch
+    // kernel's for the groups of up to 64.
     constexpr int kGroupedPassTokens = 64;
+    if (!cfg && decode == TUNA_DECODE_GEMM) {
+        BroadPlan plan;
+        BroadGroups groups;
+        if (grouped_broad_pays(m_group, n_groups, k, offsets, max_tok, &plan, &groups)) {
+            BroadArgs &a = plan.args;
+            a.q = static_cast<const uint8_t *>(q);
+            a.x = x;
+            a.code = static_cast<const float *>(code);
+            a.absmax = static_cast<const float *>(absmax);
+            a.out = out;
+            const hipError_t e = launch_gemm_broad(plan, &groups, stream);
+            return e == hipSuccess ? TUNA_OK : hip_fail(e, "grouped broad-tile gemm launch");
+        }
+    }
     const size_t group_q_bytes = (size_t)m_group * (size_t)k / 2;
     bool many_done = false;
     size_t many_ws = 0;  // bytes of its partial sums
@@ -2065,22 +2155,11 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
         WidePlan plan;
         memset(&plan, 0, sizeof(plan));
         WideArgs &a = plan.args;
-        a.m = m_group, a.k = k;
-        double apart = 0.0, together = 0.0;
-        for (int e = 0; e < n_groups; ++e) {
-            const int cnt = offsets[e + 1] - offsets[e];
-            if (cnt <= kGroupedPassTokens) continue;
-            const double flops = 2.0 * m_group * cnt * k, bytes = (double)group_q_bytes + 2.0 * cnt * ((double)m_group + k);
-            const double t_flops = flops / 0.85e9, t_bytes = bytes / 3.5e6;
-            apart += 6.0 + (t_flops > t_bytes ? t_flops : t_bytes);
-            a.tok_begin[a.n_groups] = offsets[e], a.tok_count[a.n_groups] = cnt, a.id[a.n_groups] = (unsigned char)e;
-            ++a.n_groups;
-        }
         long long large, small;
-        count_wide_tiles(a, &large, &small);
+        int split;
+        grouped_many_time(m_group, n_groups, k, offsets, kGroupedPassTokens, &a, &split, &large, &small);
         const double steps = ceil_div(k, 64);
-        const int split = a.n_groups > 1 ? wide_best_split((double)large, (double)small, steps, kRoomToGrow, &together) : 0;
-        if (split && together < apart) {
+        if (split) {
             a.q = static_cast<const uint8_t *>(q);
             a.x = x;
             a.code = static_cast<const float *>(code);

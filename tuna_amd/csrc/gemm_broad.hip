@@ -17,9 +17,11 @@
 //
 // Against the launches that were chosen before, in us: 28672 x 4096 at 80 tokens 41 -> 28, at 128 42 -> 37; 8192 x 8192 at 96
 // 30 -> 25, at 160 47 -> 31, at 256 51 -> 42; 4096 x 14336 at 96 33 -> 25, at 192 46 -> 34; 5120 x 13824 at 160 47 -> 33; 11008 x
-// 2048 at 192 27 -> 17; 57344 x 8192 at 64 75 -> 70.  The floor of the first, its weights at the rate of a large copy: 12.
+// 2048 at 192 27 -> 17; 57344 x 8192 at 64 75 -> 70.  Groups: one launch over all row tiles
+// and token tiles of all groups, eight experts of 14336 x 4096 on 512 tokens 147 -> 98.  The floor of the first, its weights at the rate of a large copy: 12.
 #include "lds_dma.hpp"
 #include "row_pieces.hpp"
+#include <type_traits>
 
 namespace tuna {
 
@@ -52,11 +54,13 @@ constexpr size_t lds_bytes(int rt, int nt, int blocks)
 }
 
 // (separate scalars, the ones the first loads need in front: the first sixteen dwords arrive in scalar registers with the wave)
-template <int RT, int NT, bool BLK>
+// (GROUPS: BroadGroups, or nothing for one matrix)
+template <int RT, int NT, bool BLK, class GROUPS>
 __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *a_q, const void *a_x, const float *a_code, const float *a_absmax,
                                                                      int a_k, int a_n, int a_m, int a_part_steps, void *a_out, int a_epilogue,
-                                                                     const void *a_residual, float *a_ws, unsigned *a_counters, int a_blk_shift, int a_ticket)
+                                                                     const void *a_residual, float *a_ws, unsigned *a_counters, int a_blk_shift, int a_ticket, const GROUPS groups)
 {
+    constexpr bool GRP = !std::is_empty<GROUPS>::value;
     using P = Pieces<RT>;
     constexpr int NS = 2;      // units whose weights are on their way
     constexpr int LD = 1, LR = LD == 1 ? 2 : 4;  // table reads are that many turns ahead of their scaling's successor
@@ -103,17 +107,30 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
     const int swz = (g ^ (i16 & 7)) << 4;
     const unsigned char *const x_frag0 = smem + kLutBytes + kg * (NT * 2048) + i16 * 128 + swz, *const x_frag1 = x_frag0 - swz + (64 ^ swz);
 
-    const int tile = (int)blockIdx.x, part = (int)blockIdx.y, split = (int)gridDim.y, row_base = tile * ROWS;
-    const int tok_base = (int)blockIdx.z * (16 * NT), tokens = min(16 * NT, a_n - tok_base);
+    const int part = (int)blockIdx.y, split = (int)gridDim.y;
+    int tile = (int)blockIdx.x, tok_base = (int)blockIdx.z * (16 * NT), tokens = min(16 * NT, a_n - tok_base), group = 0;
+    if constexpr (GRP) {
+        // the group whose items are the last to begin at or in front of this one; a row tile's token tiles are neighbours
+        const bool begun = lane < groups.n && groups.item[lane] <= tile;
+        const int at = __builtin_popcountll(__ballot(begun)) - 1, count = groups.tok_count[at], tok_tiles = (count + 16 * NT - 1) / (16 * NT);
+        const int local = tile - groups.item[at];
+        tile = local / tok_tiles;
+        const int first = (local - tile * tok_tiles) * (16 * NT);
+        tok_base = groups.tok_begin[at] + first;
+        tokens = min(16 * NT, count - first);
+        group = groups.id[at];
+    }
+    const int row_base = tile * ROWS;  // (of the group's rows)
+    const size_t first_row = (size_t)group * (size_t)a_m + (size_t)row_base;
     const int s0 = part * a_part_steps, s1 = min(s0 + a_part_steps, steps_total);
     const size_t rows_left = (size_t)(a_m - row_base);
     const __amdgpu_buffer_rsrc_t q_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t *>(a_q) + (size_t)row_base * (size_t)(a_k >> 1), 0,
+        const_cast<uint8_t *>(a_q) + first_row * (size_t)(a_k >> 1), 0,
         (int)(uint32_t)min(rows_left * (size_t)(a_k >> 1), (size_t)0xffffffffu), 0x00020000);
     const u32x4 x_rsrc = buffer_at(reinterpret_cast<const f16 *>(a_x) + (size_t)tok_base * (size_t)a_k, (size_t)tokens * (size_t)a_k * 2);
     const int nblk = BLK ? a_k >> (6 + a_blk_shift) : 1;
     const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float *>(a_absmax) + (size_t)row_base * (size_t)nblk, 0, (int)(uint32_t)min(rows_left * (size_t)nblk * 4, (size_t)0xffffffffu), 0x00020000);
+        const_cast<float *>(a_absmax) + first_row * (size_t)nblk, 0, (int)(uint32_t)min(rows_left * (size_t)nblk * 4, (size_t)0xffffffffu), 0x00020000);
 
     f32x4 acc[RT][NT];
 #pragma unroll
@@ -124,7 +141,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
     // units of four steps, one per k group; the part's, from one that depends on the tile on and around (workgroups that
     // walk k in step ask the same memory channels)
     const int units = (s1 - s0 + kStepGroups - 1) / kStepGroups;
-    const int u_first = (int)(((((unsigned)tile * 2654435761u) >> 16) * (unsigned)units) >> 16);
+    const int u_first = (int)(((((unsigned)blockIdx.x * 2654435761u) >> 16) * (unsigned)units) >> 16);
     int u_w = u_first, u_x = u_first;
     auto next = [&](int u) { return u + 1 < units ? u + 1 : 0; };
 
@@ -416,11 +433,12 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
     }
 }
 
-template <int RT, int NT, bool BLK>
-hipError_t launch(const BroadPlan &plan, hipStream_t stream)
+struct OneMatrix {};
+template <int RT, int NT, bool BLK, class GROUPS>
+hipError_t launch(const BroadPlan &plan, const GROUPS &groups, hipStream_t stream)
 {
     static OptInFlag done[16];
-    const auto fn = gemm_broad_kernel<RT, NT, BLK>;
+    const auto fn = gemm_broad_kernel<RT, NT, BLK, GROUPS>;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
@@ -428,22 +446,27 @@ hipError_t launch(const BroadPlan &plan, hipStream_t stream)
     if ((e = ensure_lds_opt_in(done[dev], reinterpret_cast<const void *>(fn))) != hipSuccess) return e;
     const BroadArgs &a = plan.args;
     const size_t lds = lds_bytes(RT, NT, plan.part_blocks);
-    hipLaunchKernelGGL(fn, dim3((unsigned)plan.tiles, (unsigned)plan.split, (unsigned)plan.tok_tiles), dim3(kThreads), lds, stream, a.q, a.x, a.code, a.absmax, a.k, a.n, a.m,
-                       plan.part_steps, a.out, a.epilogue, a.residual, a.ws, a.counters, a.blk_shift, (int)lds - 16);
+    hipLaunchKernelGGL(fn, dim3((unsigned)plan.tiles, (unsigned)plan.split, (unsigned)plan.tok_tiles), dim3(kThreads), lds, stream, a.q, a.x, a.code,
+                       a.absmax, a.k, a.n, a.m, plan.part_steps, a.out, a.epilogue, a.residual, a.ws, a.counters, a.blk_shift, (int)lds - 16, groups);
     return hipGetLastError();
 }
-template <int RT>
-hipError_t launch(const BroadPlan &plan, hipStream_t stream)
+template <int RT, int NT>
+hipError_t launch(const BroadPlan &plan, const BroadGroups *groups, hipStream_t stream)
 {
-    const bool blk = plan.part_blocks != 0;
+    if constexpr (RT * NT <= 32) {
+        if (groups) return launch<RT, NT, false>(plan, *groups, stream);
+        return plan.part_blocks ? launch<RT, NT, true>(plan, OneMatrix(), stream) : launch<RT, NT, false>(plan, OneMatrix(), stream);
+    } else {
+        return hipErrorInvalidConfiguration;
+    }
+}
+template <int RT>
+hipError_t launch(const BroadPlan &plan, const BroadGroups *groups, hipStream_t stream)
+{
     switch (plan.nt) {
-    case 4: return blk ? launch<RT, 4, true>(plan, stream) : launch<RT, 4, false>(plan, stream);
-    case 5:
-        if constexpr (RT <= 6) return blk ? launch<RT, 5, true>(plan, stream) : launch<RT, 5, false>(plan, stream);
-        else return hipErrorInvalidConfiguration;
-    default:
-        if constexpr (RT <= 5) return blk ? launch<RT, 6, true>(plan, stream) : launch<RT, 6, false>(plan, stream);
-        else return hipErrorInvalidConfiguration;
+    case 4: return launch<RT, 4>(plan, groups, stream);
+    case 5: return launch<RT, 5>(plan, groups, stream);
+    default: return launch<RT, 6>(plan, groups, stream);
     }
 }
 }  // namespace
@@ -474,15 +497,29 @@ bool plan_gemm_broad(int rows, int nt, int split, int blk_shift, BroadPlan *plan
 
 size_t broad_lds_bytes(const BroadPlan &plan) { return lds_bytes(plan.rt, plan.nt, plan.part_blocks); }
 
-hipError_t launch_gemm_broad(const BroadPlan &plan, hipStream_t stream)
+bool plan_gemm_broad_groups(int rows, int nt, BroadPlan *plan, BroadGroups *groups)
+{
+    // (a.n: the largest group's tokens)
+    if (!plan_gemm_broad(rows, nt, 1, -1, plan)) return false;
+    long long items = 0;
+    for (int e = 0; e < groups->n; ++e) {
+        groups->item[e] = (int)items;
+        items += (long long)plan->tiles * ceil_div_i(groups->tok_count[e], 16 * nt);
+        if (items > 0x7fffffff) return false;
+    }
+    plan->tiles = (int)items, plan->tok_tiles = 1;
+    return items > 0;
+}
+
+hipError_t launch_gemm_broad(const BroadPlan &plan, const BroadGroups *groups, hipStream_t stream)
 {
     switch (plan.rt) {
-    case 2: return launch<2>(plan, stream);
-    case 3: return launch<3>(plan, stream);
-    case 4: return launch<4>(plan, stream);
-    case 5: return launch<5>(plan, stream);
-    case 6: return launch<6>(plan, stream);
-    default: return launch<8>(plan, stream);
+    case 2: return launch<2>(plan, groups, stream);
+    case 3: return launch<3>(plan, groups, stream);
+    case 4: return launch<4>(plan, groups, stream);
+    case 5: return launch<5>(plan, groups, stream);
+    case 6: return launch<6>(plan, groups, stream);
+    default: return launch<8>(plan, groups, stream);
     }
 }
 

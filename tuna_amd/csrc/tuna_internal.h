@@ -240,6 +240,12 @@ struct TallPlan {
     size_t ws_bytes, n_counters;
 };
 
+// Groups with tokens of a grouped launch, in order: their first workgroups, tokens and matrices.
+struct BroadGroups {
+    int n, item[kMaxGroups], tok_begin[kMaxGroups], tok_count[kMaxGroups];
+    int id[kMaxGroups];  // (an int: read through the scalar cache)
+};
+
 struct BroadPlan {
     BroadArgs args;
     int rt, nt;                   // 16-row tiles of a row group and 16-token tiles of a workgroup
@@ -367,7 +373,10 @@ bool plan_gemm_tall(int row_tiles16, int nt, int split, int blk_shift, TallPlan 
 hipError_t launch_gemm_tall(const TallPlan &plan, hipStream_t stream);
 size_t tall_lds_bytes(const TallPlan &plan);
 bool plan_gemm_broad(int rows, int nt, int split, int blk_shift, BroadPlan *plan);
-hipError_t launch_gemm_broad(const BroadPlan &plan, hipStream_t stream);
+// groups: null for one matrix, else what plan_gemm_broad_groups has filled in for the same rows, nt (k unsplit; n, tok_begin,
+// tok_count > 0 and id are the caller's).
+hipError_t launch_gemm_broad(const BroadPlan &plan, const BroadGroups *groups, hipStream_t stream);
+bool plan_gemm_broad_groups(int rows, int nt, BroadPlan *plan, BroadGroups *groups);
 size_t broad_lds_bytes(const BroadPlan &plan);
 hipError_t launch_gemm_wide32(const TiledArgs &args, hipStream_t stream);
 bool tiled_variant_exists(int tile_rows, int tile_tokens, bool mfma32);
