@@ -70,7 +70,8 @@ def test_nothing_beyond_a_tokens_k_values_or_the_tokens_enters_a_sum(k, rows, to
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k,block,rows,tokens,split", [(64, 70, 256, 64, 64, 80, 1), (112, 64, 768, 128, 64, 64, 2), (208, 128, 2304, 64, 96, 64, 3),
                                                            (400, 90, 1792, 256, 96, 80, 2), (128, 65, 4096, 64, 128, 80, 2), (1008, 100, 2816, 256, 128, 64, 3), (336, 96, 1024, 128, 160, 64, 2), (176, 70, 2560, 64, 192, 80, 3),
-                                                           (528, 65, 3840, 64, 256, 64, 4)])
+                                                           (528, 65, 3840, 64, 256, 64, 4), (272, 90, 14336, 64, 128, 80, 1), (192, 64, 2048, 1024, 96, 64, 2),
+                                                           (512, 80, 1536, 512, 192, 80, 1)])
 def test_scale_blocks(m, n, k, block, rows, tokens, split):
     import torch
 
@@ -128,7 +129,7 @@ def test_a_call_without_a_config_takes_it_where_it_is_predicted_to_be_faster():
         assert "gemm_broad_kernel" not in ops.describe_launch(*shape), shape
 
 
-@pytest.mark.parametrize("kind,off", [("broad", 4.9), ("broad blocks", 5.1)])
+@pytest.mark.parametrize("kind,off", [("broad", 4.9), ("broad blocks", 4.4)])
 def test_the_stated_errors_are_those_of_the_kept_launches(kind, off):
     """(per cent, as stated beside broad_time in csrc/api.cpp)"""
     from test_launch_models import DATA

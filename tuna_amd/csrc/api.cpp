@@ -1242,16 +1242,18 @@ static bool best_tall(int m, int n, int k, int nblk, const Room &room, tuna_gemm
 // Microseconds of a launch of the broad-tile kernel (gemm_broad.hip): tiles of `rows` rows and 16 `nt` tokens in `split` parts of k,
 // by a model read off 300 random shapes of 0.5 ... 400 MB of weights at 49 ... 640 tokens, each with up to 14 variants (4.9 per cent
 // off on average on the 440 launches kept; the pick takes 1.01 x the time of a shape's best): units of four k-steps whose time
-// is a row tile's decode and a token tile's way through LDS, more where all compute units have a workgroup; with `nblk` scales
-// a row 200 shapes with blocks of 64 and 128 (5.1 per cent; 1.01 x).
+// is a row tile's decode and a token tile's way through LDS, more where all compute units have a workgroup;
+// with `nblk` scales a row 220 shapes of 65 ... 2048 tokens with blocks of 64 and 128 (4.4 per cent; 1.01 x).
 static double broad_items_time(long long items, int k, int rt, int nt, int part, int parts, int nblk)
 {
+    // launch, round, unit, rows, KB of a workgroup's scales: one scale per row, a part's in LDS, a unit's
+    static const double kCoef[3][5] = {{3.015, 1.578, 0.1557, 0.13, 0.0}, {2.484, 3.578, 0.0761, 0.1482, 0.0332}, {1.212, 2.125, 0.3803, 0.1493, 0.0}};
+    const double *c = kCoef[!nblk ? 0 : nblk >= 4 && broad_scale_blocks(32 * rt, nt, part, parts, log2i(k / nblk) - 6) ? 1 : 2];
     const long long full = items / kMaxCus, rest = items % kMaxCus;
-    const double unit = 0.1557 + (nblk ? 0.1365 : 0.13) * rt + (k % 64 ? 0.1034 : 0.0865) * nt + 0.00105 * rt * nt;
+    const double unit = c[2] + c[3] * rt + (k % 64 ? 0.1034 : 0.0865) * nt + 0.00105 * rt * nt;
     const double work = part * ((double)full * (unit + 0.0496 * nt) + (rest ? unit + 0.0496 * nt * rest / kMaxCus : 0.0));
-    const double scales = nblk ? 0.0298 * 0.125 * rt * ceil(part * 256.0 * nblk / k) : 0.0;
-    return (nblk ? 4.096 : 3.015) + (double)(full + (rest ? 1 : 0)) * (1.578 + 0.0809 * rt * nt + scales) + work +
-           (parts > 1 ? 1.831 + 0.0343 * parts * nt * rt : 0.0);
+    const double scales = nblk ? c[4] * 0.125 * rt * ceil(part * 256.0 * nblk / k) : 0.0;
+    return c[0] + (double)(full + (rest ? 1 : 0)) * (c[1] + 0.0809 * rt * nt + scales) + work + (parts > 1 ? 1.831 + 0.0343 * parts * nt * rt : 0.0);
 }
 static double broad_time(int m, int n, int k, int rows, int nt, int split, int nblk = 0)
 {
@@ -1472,12 +1474,16 @@ static int select_config_for(int m, int n, int k, int decode, tuna_gemm_config *
     return TUNA_OK;
 }
 
-// From 49 to 512 tokens, last: broad tiles where their model is ahead of the pick's.  On 249 random shapes of 65 ... 640 tokens
+// From 49 tokens on, last: broad tiles where their model is ahead of the pick's.  On 249 random shapes of 65 ... 640 tokens
 // it takes 152, 1.28 x faster (many-token tiles 1.26 x, streaming ones 1.2 x, 256 x 256 tiles split over k 1.2 x; worst 0.84:
-// 8192 x 28672 at 303 tokens in three rounds, hence less trust in those).  What the table holds of narrow rows stays.
+// 8192 x 28672 at 303 tokens in three rounds, hence less trust in those).  Above 512 tokens on 141 shapes of up to 16384 rows, the
+// models being 6 per cent off, it takes 33, 1.22 x faster (4096 x 14336 at 777 tokens 133 -> 100, 5120 x 5120 at 594 55 -> 39, 3712 x
+// 3072 at 608 34 -> 22; nothing slower); with more activations than the L2s hold (32 MB) launches take up to 1.4 x what the model says.
+// What the table holds of narrow rows stays.
 static bool broad_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, double flow_us, const Room &room, tuna_gemm_config *broad)
 {
-    if (n < 49 || n > 512) return false;
+    // (with a given workspace many tokens keep the selected tile, with as many parts of k as the sums fit for)
+    if (n < 49 || (n > 512 && room.bytes != kRoomToGrow.bytes)) return false;
     double price;
     if (is_flow(c)) price = flow_us;
     else if (is_tall(c)) price = tall_time(m, n, k, c.rows_per_wave / 16, c.split_k);
@@ -1486,7 +1492,7 @@ static bool broad_instead(int m, int n, int k, const tuna_gemm_config &c, bool f
     double us = 0.0;
     if (price == 0.0 || !best_broad(m, n, k, 0, room, broad, &us)) return false;
     const double rounds = ceil((double)ceil_div(m, broad->rows_per_wave) * ceil_div(n, 16 * broad->token_tiles) / kMaxCus);
-    return us < (rounds > 2 ? 0.88 : 0.95) * price;
+    return us < (n > 512 && 2e-6 * n * k > 32 ? 0.78 : n > 512 || rounds > 2 ? 0.88 : 0.95) * price;
 }
 
 // The config a launch without an explicit one runs: the selected one, or a newer kernel in its place - one whose partial
@@ -2877,12 +2883,12 @@ static bool blockwise_tall_instead(const BlockwiseCall &b, const tuna_gemm_confi
     return !best_narrow_any(b.m, b.n, b.k, nblk, us, &any);
 }
 
-// From 65 to 384 tokens: broad tiles (gemm_broad.hip) where their model is ahead of the derived config's.  Of 180
-// random shapes of 49 ... 640 tokens with blocks of 64 and 128 it takes 64, 1.23 x faster (worst 0.87: 24384 x 3584 at
-// 217 tokens, which puts 508 tiles on 256 compute units; above 384 tokens it loses as often as it gains).
+// From 65 tokens on: broad tiles (gemm_broad.hip) where their model is ahead of the derived config's.  Of 170 random shapes
+// of 65 ... 2500 tokens with blocks of 64 and 128 it takes 68, 1.28 x faster (3712 x 16384 at 297 tokens 94 -> 60, 22016 x 4096 at 72
+// 44 -> 28; worst 0.93: 10496 x 12032 at 243); less trust in the model above 384 tokens, in several rounds and beyond the L2s.
 static bool blockwise_broad_instead(const BlockwiseCall &b, const tuna_gemm_config &c, const Room &room, tuna_gemm_config *broad)
 {
-    if (b.n <= 64 || b.n > 384) return false;
+    if (b.n <= 64) return false;
     const int nblk = b.k / b.block_size, tokens = 16 * c.token_tiles;
     double price = 0.0;
     if (blockwise_family(c) == kBlkNarrow) {
@@ -2899,7 +2905,7 @@ static bool blockwise_broad_instead(const BlockwiseCall &b, const tuna_gemm_conf
     double us = 0.0;
     if (price == 0.0 || !best_broad(b.m, b.n, b.k, nblk, room, broad, &us)) return false;
     const double rounds = ceil((double)ceil_div(b.m, broad->rows_per_wave) * ceil_div(b.n, 16 * broad->token_tiles) / kMaxCus);
-    return us < (rounds > 2 ? 0.88 : 0.95) * price;
+    return us < (2e-6 * b.n * b.k > 32 ? 0.78 : b.n > 384 || rounds > 2 ? 0.86 : 0.95) * price;
 }
 
 // Tuned entry for (m, n, k, block_size) if the table has one that can run the call, else the derived config.

@@ -1,4 +1,4 @@
-// Fused FP16 x 4-bit-codebook GEMM for 49 ... 512 tokens, where an MFMA tile of 16 tokens no longer waits for its weights but a
+// Fused FP16 x 4-bit-codebook GEMM from 49 tokens on, where an MFMA tile of 16 tokens no longer waits for its weights but a
 // token tile of 128 or 256 leaves compute units idle or takes k in many parts: a workgroup is 32 RT rows (RT 2 .. 8) x 64, 80 or
 // 96 tokens in one of `split` parts of k.
 //
@@ -18,7 +18,8 @@
 // Against the launches that were chosen before, in us: 28672 x 4096 at 80 tokens 41 -> 28, at 128 42 -> 37; 8192 x 8192 at 96
 // 30 -> 25, at 160 47 -> 31, at 256 51 -> 42; 4096 x 14336 at 96 33 -> 25, at 192 46 -> 34; 5120 x 13824 at 160 47 -> 33; 11008 x
 // 2048 at 192 27 -> 17; 57344 x 8192 at 64 75 -> 70.  Groups: one launch over all row tiles
-// and token tiles of all groups, eight experts of 14336 x 4096 on 512 tokens 147 -> 98.  The floor of the first, its weights at the rate of a large copy: 12.
+// and token tiles of all groups, eight experts of 14336 x 4096 on 512 tokens 147 -> 98.  Scales in blocks: 4096 x
+// 14336 at 777 tokens 125 -> 116, 5120 x 5120 at 594 56 -> 43.  The floor of the first, its weights at the rate of a large copy: 12.
 #include "lds_dma.hpp"
 #include "row_pieces.hpp"
 #include <type_traits>
@@ -43,19 +44,21 @@ constexpr size_t end_bytes(int rt, int nt)
     const size_t red = (size_t)kWaves * rt * red_tiles(rt, nt) * 1024, out = (size_t)16 * nt * (kRowGroups * 16 * rt + 4) * 4;
     return red > out ? red : out;
 }
-// Scales in blocks of 64 << blk_shift weights: those of a tile's part of k lie behind the activations, two bytes each and a
-// lane's of a block together: [block][row group][16 lanes][scale_dwords].
+// Scales in blocks of 64 << blk_shift weights lie behind the activations, two bytes each and a lane's of a block together: [block][row
+// group][16 lanes][scale_dwords].  Where they fit all those of a tile's part of k (SCALES_PART), else a unit's, four, two or one
+// a row, in the other of two slots (SCALES_UNIT: 0.2 us more a unit).
+enum { SCALES_ROW, SCALES_PART, SCALES_UNIT };
 constexpr int scale_dwords(int rt) { return rt <= 2 ? 1 : rt <= 4 ? 2 : 4; }
+constexpr int scale_block(int rt) { return kRowGroups * 64 * scale_dwords(rt); }
+constexpr size_t loop_bytes(int rt, int nt, int blocks) { return kLutBytes + x_bytes(nt) + (size_t)blocks * scale_block(rt); }
 constexpr size_t lds_bytes(int rt, int nt, int blocks)
 {
-    const size_t loop = kLutBytes + x_bytes(nt) + (size_t)blocks * kRowGroups * 64 * scale_dwords(rt);
-    const size_t end = end_bytes(rt, nt) + 16;
+    const size_t loop = loop_bytes(rt, nt, blocks), end = end_bytes(rt, nt) + 16;
     return loop > end ? loop : end;
 }
 
-// (separate scalars, the ones the first loads need in front: the first sixteen dwords arrive in scalar registers with the wave)
 // (GROUPS: BroadGroups, or nothing for one matrix)
-template <int RT, int NT, bool BLK, class GROUPS>
+template <int RT, int NT, int BLK, class GROUPS>
 __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *a_q, const void *a_x, const float *a_code, const float *a_absmax,
                                                                      int a_k, int a_n, int a_m, int a_part_steps, void *a_out, int a_epilogue,
                                                                      const void *a_residual, float *a_ws, unsigned *a_counters, int a_blk_shift, int a_ticket, const GROUPS groups)
@@ -222,32 +225,77 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
             __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[tau & 1], fb[tau / RT][t], acc[tau % RT][t], 0, 0, 0);  \
         BROAD_SCALE(u, tau + 1)                                                                               \
         _Pragma("unroll") for (int t = 0; t < NT; ++t) if (tau == t * (RT - 1) / NT) BROAD_READ_B(1, ((u) & 1) * STAGE, t) \
-        if (tau == RT) {                                                                                   \
+        if (BLK == SCALES_UNIT && tau == RT - 1) BROAD_STORE_SCALES(((u) + 1) & 1)                                           \
+        if (tau == RT) {                                                                                      \
             __builtin_amdgcn_sched_barrier(0);                                                                \
             __builtin_amdgcn_s_waitcnt(0x0070 | (2 * P::count)); /* (for the compiler to know, and lgkmcnt(0)) */ \
             wait_loads<2 * P::count>();                                                                       \
             __builtin_amdgcn_s_barrier();                                                                     \
             asm volatile("" ::: "memory");                                                                    \
             BROAD_LOAD_X(((u) & 1) * STAGE)                                                                   \
-            if (BLK) BROAD_READ_SCALES(((u) + 1) % NS)                                                        \
+            if (BLK) {                                                                                        \
+                if (BLK == SCALES_UNIT) BROAD_LOAD_SCALES()                                                                           \
+                BROAD_READ_SCALES(((u) + 1) & 1)                                                              \
+            }                                                                                                 \
         }                                                                                                     \
         _Pragma("unroll") for (int t = 0; t < NT; ++t) if (tau == RT + t * (RT - 1) / NT) BROAD_READ_B(0, (((u) + 1) & 1) * STAGE, t) \
         BROAD_LUT(u, tau + 1 + LD)                                                                                 \
         __builtin_amdgcn_sched_barrier(0);                                                                    \
     }
-    // (the scales of the unit after the one at hand)
-#define BROAD_READ_SCALES(set)                                                                                \
-    {                                                                                                         \
-        u_sc = next(u_sc);                                                                                    \
-        const lds_u32 *const from_ = sc_lane + ((min(s0 + u_sc * kStepGroups + kg, s1 - 1) >> a_blk_shift) - b0) * (kRowGroups * 16 * SD); \
-        _Pragma("unroll") for (int j = 0; j < (RT + 1) / 2; ++j) sc[BLK ? (set) : 0][j] = __builtin_bit_cast(f16x2, from_[j]); \
-    }
+    const int b0 = BLK == SCALES_PART ? s0 >> a_blk_shift : 0;
+    // SCALES_UNIT: a row a lane, 64 rows a wave; requested behind the barrier for the unit after the next, stored in front of
+    // the next one, read behind that.
     constexpr int SD = scale_dwords(RT);
-    const int b0 = BLK ? s0 >> a_blk_shift : 0;
-    int u_sc = u_first;
     unsigned char *const scales = smem + kLutBytes + 2 * STAGE;
-    const lds_u32 *const sc_lane = reinterpret_cast<const lds_u32 *>((uintptr_t)(uint32_t)(kLutBytes + 2 * STAGE + (rg * 16 + i16) * (SD * 4)));
-    if constexpr (BLK) {
+    const lds_u32 *const sc_lane = reinterpret_cast<const lds_u32 *>(
+        (uintptr_t)(uint32_t)(kLutBytes + 2 * STAGE + (((BLK == SCALES_UNIT ? kg >> a_blk_shift : 0) * kRowGroups + rg) * 16 + i16) * (SD * 4)));
+    const int sc_row = wave * 64 + lane;
+    int sc_dst = 0, u_sc = u_first;
+    if constexpr (BLK == SCALES_UNIT) {
+        const int group_ = sc_row / (16 * RT), r16 = (sc_row >> 4) - group_ * RT;
+        const int width = r16 < 4 * P::fours ? 4 : r16 < 4 * P::fours + 2 * P::twos ? 2 : 1;
+        const int first = width == 4 ? r16 & ~3 : width == 2 ? 4 * P::fours : RT - 1;
+        const int in = sc_row - 16 * (group_ * RT + first);
+        sc_dst = (group_ * 16 + in / width) * (SD * 4) + (first + in % width) * 2;
+    }
+    u32x4 sv = {0u, 0u, 0u, 0u};
+#define BROAD_LOAD_SCALES()                                                                                   \
+    {                                                                                                         \
+        if (wave * 64 < ROWS) {                                                                               \
+            const int at_ = (sc_row * nblk + ((s0 + u_sc * kStepGroups) >> a_blk_shift)) * 4;                 \
+            if (a_blk_shift == 0) {                                                                           \
+                sv = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, at_, 0, 0);                                \
+            } else if (a_blk_shift == 1) {                                                                    \
+                const u32x2 v_ = __builtin_amdgcn_raw_buffer_load_b64(s_rsrc, at_, 0, 0);                     \
+                sv[0] = v_[0], sv[1] = v_[1];                                                                 \
+            } else {                                                                                          \
+                sv[0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(s_rsrc, at_, 0, 0);                    \
+            }                                                                                                 \
+        }                                                                                                     \
+        u_sc = next(u_sc);                                                                                    \
+    }
+#define BROAD_STORE_SCALES(slot)                                                                              \
+    if (wave * 64 < ROWS && sc_row < ROWS) {                                                                  \
+        _Pragma("unroll") for (int e = 0; e < kStepGroups; ++e) {                                             \
+            const uint32_t bits_ = sv[e]; /* (a copy: a bit cast of a vector's element would take the first) */ \
+            if (e << a_blk_shift < kStepGroups)                                                               \
+                *reinterpret_cast<f16 *>(scales + (slot) * (kStepGroups * scale_block(RT)) + e * (kRowGroups * 64 * SD) + sc_dst) = (f16)__builtin_bit_cast(float, bits_); \
+        }                                                                                                     \
+    }
+#define BROAD_READ_SCALES(slot)                                                                               \
+    {                                                                                                         \
+        const lds_u32 *from_ = sc_lane + (slot) * (kStepGroups * scale_block(RT) / 4);                        \
+        if (BLK == SCALES_PART) {                                                                             \
+            from_ = sc_lane + ((min(s0 + u_sc * kStepGroups + kg, s1 - 1) >> a_blk_shift) - b0) * (scale_block(RT) / 4); \
+            u_sc = next(u_sc);                                                                                \
+        }                                                                                                     \
+        _Pragma("unroll") for (int j = 0; j < (RT + 1) / 2; ++j) sc[BLK ? (slot) : 0][j] = __builtin_bit_cast(f16x2, from_[j]); \
+    }
+    if constexpr (BLK == SCALES_UNIT) {
+        BROAD_LOAD_SCALES()
+        BROAD_STORE_SCALES(0)
+    }
+    if constexpr (BLK == SCALES_PART) {
         // Four blocks of a row a lane, 64 rows a wave: the LDS banks of a store are those of 16 lanes and two or four pairs of
         // row tiles.  (The last four of a row where four from here on would go beyond it: what is in front of the part or
         // behind it isn't stored.)
@@ -263,16 +311,16 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
 #pragma unroll
             for (int i = 0; i < PIECES; ++i) {
                 const int j = min(j0 + kWaves * i, RG * quads - 1), c = min(b0 + 4 * (j / RG), nblk - 4) - b0;
-                const int row = 64 * (j % RG) + lane, group = row / (16 * RT), r16 = (row >> 4) - group * RT;
+                const int row = 64 * (j % RG) + lane, rows_of = row / (16 * RT), r16 = (row >> 4) - rows_of * RT;
                 const int width = r16 < 4 * P::fours ? 4 : r16 < 4 * P::fours + 2 * P::twos ? 2 : 1;
                 const int first = width == 4 ? r16 & ~3 : width == 2 ? 4 * P::fours : RT - 1;
-                const int in = row - 16 * (group * RT + first), lane16 = in / width, r = first + in % width;
+                const int in = row - 16 * (rows_of * RT + first), lane16 = in / width, r = first + in % width;
                 if (row < ROWS)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const uint32_t bits = v[i][e];  // (a copy: a bit cast of a vector's element would take the first)
                         if (c + e >= 0 && c + e < nb)
-                            *reinterpret_cast<f16 *>(scales + (((c + e) * kRowGroups + group) * 16 + lane16) * (SD * 4) + r * 2) = (f16)__builtin_bit_cast(float, bits);
+                            *reinterpret_cast<f16 *>(scales + (((c + e) * kRowGroups + rows_of) * 16 + lane16) * (SD * 4) + r * 2) = (f16)__builtin_bit_cast(float, bits);
                     }
             }
         }
@@ -283,11 +331,10 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
     __builtin_amdgcn_s_waitcnt(0x0F70 | P::count);
     __syncthreads();
     BROAD_LOAD_X(STAGE)
+    if constexpr (BLK == SCALES_UNIT) BROAD_LOAD_SCALES()
     BROAD_LOAD_W(1, 1)  // (behind the activations, as in the loop: its count of loads is exact)
     if constexpr (BLK) {
-        const lds_u32 *const from = sc_lane + ((min(s0 + u_sc * kStepGroups + kg, s1 - 1) >> a_blk_shift) - b0) * (kRowGroups * 16 * SD);
-#pragma unroll
-        for (int j = 0; j < (RT + 1) / 2; ++j) sc[0][j] = __builtin_bit_cast(f16x2, from[j]);
+        BROAD_READ_SCALES(0)
     } else {
 #pragma unroll
         for (int r = 0; r < RT; ++r) sc[0][r / 2][r & 1] = (f16)sc32[r];
@@ -313,6 +360,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
     wait_loads<0>();  // (no activations on their way to where the sums go)
 #undef BROAD_STEP
 #undef BROAD_READ_SCALES
+#undef BROAD_STORE_SCALES
+#undef BROAD_LOAD_SCALES
 #undef BROAD_READ_B
 #undef BROAD_SCALE
 #undef BROAD_LUT
@@ -434,7 +483,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
 }
 
 struct OneMatrix {};
-template <int RT, int NT, bool BLK, class GROUPS>
+template <int RT, int NT, int BLK, class GROUPS>
 hipError_t launch(const BroadPlan &plan, const GROUPS &groups, hipStream_t stream)
 {
     static OptInFlag done[16];
@@ -445,7 +494,7 @@ hipError_t launch(const BroadPlan &plan, const GROUPS &groups, hipStream_t strea
     if (dev < 0 || dev >= 16) return hipErrorInvalidDevice;
     if ((e = ensure_lds_opt_in(done[dev], reinterpret_cast<const void *>(fn))) != hipSuccess) return e;
     const BroadArgs &a = plan.args;
-    const size_t lds = lds_bytes(RT, NT, plan.part_blocks);
+    const size_t lds = lds_bytes(RT, NT, plan.blocks);
     hipLaunchKernelGGL(fn, dim3((unsigned)plan.tiles, (unsigned)plan.split, (unsigned)plan.tok_tiles), dim3(kThreads), lds, stream, a.q, a.x, a.code,
                        a.absmax, a.k, a.n, a.m, plan.part_steps, a.out, a.epilogue, a.residual, a.ws, a.counters, a.blk_shift, (int)lds - 16, groups);
     return hipGetLastError();
@@ -454,8 +503,11 @@ template <int RT, int NT>
 hipError_t launch(const BroadPlan &plan, const BroadGroups *groups, hipStream_t stream)
 {
     if constexpr (RT * NT <= 32) {
-        if (groups) return launch<RT, NT, false>(plan, *groups, stream);
-        return plan.part_blocks ? launch<RT, NT, true>(plan, OneMatrix(), stream) : launch<RT, NT, false>(plan, OneMatrix(), stream);
+        if (groups) return launch<RT, NT, SCALES_ROW>(plan, *groups, stream);
+        if (!plan.blocks) return launch<RT, NT, SCALES_ROW>(plan, OneMatrix(), stream);
+        if (!plan.unit_scales) return launch<RT, NT, SCALES_PART>(plan, OneMatrix(), stream);
+        if constexpr (NT <= 5) return launch<RT, NT, SCALES_UNIT>(plan, OneMatrix(), stream);
+        else return hipErrorInvalidConfiguration;
     } else {
         return hipErrorInvalidConfiguration;
     }
@@ -485,17 +537,25 @@ bool plan_gemm_broad(int rows, int nt, int split, int blk_shift, BroadPlan *plan
     const long long items = (long long)plan->tiles * tok_tiles;
     plan->ws_bytes = plan->split > 1 ? (size_t)items * plan->split * kRowGroups * rt * nt * 1024 : 0;
     plan->n_counters = plan->split > 1 ? (size_t)items : 0;
-    plan->part_blocks = 0;
+    plan->blocks = 0, plan->unit_scales = false, a.blk_shift = 0;
     if (blk_shift >= 0) {
-        const int size = 1 << blk_shift, nblk = a.k >> (6 + blk_shift);
-        if (a.k % (64 << blk_shift) || nblk < 4) return false;
-        plan->part_blocks = ceil_div_i(plan->part_steps, size) + (plan->split > 1 && plan->part_steps % size ? 1 : 0);
+        if (a.k % 256 || a.k % (64 << blk_shift)) return false;  // (whole units, whole blocks)
+        plan->blocks = broad_scale_blocks(rows, nt, plan->part_steps / kStepGroups, plan->split, blk_shift);
+        plan->unit_scales = !plan->blocks || a.k >> (6 + blk_shift) < 4;  // (a part's are loaded four blocks at a time)
+        if (plan->unit_scales) plan->blocks = 2 * kStepGroups;
         a.blk_shift = blk_shift;
     }
-    return lds_bytes(rt, nt, plan->part_blocks) <= (size_t)kLdsLimit;
+    return loop_bytes(rt, nt, plan->blocks) <= (size_t)kLdsLimit;
 }
 
-size_t broad_lds_bytes(const BroadPlan &plan) { return lds_bytes(plan.rt, plan.nt, plan.part_blocks); }
+int broad_scale_blocks(int rows, int nt, int part_units, int parts, int blk_shift)
+{
+    // the blocks that a part touches: one more than it fills where it starts inside one
+    const int steps = part_units * kStepGroups, size = 1 << blk_shift, blocks = ceil_div_i(steps, size) + (parts > 1 && steps % size ? 1 : 0);
+    return loop_bytes(rows / (16 * kRowGroups), nt, blocks) <= (size_t)kLdsLimit ? blocks : 0;
+}
+
+size_t broad_lds_bytes(const BroadPlan &plan) { return lds_bytes(plan.rt, plan.nt, plan.blocks); }
 
 bool plan_gemm_broad_groups(int rows, int nt, BroadPlan *plan, BroadGroups *groups)
 {

@@ -251,7 +251,8 @@ struct BroadPlan {
     int rt, nt;                   // 16-row tiles of a row group and 16-token tiles of a workgroup
     int tiles, tok_tiles, split;  // row tiles and token tiles; k parts of each
     int part_steps;               // k-steps of 64 of a part, whole units of four (the last may have fewer)
-    int part_blocks;              // as of TallPlan
+    int blocks;                   // blocks of 64 << args.blk_shift weights whose scales LDS holds; 0: one scale per row
+    bool unit_scales;             // those of two units of four k-steps, not of a part of k
     size_t ws_bytes, n_counters;
 };
 
@@ -378,6 +379,8 @@ bool plan_gemm_broad(int rows, int nt, int split, int blk_shift, BroadPlan *plan
 hipError_t launch_gemm_broad(const BroadPlan &plan, const BroadGroups *groups, hipStream_t stream);
 bool plan_gemm_broad_groups(int rows, int nt, BroadPlan *plan, BroadGroups *groups);
 size_t broad_lds_bytes(const BroadPlan &plan);
+// Blocks whose scales a part of k needs in LDS, 0 if they don't fit there.
+int broad_scale_blocks(int rows, int nt, int part_units, int parts, int blk_shift);
 hipError_t launch_gemm_wide32(const TiledArgs &args, hipStream_t stream);
 bool tiled_variant_exists(int tile_rows, int tile_tokens, bool mfma32);
 size_t tiled_lds_bytes(int tile_rows, int tile_tokens);

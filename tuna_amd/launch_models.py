@@ -118,9 +118,16 @@ def tall(r, c):
 
 
 # launch, round, unit, rows, tokens, both, tokens where rows of x start inside a cache line, with every compute unit at work,
-# hand-over, its parts, sums, output, KB of a workgroup's scales
-BROAD = (3.015, 1.578, 0.1557, 0.13, 0.0865, 0.00105, 0.1034, 0.0496, 1.831, 0.0343, 0.0809, 0.8826, 0.0)
-BROAD_BLOCKS = (4.096, 1.578, 0.1557, 0.1365, 0.0865, 0.00105, 0.1034, 0.0496, 1.831, 0.0343, 0.0809, 0.8826, 0.0298)
+# hand-over, its parts, sums, output; with scales in blocks launch, round, unit, rows and KB of scales where LDS holds a part's,
+# then the first four where it holds a unit's
+BROAD = (3.015, 1.578, 0.1557, 0.13, 0.0865, 0.00105, 0.1034, 0.0496, 1.831, 0.0343, 0.0809, 0.8826)
+BROAD_BLOCKS = BROAD + (2.484, 3.578, 0.0761, 0.1482, 0.0332, 1.212, 2.125, 0.3803, 0.1493)
+
+
+def _broad_scales_fit(rt, nt, part, parts, block):
+    steps, size = 4 * part, block // 64
+    blocks = _cd(steps, size) + (1 if parts > 1 and steps % size else 0)
+    return 65536 + 16384 * nt + blocks * 128 * (1 if rt <= 2 else 2 if rt <= 4 else 4) <= 160 * 1024
 
 
 def broad(r, c):
@@ -128,12 +135,16 @@ def broad(r, c):
     rt, units, nblk = r["rows"] // 32, _cd(_cd(k, 64), 4), k // r["block"] if r["block"] else 0
     part = _cd(units, split)
     parts = _cd(units, part)
+    own, kb = c[:4], 0.0
+    if nblk:
+        in_lds = nblk >= 4 and _broad_scales_fit(rt, nt, part, parts, r["block"])
+        own, kb = (c[12:16], c[16]) if in_lds else (c[17:21], 0.0)
     full, rest = divmod(_cd(m, r["rows"]) * _cd(n, 16 * nt) * parts, CUS)
-    unit = c[2] + c[3] * rt + (c[6] if k % 64 else c[4]) * nt + c[5] * rt * nt
+    unit = own[2] + own[3] * rt + (c[6] if k % 64 else c[4]) * nt + c[5] * rt * nt
     work = part * (full * (unit + c[7] * nt) + (unit + c[7] * nt * rest / CUS if rest else 0.0))
-    scales = c[12] * 0.125 * rt * math.ceil(part * 256.0 * nblk / k) if nblk else 0.0
+    scales = kb * 0.125 * rt * math.ceil(part * 256.0 * nblk / k) if nblk else 0.0
     over = c[8] + c[9] * parts * nt * rt if parts > 1 else 0.0
-    return c[0] + (full + (1 if rest else 0)) * (c[1] + c[10] * rt * nt + scales) + work + over + c[11] * 1e-6 * n * m
+    return own[0] + (full + (1 if rest else 0)) * (own[1] + c[10] * rt * nt + scales) + work + over + c[11] * 1e-6 * n * m
 
 
 MODELS = {"flow": (flow, FLOW), "narrow": (narrow, NARROW), "narrow blocks": (narrow, NARROW_BLOCKS), "wide": (wide, WIDE),
@@ -201,7 +212,7 @@ def launches(kind, rng, per_shape):
             for rows in (64, 96, 128, 160, 192, 256):
                 items = _cd(m, rows) * _cd(n, 16 * nt)
                 most = max(1, min(CUS // items, 16, k // 1024))
-                if rows * nt <= 1024 and items * most <= 1200:
+                if rows * nt <= 1024 and items * most <= 1200 and not (block and nt == 6):
                     fit += [(rows, nt, split) for split in sorted({most, max(1, most - 1), max(1, most // 2)})]
         return [row(m, n, k, block, rows=rows, token_tiles=nt, split=split) for rows, nt, split in rng.sample(fit, min(per_shape, len(fit)))]
     if kind in ("tall", "tall blocks"):
