@@ -1345,8 +1345,8 @@ static bool narrow_any_instead(int m, int n, int k, const tuna_gemm_config &c, b
 }
 
 // Up to 64 tokens, after all of these: tall tiles where their model is ahead of the price of what is picked so far - that
-// kernel's model, or straight lines in MB of weights.  Against the picks without it on 700 random shapes, as far as they
-// differ: decode-batch picks 1.3 x, many-token tiles 1.9 x, general 1.6 x, narrow rows 1.07 x.  Lean and batched launches are
+// kernel's model, or straight lines in MB of weights.  Against the picks without it on 1100 random shapes, as far as they
+// differ (465, 1.34 x): decode-batch picks 1.3 x, many-token tiles 1.9 x, general 1.6 x, narrow rows 1.07 x.  Lean and batched launches are
 // left alone, and so is what the table holds for one token tile a workgroup of narrow rows.
 static bool tall_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, double flow_us, const Room &room, tuna_gemm_config *tall)
 {
