@@ -1490,7 +1490,7 @@ static bool broad_instead(int m, int n, int k, const tuna_gemm_config &c, bool f
     else if (is_narrow(c) || is_narrow_any(c)) price = n > 64 && !from_table ? narrow_time(m, n, k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles) : 0.0;
     else price = n > 64 ? many_token_price(m, n, k, c) : 0.0;
     double us = 0.0;
-    if (price == 0.0 || !best_broad(m, n, k, 0, room, broad, &us)) return false;
+    if (price < 6.0 || !best_broad(m, n, k, 0, room, broad, &us)) return false;  // (less than the model gives to any launch)
     const double rounds = ceil((double)ceil_div(m, broad->rows_per_wave) * ceil_div(n, 16 * broad->token_tiles) / kMaxCus);
     return us < (n > 512 && 2e-6 * n * k > 32 ? 0.78 : n > 512 || rounds > 2 ? 0.88 : 0.95) * price;
 }
@@ -2903,7 +2903,7 @@ static bool blockwise_broad_instead(const BlockwiseCall &b, const tuna_gemm_conf
                 price = kBlockwiseCostUs * b.k * blockwise_tile_cost(t, c.split_k, (long long)ceil_div(b.m, t.rows) * ceil_div(b.n, tokens) * c.split_k, b.k);
     }
     double us = 0.0;
-    if (price == 0.0 || !best_broad(b.m, b.n, b.k, nblk, room, broad, &us)) return false;
+    if (price < 6.0 || !best_broad(b.m, b.n, b.k, nblk, room, broad, &us)) return false;  // (as in broad_instead)
     const double rounds = ceil((double)ceil_div(b.m, broad->rows_per_wave) * ceil_div(b.n, 16 * broad->token_tiles) / kMaxCus);
     return us < (2e-6 * b.n * b.k > 32 ? 0.78 : b.n > 384 || rounds > 2 ? 0.86 : 0.95) * price;
 }
