@@ -505,8 +505,9 @@ hipError_t launch(const BroadPlan &plan, const BroadGroups *groups, hipStream_t 
     if constexpr (RT * NT <= 32) {
         if (groups) return launch<RT, NT, SCALES_ROW>(plan, *groups, stream);
         if (!plan.blocks) return launch<RT, NT, SCALES_ROW>(plan, OneMatrix(), stream);
-        if (!plan.unit_scales) return launch<RT, NT, SCALES_PART>(plan, OneMatrix(), stream);
-        if constexpr (NT <= 5) return launch<RT, NT, SCALES_UNIT>(plan, OneMatrix(), stream);
+        // (beside the table and the activations of 96 tokens there is no room for scales)
+        if constexpr (NT <= 5)
+            return plan.unit_scales ? launch<RT, NT, SCALES_UNIT>(plan, OneMatrix(), stream) : launch<RT, NT, SCALES_PART>(plan, OneMatrix(), stream);
         else return hipErrorInvalidConfiguration;
     } else {
         return hipErrorInvalidConfiguration;
