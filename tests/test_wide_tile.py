@@ -155,7 +155,7 @@ def test_groups_of_many_tokens_in_one_launch(m, k, counts):
 
 # scale blocks: one block per step and several steps per block, odd numbers of steps, splits, small last tiles
 @pytest.mark.parametrize("m,n,k,block,split", [(256, 200, 256, 64, 1), (528, 300, 1280, 64, 1), (272, 70, 768, 256, 1), (512, 385, 2048, 128, 3),
-                                               (1024, 129, 1792, 64, 2)])
+                                               (1024, 129, 1792, 64, 2), (1280, 768, 5632, 64, 3)])
 def test_scale_blocks(m, n, k, block, split):
     import torch
 
@@ -166,3 +166,20 @@ def test_scale_blocks(m, n, k, block, split):
     ops.matmul_blockwise(x, q, s, code, out, m, n, k, block, config=_cfg(split))
     torch.cuda.synchronize()
     _check(out, q, s, x, code, k, block=block)
+
+
+# the same in launches whose last tiles are shared: segments of any number of steps, full token tiles and small last ones
+@pytest.mark.parametrize("m,n,k,block", [(9728, 1024, 8192, 64), (8448, 1100, 4352, 128), (5120, 2000, 13824, 64)])
+def test_scale_blocks_of_shared_tiles(m, n, k, block):
+    import torch
+
+    from tuna_amd import ops
+
+    assert "last tiles shared" in ops.describe_launch(m, n, k, _cfg(1))
+    q, s, x, code = _inputs(m, n, k, seed=k + n, block=block)
+    outs = [_out(n, m) for _ in range(3)]
+    for o in outs:
+        ops.matmul_blockwise(x, q, s, code, o, m, n, k, block, config=_cfg(1))
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    _check(outs[0], q, s, x, code, k, block=block)

@@ -226,8 +226,14 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
         WIDE_HALF(0, s, 0)
         WIDE_HALF(0, s, 1)
     }
-    // (the requests beyond the last step have arrived: their LDS and registers are free)
+    // The requests beyond the last step have arrived: their LDS and registers are free.  Every set passes through this wait,
+    // used or not: a register that the compiler takes for free while its load is on its way would be overwritten under whatever
+    // it holds by then (the scales of a segment's last step came to lie on a token fragment).
     asm volatile("s_waitcnt vmcnt(0)" : "+v"(wq[0][0]), "+v"(wq[0][1]), "+v"(wq[1][0]), "+v"(wq[1][1])::"memory");
+    if (BLK) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) asm volatile("" : "+v"(sq[BLK ? i : 0][0]), "+v"(sq[BLK ? i : 0][1]), "+v"(sq[BLK ? i : 0][2]), "+v"(sq[BLK ? i : 0][3]));
+    }
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMAs have written their accumulators
     // (pinned once more: no copy of an accumulator moves up between the MFMAs, whose latency the compiler does not know)
 #pragma unroll

@@ -2,8 +2,10 @@
 // return their data over one path: 8 KB per wave of loads and 56 table reads take 64 and 55 ns apart and 118 together, with
 // the loads going to LDS 66 (256 workgroups of eight waves).  The kernels that read LDS most of the time therefore have
 // their activations brought into LDS directly.  The compiler, seeing such loads, would wait for all of them at every use of a
-// loaded register and at every LDS store: here they are instructions it does not look into, so every wait is written out,
-// and a register that such a load fills is passed through the wait that makes it valid.
+// loaded register and at every LDS store: here they are instructions it does not look into, so every wait is written out.
+// For the compiler a register that such a load fills holds its value at once, and is free from its last use on.  So every
+// destination is passed ("+v") through a wait that covers its load, on EVERY path from there, also where nothing uses what was
+// loaded (tests/test_async_loads.py follows the assembly).
 #pragma once
 #include "epilogue.hpp"
 
