@@ -398,7 +398,7 @@ def time_blockwise(ops, synth, torch, dev, names=("mistral_qkv", "mistral_gate_u
         torch.cuda.synchronize()
         took = [L.tuna_blockwise_launches(i) - before[i] for i in range(6)]
         kernel = ("tuna::gemm_narrow_kernel", "tuna::gemm_multi_kernel", "tuna::gemm_tiled_kernel", "tuna::gemm_mid_kernel",
-                  "tuna::gemm_flow_kernel_tall", "tuna::gemm_broad_kernel")[took.index(max(took))]
+                  "tuna::gemm_tall_kernel", "tuna::gemm_broad_kernel")[took.index(max(took))]
         for _ in range(3):
             graph.replay()
         torch.cuda.synchronize()

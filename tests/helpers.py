@@ -4,7 +4,7 @@ import numpy as np
 from oracle import oracle as O
 from tuna_amd.synth import make_inputs_np
 
-# GEMM tolerance of the north star: max relative error 1e-2 (fp16 output, fp32
+# GEMM tolerance: max relative error 1e-2 (fp16 output, fp32
 # accumulate, any split-K order).  "Relative" is |y - y_ref| / max(|y_ref|, FLOOR * max|y_ref|):
 # outputs are sums of ~k zero-mean terms, so a few land arbitrarily close to zero, where a
 # pure ratio is meaningless; below FLOOR (0.1 % of the largest output) the error is measured
@@ -78,5 +78,28 @@ def run_dequant(q, code, absmax, m, k, decode_mode=2):
     return out.cpu().numpy().view(np.uint16)
 
 
+def launched(m, n, k):
+    """(kernel, bytes of partial sums) of a launch without a config where the workspace can grow, for the kernels whose tiles
+    several workgroups may share; (kernel, 0) for the others."""
+    import re
+
+    from tuna_amd import launch_models, ops
+
+    d = ops.describe_launch(m, n, k)
+    kernel = re.match(r"\w+", d).group(0)
+    numbers = [int(v) for v in re.findall(r"\d+", d.split(" in place of")[0])]
+    if kernel == "gemm_flow_kernel":
+        r = dict(kind="flow", token_tiles=numbers[0], split=numbers[1])
+    elif kernel == "gemm_tall_kernel":
+        r = dict(kind="tall", rows=numbers[0], token_tiles=numbers[1], split=numbers[2])
+    elif kernel == "gemm_broad_kernel":
+        r = dict(kind="broad", rows=numbers[0], token_tiles=numbers[1] // 16, split=numbers[2])
+    elif kernel == "gemm_wide_kernel":
+        r = dict(kind="wide", token_tiles=16, split=numbers[2])
+    else:
+        return kernel, 0
+    return kernel, ops.config_footprint(m, n, k, launch_models.config_of(r))[1]
+
+
 __all__ = ["O", "make_inputs_np", "rel_err", "REL_TOL", "REL_FLOOR_D2", "f16_bits_to_f64", "ulp_diff_f16", "to_dev", "run_gemm",
-           "run_dequant"]
+           "run_dequant", "launched"]

@@ -5,6 +5,7 @@ import random
 import numpy as np
 import pytest
 
+from helpers import launched
 from test_wide_tile import _check, _inputs, _out
 from tuna_amd import _lib, ops
 
@@ -27,34 +28,52 @@ def test_the_static_entry_point_refuses_no_pick_of_the_library_for_its_workspace
     assert not refused, refused[:5]
 
 
+# (kernel, m, n, k) whose partial sums fit the static scratch: decode-batch shares that cross tiles and equal parts of tiles, tall
+# and broad tiles in parts of k
+SHARED = [("gemm_flow_kernel", 33352, 24, 1088), ("gemm_flow_kernel", 33832, 16, 6336), ("gemm_flow_kernel", 33056, 35, 1024),
+          ("gemm_tall_kernel", 4096, 64, 14336), ("gemm_tall_kernel", 5120, 37, 13824), ("gemm_broad_kernel", 8192, 160, 8192)]
+# ... and whole tiles
+WHOLE = [("gemm_tall_kernel", *s) for s in ((22016, 33, 4096), (27648, 40, 5120), (17024, 24, 1936), (17728, 50, 4096), (17664, 14, 5056))]
+
+
+def test_these_launches_are_what_they_are_here_for():
+    for kernel, *shape in SHARED + WHOLE:
+        ran, sums = launched(*shape)
+        assert ran == kernel and (0 < sums <= 16 << 20 if (kernel, *shape) in SHARED else sums == 0), (shape, ran, sums)
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k", [(22016, 33, 4096), (27648, 40, 5120), (17024, 24, 1936), (17728, 50, 4096), (17664, 14, 5056)])
-def test_static_entry_point(m, n, k):
+@pytest.mark.parametrize("kernel,m,n,k", SHARED + WHOLE)
+def test_static_entry_point(kernel, m, n, k):
     import torch
 
-    assert "gemm_flow_kernel" in ops.describe_launch(m, n, k)
+    assert launched(m, n, k)[0] == kernel
     q, s, x, code = _inputs(m, n, k, seed=n)
-    out, again = _out(n, m), _out(n, m)
+    out, again, grown = (_out(n, m) for _ in range(3))
     ops.matmul_static(x, q, s, code, out, m, n, k)
     ops.matmul_static(x, q, s, code, again, m, n, k)
+    ops.matmul(x, q, s, code, grown, m, n, k)
     torch.cuda.synchronize()
-    assert torch.equal(out, again)
+    assert torch.equal(out, again) and torch.equal(out, grown)  # (the same launch: its sums fit both workspaces)
     _check(out, q, s, x, code, k)
 
 
 def _calls():
-    """(name, kernel that an eager call takes, call, output, check)"""
-    for m, n, k in ((22016, 33, 4096), (17024, 24, 1936), (17664, 14, 5056), (8832, 497, 3456)):
+    """(name, bytes of partial sums of an eager call, call, output, check, whether there is a launch without partial sums)"""
+    for _kernel, m, n, k in SHARED + [("gemm_flow_kernel", 33136, 41, 1088), ("gemm_wide_kernel", 8832, 497, 3456)]:
         q, s, x, code = _inputs(m, n, k, seed=n)
         out = _out(n, m)
-        yield (f"matmul {m} {n} {k}", ops.describe_launch(m, n, k), lambda q=q, s=s, x=x, code=code, out=out, m=m, n=n, k=k:
-               ops.matmul(x, q, s, code, out, m, n, k), out, lambda q=q, s=s, x=x, code=code, out=out, k=k: _check(out, q, s, x, code, k))
-    m, n, k, block = 8832, 467, 3328, 64
-    cfg, _hit = ops.select_config_blockwise(m, n, k, block)
-    q, s, x, code = _inputs(m, n, k, seed=n, block=block)
-    out = _out(n, m)
-    yield (f"matmul_blockwise {m} {n} {k}", f"gemm_wide_kernel split_k={cfg.split_k}" if cfg.lds_tile_rows == 256 and cfg.split_k > 1 else "",
-           lambda: ops.matmul_blockwise(x, q, s, code, out, m, n, k, block), out, lambda: _check(out, q, s, x, code, k, block=block))
+        yield (f"matmul {m} {n} {k}", launched(m, n, k)[1], lambda q=q, s=s, x=x, code=code, out=out, m=m, n=n, k=k:
+               ops.matmul(x, q, s, code, out, m, n, k), out, lambda q=q, s=s, x=x, code=code, out=out, k=k: _check(out, q, s, x, code, k),
+               ops.config_footprint(m, n, k, ops.select_config(m, n, k)[0])[1] == 0 or _kernel == "gemm_wide_kernel")
+    # (scale blocks: 256 x 256 tiles split in parts, tall tiles and broad tiles in parts of k)
+    for tile_rows, m, n, k, block in ((256, 8832, 467, 3328, 64), (-6, 4096, 48, 14336, 64), (-7, 4096, 160, 14336, 128)):
+        cfg, _hit = ops.select_config_blockwise(m, n, k, block)
+        q, s, x, code = _inputs(m, n, k, seed=n, block=block)
+        out = _out(n, m)
+        yield (f"matmul_blockwise {m} {n} {k}", ops.config_footprint(m, n, k, cfg)[1] if cfg.lds_tile_rows == tile_rows else 0,
+               lambda q=q, s=s, x=x, code=code, out=out, m=m, n=n, k=k, block=block: ops.matmul_blockwise(x, q, s, code, out, m, n, k, block),
+               out, lambda q=q, s=s, x=x, code=code, out=out, k=k, block=block: _check(out, q, s, x, code, k, block=block), tile_rows > 0)
 
 
 @pytest.mark.gpu
@@ -64,9 +83,11 @@ def test_capture(warm):
     Warm: the shape ran there once, and the graph replays the bits of that run."""
     import torch
 
-    for name, kernel, call, out, check in _calls():
-        print(name, "warm" if warm else "cold", kernel, flush=True)
-        assert kernel.startswith(("gemm_flow_kernel", "gemm_wide_kernel"))
+    for name, sums, call, out, check, runs_without in _calls():
+        print(name, "warm" if warm else "cold", sums, flush=True)
+        assert sums > 0
+        if not warm and not runs_without:  # (what the pick stands in for splits k itself: such a call asks for the workspace)
+            continue
         torch.cuda.synchronize()
         assert _lib.lib().tuna_release_workspaces() == _lib.OK
         side, g, eager = torch.cuda.Stream(), torch.cuda.CUDAGraph(), None

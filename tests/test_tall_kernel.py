@@ -26,7 +26,7 @@ def test_tiles(m, n, k, rows, split, epilogue):
 
     from tuna_amd import _lib, ops
 
-    assert f"gemm_flow_kernel_tall<{rows} rows" in ops.describe_launch(m, n, k, _cfg(rows, n, split))
+    assert f"gemm_tall_kernel<{rows} rows" in ops.describe_launch(m, n, k, _cfg(rows, n, split))
     q, s, x, code = _inputs(m, n, k, seed=m + n)
     plain, again = _out(n, m), _out(n, m)
     ops.matmul(x, q, s, code, plain, m, n, k, config=_cfg(rows, n, split))
@@ -108,9 +108,9 @@ def test_a_call_without_a_config_takes_it_where_it_is_predicted_to_be_faster():
     from tuna_amd import ops
 
     for shape in ((5120, 37, 13824), (28672, 64, 4096), (4096, 64, 14336), (8192, 24, 28672), (11008, 20, 4104)):
-        assert "gemm_flow_kernel_tall" in ops.describe_launch(*shape), shape
+        assert "gemm_tall_kernel" in ops.describe_launch(*shape), shape
     for shape in ((4096, 1, 4096), (6144, 16, 4096), (4096, 64, 4096), (57344, 16, 8192), (229376, 64, 4096), (4096, 65, 14336)):
-        assert "gemm_flow_kernel_tall" not in ops.describe_launch(*shape), shape
+        assert "gemm_tall_kernel" not in ops.describe_launch(*shape), shape
 
 
 @pytest.mark.parametrize("kind,off", [("tall", 5.1), ("tall blocks", 4.7)])

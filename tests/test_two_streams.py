@@ -2,19 +2,25 @@
 its own, and the bits are those of a launch alone."""
 import pytest
 
+from helpers import launched
 from test_wide_tile import _check, _inputs, _out
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("kernel,m,n,k", [("gemm_flow_kernel", 22016, 33, 4096), ("gemm_flow_kernel", 17664, 14, 5056),
-                                          ("last tiles shared", 8448, 1100, 4096), ("split_k=3 in place", 8832, 497, 3456)])
+# decode-batch shares that cross tiles (three and one token tile) and equal parts of tiles; tall and broad tiles in parts of k;
+# 256 x 256 tiles with the last ones shared, and split in three
+@pytest.mark.parametrize("kernel,m,n,k", [("gemm_flow_kernel", 33136, 41, 1088), ("gemm_flow_kernel", 33832, 16, 6336),
+                                          ("gemm_flow_kernel", 33056, 35, 1024), ("gemm_tall_kernel", 4096, 64, 14336),
+                                          ("gemm_tall_kernel", 5120, 37, 13824), ("gemm_broad_kernel", 8192, 160, 8192),
+                                          ("gemm_wide_kernel", 8448, 1100, 4096), ("gemm_wide_kernel", 8832, 497, 3456)])
 def test_two_streams(kernel, m, n, k):
     import torch
 
     from tuna_amd import ops
 
-    assert kernel in ops.describe_launch(m, n, k)
+    ran, sums = launched(m, n, k)
+    assert ran == kernel and sums > 0
     calls = [_inputs(m, n, k, seed=seed) for seed in (n, n + 1)]
     alone = [_out(n, m) for _ in calls]
     for (q, s, x, code), out in zip(calls, alone):
@@ -34,12 +40,15 @@ def test_two_streams(kernel, m, n, k):
             assert torch.equal(o, want)
 
 
-@pytest.mark.parametrize("m,k,counts", [(14336, 1024, (3, 0, 17, 33, 1, 16, 8, 2)), (4096, 1024, (400, 100, 777, 90))])
+# decode-batch shares that are equal parts of tiles, and that cross them; 256 x 256 tiles split in two and with shared last
+# tiles, with decode-batch shares that need partial sums behind theirs
+@pytest.mark.parametrize("m,k,counts", [(2816, 2048, (3, 0, 17, 32, 1, 16, 8, 2)), (4096, 4096, (3, 0, 17, 32, 1, 16, 8, 2)),
+                                        (4608, 2688, (5, 1250, 0, 420, 30)), (5120, 1024, (157, 232, 14, 1207, 1494, 4))])
 def test_groups_on_two_streams(m, k, counts):
     import numpy as np
     import torch
 
-    from tuna_amd import ops
+    from tuna_amd import _lib, ops
 
     offs = np.concatenate([[0], np.cumsum(counts)]).tolist()
     calls = [_inputs(m * len(counts), offs[-1], k, seed=seed) for seed in (k, k + 1)]
@@ -47,6 +56,16 @@ def test_groups_on_two_streams(m, k, counts):
     for (q, s, x, code), out in zip(calls, alone):
         ops.matmul_grouped(x, q, s, code, out, m, len(counts), k, offs)
         torch.cuda.synchronize()
+        for e, (lo, hi) in enumerate(zip(offs, offs[1:])):
+            if hi > lo:
+                _check(out[lo:hi], q, s, x[lo:hi], code, k, first_row=e * m, rows=m)
+    # (all kernels are loaded: a call that has no workspace yet takes memory for nothing else)
+    assert _lib.lib().tuna_release_workspaces() == _lib.OK
+    free = torch.cuda.mem_get_info()[0]
+    q, s, x, code = calls[0]
+    ops.matmul_grouped(x, q, s, code, alone[0], m, len(counts), k, offs)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] >= 8 << 20
     streams = [torch.cuda.Stream() for _ in calls]
     outs = [[_out(offs[-1], m) for _ in range(4)] for _ in calls]
     torch.cuda.synchronize()

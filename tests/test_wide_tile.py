@@ -135,7 +135,7 @@ def test_a_capturing_stream_without_workspace_takes_whole_tiles():
 
 
 @pytest.mark.parametrize("m,k,counts", [(512, 512, (200, 65, 0, 128, 129, 256, 257, 70)), (320, 1032, (300, 66, 64, 80, 100, 512)),
-                                        (2048, 1024, (400, 1, 777, 90))])
+                                        (2048, 1024, (400, 1, 777, 90)), (4608, 2688, (5, 1250, 0, 420, 30))])
 def test_groups_of_many_tokens_in_one_launch(m, k, counts):
     import torch
 

@@ -3292,7 +3292,7 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
                            ? describe_narrow_any(np, n, buf, len, " in place of ")
                        : is_flow(w) ? snprintf(buf, len, "gemm_flow_kernel<NT=%d> %d shares in place of ", w.token_tiles, w.split_k)
                        : is_broad(w) ? snprintf(buf, len, "gemm_broad_kernel<%d rows x %d tokens> split_k=%d in place of ", w.rows_per_wave, 16 * w.token_tiles, w.split_k)
-                       : is_tall(w) ? snprintf(buf, len, "gemm_flow_kernel_tall<%d rows,NT=%d> split_k=%d in place of ", w.rows_per_wave, w.token_tiles, w.split_k)
+                       : is_tall(w) ? snprintf(buf, len, "gemm_tall_kernel<%d rows,NT=%d> split_k=%d in place of ", w.rows_per_wave, w.token_tiles, w.split_k)
                                     : snprintf(buf, len, "gemm_wide_kernel<256 rows x 256 tokens> split_k=%d in place of ", w.split_k);
         return at < 0 || (size_t)at + 16 > len ? TUNA_OK : tuna_describe_launch(m, n, k, &c, decode_mode, buf + at, len - (size_t)at);
     }
@@ -3314,7 +3314,7 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
     if (is_tall(c)) {
         TallPlan tp;
         if ((rc = plan_tall(m, n, k, c, decode_mode, &tp))) return rc;
-        snprintf(buf, len, "gemm_flow_kernel_tall<%d rows,NT=%d> split_k=%d", 16 * tp.rt, tp.nt, tp.split);
+        snprintf(buf, len, "gemm_tall_kernel<%d rows,NT=%d> split_k=%d", 16 * tp.rt, tp.nt, tp.split);
         return TUNA_OK;
     }
     if (is_broad(c)) {

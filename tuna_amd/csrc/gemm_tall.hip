@@ -59,7 +59,7 @@ constexpr size_t lds_bytes(int rt, int nt, int blocks)
 
 // (separate scalars, the ones the first loads need in front: the first sixteen dwords arrive in scalar registers with the wave)
 template <int RT, int NT, bool BLK>
-__global__ __launch_bounds__(kThreads, 2) void gemm_flow_kernel_tall(const uint8_t *a_q, const void *a_x, const float *a_code, const float *a_absmax,
+__global__ __launch_bounds__(kThreads, 2) void gemm_tall_kernel(const uint8_t *a_q, const void *a_x, const float *a_code, const float *a_absmax,
                                                                      int a_k, int a_n, int a_m, int a_part_steps, void *a_out, int a_epilogue,
                                                                      const void *a_residual, float *a_ws, unsigned *a_counters, int a_blk_shift, int a_ticket)
 {
@@ -401,7 +401,7 @@ template <int RT, int NT, bool BLK>
 hipError_t launch(const TallPlan &plan, hipStream_t stream)
 {
     static OptInFlag done[16];
-    const auto fn = gemm_flow_kernel_tall<RT, NT, BLK>;
+    const auto fn = gemm_tall_kernel<RT, NT, BLK>;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
