@@ -1213,11 +1213,27 @@ static double tall_time(int m, int n, int k, int rt, int split, int nblk = 0)
            (parts > 1 ? 2.371 + 0.02158 * parts * nt * rt : 0.0) + 3.18e-6 * n * m;
 }
 
-// The tile height and the number of k parts that take least time with partial sums that `room` holds, and that time in *us.
-static bool best_tall(int m, int n, int k, int nblk, const Room &room, tuna_gemm_config *tall, double *us)
+// Less than tall_time of any launch that best_tall considers: one round of the lowest tiles, and their steps unsplit or those
+// of the shortest part it makes with the hand-over.
+static double tall_time_least(int m, int n, int k, int nblk)
 {
+    const int nt = ceil_div(n, 16), steps = ceil_div(k, 64), most = std::max(1, std::min(16, k / 512));
+    const double step = (nblk ? 0.2332 + 0.05657 * 2 : 0.2405 + 0.04922 * 2) + (0.1367 + 0.0191 * 2) * nt;
+    const double stream = 0.1662 * (0.5e-6 * m * k + 4e-6 * m * nblk), whole = ceil_div(steps, 8) * step, part = ceil_div(ceil_div(steps, most), 8) * step;
+    const double divided = (part > stream ? part : stream) + 2.371 + 0.02158 * 2 * nt * 2, undivided = whole > stream ? whole : stream;
+    return (nblk ? 2.622 : 1.519) + 2.036 + 0.02599 * 2 * nt + (undivided < divided ? undivided : divided) + 3.18e-6 * n * m;
+}
+
+// The tile height and the number of k parts that take least time, less than `limit` us, with partial sums that `room` holds,
+// and that time in *us.
+static bool best_tall(int m, int n, int k, int nblk, const Room &room, double limit, tuna_gemm_config *tall, double *us)
+{
+    // (small shapes end here: the pick for 1024 x 4096 at 4 tokens, which host time bounds, 2.9 us with a Python call around it; 3.8
+    // with the search)
+    if (tall_time_least(m, n, k, nblk) >= limit) return false;
     const int nt = ceil_div(n, 16), blk_shift = nblk ? log2i(k / nblk) - 6 : -1;
     bool found = false;
+    *us = limit;
     for (int rt = 2; rt <= 8; ++rt) {
         const int tiles = ceil_div(m, 16 * rt);
         if (rt * nt > 28) continue;
@@ -1226,7 +1242,7 @@ static bool best_tall(int m, int n, int k, int nblk, const Room &room, tuna_gemm
         for (int split = most; split >= 1; split = split > 2 ? std::max(split / 2, split == most ? split - 1 : 1) : split - 1) {
             if (split > 1 && !room.holds((size_t)tiles * split * rt * nt * 1024, (size_t)tiles)) continue;
             const double t = tall_time(m, n, k, rt, split, nblk);
-            if (found && t >= *us) continue;
+            if (t >= *us) continue;
             tuna_gemm_config c;
             memset(&c, 0, sizeof(c));
             c.rows_per_wave = 16 * rt, c.waves_m = 1, c.waves_k = 8, c.prefetch = 2, c.x_chunk = 64, c.token_tiles = nt;
@@ -1370,9 +1386,8 @@ static bool tall_instead(int m, int n, int k, const tuna_gemm_config &c, bool fr
         else if (plan.ws_bytes) price = 0.88 * (9.0 + (nt > 1 ? nt : 0) + kMid[nt] * mb); // (split: with the hand-over of its sums)
         else price = 0.85 * (6.0 + (nt > 1 ? nt : 0) + kMid[nt] * mb);
     }
-    if (4.0 + 0.1662 * mb > price) return false; // (below what the model gives to any launch)
     double us = 0.0;
-    return best_tall(m, n, k, 0, room, tall, &us) && us < price;
+    return best_tall(m, n, k, 0, room, price, tall, &us);
 }
 
 // What a config for more than 64 tokens takes by its kernel's model, in microseconds: 256 x 256 tiles by theirs, many-token and
@@ -2878,7 +2893,7 @@ static bool blockwise_tall_instead(const BlockwiseCall &b, const tuna_gemm_confi
     }
     price *= 0.95;
     double us = 0.0;
-    if (4.0 + 0.1662 * mb > price || !best_tall(b.m, b.n, b.k, nblk, room, tall, &us) || us >= price) return false;
+    if (!best_tall(b.m, b.n, b.k, nblk, room, price, tall, &us)) return false;
     tuna_gemm_config any;
     return !best_narrow_any(b.m, b.n, b.k, nblk, us, &any);
 }
