@@ -67,13 +67,13 @@ def _calls():
                ops.matmul(x, q, s, code, out, m, n, k), out, lambda q=q, s=s, x=x, code=code, out=out, k=k: _check(out, q, s, x, code, k),
                ops.config_footprint(m, n, k, ops.select_config(m, n, k)[0])[1] == 0 or _kernel == "gemm_wide_kernel")
     # (scale blocks: 256 x 256 tiles split in parts, tall tiles and broad tiles in parts of k)
-    for tile_rows, m, n, k, block in ((256, 8832, 467, 3328, 64), (-6, 4096, 48, 14336, 64), (-7, 4096, 160, 14336, 128)):
+    for tile_rows, m, n, k, block in ((256, 8832, 467, 3328, 64), (-6, 4096, 32, 14336, 128), (-6, 4096, 48, 14336, 64), (-7, 4096, 160, 14336, 128)):
         cfg, _hit = ops.select_config_blockwise(m, n, k, block)
         q, s, x, code = _inputs(m, n, k, seed=n, block=block)
         out = _out(n, m)
         yield (f"matmul_blockwise {m} {n} {k}", ops.config_footprint(m, n, k, cfg)[1] if cfg.lds_tile_rows == tile_rows else 0,
                lambda q=q, s=s, x=x, code=code, out=out, m=m, n=n, k=k, block=block: ops.matmul_blockwise(x, q, s, code, out, m, n, k, block),
-               out, lambda q=q, s=s, x=x, code=code, out=out, k=k, block=block: _check(out, q, s, x, code, k, block=block), tile_rows > 0)
+               out, lambda q=q, s=s, x=x, code=code, out=out, k=k, block=block: _check(out, q, s, x, code, k, block=block), tile_rows != -7)
 
 
 @pytest.mark.gpu

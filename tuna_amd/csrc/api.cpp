@@ -2873,6 +2873,24 @@ static int derive_blockwise(const BlockwiseCall &b, const Room &room, tuna_gemm_
     return TUNA_OK;
 }
 
+// Whether `room` holds the partial sums of a config of the batched kernel or of many-token tiles (others have none).
+static bool blockwise_sums_fit(const BlockwiseCall &b, const tuna_gemm_config &c, const Room &room)
+{
+    if (room.bytes == kRoomToGrow.bytes) return true;
+    if (blockwise_family(c) == kBlkTiled) {
+        tuna_gemm_config t = c;
+        t.rows_per_wave = 64;
+        TiledPlan tp;
+        return plan_tiled(b.m, b.n, b.k, t, TUNA_DECODE_GEMM, &tp) != TUNA_OK || room.holds(tp.ws_bytes, tp.n_counters);
+    }
+    if (blockwise_family(c) != kBlkMulti) return true;
+    const int chunks = ceil_div(b.n, 16), cnt = chunks < kMaxMultiProblems ? chunks : kMaxMultiProblems;
+    tuna_gemm_problem probs[kMaxMultiProblems];
+    for (int ch = 0; ch < cnt; ++ch) probs[ch] = {b.q ? b.q : b.out, b.x, b.code, b.absmax, b.out, b.m, std::min(16, b.n - 16 * ch), b.k};
+    MultiPlan plan;
+    return !plan_multi(probs, cnt, planned_cus(), &plan, c.waves_m, c.prefetch, log2i(b.block_size) - 6) || room.holds(plan.ws_bytes, plan.n_counters);
+}
+
 // Up to 64 tokens: tall tiles (gemm_tall.hip) where their model is ahead of `c`'s price - the narrow-row kernel's model, of
 // its variants for any k too, or straight lines over the bytes of the weights (28672 x 4096 with blocks of 64: at 16 tokens
 // 20.2 -> 18.2 us, at 64 37.1 -> 27.6; 5440 x 21760 at 46 tokens 53.9 -> 26.8, 4224 x 21248 at 16 31.4 -> 17.1; 220 random
@@ -2893,6 +2911,8 @@ static bool blockwise_tall_instead(const BlockwiseCall &b, const tuna_gemm_confi
     }
     price *= 0.95;
     double us = 0.0;
+    // (a pick that cannot run gives way to any launch that can)
+    if (!blockwise_sums_fit(b, c, room)) return best_tall(b.m, b.n, b.k, nblk, room, 1e30, tall, &us);
     if (!best_tall(b.m, b.n, b.k, nblk, room, price, tall, &us)) return false;
     tuna_gemm_config any;
     return !best_narrow_any(b.m, b.n, b.k, nblk, us, &any);
