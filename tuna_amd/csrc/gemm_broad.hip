@@ -66,7 +66,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
     constexpr bool GRP = !std::is_empty<GROUPS>::value;
     using P = Pieces<RT>;
     constexpr int NS = 2;      // units whose weights are on their way
-    constexpr int LD = 1, LR = LD == 1 ? 2 : 4;  // table reads are that many turns ahead of their scaling's successor
     constexpr int T = 2 * RT;  // turns of a step: a row tile of a half each
     constexpr int ROWS = kRowGroups * 16 * RT, STAGE = kStepGroups * NT * 2048;  // activations of a unit
     extern __shared__ __align__(16) unsigned char smem[];
@@ -192,18 +191,18 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
     BROAD_LOAD_W(0, 1)
     f16x2 sc[BLK ? 2 : 1][(RT + 1) / 2];  // of the step at hand and of the next one
     f16x8 fa[2], fb[2][NT];
-    uint32_t lt[LR][4];
+    uint32_t lt[2][4];  // table reads of a turn and of the next one
     // (turn tau of step u: row tile tau % RT of half tau / RT; u and tau may run over into the next step)
 #define BROAD_LUT(u, tau)                                                                                      \
     {                                                                                                         \
-        const int u_ = ((u) + (tau) / T) % NS, h_ = (tau) % T / RT, r_ = (tau) % RT, l_ = ((u) * T + (tau)) % LR; \
+        const int u_ = ((u) + (tau) / T) % NS, h_ = (tau) % T / RT, r_ = (tau) % RT, l_ = ((u) * T + (tau)) % 2; \
         _Pragma("unroll") for (int b = 0; b < 4; ++b) lt[l_][b] = *reinterpret_cast<const lds_u32 *>(         \
             (uintptr_t)__builtin_amdgcn_perm(wq[u_][h_][r_], lane4, 0x0c0c0400u + 0x100u * b));               \
         if (r_ == RT - 1) BROAD_LOAD_W(u_, h_) /* the half's registers are free */                             \
     }
 #define BROAD_SCALE(u, tau)                                                                                    \
     {                                                                                                         \
-        const int r_ = (tau) % RT, l_ = ((u) * T + (tau)) % LR, f_ = (tau) & 1; /* (as for BROAD_LUT) */       \
+        const int r_ = (tau) % RT, l_ = ((u) * T + (tau)) % 2, f_ = (tau) & 1; /* (as for BROAD_LUT) */       \
         _Pragma("unroll") for (int b = 0; b < 4; ++b)                                                         \
         {                                                                                                     \
             f16x2 v_;                                                                                         \
@@ -239,7 +238,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
             }                                                                                                 \
         }                                                                                                     \
         _Pragma("unroll") for (int t = 0; t < NT; ++t) if (tau == RT + t * (RT - 1) / NT) BROAD_READ_B(0, (((u) + 1) & 1) * STAGE, t) \
-        BROAD_LUT(u, tau + 1 + LD)                                                                                 \
+        BROAD_LUT(u, tau + 2)                                                                                 \
         __builtin_amdgcn_sched_barrier(0);                                                                    \
     }
     const int b0 = BLK == SCALES_PART ? s0 >> a_blk_shift : 0;
@@ -341,8 +340,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
     }
     BROAD_LUT(0, 0)
     BROAD_SCALE(0, 0)
-#pragma unroll
-    for (int l = 1; l <= LD; ++l) BROAD_LUT(0, l)
+    BROAD_LUT(0, 1)
 #pragma unroll
     for (int t = 0; t < NT; ++t) BROAD_READ_B(0, 0, t)
     {

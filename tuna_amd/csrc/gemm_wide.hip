@@ -102,8 +102,8 @@ __device__ __forceinline__ void wide_steps(f32x4 (&acc)[4][16], const WideTile &
     {                                                                                                         \
         const int s_ = min((s), s_last);                                                                      \
         const bool t_ = KTAIL && s_ == s_last;                                                                \
-        load_async<false>(wq[set][0], q_rsrc, t_ ? a_off - a_back0 : a_off, (uint32_t)wide_weight_uniform(s_, 0, t_, slot_last)); \
-        load_async<false>(wq[set][1], q_rsrc, t_ ? a_off - a_back1 : a_off, (uint32_t)wide_weight_uniform(s_, 1, t_, slot_last)); \
+        load_async(wq[set][0], q_rsrc, t_ ? a_off - a_back0 : a_off, (uint32_t)wide_weight_uniform(s_, 0, t_, slot_last)); \
+        load_async(wq[set][1], q_rsrc, t_ ? a_off - a_back1 : a_off, (uint32_t)wide_weight_uniform(s_, 1, t_, slot_last)); \
         if (BLK)                                                                                              \
             _Pragma("unroll") for (int j = 0; j < 4; ++j) load_async(sq[set][j], s_rsrc, s_off[j], (uint32_t)min(s_ >> w.blk_shift, nblk - 1) * 4u); \
     }

@@ -22,13 +22,12 @@ __device__ __forceinline__ u32x4 buffer_at(const void *base, size_t bytes)
 // 16 bytes a lane into LDS, lane l's at lds + 16 l.
 __device__ __forceinline__ void load_to_lds(const u32x4 &rsrc, uint32_t offset, uint32_t uniform, uint32_t lds)
 {
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(offset), "s"(rsrc), "s"(uniform), "s"(lds));
+    // (the address in M0 is an operand: the compiler writes that register itself and knows when it has changed)
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(offset), "s"(rsrc), "s"(uniform), "{m0}"(lds));
 }
-template <bool NONTEMPORAL>
 __device__ __forceinline__ void load_async(u32x4 &dst, const u32x4 &rsrc, uint32_t offset, uint32_t uniform)
 {
-    if (NONTEMPORAL) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen nt" : "=v"(dst) : "v"(offset), "s"(rsrc), "s"(uniform));
-    else asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen" : "=v"(dst) : "v"(offset), "s"(rsrc), "s"(uniform));
+    asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen" : "=v"(dst) : "v"(offset), "s"(rsrc), "s"(uniform));
 }
 __device__ __forceinline__ void load_async(uint32_t &dst, const u32x4 &rsrc, uint32_t offset, uint32_t uniform)
 {
