@@ -696,8 +696,9 @@ static bool narrow_round(int m, int n, int k, tuna_gemm_config *out)
 
 
 // Microseconds of a launch of 256 x 256 many-token tiles (gemm_wide.hip) by a model read off 320 random shapes of 1024 ...
-// 57344 rows and 65 ... 4096 tokens (14 per cent off on average, and at 0.89 of the measured time, on the 323 launches kept in
-// profiles/launch_model_times.csv, which tuna_amd/launch_models.py times and fits models to, this one and those below): a k-step of
+// 57344 rows and 65 ... 4096 tokens when that kernel still stored its activations to LDS (the 323 launches kept in
+// profiles/launch_model_times.csv, which tuna_amd/launch_models.py times and fits models to, this one and those below, are of the
+// present kernel: 9.6 per cent off on average, at 0.97 of the measured time, 0.93 unsplit): a k-step of
 // a tile takes longer the more workgroups share the chip's power, a whole tile ends with 12 us of stores, a shared one
 // with as long for the partial sums and more for every further share of it.  split: 1 whole tiles, 2 ... that many equal shares of
 // every tile, 0 the last rounds of tiles shared evenly between the compute units.
@@ -1419,7 +1420,8 @@ static bool wide_instead(int m, int n, int k, const tuna_gemm_config &c, const R
     const double price = many_token_price(m, n, k, c);
     double us = 0.0;
     const int split = price == 0.0 ? 0 : wide_best_split(t.large, t.small, t.steps, room, &us);
-    // (four parts and more: what their hand-over costs beyond the model)
+    // (four parts and more: what their hand-over cost beyond the model with the kernel it was read off; at 0.98 of the measured
+    // time now)
     if (!split || us * (split >= 4 ? 1.1 : 1.0) >= 0.96 * price) return false;
     memset(wide, 0, sizeof(*wide));
     wide->rows_per_wave = 64, wide->waves_m = 1, wide->waves_k = 1, wide->prefetch = 2, wide->x_chunk = 64, wide->token_tiles = 16;
@@ -2045,7 +2047,9 @@ static int grouped_flow_shares(int m_group, int n_active, int nt, int k)
 }
 
 // What the groups with more than `pass` tokens take as a launch each, or in one of 256 x 256 tiles (its split in *split, 0 if
-// that is no option or slower; its tiles in a): 6 us and the larger of 0.85 PFLOP/s and 3.5 TB/s apart, wide_time together.
+// that is no option or slower; its tiles in a): 6 us and the larger of 0.85 PFLOP/s and 3.5 TB/s apart, wide_time together.  (The
+// former is 0.85 of what dense calls take, 26 per cent off, on 90 random shapes of 65 ... 1200 tokens.  The latter a tenth higher made
+// the choices that changed 1.03 x slower, on 130 random launches of 48 to 400 tokens per group.)
 static double grouped_many_time(int m_group, int n_groups, int k, const int32_t *offsets, int pass, WideArgs *a, int *split, long long *large, long long *small)
 {
     a->m = m_group, a->k = k, a->n_groups = 0;
@@ -2680,8 +2684,10 @@ static int run_blockwise(const BlockwiseCall &b, const tuna_gemm_config &c, hipS
 }
 
 // Many-token tiles with scale blocks and their factors in the model of derive_config, what a launch of `tiles` workgroups costs
-// in units of 5.68e-7 us per k, and the 256 x 256 tile by its per-row time: 1.07 x, more where k is split (four parts and more
-// cost a quarter more than the model says: 4032 x 6400 at 580 tokens 73 us, the best other tile 56).
+// in units of 5.68e-7 us per k, and the 256 x 256 tile by its per-row time: 1.07 x, more where k is split.  (Of 110 random launches
+// those with scale blocks take 1.12 x the time of those without; this price is at 1.00 of the measured time unsplit, 5 per cent off,
+// at 1.01 in two and three parts, 10 per cent off, and at 1.24 in four and more: the quarter was measured before the kernel's
+// activations were loaded into LDS directly - 4032 x 6400 at 580 tokens 73 us, the best other tile 56.)
 struct BlockwiseTile {
     int rows, tokens;
     double factor;

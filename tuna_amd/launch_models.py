@@ -2,6 +2,7 @@
 they are read off, how far they are from them, and the fit of their coefficients.
 
     python -m tuna_amd.launch_models --measure times.csv    # on a GPU: random shapes, several launches each
+    python -m tuna_amd.launch_models --again wide times.csv # on a GPU: one kind's launches of the file once more
     python -m tuna_amd.launch_models times.csv              # anywhere: the models' errors, and refitted coefficients
 
 A model is a function of a launch and a list of coefficients (below, the forms of api.cpp with its coefficients); the fit
@@ -227,40 +228,64 @@ def launches(kind, rng, per_shape):
     return [row(m, n, k, block, *v, split=1) for v in rng.sample(fit, min(per_shape, len(fit)))]
 
 
-def measure(path, shapes, per_shape, seed, log=print):
+def _timer():
+    """A function that times a launch: microseconds, the median of three runs."""
     import torch
 
     from . import _lib, ops
     from .quantize import nf4_codebook
 
     _lib.use_diagnostic_build()
-    dev, rng = torch.device("cuda:0"), random.Random(seed)
+    dev = torch.device("cuda:0")
     code = nf4_codebook(dev)
     pool = torch.randint(0, 256, (1 << 30,), dtype=torch.uint8, device=dev)  # weights: as many matrices as fit, in turn
     scales = torch.rand(1 << 26, device=dev) * 0.015 + 0.005
     xs = torch.randn(1 << 27, device=dev, dtype=torch.float16)
     out = torch.empty(1 << 28, dtype=torch.float16, device=dev)
+
+    def time(r):
+        m, n, k, block = r["m"], r["n"], r["k"], r["block"]
+        sets = max(1, min(40, (1 << 30) // (m * k // 2)))
+        q = [pool[j * (m * k // 2):(j + 1) * (m * k // 2)].view(m // 8, k // 8, 32) for j in range(sets)]
+        s = [scales[:m * (k // block if block else 1)]] * sets
+        x, o, cfg = xs[:n * k].view(n, k), out[:n * m].view(n, m), config_of(r)
+        iters = max(10, min(100, int(4e11 / (2.0 * m * n * k + 2e9))))
+        us = []
+        for _ in range(3):
+            ms = (ops.time_matmul_blockwise(q, s, x, code, o, m, n, k, block, config=cfg, warmup=4, iters=iters) if block else
+                  ops.time_matmul(q, s, x, code, o, m, n, k, config=cfg, warmup=4, iters=iters))
+            us.append(ms * 1e3 / iters)
+        return round(sorted(us)[1], 2)
+
+    return time
+
+
+def measure(path, shapes, per_shape, seed, log=print):
+    time, rng = _timer(), random.Random(seed)
     with open(path, "w", newline="") as f:
         w = csv.DictWriter(f, FIELDS)
         w.writeheader()
         for kind in MODELS:
             for i in range(shapes):
                 for r in launches(kind, rng, per_shape):
-                    m, n, k, block = r["m"], r["n"], r["k"], r["block"]
-                    sets = max(1, min(40, (1 << 30) // (m * k // 2)))
-                    q = [pool[j * (m * k // 2):(j + 1) * (m * k // 2)].view(m // 8, k // 8, 32) for j in range(sets)]
-                    s = [scales[:m * (k // block if block else 1)]] * sets
-                    x, o, cfg = xs[:n * k].view(n, k), out[:n * m].view(n, m), config_of(r)
-                    iters = max(10, min(100, int(4e11 / (2.0 * m * n * k + 2e9))))
-                    us = []
-                    for _ in range(3):
-                        ms = (ops.time_matmul_blockwise(q, s, x, code, o, m, n, k, block, config=cfg, warmup=4, iters=iters) if block else
-                              ops.time_matmul(q, s, x, code, o, m, n, k, config=cfg, warmup=4, iters=iters))
-                        us.append(ms * 1e3 / iters)
-                    w.writerow(dict(r, us=round(sorted(us)[1], 2)))
+                    w.writerow(dict(r, us=time(r)))
                 if i % 20 == 19:
                     log(f"{kind}: {i + 1} of {shapes} shapes")
                     f.flush()
+
+
+def measure_again(path, kind, log=print):
+    """The launches of `kind` in the file, timed again in place (that kernel has changed)."""
+    rows, time = read(path), _timer()
+    mine = [r for r in rows if r["kind"] == kind]
+    for i, r in enumerate(mine):
+        r["us"] = time(r)
+        if i % 50 == 49:
+            log(f"{kind}: {i + 1} of {len(mine)} launches")
+    with open(path, "w", newline="") as f:
+        w = csv.DictWriter(f, FIELDS)
+        w.writeheader()
+        w.writerows(rows)
 
 
 # ---- errors and fit ---------------------------------------------------------------------------------------------------
@@ -295,12 +320,15 @@ def main(argv=None):
     ap = argparse.ArgumentParser(description=__doc__, formatter_class=argparse.RawDescriptionHelpFormatter)
     ap.add_argument("csv")
     ap.add_argument("--measure", action="store_true")
+    ap.add_argument("--again", metavar="KIND", help="time the launches of one kind in the file again")
     ap.add_argument("--shapes", type=int, default=100, help="random shapes per model")
     ap.add_argument("--per-shape", type=int, default=4, help="launches per shape")
     ap.add_argument("--seed", type=int, default=1)
     a = ap.parse_args(argv)
     if a.measure:
         return measure(a.csv, a.shapes, a.per_shape, a.seed, log=lambda s: print(s, flush=True))
+    if a.again:
+        return measure_again(a.csv, a.again, log=lambda s: print(s, flush=True))
     rows = read(a.csv)
     for kind, (model, coefficients) in MODELS.items():
         mine = [r for r in rows if r["kind"] == kind]
