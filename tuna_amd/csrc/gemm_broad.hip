@@ -30,8 +30,6 @@ namespace {
 constexpr int kRowGroups = 2, kStepGroups = 4;  // the waves: two along the rows, four along k
 constexpr int kWaves = kRowGroups * kStepGroups, kThreads = 64 * kWaves;
 
-template <int RT, int NT>
-constexpr size_t slot_bytes() { return (size_t)kRowGroups * RT * NT * 1024; }
 constexpr size_t x_bytes(int nt) { return (size_t)2 * kStepGroups * nt * 2048; }  // two units' activations
 // In the end, over the table and the activations: the waves' sums, as many token tiles at a time as fit, then the outputs.
 constexpr int red_tiles(int rt, int nt)
@@ -79,17 +77,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
     unsigned char *const work = smem + kLutBytes;
     volatile unsigned *const ticket = reinterpret_cast<volatile unsigned *>(smem + a_ticket);
     const float code_lane = a_code[lane & 15];
-    auto build_table = [&]() {  // as in the streaming kernels
-        const int code_bits = (int)(uint32_t)__builtin_bit_cast(uint16_t, (f16)code_lane);
-#pragma unroll 4
-        for (int p = tid; p < kLutBytes / 16; p += kThreads) {
-            const int e = p >> 4;
-            const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute((e >> 4) << 2, code_bits);
-            const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute((e & 15) << 2, code_bits);
-            const uint32_t v = hi | (lo << 16);
-            reinterpret_cast<u32x4 *>(smem)[p] = u32x4{v, v, v, v};
-        }
-    };
 
     // weights, per lane and piece: rows LW i16 .. + LW - 1 of the piece's, block column g of a half
     uint32_t w_off[P::count];
@@ -252,8 +239,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
     int sc_dst = 0, u_sc = u_first;
     if constexpr (BLK == SCALES_UNIT) {
         const int group_ = sc_row / (16 * RT), r16 = (sc_row >> 4) - group_ * RT;
-        const int width = r16 < 4 * P::fours ? 4 : r16 < 4 * P::fours + 2 * P::twos ? 2 : 1;
-        const int first = width == 4 ? r16 & ~3 : width == 2 ? 4 * P::fours : RT - 1;
+        const int width = P::width_at(r16), first = P::first_at(r16);
         const int in = sc_row - 16 * (group_ * RT + first);
         sc_dst = (group_ * 16 + in / width) * (SD * 4) + (first + in % width) * 2;
     }
@@ -311,8 +297,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
             for (int i = 0; i < PIECES; ++i) {
                 const int j = min(j0 + kWaves * i, RG * quads - 1), c = min(b0 + 4 * (j / RG), nblk - 4) - b0;
                 const int row = 64 * (j % RG) + lane, rows_of = row / (16 * RT), r16 = (row >> 4) - rows_of * RT;
-                const int width = r16 < 4 * P::fours ? 4 : r16 < 4 * P::fours + 2 * P::twos ? 2 : 1;
-                const int first = width == 4 ? r16 & ~3 : width == 2 ? 4 * P::fours : RT - 1;
+                const int width = P::width_at(r16), first = P::first_at(r16);
                 const int in = row - 16 * (rows_of * RT + first), lane16 = in / width, r = first + in % width;
                 if (row < ROWS)
 #pragma unroll
@@ -324,7 +309,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
             }
         }
     }
-    build_table();
+    build_pair_table<kThreads>(smem, tid, code_lane);
     BROAD_LOAD_W(1, 0)
     wait_loads<P::count>();
     __builtin_amdgcn_s_waitcnt(0x0F70 | P::count);
@@ -395,89 +380,10 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_broad_kernel(const uint8_t *
             }
         }
     }
-    bool store = true;
-    if (split > 1) {
-        // k parts: the last workgroup of a tile to arrive adds all parts' sums in k order
-        const int item = (int)blockIdx.z * (int)gridDim.x + tile;
-        unsigned *const counter = a_counters + item;
-        auto slot = [&](int p) {
-            return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char *>(a_ws) + ((size_t)item * split + p) * slot_bytes<RT, NT>(), 0,
-                                                     (int)slot_bytes<RT, NT>(), 0x00020000);
-        };
-        const int at = (wave * NT * 64 + lane) * 16;
-        const auto dst = slot(part);
-#pragma unroll
-        for (int w = 0; w < TW; ++w)
-            if (wave + w * kWaves < TILES) {
-#pragma unroll
-                for (int t = 0; t < NT; ++t)
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sum[w][t]), dst, at, (w * kWaves * NT + t) * 1024, 16);
-            }
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the sums have left this CU
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __syncthreads();
-        if (tid == 0) *ticket = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        store = *ticket == (unsigned)split - 1;
-        if (store && tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (store) {
-            constexpr int PB = NT <= 5 ? 3 : 2;  // parts whose loads are issued before the first is awaited
-#pragma unroll
-            for (int w = 0; w < TW; ++w) {
-                if (wave + w * kWaves >= TILES) continue;
-#pragma unroll
-                for (int t = 0; t < NT; ++t) sum[w][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-                for (int p = 0; p < split; p += PB) {
-                    f32x4 v[PB][NT];
-#pragma unroll
-                    for (int b = 0; b < PB; ++b) {
-                        const auto src = slot(min(p + b, split - 1));
-#pragma unroll
-                        for (int t = 0; t < NT; ++t)
-                            v[b][t] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(src, at, (w * kWaves * NT + t) * 1024, 16));
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int b = 0; b < PB; ++b)
-                        if (p + b < split) {
-#pragma unroll
-                            for (int t = 0; t < NT; ++t) sum[w][t] += v[b][t];
-                        }
-                }
-            }
-        }
-    }
-    if (store) {
-        // through LDS into rows of eight consecutive features
-        constexpr int PITCH = ROWS + 4;
-        float *const ob = reinterpret_cast<float *>(smem);
-        __syncthreads();
-#pragma unroll
-        for (int w = 0; w < TW; ++w) {
-            const int r = wave + w * kWaves, group = r >= RT ? 1 : 0, r16 = r - group * RT;
-            if (r < TILES) {
-                const int width = r16 < 4 * P::fours ? 4 : r16 < 4 * P::fours + 2 * P::twos ? 2 : 1;
-                const int first = width == 4 ? r16 & ~3 : width == 2 ? 4 * P::fours : RT - 1;
-#pragma unroll
-                for (int t = 0; t < NT; ++t)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        ob[(16 * t + i16) * PITCH + 16 * (group * RT + first) + width * (4 * g + v) + r16 - first] = sum[w][t][v];
-            }
-        }
-        __syncthreads();
-        f16 *outp = reinterpret_cast<f16 *>(a_out);
-        const f16 *resp = reinterpret_cast<const f16 *>(a_residual);
-        for (int c = tid; c < 16 * NT * 2 * TILES; c += kThreads) {
-            const int tok = c / (2 * TILES), r8 = c - tok * (2 * TILES), row = row_base + 8 * r8;
-            if (tok < tokens && row + 8 <= a_m) {
-                const float *src = ob + tok * PITCH + 8 * r8;
-                store_features8(outp, resp, a_epilogue, (size_t)(tok_base + tok), a_m, row, *reinterpret_cast<const f32x4 *>(src),
-                                *reinterpret_cast<const f32x4 *>(src + 4));
-            }
-        }
-    }
+    // parts of k: the last workgroup of a tile to arrive adds all parts' sums in k order
+    const int item = (int)blockIdx.z * (int)gridDim.x + tile;
+    if (split > 1 && !add_parts<kWaves, TILES, NT, NT <= 5 ? 3 : 2>(sum, a_ws, a_counters + item, (size_t)item, part, split, tid, wave, ticket)) return;
+    store_tile<kWaves, TILES, NT, RT>(sum, reinterpret_cast<float *>(smem), tid, wave, a_out, a_residual, a_epilogue, row_base, a_m, tok_base, tokens);
 }
 
 struct OneMatrix {};

@@ -33,8 +33,6 @@ namespace tuna {
 namespace {
 constexpr int kWaves = 8, kThreads = 64 * kWaves;
 
-template <int RT, int NT>
-constexpr size_t slot_bytes() { return (size_t)RT * NT * 1024; }
 // Token tiles whose sums the waves exchange at a time: as many as fit beside the table.
 constexpr int red_tiles(int rt, int nt)
 {
@@ -79,17 +77,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tall_kernel(const uint8_t *a
     unsigned char *const work = smem + kLutBytes;
     volatile unsigned *const ticket = reinterpret_cast<volatile unsigned *>(smem + a_ticket);
     const float code_lane = a_code[lane & 15];
-    auto build_table = [&]() {  // as in the streaming kernels
-        const int code_bits = (int)(uint32_t)__builtin_bit_cast(uint16_t, (f16)code_lane);
-#pragma unroll 4
-        for (int p = tid; p < kLutBytes / 16; p += kThreads) {
-            const int e = p >> 4;
-            const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute((e >> 4) << 2, code_bits);
-            const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute((e & 15) << 2, code_bits);
-            const uint32_t v = hi | (lo << 16);
-            reinterpret_cast<u32x4 *>(smem)[p] = u32x4{v, v, v, v};
-        }
-    };
 
     // weights, per lane and piece: rows LW i16 .. + LW - 1 of the piece's, block column g of a half
     uint32_t w_off[P::count];
@@ -247,8 +234,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tall_kernel(const uint8_t *a
             for (int i = 0; i < PIECES; ++i) {
                 const int j = min(j0 + kWaves * i, RG * quads - 1), rg = RG == 1 ? 0 : j & 1, c = min(b0 + 4 * (RG == 1 ? j : j >> 1), nblk - 4) - b0;
                 const int row = 64 * rg + lane, r16 = row >> 4;
-                const int width = r16 < 4 * P::fours ? 4 : r16 < 4 * P::fours + 2 * P::twos ? 2 : 1;
-                const int first = width == 4 ? r16 & ~3 : width == 2 ? 4 * P::fours : RT - 1;
+                const int width = P::width_at(r16), first = P::first_at(r16);
                 const int in = row - 16 * first, lane16 = in / width, r = first + in % width;
                 if (row < ROWS)
 #pragma unroll
@@ -260,7 +246,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tall_kernel(const uint8_t *a
             }
         }
     }
-    build_table();
+    build_pair_table<kThreads>(smem, tid, code_lane);
     TALL_LOAD_W(1, 0)
     TALL_LOAD_W(1, 1)
     __syncthreads();
@@ -303,7 +289,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tall_kernel(const uint8_t *a
 #undef TALL_LOAD_W
 
     // ---- the waves' sums, added in wave order: wave r ends with row tile r ------------------------------------
-    f32x4 sum[NT];
+    f32x4 sum[1][NT];
     f32x4 *const red = reinterpret_cast<f32x4 *>(work);
     constexpr int TP = red_tiles(RT, NT);  // token tiles a pass
 #pragma unroll
@@ -320,81 +306,15 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tall_kernel(const uint8_t *a
                 f32x4 v[kWaves];
 #pragma unroll
                 for (int w = 0; w < kWaves; ++w) v[w] = red[((w * TP + t - t0) * RT + wave) * 64 + lane];
-                sum[t] = v[0];
+                sum[0][t] = v[0];
 #pragma unroll
-                for (int w = 1; w < kWaves; ++w) sum[t] += v[w];
+                for (int w = 1; w < kWaves; ++w) sum[0][t] += v[w];
             }
         }
     }
-    bool store = true;
-    if (split > 1) {
-        // k parts: the last workgroup of a tile to arrive adds all parts' sums in k order
-        unsigned *const counter = a_counters + tile;
-        auto slot = [&](int p) {
-            return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char *>(a_ws) + ((size_t)tile * split + p) * slot_bytes<RT, NT>(), 0,
-                                                     (int)slot_bytes<RT, NT>(), 0x00020000);
-        };
-        const int at = (wave * NT * 64 + lane) * 16;
-        if (wave < RT) {
-            const auto dst = slot(part);
-#pragma unroll
-            for (int t = 0; t < NT; ++t) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sum[t]), dst, at, t * 1024, 16);
-        }
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the sums have left this CU
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __syncthreads();
-        if (tid == 0) *ticket = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        store = *ticket == (unsigned)split - 1;
-        if (store && tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (store && wave < RT) {
-            constexpr int PB = 16 / NT;  // parts whose loads are issued before the first is awaited
-#pragma unroll
-            for (int t = 0; t < NT; ++t) sum[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-            for (int p = 0; p < split; p += PB) {
-                f32x4 v[PB][NT];
-#pragma unroll
-                for (int b = 0; b < PB; ++b) {
-                    const auto src = slot(min(p + b, split - 1));
-#pragma unroll
-                    for (int t = 0; t < NT; ++t) v[b][t] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(src, at, t * 1024, 16));
-                }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int b = 0; b < PB; ++b)
-                    if (p + b < split) {
-#pragma unroll
-                        for (int t = 0; t < NT; ++t) sum[t] += v[b][t];
-                    }
-            }
-        }
-    }
-    if (store) {
-        // through LDS into rows of eight consecutive features
-        constexpr int PITCH = ROWS + 4;
-        float *const ob = reinterpret_cast<float *>(work);
-        __syncthreads();
-        if (wave < RT) {
-            const int width = wave < 4 * P::fours ? 4 : wave < 4 * P::fours + 2 * P::twos ? 2 : 1;
-            const int first = width == 4 ? wave & ~3 : width == 2 ? 4 * P::fours : RT - 1;
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) ob[(16 * t + i16) * PITCH + 16 * first + width * (4 * g + v) + wave - first] = sum[t][v];
-        }
-        __syncthreads();
-        f16 *outp = reinterpret_cast<f16 *>(a_out);
-        const f16 *resp = reinterpret_cast<const f16 *>(a_residual);
-        for (int c = tid; c < 16 * NT * 2 * RT; c += kThreads) {
-            const int tok = c / (2 * RT), r8 = c - tok * (2 * RT), row = row_base + 8 * r8;
-            if (tok < a_n && row + 8 <= a_m) {
-                const float *src = ob + tok * PITCH + 8 * r8;
-                store_features8(outp, resp, a_epilogue, (size_t)tok, a_m, row, *reinterpret_cast<const f32x4 *>(src),
-                                *reinterpret_cast<const f32x4 *>(src + 4));
-            }
-        }
-    }
+    // parts of k: the last workgroup of a tile to arrive adds all parts' sums in k order
+    if (split > 1 && !add_parts<kWaves, RT, NT, 16 / NT>(sum, a_ws, a_counters + tile, (size_t)tile, part, split, tid, wave, ticket)) return;
+    store_tile<kWaves, RT, NT, RT>(sum, reinterpret_cast<float *>(work), tid, wave, a_out, a_residual, a_epilogue, row_base, a_m, 0, a_n);
 }
 
 template <int RT, int NT, bool BLK>
