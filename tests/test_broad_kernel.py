@@ -129,6 +129,17 @@ def test_a_call_without_a_config_takes_it_where_it_is_predicted_to_be_faster():
         assert "gemm_broad_kernel" not in ops.describe_launch(*shape), shape
 
 
+def test_256_x_256_tiles_stay_where_their_price_is_known_to_be_too_high():
+    """Tiles of both kinds over long k, and four parts and more with scale blocks: broad tiles take 1.13 x and 1.14 x the time there."""
+    from tuna_amd import ops
+
+    for shape in ((8192, 384, 28672), (7744, 331, 24256), (16064, 264, 23704)):
+        assert ops.describe_launch(*shape).startswith("gemm_wide_kernel"), shape
+    for shape in ((12672, 254, 13056, 128), (15552, 229, 23040, 128), (8064, 355, 24064, 64)):
+        c, _hit = ops.select_config_blockwise(*shape)
+        assert (c.lds_tile_rows, c.token_tiles) == (256, 16), shape
+
+
 @pytest.mark.parametrize("kind,off", [("broad", 4.9), ("broad blocks", 4.4)])
 def test_the_stated_errors_are_those_of_the_kept_launches(kind, off):
     """(per cent, as stated beside broad_time in csrc/api.cpp)"""

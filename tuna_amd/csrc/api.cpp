@@ -1496,6 +1496,9 @@ static int select_config_for(int m, int n, int k, int decode, tuna_gemm_config *
 // 8192 x 28672 at 303 tokens in three rounds, hence less trust in those).  Above 512 tokens on 141 shapes of up to 16384 rows, the
 // models being 6 per cent off, it takes 33, 1.22 x faster (4096 x 14336 at 777 tokens 133 -> 100, 5120 x 5120 at 594 55 -> 39, 3712 x
 // 3072 at 608 34 -> 22; nothing slower); with more activations than the L2s hold (32 MB) launches take up to 1.4 x what the model says.
+// Ahead of 256 x 256 tiles for 257 ... 384 tokens that holds from 10 MB on: wide_time exceeds what such launches take, of large and
+// small tiles in shares of one size (8192 x 28672 at 384 tokens 167 us, 215 with broad tiles; the 51 of 26400 random shapes whose pick
+// that changes 1.13 x, one of them 3 per cent slower).
 // What the table holds of narrow rows stays.
 static bool broad_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, double flow_us, const Room &room, tuna_gemm_config *broad)
 {
@@ -1509,7 +1512,9 @@ static bool broad_instead(int m, int n, int k, const tuna_gemm_config &c, bool f
     double us = 0.0;
     if (price < 6.0 || !best_broad(m, n, k, 0, room, broad, &us)) return false;  // (less than the model gives to any launch)
     const double rounds = ceil((double)ceil_div(m, broad->rows_per_wave) * ceil_div(n, 16 * broad->token_tiles) / kMaxCus);
-    return us < (n > 512 && 2e-6 * n * k > 32 ? 0.78 : n > 512 || rounds > 2 ? 0.88 : 0.95) * price;
+    const bool from_wide = c.lds_tile_rows == 256 && c.token_tiles == 16 && c.rows_per_wave != 32;
+    const double x_mb = 2e-6 * n * k, limit = n > 512 ? 32 : from_wide && n > 256 && n <= 384 ? 10 : 1e9;
+    return us < (x_mb > limit ? 0.78 : n > 512 || rounds > 2 ? 0.88 : 0.95) * price;
 }
 
 // The config a launch without an explicit one runs: the selected one, or a newer kernel in its place - one whose partial
@@ -2937,7 +2942,11 @@ static bool blockwise_broad_instead(const BlockwiseCall &b, const tuna_gemm_conf
     } else if (blockwise_family(c) == kBlkTiled) {
         if (c.lds_tile_rows == 256 && tokens == 256) {
             const WideTiles t(b.m, b.n, b.k);
-            price = blockwise_wide_time(wide_time(t.large, t.small, t.steps, c.split_k == 1 && wide_balance_pays(b.m, b.n, b.k) ? 0 : c.split_k), c.split_k);
+            // (between 129 and 384 tokens without the quarter for four parts and more, which that price exceeds the measured time by: 12672 x
+            // 13056 at 254 with blocks of 128 took 122 us for 100, 76 such random shapes 1.14 x; below and above it makes up for what broad
+            // launches take beyond their model)
+            price = blockwise_wide_time(wide_time(t.large, t.small, t.steps, c.split_k == 1 && wide_balance_pays(b.m, b.n, b.k) ? 0 : c.split_k),
+                                        b.n > 128 && b.n <= 384 ? std::min(c.split_k, 3) : c.split_k);
         }
         for (const BlockwiseTile &t : kBlockwiseTiles)
             if (t.rows == c.lds_tile_rows && t.tokens == tokens)
