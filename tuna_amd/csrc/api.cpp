@@ -2904,7 +2904,7 @@ static bool blockwise_sums_fit(const BlockwiseCall &b, const tuna_gemm_config &c
 
 // Up to 64 tokens: tall tiles (gemm_tall.hip) where their model is ahead of `c`'s price - the narrow-row kernel's model, of
 // its variants for any k too, or straight lines over the bytes of the weights (28672 x 4096 with blocks of 64: at 16 tokens
-// 20.2 -> 18.2 us, at 64 37.1 -> 27.6; 5440 x 21760 at 46 tokens 53.9 -> 26.8, 4224 x 21248 at 16 31.4 -> 17.1; 220 random
+// 19.2 -> 17.3 us, at 64 33.5 -> 25.9; 5440 x 21760 at 46 tokens 53.9 -> 26.8, 4224 x 21248 at 16 31.4 -> 17.1; 220 random
 // shapes 1.26 x, 1.4 x where the choice changes).
 static bool blockwise_tall_instead(const BlockwiseCall &b, const tuna_gemm_config &c, const Room &room, tuna_gemm_config *tall)
 {

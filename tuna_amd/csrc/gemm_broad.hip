@@ -15,11 +15,11 @@
 // 4096 at 80 tokens, 24 are left without the loads, 27 with either kind.  No gain, and not kept: table reads three and four turns
 // ahead, the matrix instructions dealt out between the decode of byte pairs, the barrier two turns before a unit's end.
 //
-// Against the launches that were chosen before, in us: 28672 x 4096 at 80 tokens 41 -> 28, at 128 42 -> 37; 8192 x 8192 at 96
-// 30 -> 25, at 160 47 -> 31, at 256 51 -> 42; 4096 x 14336 at 96 33 -> 25, at 192 46 -> 34; 5120 x 13824 at 160 47 -> 33; 11008 x
-// 2048 at 192 27 -> 17; 57344 x 8192 at 64 75 -> 70.  Groups: one launch over all row tiles
-// and token tiles of all groups, eight experts of 14336 x 4096 on 512 tokens 147 -> 98.  Scales in blocks: 4096 x
-// 14336 at 777 tokens 125 -> 116, 5120 x 5120 at 594 56 -> 43.  The floor of the first, its weights at the rate of a large copy: 12.
+// Against the launches that were chosen before, in us on one box: 28672 x 4096 at 80 tokens 44 -> 29, at 128 43 -> 37; 8192 x 8192
+// at 96 29 -> 24, at 160 47 -> 30, at 256 52 -> 43; 4096 x 14336 at 192 45 -> 32; 5120 x 13824 at 160 45 -> 34; 11008 x 2048 at 192
+// 27 -> 17; 57344 x 8192 at 64 88 -> 73.  Groups: one launch over all row tiles and token tiles of all groups, eight experts of
+// 14336 x 4096 on 512 tokens 147 -> 98.  Scales in blocks of 128: 4096 x 14336 at 777 tokens 126 -> 115, 5120 x 5120 at 594
+// 55 -> 42.  The floor of the first, its weights at the rate of a large copy: 12.
 #include "lds_dma.hpp"
 #include "row_pieces.hpp"
 #include <type_traits>

@@ -15,16 +15,16 @@
 // channels: 101 us became 83 for the weights of 229376 x 4096 alone).  The waves' sums meet in LDS in wave order, parts of k in
 // the workspace, added by the last to arrive in k order: results don't depend on the order of arrival.
 //
-// Measured against the launches that were chosen before, in us (m x k at 16 NT tokens): 5120 x 13824: 19.3 -> 14.4, 28.9 -> 16.1,
-// 29.3 -> 19.4, 34.7 -> 22.0 for NT 1 .. 4; 8192 x 28672: 32 -> 29, 40 -> 32, 57 -> 39, 56 -> 47; 28672 x 4096: 16.2 -> 15.5,
-// 22 -> 18.8, 31 -> 22.2, 31 -> 25.1; 4096 x 14336 at NT 4: 23.7 -> 18.9.  Its floor, the weights at the rate of a large copy:
-// 7, 23, 12 and 6.  Compute alone (table, scaling, MFMA) runs at 29 .. 36 ns per KB and CU, which is what is left.  Not better,
+// Measured against the launches that were chosen before, in us on one box (m x k at 16 NT tokens): 5120 x 13824: 19.0 -> 14.4,
+// 28.7 -> 15.7, 28.0 -> 18.1, 33.8 -> 20.4 for NT 1 .. 4; for NT 2 .. 4 8192 x 28672: 39 -> 32, 55 -> 37, 54 -> 47; for NT 3 and
+// 4 28672 x 4096: 27.8 -> 21.0, 27.7 -> 24.0, 4096 x 14336: 22.9 -> 16.5, 22.6 -> 18.5.  Floors, the weights at the rate of a large
+// copy: 7, 23, 12 and 6.  Compute alone (table, scaling, MFMA) runs at 29 .. 36 ns per KB and CU, which is what is left.  Not better,
 // and not kept: activations straight into LDS (pieces of 64 bytes 28.4 for 24.9 us at NT 4, of 128 equal), four steps ahead, a
 // deeper ring of table reads, part of the decode on the VALU (5 .. 14 per cent slower).
 //
 // Scales finer than a row (BLK): a part's scales go to LDS once, two bytes each and a lane's of a block together, and a step's
-// are read half a step ahead.  28672 x 4096 with blocks of 64: 20.2 -> 18.2 us at 16 tokens, 37 -> 27.6 at 64; 8192 x 28672 at 32
-// tokens 58 -> 39.
+// are read half a step ahead.  28672 x 4096 with blocks of 64: 19.2 -> 17.3 us at 16 tokens, 33.5 -> 25.9 at 64; 8192 x 28672 at 32
+// tokens 57 -> 34.
 #include "epilogue.hpp"
 #include "row_pieces.hpp"
 
