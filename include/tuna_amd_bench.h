@@ -177,7 +177,7 @@ unsigned long long tuna_lean_launches(void);
  * and 8- or 16-wave launches with more token tiles (the streaming kernel of gemm_mid.hpp, ring depth 2 or 4) stage the packed weights through
  * LDS (global_load_lds_dwordx4 into a per-wave ring, ds_read_b128 when a slot is consumed) instead
  * of loading them into registers.  Same access pattern, ring depth, arithmetic and results; it
- * exists so that the two weight paths can be timed against each other on one box (the reference
+ * exists so that the two weight paths can be timed against each other on one card (the reference
  * stages its packed weights through shared memory, kernel.cu:1997-2042).  Returns the previous
  * setting.  tuna_describe_launch names the path a launch would take. */
 int tuna_set_weight_path(int through_lds);

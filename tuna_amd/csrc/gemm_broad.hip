@@ -15,7 +15,7 @@
 // 4096 at 80 tokens, 24 are left without the loads, 27 with either kind.  No gain, and not kept: table reads three and four turns
 // ahead, the matrix instructions dealt out between the decode of byte pairs, the barrier two turns before a unit's end.
 //
-// Against the launches that were chosen before, in us on one box: 28672 x 4096 at 80 tokens 44 -> 29, at 128 43 -> 37; 8192 x 8192
+// Against the launches that were chosen before, in us on one card: 28672 x 4096 at 80 tokens 44 -> 29, at 128 43 -> 37; 8192 x 8192
 // at 96 29 -> 24, at 160 47 -> 30, at 256 52 -> 43; 4096 x 14336 at 192 45 -> 32; 5120 x 13824 at 160 45 -> 34; 11008 x 2048 at 192
 // 27 -> 17; 57344 x 8192 at 64 88 -> 73.  Groups: one launch over all row tiles and token tiles of all groups, eight experts of
 // 14336 x 4096 on 512 tokens 147 -> 98.  Scales in blocks of 128: 4096 x 14336 at 777 tokens 126 -> 115, 5120 x 5120 at 594

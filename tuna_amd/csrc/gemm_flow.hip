@@ -17,7 +17,7 @@
 // of that (229376 x 4096 at 32 tokens 132 us on 256 shares, 107 on 512), but costs more for short launches.  Around the loop 6 us
 // in all, and 3 .. 10 for handing over tiles that several shares contribute to (120064 x 3968 at 16 tokens: 46 us on 469 shares of
 // a tile each, 59 on 512; without the hand-over 47).  No gain: each share's part of a tile walked from elsewhere in k on.
-// Against the kernels the launches took before (general, streaming, many-token; one box, launch loop): 17920 x 23168 at 30
+// Against the kernels the launches took before (general, streaming, many-token; one card, launch loop): 17920 x 23168 at 30
 // tokens 154 -> 60 us, 32128 x 13312 at 36 tokens 129 -> 68, 28672 x 8192 at 37 tokens 51 -> 43; eight experts of 28672 x 4096 on 128 tokens 148 -> 128, and 100 on 512 shares (117 on 256 on that box).
 #include "epilogue.hpp"
 

@@ -15,7 +15,7 @@
 // channels: 101 us became 83 for the weights of 229376 x 4096 alone).  The waves' sums meet in LDS in wave order, parts of k in
 // the workspace, added by the last to arrive in k order: results don't depend on the order of arrival.
 //
-// Measured against the launches that were chosen before, in us on one box (m x k at 16 NT tokens): 5120 x 13824: 19.0 -> 14.4,
+// Measured against the launches that were chosen before, in us on one card (m x k at 16 NT tokens): 5120 x 13824: 19.0 -> 14.4,
 // 28.7 -> 15.7, 28.0 -> 18.1, 33.8 -> 20.4 for NT 1 .. 4; for NT 2 .. 4 8192 x 28672: 39 -> 32, 55 -> 37, 54 -> 47; for NT 3 and
 // 4 28672 x 4096: 27.8 -> 21.0, 27.7 -> 24.0, 4096 x 14336: 22.9 -> 16.5, 22.6 -> 18.5.  Floors, the weights at the rate of a large
 // copy: 7, 23, 12 and 6.  Compute alone (table, scaling, MFMA) runs at 29 .. 36 ns per KB and CU, which is what is left.  Not better,

@@ -14,9 +14,9 @@
 // What bounds it: in the loop the matrix pipes, busy 75 % of the cycles at the 1.68 GHz that the power limit leaves (with the
 // activations loaded into registers and stored to LDS 68 % at 1.72 GHz); around it the start and end of a tile, 12 us by
 // wide_time's fit, which nothing overlaps - one workgroup per compute unit - and compute units without a tile in the last round.
-// The power limit alone explains less: torch's fp16 product of the first two shapes takes 187 and 367 us on the box of these
+// The power limit alone explains less: torch's fp16 product of the first two shapes takes 187 and 367 us on the card of these
 // figures.  8192 x 8192 at 2048 tokens 241 -> 224 us, 28672 x 4096 at 2000 tokens 403 -> 381, 4096 x 14336 at 2000 200 -> 190,
-// 6144 x 4096 at 2000 101 -> 93, 8192 x 8200 at 4096 468 -> 420 (one box, launch loop).
+// 6144 x 4096 at 2000 101 -> 93, 8192 x 8200 at 4096 468 -> 420 (one card, launch loop).
 //
 // Tiles of 1 .. 128 tokens (the last of a group) run the same steps with half the token tiles.  How tiles become
 // workgroups is plan_gemm_wide's choice.  KTAIL: k is any multiple of 8 - the slots of the last k-step beyond k load
