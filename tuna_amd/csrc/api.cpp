@@ -1494,8 +1494,8 @@ static int select_config_for(int m, int n, int k, int decode, tuna_gemm_config *
 // From 49 tokens on, last: broad tiles where their model is ahead of the pick's.  On 249 random shapes of 65 ... 640 tokens
 // it takes 152, 1.28 x faster (many-token tiles 1.26 x, streaming ones 1.2 x, 256 x 256 tiles split over k 1.2 x; worst 0.84:
 // 8192 x 28672 at 303 tokens in three rounds, hence less trust in those).  Above 512 tokens on 141 shapes of up to 16384 rows, the
-// models being 6 per cent off, it takes 33, 1.22 x faster (4096 x 14336 at 777 tokens 133 -> 100, 5120 x 5120 at 594 55 -> 39, 3712 x
-// 3072 at 608 34 -> 22; nothing slower); with more activations than the L2s hold (32 MB) launches take up to 1.4 x what the model says.
+// models being 6 per cent off, it takes 33, 1.22 x faster (5120 x 5120 at 594 tokens 54 -> 40, 3712 x 3072 at 608 34 -> 25;
+// nothing slower); with more activations than the L2s hold (32 MB) launches take up to 1.4 x what the model says.
 // Ahead of 256 x 256 tiles for 257 ... 384 tokens that holds from 10 MB on: wide_time exceeds what such launches take, of large and
 // small tiles in shares of one size (8192 x 28672 at 384 tokens 167 us, 215 with broad tiles; the 51 of 26400 random shapes whose pick
 // that changes 1.13 x, one of them 3 per cent slower).
@@ -2930,8 +2930,8 @@ static bool blockwise_tall_instead(const BlockwiseCall &b, const tuna_gemm_confi
 }
 
 // From 65 tokens on: broad tiles (gemm_broad.hip) where their model is ahead of the derived config's.  Of 170 random shapes
-// of 65 ... 2500 tokens with blocks of 64 and 128 it takes 68, 1.28 x faster (3712 x 16384 at 297 tokens 94 -> 60, 22016 x 4096 at 72
-// 44 -> 28; worst 0.93: 10496 x 12032 at 243); less trust in the model above 384 tokens, in several rounds and beyond the L2s.
+// of 65 ... 2500 tokens with blocks of 64 and 128 it takes 68, 1.28 x faster (3712 x 16384 at 297 tokens 92 -> 57, 22016 x 4096 at 72
+// 44 -> 30; worst 0.93: 10496 x 12032 at 243); less trust in the model above 384 tokens, in several rounds and beyond the L2s.
 static bool blockwise_broad_instead(const BlockwiseCall &b, const tuna_gemm_config &c, const Room &room, tuna_gemm_config *broad)
 {
     if (b.n <= 64) return false;
