@@ -17,18 +17,20 @@ struct Pieces {
     static __device__ __forceinline__ int first_at(int r) { return r < 4 * fours ? r & ~3 : r < 4 * fours + 2 * twos ? 4 * fours : RT - 1; }
 };
 
-// The decode table at LDS address 0: each of the 256 pairs of codes for each bank (as in the streaming kernels).
+// The decode table at LDS address 0: each of the 256 pairs of codes for each bank (as in the streaming kernels).  A thread's entries
+// share their low code; the high ones are the same for a whole wave: seven instructions an entry of four banks instead of eighteen,
+// 0.7 -> 0.3 us of a launch's start with eight waves.
 template <int THREADS>
 __device__ __forceinline__ void build_pair_table(unsigned char *smem, int tid, float code_lane)
 {
+    static_assert(THREADS % 256 == 0 && kLutBytes % (16 * THREADS) == 0, "threads");
     const int code_bits = (int)(uint32_t)__builtin_bit_cast(uint16_t, (f16)code_lane);
-#pragma unroll 4
-    for (int p = tid; p < kLutBytes / 16; p += THREADS) {
-        const int e = p >> 4;
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute((e >> 4) << 2, code_bits);
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute((e & 15) << 2, code_bits);
-        const uint32_t v = hi | (lo << 16);
-        reinterpret_cast<u32x4 *>(smem)[p] = u32x4{v, v, v, v};
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(((tid >> 4) & 15) << 2, code_bits) << 16;
+    const int high = __builtin_amdgcn_readfirstlane(tid >> 8);
+#pragma unroll
+    for (int i = 0; i < kLutBytes / (16 * THREADS); ++i) {
+        const uint32_t v = lo | (uint32_t)__builtin_amdgcn_readlane(code_bits, high + i * (THREADS / 256));
+        reinterpret_cast<u32x4 *>(smem)[tid + i * THREADS] = u32x4{v, v, v, v};
     }
 }
 
@@ -58,7 +60,8 @@ __device__ __forceinline__ bool add_parts(f32x4 (&sum)[(TILES + WAVES - 1) / WAV
     __syncthreads();
     if (tid == 0) *ticket = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    if (*ticket != (unsigned)split - 1) return false;
+    // (one value for the wave: a branch that could differ between lanes makes the slots below look as if they did)
+    if (__builtin_amdgcn_readfirstlane((int)*ticket) != split - 1) return false;
     if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
     for (int w = 0; w < TW; ++w) {
