@@ -95,7 +95,11 @@ typedef struct tuna_gemm_config {
                               (tiles of at least 32 tokens), any other value with 16 x 16 x 32
                               (the reference's counterpart: its MMA shapes, kernel.cu:411-465).
                               256 rows x 256 tokens is a kernel of its own (one wave per SIMD, a
-                              wave owns 64 x 256, or 128 x 128 with 32 x 32 MFMA tiles).  -4: the
+                              wave owns 64 x 256, or 128 x 128 with 32 x 32 MFMA tiles); with waves_m
+                              8 .. 16 (and 16 x 16 MFMA tiles) its tiles have up to waves_m x 16 tokens,
+                              n divided evenly between as few as that makes, each whole (split_k 1),
+                              in split_k parts of k, or (split_k 0) the last ones shared between the
+                              compute units.  -4: the
                               decode-batch kernel - 256 rows x token_tiles (1 .. 4) x 16 tokens per
                               workgroup, the k-steps of all row tiles divided into split_k shares (1 ..
                               512 workgroups); no other field is read.  -5: the narrow-row
@@ -219,7 +223,7 @@ int tuna_matmul_multi_blockwise(const tuna_gemm_problem *problems, int count, in
  * cannot grow -, and the groups of more than 64 tokens (prefill sizes) leave the grouped launch, which would stream their weights once per 64 tokens: each runs
  * as a dense GEMM of its own on the same stream - tuna_matmul on its slices of q, absmax, x and
  * out, bit-identical to that call - or, several of them where that is predicted to be faster, all
- * in one launch of 256 x 256 tiles, within the GEMM's tolerance of it.  No counterpart in the reference, whose 8-expert
+ * in one launch of 256-row tiles, within the GEMM's tolerance of it.  No counterpart in the reference, whose 8-expert
  * benchmark applies every expert to every token (README.md:16-18); this is the op a
  * router-driven Mixtral layer needs. */
 int tuna_matmul_grouped(const void *q, const void *x, const void *code, const void *absmax,
@@ -288,7 +292,7 @@ int tuna_blockwise_table_entry(int i, int *m, int *n_lo, int *n_hi, int *k, int 
  * configs.cu:56-3331 by a table lookup on (m, n-bucket, k) with a derived fallback.
  * Runs on the host only (no device needed).  Returns 1 in *from_table when the shape
  * hit a tuned entry.  A call without a config runs it, except that the decode-batch kernel or the
- * narrow-row kernel's variants for any k (up to 64 tokens) or 256 x 256 tiles (from 65) take its place where they are predicted to be faster
+ * narrow-row kernel's variants for any k (up to 64 tokens) or 256-row tiles (from 65) take its place where they are predicted to be faster
  * (tuna_describe_launch says so). */
 int tuna_select_config(int m, int n, int k, tuna_gemm_config *cfg, int *from_table);
 /* The config tuna_matmul_ex(cfg = NULL, decode_mode) runs: the table lookup above for

@@ -232,13 +232,49 @@ static int planned_cus()
     return kMaxCus;
 }
 
-static bool wide_balance_pays(int m, int n, int k);
+static bool wide_shares_last(int m, int n, int k);
 static bool stream_applies(const tuna_gemm_config &c, int n, int decode);
 static bool plan_wide_dense(int m, int n, int k, int split, WidePlan *plan)
 {
+    // tiles of 256 tokens, the last of 129 ... 256 among them; 1 ... 128 tokens behind them are tiles of another kind
     memset(plan, 0, sizeof(*plan));
-    plan->args.m = m, plan->args.k = k, plan->args.n_groups = 1, plan->args.tok_count[0] = n;
+    WideArgs &a = plan->args;
+    a.m = m, a.k = k;
+    const int large = (int)(((long long)n + 127) >> 8), full = large < 0x7fffffff >> 8 && large * 256 < n ? large * 256 : n;
+    if (large) a.g.tok_count[0] = full, a.g.width[0] = 256, a.n_groups = 1;
+    if (!large || full < n) {
+        const int g = a.n_groups++;
+        a.g.tok_begin[g] = large ? full : 0, a.g.tok_count[g] = n - a.g.tok_begin[g], a.g.width[g] = 128;
+    }
     return plan_gemm_wide(split, planned_cus(), plan);
+}
+
+// 256 x 256 tiles with waves_m 8 ... 16: of up to 16 * waves_m tokens each, the tokens divided evenly between as many tiles as that takes
+// (gemm_wide.hip, gemm_wide_whole.hip)
+static inline bool is_width(const tuna_gemm_config &c)
+{
+    return c.lds_tile_rows == 256 && c.token_tiles == 16 && c.rows_per_wave != 32 && c.waves_m >= 8 && c.waves_m <= 16;
+}
+struct WidthTiles {
+    int count, width, nt;  // token tiles, tokens of one, token tiles of 16 that it runs
+    WidthTiles(int n, int token_tiles)
+        : count(ceil_div(n, 16 * token_tiles)), width((ceil_div(n, count) + 15) / 16 * 16), nt(wide_token_tiles(width))
+    {
+    }
+};
+static int plan_width(int m, int n, int k, const tuna_gemm_config &c, int decode, WidePlan *plan)
+{
+    int rc = check_shape(m, n, k);
+    if (rc) return rc;
+    if (decode != TUNA_DECODE_GEMM) return fail(TUNA_ERR_UNSUPPORTED, "256-row tiles implement TUNA_DECODE_GEMM only");
+    const int steps = ceil_div(k, 64);
+    if (c.split_k < 0 || c.split_k > steps)
+        return fail(TUNA_ERR_UNSUPPORTED, "256-row tiles: split_k=%d must be in 0 (the last tiles shared between the compute units) .. %d", c.split_k, steps);
+    memset(plan, 0, sizeof(*plan));
+    WideArgs &a = plan->args;
+    a.m = m, a.k = k, a.n_groups = 1, a.g.tok_count[0] = n, a.g.width[0] = WidthTiles(n, c.waves_m).width;
+    if (!plan_gemm_wide(c.split_k, planned_cus(), plan)) return fail(TUNA_ERR_UNSUPPORTED, "m=%d n=%d k=%d has too many 256-row tiles for one launch", m, n, k);
+    return TUNA_OK;
 }
 
 static int plan_tiled(int m, int n, int k, const tuna_gemm_config &c, int decode, TiledPlan *plan)
@@ -274,7 +310,7 @@ static int plan_tiled(int m, int n, int k, const tuna_gemm_config &c, int decode
     a.steps_per_split = ceil_div(steps, c.split_k);
     if (wide) {
         plan->wide = true;
-        if (!plan_wide_dense(m, n, k, c.split_k == 1 && wide_balance_pays(m, n, k) ? 0 : c.split_k, &plan->wide_plan))
+        if (!plan_wide_dense(m, n, k, c.split_k == 1 && wide_shares_last(m, n, k) ? 0 : c.split_k, &plan->wide_plan))
             return fail(TUNA_ERR_UNSUPPORTED, "m=%d n=%d k=%d has too many 256 x 256 tiles for one launch", m, n, k);
         plan->ws_bytes = plan->wide_plan.ws_bytes;
         plan->n_counters = plan->wide_plan.n_counters;
@@ -315,6 +351,24 @@ static int launch_tiled(TiledPlan &tp, const void *q, const void *x, const void 
         e = launch_gemm_tiled(tp.args, tp.tile_rows, tp.tile_tokens, tp.mfma32, stream, blk_shift >= 0);
     }
     return e == hipSuccess ? TUNA_OK : hip_fail(e, "many-token gemm launch");
+}
+
+static int launch_width(WidePlan &plan, const void *q, const void *x, const void *code, const void *absmax, void *out, int epilogue,
+                        const void *residual, int blk_shift, bool static_ws, hipStream_t stream)
+{
+    WideArgs &a = plan.args;
+    a.q = static_cast<const uint8_t *>(q);
+    a.x = x;
+    a.code = static_cast<const float *>(code);
+    a.absmax = static_cast<const float *>(absmax);
+    a.out = out;
+    a.epilogue = epilogue;
+    a.residual = residual;
+    a.blk_shift = blk_shift < 0 ? 0 : blk_shift;
+    if (plan.ws_bytes)
+        if (const int rc = provide_workspace(static_ws, stream, plan.ws_bytes, plan.n_counters, &a.ws, &a.counters)) return rc;
+    const hipError_t e = launch_gemm_wide(plan, blk_shift >= 0, stream);
+    return e == hipSuccess ? TUNA_OK : hip_fail(e, "256-row tile gemm launch");
 }
 
 // lds_tile_rows -4: the decode-batch kernel (gemm_flow.hip), its k-steps divided into split_k shares
@@ -745,6 +799,126 @@ static bool wide_balance_pays(int m, int n, int k)
     return wide_balance_pays(t.large, t.small, t.steps);
 }
 
+// The same kernel's tiles of any width, and gemm_wide_whole.hip's, by a model read off 958 launches of 200 random shapes of 1024 ... 57344
+// rows and 65 ... 4096 tokens (with blocks of 64 and 128 943): on the 440 and 440 kept in profiles/launch_model_times.csv 2.9 and 3.8 per cent off on
+// average, their pick 1.004 and 1.003 x the best.  (Several kinds: 900 grouped launches, 5.)  A k-step costs its decode, and its token tiles the more the
+// larger a share of the compute units is at work, over the whole launch: the power limit lowers the clock of all; the end of a tile goes with its token tiles; a divided one is handed over, and shares that
+// cross tiles meet fewer of their neighbours' activations in the L2.
+struct WideKind {
+    long long tiles;
+    int nt;
+};
+struct WidthCosts {
+    double step, tokens, power, end, over, parts, sums, cross, ragged;
+};
+static const WidthCosts kWidthCosts[2] = {{0.3629, 0.04097, 0.02435, 0.5872, 7.453, 0.1832, 0.5656, 0.4398, 1.058},
+                                          {0.4656, 0.04306, 0.02143, 0.431, 7.898, 0.2, 0.6377, 0.557, 1.034}};
+// (kinds: the widest tiles first; split as in a config of such tiles)
+static double wide_kinds_time(const WideKind *kinds, int n_kinds, int steps, int split, bool blocks)
+{
+    const WidthCosts &c = kWidthCosts[blocks];
+    const double cus = kMaxCus;
+    auto run = [&](int i) { return split == 1 ? kinds[i].nt : wide_divided_token_tiles(kinds[i].nt); };
+    long long tiles = 0, weight = 0;
+    for (int i = 0; i < n_kinds; ++i) tiles += kinds[i].tiles, weight += kinds[i].tiles * wide_step_weight(run(i)) * steps;
+    auto busy = [&](double wgs) { return wgs / (ceil(wgs / cus) * cus); };  // share of the compute units at work, over all rounds
+    auto step_us = [&](int nt, double u) { return c.step + nt * (c.tokens + c.power * u * u); };
+    const int widest = run(0);
+    if (split == 1) {
+        // dealt out in order to the first compute unit that is free: `free_cus` of them at `now`, the others at `later`
+        double now = 0.0, later = 0.0;
+        long long free_cus = kMaxCus;
+        for (int i = 0; i < n_kinds; ++i) {
+            const double us = steps * step_us(run(i), busy((double)tiles)) + c.end * run(i);
+            long long left = kinds[i].tiles;
+            if (free_cus == kMaxCus && left >= kMaxCus) now += left / kMaxCus * us, left %= kMaxCus;
+            while (left > 0) {
+                if (left < free_cus) {
+                    free_cus -= left, later = later > now + us ? later : now + us;
+                    break;
+                }
+                left -= free_cus;
+                if (free_cus == kMaxCus) now += us;
+                else if (now + us <= later) now += us;
+                else {
+                    const double end = now + us;
+                    now = later, later = end, free_cus = kMaxCus - free_cus;
+                }
+            }
+        }
+        return (free_cus == kMaxCus ? now : later) * (n_kinds > 1 ? 1.045 : 1.0);  // (tiles of two kinds do not meet in step)
+    }
+    auto over = [&](double parts, double wgs) { return c.over + c.parts * widest * (parts > 2 ? parts - 2 : 0) + c.sums * widest * (wgs < cus ? wgs : cus) / cus; };
+    if (split > 1) {
+        const double wgs = (double)tiles * split;
+        double work = 0.0;
+        for (int i = 0; i < n_kinds; ++i) work += kinds[i].tiles * (steps * step_us(run(i), busy(wgs)) / split + c.end * run(i));
+        if (n_kinds > 1) return 1.09 * (ceil(wgs / cus) * work / tiles * c.ragged + c.end * widest * c.cross + over(split + 1, wgs));  // (shares cross tiles)
+        return ceil(wgs / cus) * work / tiles + over(split, wgs);
+    }
+    int whole, shares;
+    wide_balance(tiles, kinds[0].tiles, weight, wide_step_weight(widest), steps, kMaxCus, &whole, &shares);
+    double us = whole / kMaxCus * (steps * step_us(widest, 1.0) + c.end * widest);
+    if (!shares) return us;
+    const long long divided = tiles - whole;
+    const bool ragged = n_kinds > 1 || (shares % divided && divided % shares);
+    double work = 0.0;
+    for (int i = 0; i < n_kinds; ++i) work += (double)(kinds[i].tiles - (i ? 0 : whole)) * steps * step_us(run(i), shares / cus);
+    us += work / shares * (ragged ? c.ragged : 1.0) + c.end * widest * (ragged ? 1.0 + c.cross : 1.0);
+    return n_kinds > 1 || divided % shares ? us + over(ragged ? (double)shares / divided + 1.0 : (double)shares / divided, shares) : us;
+}
+// (a config's 256 x 256 tiles: the last 1 ... 128 tokens of a row of them are narrower ones)
+static double wide_width_time(int m, int n, int k, int split_k, int nblk)
+{
+    const WideTiles t(m, n, k);
+    WideKind kinds[2];
+    int n_kinds = 0;
+    if (t.large > 0) kinds[n_kinds++] = {(long long)t.large, wide_token_tiles(n < 256 ? n : 256)};
+    if (t.small > 0) kinds[n_kinds++] = {(long long)t.small, 8};
+    return wide_kinds_time(kinds, n_kinds, (int)t.steps, split_k, nblk > 0);
+}
+// Whether an unsplit config's 256 x 256 tiles are shared between the compute units in the end: as above, and from a quarter of a round on
+// by the model of any width (8832 x 3456 at 497 tokens, 70 tiles: 63 us whole, 59.5).
+static bool wide_shares_last(int m, int n, int k)
+{
+    const WideTiles t(m, n, k);
+    return wide_balance_pays(m, n, k) || (t.large + t.small > kMaxCus / 4 && t.large + t.small <= kMaxCus / 2 &&
+                                          wide_width_time(m, n, k, 0, 0) < wide_width_time(m, n, k, 1, 0));
+}
+static double width_time(int m, int n, int k, int token_tiles, int split, int nblk)
+{
+    const WidthTiles t(n, token_tiles);
+    const WideKind kind = {(long long)ceil_div(m, 256) * t.count, t.nt};
+    return wide_kinds_time(&kind, 1, ceil_div(k, 64), split, nblk > 0);
+}
+static const int kWidthSplits[7] = {1, 0, 2, 3, 4, 6, 8};
+// Whether so many tiles are divided so: not into parts of less than eight steps, and no more than 400.
+static bool width_split_sensible(long long tiles, int steps, int split)
+{
+    return split == 0 ? tiles > kMaxCus / 2 : split == 1 ? tiles >= 16 : tiles * split >= 16 && tiles * split <= 400 && steps / split >= 8;
+}
+// The launch of such tiles that takes least time, below *us, with partial sums that `room` holds.
+static bool best_width(int m, int n, int k, int nblk, const Room &room, tuna_gemm_config *width, double *us)
+{
+    bool found = false;
+    for (int tt = 16; tt >= 8; --tt) {
+        const WidthTiles t(n, tt);
+        if (t.nt != tt) continue;  // (that many token tiles, evenly divided, are narrower ones)
+        for (const int split : kWidthSplits) {
+            if (!width_split_sensible((long long)ceil_div(m, 256) * t.count, ceil_div(k, 64), split)) continue;
+            const double time = width_time(m, n, k, tt, split, nblk);
+            if (time >= *us) continue;
+            tuna_gemm_config c;
+            memset(&c, 0, sizeof(c));
+            c.rows_per_wave = 64, c.waves_m = tt, c.waves_k = 1, c.prefetch = 2, c.x_chunk = 64, c.token_tiles = 16, c.split_k = split, c.lds_tile_rows = 256;
+            WidePlan plan;
+            if (plan_width(m, n, k, c, TUNA_DECODE_GEMM, &plan) != TUNA_OK || !room.holds(plan.ws_bytes, plan.n_counters)) continue;
+            *width = c, *us = time, found = true;
+        }
+    }
+    return found;
+}
+
 // The split (as above; 1 where the launch then shares its last tiles by itself) that takes these tiles least time with
 // partial sums that `room` holds, and that time in *us; 0 if there are too few of them.
 static int wide_best_split(double large, double small, double steps, const Room &room, double *us)
@@ -1058,6 +1232,10 @@ static tuna_gemm_config derive_config(int m, int n, int k)
 // Whether config c can run the shape (the checks of the three planners).
 static bool config_runs(int m, int n, int k, const tuna_gemm_config &c)
 {
+    if (is_width(c)) {
+        WidePlan wp;
+        return plan_width(m, n, k, c, TUNA_DECODE_GEMM, &wp) == TUNA_OK;
+    }
     if (c.lds_tile_rows > 0) {
         TiledPlan tp;
         return plan_tiled(m, n, k, c, TUNA_DECODE_GEMM, &tp) == TUNA_OK;
@@ -1308,6 +1486,7 @@ double predicted_us(int m, int n, int k, const tuna_gemm_config &c, int nblk)
 {
     if (is_tall(c)) return tall_time(m, n, k, c.rows_per_wave / 16, c.split_k, nblk);
     if (is_broad(c)) return broad_time(m, n, k, c.rows_per_wave, c.token_tiles, c.split_k, nblk);
+    if (is_width(c)) return width_time(m, n, k, c.waves_m, c.split_k, nblk);
     if (is_flow(c)) return flow_time(ceil_div(m, 256), ceil_div(ceil_div(k, 64), 4), c.token_tiles, c.split_k);
     if (is_narrow_any(c) || is_narrow(c)) return narrow_time(m, n, k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles, nblk);
     if (c.lds_tile_rows == 256 && c.token_tiles == 16 && c.rows_per_wave != 32) {
@@ -1407,28 +1586,6 @@ static double many_token_price(int m, int n, int k, const tuna_gemm_config &c)
     return 0.0;
 }
 
-// What a launch without an explicit config runs from 65 tokens on: the selected config, or 256 x 256 tiles of gemm_wide.hip
-// in its place where their model is ahead of the grid cost model's price of that config by more than the models' error
-// (26624 x 5888 at 665 tokens 265 -> 219 us, 4096 x 14336 at 777 tokens 135 -> 117, 46848 x 5120 at 295 tokens 205 -> 175;
-// the table and the cost model were measured before that kernel and still pick the best of the other tiles).  Configs of
-// kernels that the model does not price - narrow rows, k split over lean workgroups - are left alone: they are picked
-// for shapes too small for such tiles.
-static bool wide_instead(int m, int n, int k, const tuna_gemm_config &c, const Room &room, tuna_gemm_config *wide)
-{
-    if (n <= 64 || is_narrow(c)) return false;
-    const WideTiles t(m, n, k);
-    const double price = many_token_price(m, n, k, c);
-    double us = 0.0;
-    const int split = price == 0.0 ? 0 : wide_best_split(t.large, t.small, t.steps, room, &us);
-    // (four parts and more: what their hand-over cost beyond the model with the kernel it was read off; at 0.98 of the measured
-    // time now)
-    if (!split || us * (split >= 4 ? 1.1 : 1.0) >= 0.96 * price) return false;
-    memset(wide, 0, sizeof(*wide));
-    wide->rows_per_wave = 64, wide->waves_m = 1, wide->waves_k = 1, wide->prefetch = 2, wide->x_chunk = 64, wide->token_tiles = 16;
-    wide->lds_tile_rows = 256, wide->split_k = split;
-    return config_runs(m, n, k, *wide);
-}
-
 // The table's buckets are the reference dispatcher's (kernel.cu:3022-3155) and every entry is tuned at the lower edge
 // of its bucket.  A token count inside a bucket often runs faster with the entry of the NEXT bucket, which is tuned for
 // more tokens per pass over the weights (8192 x 28672 at 17 tokens 79 -> 40 us, 8192 x 8192 at 20 tokens 23.8 -> 14.8,
@@ -1517,6 +1674,22 @@ static bool broad_instead(int m, int n, int k, const tuna_gemm_config &c, bool f
     return us < (x_mb > limit ? 0.78 : n > 512 || rounds > 2 ? 0.88 : 0.95) * price;
 }
 
+// From 65 tokens on, after all others: 256-row tiles of the width and the division that take least time by their model, where that is
+// below 0.97 (256 x 256 tiles, priced by the same model) or 0.96 of what is picked so far takes by its own.  Against the picks without it on 64
+// random shapes of 65 ... 4096 tokens 1.06 x, with scale blocks on 98 1.10 x (up to 1.49), groups on 150 1.08 x; slower is nothing
+// by more than the runs differ.
+static bool width_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, const Room &room, tuna_gemm_config *width)
+{
+    if (n <= 64) return false;
+    const bool wide = c.lds_tile_rows == 256 && c.token_tiles == 16 && c.rows_per_wave != 32;
+    double price;
+    if (wide) price = 0.97 * wide_width_time(m, n, k, c.split_k == 1 && wide_shares_last(m, n, k) ? 0 : c.split_k, 0);
+    else if (is_broad(c)) price = 0.96 * broad_time(m, n, k, c.rows_per_wave, c.token_tiles, c.split_k);
+    else if (is_narrow(c) || is_narrow_any(c)) price = from_table ? 0.0 : 0.96 * narrow_time(m, n, k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles);
+    else price = 0.96 * many_token_price(m, n, k, c);
+    return price > 12.0 && best_width(m, n, k, 0, room, width, &price);  // (12: less than any such launch takes)
+}
+
 // The config a launch without an explicit one runs: the selected one, or a newer kernel in its place - one whose partial
 // sums `room` holds.
 static void select_launch(int m, int n, int k, int decode, const Room &room, tuna_gemm_config *c)
@@ -1526,15 +1699,20 @@ static void select_launch(int m, int n, int k, int decode, const Room &room, tun
     tuna_gemm_config other;
     double flow_us = 0.0;
     if (decode != TUNA_DECODE_GEMM) return;
-    if (wide_instead(m, n, k, *c, room, &other) || flow_instead(m, n, k, *c, from_table != 0, room, &other, &flow_us)) *c = other;
+    if (flow_instead(m, n, k, *c, from_table != 0, room, &other, &flow_us)) *c = other;
     if (narrow_any_instead(m, n, k, *c, from_table != 0, flow_us, &other)) *c = other;
     if (tall_instead(m, n, k, *c, from_table != 0, flow_us, room, &other)) *c = other;
     if (broad_instead(m, n, k, *c, from_table != 0, flow_us, room, &other)) *c = other;
+    if (width_instead(m, n, k, *c, from_table != 0, room, &other)) *c = other;
 }
 
 // The checks of the planner `c` belongs to, for a decode mode.
 static int validate_for(int m, int n, int k, const tuna_gemm_config &c, int decode)
 {
+    if (is_width(c)) {
+        WidePlan wp;
+        return plan_width(m, n, k, c, decode, &wp);
+    }
     if (c.lds_tile_rows > 0) {
         TiledPlan tp;
         return plan_tiled(m, n, k, c, decode, &tp);
@@ -1880,6 +2058,11 @@ static int matmul_impl(const void *q, const void *x, const void *code, const voi
         const Room room = workspace_room(stream);
         return matmul_impl(q, x, code, absmax, out, m, n, k, cfg, decode, stream, epilogue, residual, false, &room);
     };
+    if (is_width(c)) {
+        WidePlan wp;
+        if ((rc = plan_width(m, n, k, c, decode, &wp))) return rc;
+        return or_with_less(launch_width(wp, q, x, code, absmax, out, epilogue, residual, -1, static_ws, stream));
+    }
     if (c.lds_tile_rows > 0) {
         TiledPlan tp;
         if ((rc = plan_tiled(m, n, k, c, decode, &tp))) return rc;
@@ -2051,28 +2234,61 @@ static int grouped_flow_shares(int m_group, int n_active, int nt, int k)
     return flow_best_shares((long long)ceil_div(m_group, 256) * n_active, ceil_div(ceil_div(k, 64), 4), nt, kRoomToGrow, &us);
 }
 
-// What the groups with more than `pass` tokens take as a launch each, or in one of 256 x 256 tiles (its split in *split, 0 if
-// that is no option or slower; its tiles in a): 6 us and the larger of 0.85 PFLOP/s and 3.5 TB/s apart, wide_time together.  (The
-// former is 0.85 of what dense calls take, 26 per cent off, on 90 random shapes of 65 ... 1200 tokens.  The latter a tenth higher made
-// the choices that changed 1.03 x slower, on 130 random launches of 48 to 400 tokens per group.)
-static double grouped_many_time(int m_group, int n_groups, int k, const int32_t *offsets, int pass, WideArgs *a, int *split, long long *large, long long *small)
+// What the groups with more than `pass` tokens take as a launch each, or in one of 256-row tiles (its split in *split, -1 if
+// that is no option or slower; its groups in a): 8 us and the larger of 0.95 PFLOP/s and 1.9 TB/s apart, wide_kinds_time together,
+// tiles as wide as that makes best.  (The former is what dense calls of 65 ... 100 tokens take: 21888 x 4224 at 68 33 us, 9728 x 7680 28.)
+static double grouped_many_time(int m_group, int n_groups, int k, const int32_t *offsets, int pass, WideArgs *a, int *split)
 {
-    a->m = m_group, a->k = k, a->n_groups = 0;
+    int many = 0;
     double apart = 0.0, together = 0.0;
+    *split = -1;
     for (int e = 0; e < n_groups; ++e) {
         const int cnt = offsets[e + 1] - offsets[e];
         if (cnt <= pass) continue;
         const double flops = 2.0 * m_group * cnt * k, bytes = 0.5 * m_group * k + 2.0 * cnt * ((double)m_group + k);
-        const double t_flops = flops / 0.85e9, t_bytes = bytes / 3.5e6;
-        apart += 6.0 + (t_flops > t_bytes ? t_flops : t_bytes);
-        a->tok_begin[a->n_groups] = offsets[e], a->tok_count[a->n_groups] = cnt, a->id[a->n_groups] = (unsigned char)e;
-        ++a->n_groups;
+        const double t_flops = flops / 0.95e9, t_bytes = bytes / 1.9e6;
+        apart += 8.0 + (t_flops > t_bytes ? t_flops : t_bytes);
+        ++many;
     }
-    count_wide_tiles(*a, large, small);
-    *split = a->n_groups > 1 ? wide_best_split((double)*large, (double)*small, ceil_div(k, 64), kRoomToGrow, &together) : 0;
-    if (*split && together < apart) return together;
-    *split = 0;
-    return apart;
+    if (many < 2) return apart;
+    const int row_tiles = ceil_div(m_group, 256), steps = ceil_div(k, 64);
+    int best = 0;
+    for (int tt = 16; tt >= 8; --tt) {
+        long long of[17] = {0}, tiles = 0;
+        for (int e = 0; e < n_groups; ++e) {
+            const int cnt = offsets[e + 1] - offsets[e];
+            if (cnt <= pass) continue;
+            const WidthTiles t(cnt, tt);
+            of[t.nt] += (long long)row_tiles * t.count, tiles += (long long)row_tiles * t.count;
+        }
+        WideKind kinds[9];
+        int n_kinds = 0;
+        for (int nt = 16; nt >= 8; --nt)
+            if (of[nt]) kinds[n_kinds++] = {of[nt], nt};
+        for (const int s : kWidthSplits) {
+            if (!width_split_sensible(tiles, steps, s)) continue;
+            // (up to 16 steps, where the model is at its worst - 5120 x 1024 on 157 to 1494 tokens 40 us, 53 measured: whole tiles go to
+            // the XCDs in turn, the widest ones first - the last tiles of 256 tokens are shared)
+            if (steps <= 16 && (tt < 16 || s != (tiles > kMaxCus / 2 ? 0 : 1))) continue;
+            const double us = wide_kinds_time(kinds, n_kinds, steps, s, false);
+            if (!best || us < together) best = tt, together = us, *split = s;
+        }
+    }
+    if (!best || together >= apart) {
+        *split = -1;
+        return apart;
+    }
+    a->m = m_group, a->k = k, a->n_groups = 0;
+    for (int nt = 16; nt >= 8; --nt)  // (the widest tiles first)
+        for (int e = 0; e < n_groups; ++e) {
+            const int cnt = offsets[e + 1] - offsets[e];
+            if (cnt <= pass) continue;
+            const WidthTiles t(cnt, best);
+            if (t.nt != nt) continue;
+            const int g = a->n_groups++;
+            a->g.tok_begin[g] = offsets[e], a->g.tok_count[g] = cnt, a->g.width[g] = t.width, a->g.id[g] = e;
+        }
+    return together;
 }
 
 // One launch of broad tiles for all groups with tokens, where broad_time of its workgroups - a row tile and up to 96 tokens of a
@@ -2099,8 +2315,7 @@ static bool grouped_broad_pays(int m_group, int n_groups, int k, const int32_t *
     if (groups->n > few) {
         WideArgs wide;
         int split;
-        long long large, small;
-        price += grouped_many_time(m_group, n_groups, k, offsets, 64, &wide, &split, &large, &small);
+        price += grouped_many_time(m_group, n_groups, k, offsets, 64, &wide, &split);
     }
     if (few) {
         if (!flow_best_shares((long long)ceil_div(m_group, 256) * few, ceil_div(ceil_div(k, 64), 4), ceil_div(few_tok, 16), kRoomToGrow, &us)) return false;
@@ -2185,20 +2400,17 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
         WidePlan plan;
         memset(&plan, 0, sizeof(plan));
         WideArgs &a = plan.args;
-        long long large, small;
         int split;
-        grouped_many_time(m_group, n_groups, k, offsets, kGroupedPassTokens, &a, &split, &large, &small);
-        const double steps = ceil_div(k, 64);
-        if (split) {
+        grouped_many_time(m_group, n_groups, k, offsets, kGroupedPassTokens, &a, &split);
+        if (split >= 0) {
             a.q = static_cast<const uint8_t *>(q);
             a.x = x;
             a.code = static_cast<const float *>(code);
             a.absmax = static_cast<const float *>(absmax);
             a.out = out;
-            const bool balance = split == 1 && wide_balance_pays((double)large, (double)small, steps);
-            rc = plan_gemm_wide(balance ? 0 : split, planned_cus(), &plan) ? TUNA_OK : TUNA_ERR_UNSUPPORTED;
+            rc = plan_gemm_wide(split, planned_cus(), &plan) ? TUNA_OK : TUNA_ERR_UNSUPPORTED;
             if (!rc && plan.ws_bytes) rc = provide_workspace(false, stream, plan.ws_bytes, plan.n_counters, &a.ws, &a.counters);
-            if (rc && balance)  // (a stream that is capturing, with too small a workspace: whole tiles)
+            if (rc && split != 1)  // (a stream that is capturing, with too small a workspace: whole tiles)
                 rc = plan_gemm_wide(1, planned_cus(), &plan) ? TUNA_OK : TUNA_ERR_UNSUPPORTED;
             if (!rc) {
                 const hipError_t e = launch_gemm_wide(plan, false, stream);
@@ -2542,10 +2754,11 @@ TUNA_EXPORT int tuna_quantize_blockwise(const void *w, const void *code, void *q
 // A config comes from the caller (tuna_matmul_blockwise_ex), from the table of tuned entries keyed by (m, token bucket,
 // k, block_size) (config_table.cpp, written by the tuner), or from the rules of derive_blockwise below.
 // ---------------------------------------------------------------------------------------
-enum BlockwiseFamily { kBlkNarrow = 0, kBlkMulti = 1, kBlkTiled = 2, kBlkMid = 3, kBlkFlow = 4, kBlkNarrowAny = 5, kBlkTall = 6, kBlkBroad = 7 };
+enum BlockwiseFamily { kBlkNarrow = 0, kBlkMulti = 1, kBlkTiled = 2, kBlkMid = 3, kBlkFlow = 4, kBlkNarrowAny = 5, kBlkTall = 6, kBlkBroad = 7, kBlkWidth = 8 };
 
 static BlockwiseFamily blockwise_family(const tuna_gemm_config &c)
 {
+    if (is_width(c)) return kBlkWidth;
     if (c.lds_tile_rows > 0) return kBlkTiled;
     if (is_flow(c)) return kBlkFlow;
     if (is_tall(c)) return kBlkTall;
@@ -2655,6 +2868,14 @@ static int run_blockwise(const BlockwiseCall &b, const tuna_gemm_config &c, hipS
         if (dry) return TUNA_OK;
         if ((rc = launch_broad(bp, b.q, b.x, b.code, b.absmax, b.out, TUNA_EPILOGUE_NONE, nullptr, false, st))) return rc;
         diag::count(diag::kBlockwiseBroad);
+        return TUNA_OK;
+    }
+    case kBlkWidth: {
+        WidePlan wp;
+        if ((rc = plan_width(m, n, k, c, TUNA_DECODE_GEMM, &wp))) return rc;
+        if (dry) return TUNA_OK;
+        if ((rc = launch_width(wp, b.q, b.x, b.code, b.absmax, b.out, TUNA_EPILOGUE_NONE, nullptr, shift, false, st))) return rc;
+        diag::count(diag::kBlockwiseTiled);
         return TUNA_OK;
     }
     case kBlkNarrowAny: {
@@ -2929,33 +3150,54 @@ static bool blockwise_tall_instead(const BlockwiseCall &b, const tuna_gemm_confi
     return !best_narrow_any(b.m, b.n, b.k, nblk, us, &any);
 }
 
+// What the grid cost model gives a many-token tile with scale blocks; 0 for one that it has no factor for.
+static double blockwise_tiled_price(const BlockwiseCall &b, const tuna_gemm_config &c)
+{
+    const int tokens = 16 * c.token_tiles;
+    for (const BlockwiseTile &t : kBlockwiseTiles)
+        if (t.rows == c.lds_tile_rows && t.tokens == tokens)
+            return kBlockwiseCostUs * b.k * blockwise_tile_cost(t, c.split_k, (long long)ceil_div(b.m, t.rows) * ceil_div(b.n, tokens) * c.split_k, b.k);
+    return 0.0;
+}
+
 // From 65 tokens on: broad tiles (gemm_broad.hip) where their model is ahead of the derived config's.  Of 170 random shapes
 // of 65 ... 2500 tokens with blocks of 64 and 128 it takes 68, 1.28 x faster (3712 x 16384 at 297 tokens 92 -> 57, 22016 x 4096 at 72
 // 44 -> 30; worst 0.93: 10496 x 12032 at 243); less trust in the model above 384 tokens, in several rounds and beyond the L2s.
 static bool blockwise_broad_instead(const BlockwiseCall &b, const tuna_gemm_config &c, const Room &room, tuna_gemm_config *broad)
 {
     if (b.n <= 64) return false;
-    const int nblk = b.k / b.block_size, tokens = 16 * c.token_tiles;
+    const int nblk = b.k / b.block_size;
     double price = 0.0;
     if (blockwise_family(c) == kBlkNarrow) {
         price = narrow_time(b.m, b.n, b.k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles, nblk);
     } else if (blockwise_family(c) == kBlkTiled) {
-        if (c.lds_tile_rows == 256 && tokens == 256) {
+        if (c.lds_tile_rows == 256 && 16 * c.token_tiles == 256) {
             const WideTiles t(b.m, b.n, b.k);
             // (between 129 and 384 tokens without the quarter for four parts and more, which that price exceeds the measured time by: 12672 x
             // 13056 at 254 with blocks of 128 took 122 us for 100, 76 such random shapes 1.14 x; below and above it makes up for what broad
             // launches take beyond their model)
             price = blockwise_wide_time(wide_time(t.large, t.small, t.steps, c.split_k == 1 && wide_balance_pays(b.m, b.n, b.k) ? 0 : c.split_k),
                                         b.n > 128 && b.n <= 384 ? std::min(c.split_k, 3) : c.split_k);
-        }
-        for (const BlockwiseTile &t : kBlockwiseTiles)
-            if (t.rows == c.lds_tile_rows && t.tokens == tokens)
-                price = kBlockwiseCostUs * b.k * blockwise_tile_cost(t, c.split_k, (long long)ceil_div(b.m, t.rows) * ceil_div(b.n, tokens) * c.split_k, b.k);
+        } else price = blockwise_tiled_price(b, c);
     }
     double us = 0.0;
     if (price < 6.0 || !best_broad(b.m, b.n, b.k, nblk, room, broad, &us)) return false;  // (as in broad_instead)
     const double rounds = ceil((double)ceil_div(b.m, broad->rows_per_wave) * ceil_div(b.n, 16 * broad->token_tiles) / kMaxCus);
     return us < (2e-6 * b.n * b.k > 32 ? 0.78 : b.n > 384 || rounds > 2 ? 0.86 : 0.95) * price;
+}
+
+// After all others, 256-row tiles as in width_instead.
+static bool blockwise_width_instead(const BlockwiseCall &b, const tuna_gemm_config &c, const Room &room, tuna_gemm_config *width)
+{
+    if (b.n <= 64) return false;
+    const int nblk = b.k / b.block_size;
+    const bool wide = blockwise_family(c) == kBlkTiled && c.lds_tile_rows == 256 && c.token_tiles == 16;
+    double price = 0.0;
+    if (wide) price = 0.97 * wide_width_time(b.m, b.n, b.k, c.split_k == 1 && wide_shares_last(b.m, b.n, b.k) ? 0 : c.split_k, nblk);
+    else if (is_broad(c)) price = 0.96 * broad_time(b.m, b.n, b.k, c.rows_per_wave, c.token_tiles, c.split_k, nblk);
+    else if (blockwise_family(c) == kBlkNarrow) price = 0.96 * narrow_time(b.m, b.n, b.k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles, nblk);
+    else if (blockwise_family(c) == kBlkTiled) price = 0.96 * blockwise_tiled_price(b, c);
+    return price > 12.0 && best_width(b.m, b.n, b.k, nblk, room, width, &price);
 }
 
 // Tuned entry for (m, n, k, block_size) if the table has one that can run the call, else the derived config.
@@ -2979,6 +3221,7 @@ static int select_blockwise(const BlockwiseCall &b, const Room &room, tuna_gemm_
     }
     const int rc = derive_blockwise(b, room, cfg);
     if (!rc && (blockwise_tall_instead(b, *cfg, room, &tall) || blockwise_broad_instead(b, *cfg, room, &tall))) *cfg = tall;
+    if (!rc && blockwise_width_instead(b, *cfg, room, &tall)) *cfg = tall;
     return rc;
 }
 
@@ -3145,6 +3388,14 @@ TUNA_EXPORT int tuna_config_footprint(int m, int n, int k, const tuna_gemm_confi
                                       size_t *workspace_bytes)
 {
     if (!cfg) return fail(TUNA_ERR_INVALID_ARG, "cfg is null");
+    if (is_width(*cfg)) {
+        WidePlan wp;
+        int rc = plan_width(m, n, k, *cfg, TUNA_DECODE_GEMM, &wp);
+        if (rc) return rc;
+        if (lds_bytes) *lds_bytes = wide_lds_bytes();
+        if (workspace_bytes) *workspace_bytes = wp.ws_bytes;
+        return TUNA_OK;
+    }
     if (cfg->lds_tile_rows > 0) {
         TiledPlan tp;
         int rc = plan_tiled(m, n, k, *cfg, TUNA_DECODE_GEMM, &tp);
@@ -3341,10 +3592,18 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
         const int at = is_narrow_any(w) && plan_narrow_any(m, n, k, w, decode_mode, &np) == TUNA_OK
                            ? describe_narrow_any(np, n, buf, len, " in place of ")
                        : is_flow(w) ? snprintf(buf, len, "gemm_flow_kernel<NT=%d> %d shares in place of ", w.token_tiles, w.split_k)
+                       : is_width(w) ? snprintf(buf, len, "gemm_wide_kernel<256 rows x %d tokens> split_k=%d in place of ", 16 * WidthTiles(n, w.waves_m).nt, w.split_k ? w.split_k : 1)
                        : is_broad(w) ? snprintf(buf, len, "gemm_broad_kernel<%d rows x %d tokens> split_k=%d in place of ", w.rows_per_wave, 16 * w.token_tiles, w.split_k)
                        : is_tall(w) ? snprintf(buf, len, "gemm_tall_kernel<%d rows,NT=%d> split_k=%d in place of ", w.rows_per_wave, w.token_tiles, w.split_k)
                                     : snprintf(buf, len, "gemm_wide_kernel<256 rows x 256 tokens> split_k=%d in place of ", w.split_k);
         return at < 0 || (size_t)at + 16 > len ? TUNA_OK : tuna_describe_launch(m, n, k, &c, decode_mode, buf + at, len - (size_t)at);
+    }
+    if (is_width(c)) {
+        WidePlan wp;
+        if ((rc = plan_width(m, n, k, c, decode_mode, &wp))) return rc;
+        snprintf(buf, len, "gemm_wide_kernel<256 rows x %d tokens> split_k=%d%s", 16 * wp.args.g.nt[0], c.split_k ? c.split_k : 1,
+                 !c.split_k && wp.args.n_shares ? ", last tiles shared" : "");
+        return TUNA_OK;
     }
     if (c.lds_tile_rows > 0) {
         TiledPlan tp;

@@ -29,6 +29,10 @@ __device__ __forceinline__ void load_async(u32x4 &dst, const u32x4 &rsrc, uint32
 {
     asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen" : "=v"(dst) : "v"(offset), "s"(rsrc), "s"(uniform));
 }
+__device__ __forceinline__ void load_async(u32x2 &dst, const u32x4 &rsrc, uint32_t offset, uint32_t uniform)
+{
+    asm volatile("buffer_load_dwordx2 %0, %1, %2, %3 offen" : "=v"(dst) : "v"(offset), "s"(rsrc), "s"(uniform));
+}
 __device__ __forceinline__ void load_async(uint32_t &dst, const u32x4 &rsrc, uint32_t offset, uint32_t uniform)
 {
     asm volatile("buffer_load_dword %0, %1, %2, %3 offen" : "=v"(dst) : "v"(offset), "s"(rsrc), "s"(uniform));

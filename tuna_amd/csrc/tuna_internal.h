@@ -148,10 +148,16 @@ struct TiledArgs {
     int blk_shift;        // scale-block variants: absmax is [m, k / (64 << blk_shift)], one scale per block of a row
 };
 
-// Launch arguments of the 256 x 256 many-token kernel (gemm_wide.hip): n_groups of a stack of matrices of m rows each,
-// matrix id[e] multiplying the activation rows tok_begin[e] .. + tok_count[e] - 1 (a dense GEMM is one group).  A tile is 256 rows x
-// up to 256 tokens of one group; tiles of more than 128 tokens ("large") are numbered first, group by group, row tile by
-// row tile, the token tiles of a row tile next to each other; then the groups' last tiles of 1 .. 128 tokens ("small").
+// Launch arguments of the many-token kernel with 256-row tiles (gemm_wide.hip): n_groups of a stack of matrices of m rows each,
+// matrix id[e] multiplying the activation rows tok_begin[e] .. + tok_count[e] - 1 (a dense GEMM is one group, or two: its full tiles
+// and the tokens behind them).  A group's tokens are divided into tok_tiles[e] tiles of `width[e]` each (the last may have fewer),
+// which run nt[e] token tiles of 16.  Tiles are numbered group by group, row tile by row tile, the token tiles of a row tile next to
+// each other.
+struct WideGroups {
+    int tok_begin[kMaxGroups], tok_count[kMaxGroups], tok_tiles[kMaxGroups], width[kMaxGroups];
+    int tile_end[kMaxGroups];            // tiles of the groups up to this one (INT_MAX behind the last group)
+    int id[kMaxGroups], nt[kMaxGroups];  // (ints: read through the scalar cache)
+};
 struct WideArgs {
     const uint8_t *q;
     const void *x;
@@ -165,14 +171,36 @@ struct WideArgs {
     int m, k, n_groups;
     int steps_total;     // ceil(k / 64)
     int row_tiles;       // of one group
-    int large, small;    // tiles of either kind
+    int tiles;           // of all groups
     int whole;           // tiles 0 .. whole - 1 are computed whole, one workgroup each
     int n_shares;        // the k-steps of the other tiles, laid end to end, are divided into this many equal shares (0: none)
+    unsigned share_each, share_rest;  // weight of those steps divided by n_shares, and what remains
     int slots;           // 2; 1 where every tile ends with a share, so that no share has parts of two; 0: no tile is divided
     int blk_shift;       // scale-block variants: absmax is [m, k / (64 << blk_shift)]
-    int tok_begin[kMaxGroups], tok_count[kMaxGroups];
-    unsigned char id[kMaxGroups];
+    unsigned weight_end[kMaxGroups];  // weight of the k-steps of the divided tiles of the groups up to this one (UINT_MAX behind the last)
+    WideGroups g;
 };
+
+// Weight of a k-step of nt token tiles in a share: the MFMAs, and the decode that does not depend on nt.
+__host__ __device__ inline unsigned wide_step_weight(int nt) { return (unsigned)nt + 5u; }
+// Token tiles that a tile of `tokens` tokens runs: 8 ... 16.
+inline int wide_token_tiles(int tokens) { return tokens <= 128 ? 8 : (tokens + 15) / 16; }
+// ... in a launch that divides tiles, whose kernel holds the even numbers (all nine are more code than its branches reach).
+inline int wide_divided_token_tiles(int nt) { return nt + (nt & 1); }
+
+// Shares of a launch whose last tiles are divided evenly between `cus` compute units, the tiles' k-steps weighing `weight`: as many
+// rounds of whole tiles of the first kind (`widest` of them, a step of `step` each) as leave between a quarter and one and a quarter
+// of such a tile's work per compute unit; that is shared, at most eight shares to a tile and of at least eight steps.
+inline void wide_balance(long long tiles, long long widest, long long weight, unsigned step, int steps_total, int cus, int *whole, int *n_shares)
+{
+    const double per_cu = (double)weight / ((double)step * steps_total * cus);
+    long long rounds = (long long)(per_cu - 0.25), shares = cus;
+    if (rounds > widest / cus) rounds = widest / cus;
+    if (!rounds && shares > 8 * tiles) shares = 8 * tiles;
+    if (!rounds && shares > weight / (8 * step)) shares = weight / (8 * step) + 1;
+    *whole = (int)(rounds * cus);
+    *n_shares = tiles > *whole ? (int)shares : 0;
+}
 
 // Bytes between the partial-sum slots: a tile's 256 KB and 4352 more.
 constexpr size_t kWideSlot = (size_t)256 * 256 * 4 + 4352;
@@ -359,12 +387,13 @@ hipError_t launch_gemm_tiled(const TiledArgs &args, int tile_rows, int tile_toke
 // 256 x 256 tile, one wave per SIMD: gemm_wide.hip, and gemm_wide32.hip with 32 x 32 x 16 MFMAs (reached through
 // launch_gemm_tiled)
 size_t wide_lds_bytes();
-// Fills in the launch whose shape and groups plan->args holds (m, k, n_groups, tok_begin, tok_count, id).  split: 0 = the
-// last rounds of tiles balanced over the compute units, 1 = every tile whole, else that many shares per tile.
+// Fills in the launch whose shape and groups plan->args holds (m, k, n_groups, tok_begin, tok_count, width, id; the groups with the
+// widest tiles first).  split: 0 = the last rounds of tiles balanced over the compute units, 1 = every tile whole, else that many
+// shares per tile.
 bool plan_gemm_wide(int split, int cus, WidePlan *plan);
-// Its tiles of more than 128 tokens and of 1 .. 128.
-void count_wide_tiles(const WideArgs &args, long long *large, long long *small);
 hipError_t launch_gemm_wide(const WidePlan &plan, bool scale_blocks, hipStream_t stream);
+// ... of undivided tiles (gemm_wide_whole.hip; with several groups no epilogue, and one scale per row)
+hipError_t launch_gemm_wide_whole(const WideArgs &args, bool scale_blocks, hipStream_t stream);
 // Fills in the launch whose shape and groups plan->args holds (m, k, n_groups, m_total, tok_begin, tok_count, id).
 bool plan_gemm_flow(int nt, int shares, FlowPlan *plan);
 hipError_t launch_gemm_flow(const FlowPlan &plan, bool scale_blocks, hipStream_t stream);

@@ -1,4 +1,4 @@
-"""The time models behind the choice between kernels (flow_time, narrow_time, tall_time, broad_time and wide_time of csrc/api.cpp): the launches
+"""The time models behind the choice between kernels (flow_time, narrow_time, tall_time, broad_time, wide_time and width_time of csrc/api.cpp): the launches
 they are read off, how far they are from them, and the fit of their coefficients.
 
     python -m tuna_amd.launch_models --measure times.csv    # on a GPU: random shapes, several launches each
@@ -148,8 +148,82 @@ def broad(r, c):
     return own[0] + (full + (1 if rest else 0)) * (own[1] + c[10] * rt * nt + scales) + work + over + c[11] * 1e-6 * n * m
 
 
+# a k-step's decode, its token tiles, those with every compute unit at work, a tile's end, hand-over, its parts, its sums, where shares
+# cross tiles: the ends, the steps
+WIDTH = (0.3629, 0.04097, 0.02435, 0.5872, 7.453, 0.1832, 0.5656, 0.4398, 1.058)
+WIDTH_BLOCKS = (0.4656, 0.04306, 0.02143, 0.431, 7.898, 0.2, 0.6377, 0.557, 1.034)
+
+
+def width_tiles(n, token_tiles):
+    """Tiles that n tokens make at up to 16 * token_tiles each, and the token tiles of 16 that one runs."""
+    count = _cd(n, 16 * token_tiles)
+    tokens = _cd(_cd(n, count), 16) * 16
+    return count, max(8, tokens // 16)
+
+
+def kinds_time(kinds, steps, split, c):
+    """Tiles of several kinds, (number, token tiles of 16), the widest first."""
+    if split != 1:  # (the kernel that divides tiles runs even numbers)
+        kinds = [(t, nt + nt % 2) for t, nt in kinds]
+    tiles, widest, several = sum(t for t, _ in kinds), kinds[0][1], len(kinds) > 1
+
+    def busy(workgroups):  # share of the compute units at work, over all rounds
+        return workgroups / (_cd(workgroups, CUS) * CUS)
+
+    def step(nt, u):
+        return c[0] + nt * (c[1] + c[2] * u * u)
+
+    def over(parts, workgroups):
+        return c[4] + c[5] * widest * max(0, parts - 2) + c[6] * widest * min(workgroups, CUS) / CUS
+
+    if split == 1:
+        now, later, free = 0.0, 0.0, CUS
+        for left, nt in kinds:
+            us = steps * step(nt, busy(tiles)) + c[3] * nt
+            if free == CUS and left >= CUS:
+                now, left = now + left // CUS * us, left % CUS
+            while left > 0:
+                if left < free:
+                    free, later = free - left, max(later, now + us)
+                    break
+                left -= free
+                if free == CUS or now + us <= later:
+                    now += us
+                else:
+                    now, later, free = later, now + us, CUS - free
+        return (now if free == CUS else later) * (1.045 if several else 1.0)
+    if split > 1:
+        wgs = tiles * split
+        work = sum(t * (steps * step(nt, busy(wgs)) / split + c[3] * nt) for t, nt in kinds)
+        if several:
+            return 1.09 * (_cd(wgs, CUS) * work / tiles * c[8] + c[3] * widest * c[7] + over(split + 1, wgs))
+        return _cd(wgs, CUS) * work / tiles + over(split, wgs)
+    # as many rounds of whole tiles as wide_balance of csrc/tuna_internal.h leaves, the others shared
+    weight, own = sum(t * (nt + 5) * steps for t, nt in kinds), widest + 5
+    rounds, shares = min(int(weight / (own * steps * CUS) - 0.25), kinds[0][0] // CUS), CUS
+    if not rounds:
+        shares = min(shares, 8 * tiles)
+        if shares > weight // (8 * own):
+            shares = weight // (8 * own) + 1
+    whole = rounds * CUS
+    us = rounds * (steps * step(widest, 1.0) + c[3] * widest)
+    if tiles <= whole:
+        return us
+    divided = tiles - whole
+    ragged = several or (shares % divided and divided % shares)
+    work = sum((t - (0 if i else whole)) * steps * step(nt, shares / CUS) for i, (t, nt) in enumerate(kinds))
+    us += work / shares * (c[8] if ragged else 1.0) + c[3] * widest * (1.0 + c[7] if ragged else 1.0)
+    return us + over(shares / divided + (1.0 if ragged else 0.0), shares) if several or divided % shares else us
+
+
+def width(r, c):
+    count, nt = width_tiles(r["n"], r["token_tiles"])
+    return kinds_time([(_cd(r["m"], 256) * count, nt)], _cd(r["k"], 64), r["split"], c)
+
+
 MODELS = {"flow": (flow, FLOW), "narrow": (narrow, NARROW), "narrow blocks": (narrow, NARROW_BLOCKS), "wide": (wide, WIDE),
-          "tall": (tall, TALL), "tall blocks": (tall, TALL_BLOCKS), "broad": (broad, BROAD), "broad blocks": (broad, BROAD_BLOCKS)}
+          "tall": (tall, TALL), "tall blocks": (tall, TALL_BLOCKS), "broad": (broad, BROAD), "broad blocks": (broad, BROAD_BLOCKS),
+          "width": (width, WIDTH), "width blocks": (width, WIDTH_BLOCKS)}
 
 
 def config_of(r):
@@ -162,6 +236,9 @@ def config_of(r):
         d = dict(rows_per_wave=r["rows"], waves_m=1, waves_k=8, split_k=r["split"], prefetch=2, x_chunk=64, lds_tile_rows=-6)
     elif r["kind"] in ("broad", "broad blocks"):
         d = dict(rows_per_wave=r["rows"], waves_m=2, waves_k=4, split_k=r["split"], prefetch=2, x_chunk=256, lds_tile_rows=-7)
+    elif r["kind"] in ("width", "width blocks"):
+        d = dict(rows_per_wave=64, waves_m=r["token_tiles"], waves_k=1, split_k=r["split"], prefetch=2, x_chunk=64, lds_tile_rows=256)
+        return GemmConfig.from_dict(dict(d, token_tiles=16, xcd_swizzle=0))
     elif r["kind"] == "wide":
         d = dict(rows_per_wave=64, waves_m=1, waves_k=1, split_k=r["split"], prefetch=2, x_chunk=64, lds_tile_rows=256)
     else:
@@ -194,6 +271,19 @@ def launches(kind, rng, per_shape):
         tiles = _cd(m, 256) * _cd(n, 256)
         splits = [s for s in (1, 2, 3, 4, 6, 8) if s == 1 or (tiles * s <= 400 and _cd(k, 64) / s >= 8)]
         return [row(m, n, k, token_tiles=16, split=s) for s in rng.sample(splits, min(per_shape, len(splits)))]
+    if kind in ("width", "width blocks"):
+        block = rng.choice((64, 128)) if kind == "width blocks" else 0
+        while True:
+            m, n = 64 * round(_log_uniform(rng, 16, 896)), round(_log_uniform(rng, 65, 4096))
+            k = 256 * round(_log_uniform(rng, 4, 112)) if block else 64 * round(_log_uniform(rng, 16, 448))
+            fit = []
+            for nt in range(8, 17):
+                count, own = width_tiles(n, nt)
+                tiles = _cd(m, 256) * count
+                fit += [(nt, s) for s in (0, 1, 2, 3, 4, 6, 8) if own == nt and
+                        (tiles > CUS / 2 if s == 0 else tiles >= 24 if s == 1 else tiles * s <= 400 and _cd(k, 64) / s >= 8)]
+            if fit and 2.0 * m * n * k <= 6e11:
+                return [row(m, n, k, block, token_tiles=nt, split=s) for nt, s in rng.sample(fit, min(per_shape, len(fit)))]
     lo, hi = (6, 390) if kind == "flow" else (0.5, 400) if kind.startswith(("tall", "broad")) else (0.5, 100)
     unit = 256 if kind.endswith("blocks") else 8
     while True:
@@ -260,12 +350,12 @@ def _timer():
     return time
 
 
-def measure(path, shapes, per_shape, seed, log=print):
+def measure(path, shapes, per_shape, seed, log=print, kinds=tuple(MODELS)):
     time, rng = _timer(), random.Random(seed)
     with open(path, "w", newline="") as f:
         w = csv.DictWriter(f, FIELDS)
         w.writeheader()
-        for kind in MODELS:
+        for kind in kinds:
             for i in range(shapes):
                 for r in launches(kind, rng, per_shape):
                     w.writerow(dict(r, us=time(r)))
@@ -323,10 +413,11 @@ def main(argv=None):
     ap.add_argument("--again", metavar="KIND", help="time the launches of one kind in the file again")
     ap.add_argument("--shapes", type=int, default=100, help="random shapes per model")
     ap.add_argument("--per-shape", type=int, default=4, help="launches per shape")
+    ap.add_argument("--kinds", default=",".join(MODELS), help="which models, for --measure")
     ap.add_argument("--seed", type=int, default=1)
     a = ap.parse_args(argv)
     if a.measure:
-        return measure(a.csv, a.shapes, a.per_shape, a.seed, log=lambda s: print(s, flush=True))
+        return measure(a.csv, a.shapes, a.per_shape, a.seed, log=lambda s: print(s, flush=True), kinds=a.kinds.split(","))
     if a.again:
         return measure_again(a.csv, a.again, log=lambda s: print(s, flush=True))
     rows = read(a.csv)
