@@ -801,7 +801,7 @@ static bool wide_balance_pays(int m, int n, int k)
 
 // The same kernel's tiles of any width, and gemm_wide_whole.hip's, by a model read off 958 launches of 200 random shapes of 1024 ... 57344
 // rows and 65 ... 4096 tokens (with blocks of 64 and 128 943): on the 440 and 440 kept in profiles/launch_model_times.csv 2.9 and 3.8 per cent off on
-// average, their pick 1.004 and 1.003 x the best.  (Several kinds: 900 grouped launches, 5.)  A k-step costs its decode, and its token tiles the more the
+// average, their pick 1.004 and 1.003 x the best.  (Several kinds: 900 grouped launches, 4.)  A k-step costs its decode, and its token tiles the more the
 // larger a share of the compute units is at work, over the whole launch: the power limit lowers the clock of all; the end of a tile goes with its token tiles; a divided one is handed over, and shares that
 // cross tiles meet fewer of their neighbours' activations in the L2.
 struct WideKind {
@@ -825,28 +825,16 @@ static double wide_kinds_time(const WideKind *kinds, int n_kinds, int steps, int
     auto step_us = [&](int nt, double u) { return c.step + nt * (c.tokens + c.power * u * u); };
     const int widest = run(0);
     if (split == 1) {
-        // dealt out in order to the first compute unit that is free: `free_cus` of them at `now`, the others at `later`
-        double now = 0.0, later = 0.0;
-        long long free_cus = kMaxCus;
+        // in rounds of a tile per compute unit, each as long as its widest tile
+        double us = 0.0;
+        long long first = 0, seen = 0;
         for (int i = 0; i < n_kinds; ++i) {
-            const double us = steps * step_us(run(i), busy((double)tiles)) + c.end * run(i);
-            long long left = kinds[i].tiles;
-            if (free_cus == kMaxCus && left >= kMaxCus) now += left / kMaxCus * us, left %= kMaxCus;
-            while (left > 0) {
-                if (left < free_cus) {
-                    free_cus -= left, later = later > now + us ? later : now + us;
-                    break;
-                }
-                left -= free_cus;
-                if (free_cus == kMaxCus) now += us;
-                else if (now + us <= later) now += us;
-                else {
-                    const double end = now + us;
-                    now = later, later = end, free_cus = kMaxCus - free_cus;
-                }
-            }
+            seen += kinds[i].tiles;
+            const long long rounds = seen > first ? (seen - first + kMaxCus - 1) / kMaxCus : 0;
+            us += rounds * (steps * step_us(run(i), busy((double)tiles)) + c.end * run(i));
+            first += rounds * kMaxCus;
         }
-        return (free_cus == kMaxCus ? now : later) * (n_kinds > 1 ? 1.045 : 1.0);  // (tiles of two kinds do not meet in step)
+        return us;
     }
     auto over = [&](double parts, double wgs) { return c.over + c.parts * widest * (parts > 2 ? parts - 2 : 0) + c.sums * widest * (wgs < cus ? wgs : cus) / cus; };
     if (split > 1) {
@@ -865,7 +853,8 @@ static double wide_kinds_time(const WideKind *kinds, int n_kinds, int steps, int
     double work = 0.0;
     for (int i = 0; i < n_kinds; ++i) work += (double)(kinds[i].tiles - (i ? 0 : whole)) * steps * step_us(run(i), shares / cus);
     us += work / shares * (ragged ? c.ragged : 1.0) + c.end * widest * (ragged ? 1.0 + c.cross : 1.0);
-    return n_kinds > 1 || divided % shares ? us + over(ragged ? (double)shares / divided + 1.0 : (double)shares / divided, shares) : us;
+    if (n_kinds > 1) return 1.03 * (us + over((double)shares / divided + 1.0, shares));
+    return divided % shares ? us + over(ragged ? (double)shares / divided + 1.0 : (double)shares / divided, shares) : us;
 }
 // (a config's 256 x 256 tiles: the last 1 ... 128 tokens of a row of them are narrower ones)
 static double wide_width_time(int m, int n, int k, int split_k, int nblk)

@@ -93,7 +93,10 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_groups_kernel(const
                                                                            void *a_out, int a_m, int a_k, const WideGroups a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    const int lane = threadIdx.x & 63, tile = wide_place();
+    // (the widest tiles come first: they go to the XCDs in turn, 32 at a time, so that each has its part of every width)
+    const int grid = (int)gridDim.x, xcd = (int)blockIdx.x & 7, local = (int)blockIdx.x >> 3, full = grid >> 8, rest = grid & 255;
+    const int lane = threadIdx.x & 63, tile = local < 32 * full ? (local >> 5) * 256 + xcd * 32 + (local & 31)
+                                                                 : 256 * full + xcd * (rest >> 3) + min(xcd, rest & 7) + local - 32 * full;
     const int tile_end = a.tile_end[lane], begin = a.tok_begin[lane], count = a.tok_count[lane], tiles = a.tok_tiles[lane], wid = a.width[lane],
               matrix = a.id[lane], tok_tiles16 = a.nt[lane];
     const int group = __builtin_popcountll(__ballot(tile_end <= tile));

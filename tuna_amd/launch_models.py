@@ -177,21 +177,13 @@ def kinds_time(kinds, steps, split, c):
         return c[4] + c[5] * widest * max(0, parts - 2) + c[6] * widest * min(workgroups, CUS) / CUS
 
     if split == 1:
-        now, later, free = 0.0, 0.0, CUS
-        for left, nt in kinds:
-            us = steps * step(nt, busy(tiles)) + c[3] * nt
-            if free == CUS and left >= CUS:
-                now, left = now + left // CUS * us, left % CUS
-            while left > 0:
-                if left < free:
-                    free, later = free - left, max(later, now + us)
-                    break
-                left -= free
-                if free == CUS or now + us <= later:
-                    now += us
-                else:
-                    now, later, free = later, now + us, CUS - free
-        return (now if free == CUS else later) * (1.045 if several else 1.0)
+        # in rounds of a tile per compute unit, each as long as its widest tile
+        us, first, seen = 0.0, 0, 0
+        for t, nt in kinds:
+            seen += t
+            rounds = max(0, _cd(seen - first, CUS))
+            us, first = us + rounds * (steps * step(nt, busy(tiles)) + c[3] * nt), first + rounds * CUS
+        return us
     if split > 1:
         wgs = tiles * split
         work = sum(t * (steps * step(nt, busy(wgs)) / split + c[3] * nt) for t, nt in kinds)
@@ -213,7 +205,9 @@ def kinds_time(kinds, steps, split, c):
     ragged = several or (shares % divided and divided % shares)
     work = sum((t - (0 if i else whole)) * steps * step(nt, shares / CUS) for i, (t, nt) in enumerate(kinds))
     us += work / shares * (c[8] if ragged else 1.0) + c[3] * widest * (1.0 + c[7] if ragged else 1.0)
-    return us + over(shares / divided + (1.0 if ragged else 0.0), shares) if several or divided % shares else us
+    if several:
+        return 1.03 * (us + over(shares / divided + 1.0, shares))
+    return us + over(shares / divided + (1.0 if ragged else 0.0), shares) if divided % shares else us
 
 
 def width(r, c):
