@@ -2229,10 +2229,12 @@ static int grouped_flow_shares(int m_group, int n_active, int nt, int k)
 static double grouped_many_time(int m_group, int n_groups, int k, const int32_t *offsets, int pass, WideArgs *a, int *split)
 {
     int many = 0;
+    bool few = false;
     double apart = 0.0, together = 0.0;
     *split = -1;
     for (int e = 0; e < n_groups; ++e) {
         const int cnt = offsets[e + 1] - offsets[e];
+        few = few || (cnt > 0 && cnt <= pass);
         if (cnt <= pass) continue;
         const double flops = 2.0 * m_group * cnt * k, bytes = 0.5 * m_group * k + 2.0 * cnt * ((double)m_group + k);
         const double t_flops = flops / 0.95e9, t_bytes = bytes / 1.9e6;
@@ -2256,9 +2258,10 @@ static double grouped_many_time(int m_group, int n_groups, int k, const int32_t 
             if (of[nt]) kinds[n_kinds++] = {of[nt], nt};
         for (const int s : kWidthSplits) {
             if (!width_split_sensible(tiles, steps, s)) continue;
-            // (up to 16 steps, where the model is at its worst - 5120 x 1024 on 157 to 1494 tokens 40 us, 53 measured: whole tiles go to
-            // the XCDs in turn, the widest ones first - the last tiles of 256 tokens are shared)
-            if (steps <= 16 && (tt < 16 || s != (tiles > kMaxCus / 2 ? 0 : 1))) continue;
+            // (up to 16 steps, with groups of up to `pass` tokens beside these: the last tiles of 256 tokens shared, as ever.  Not for
+            // speed - 5120 x 1024 on 157 to 1494 tokens takes 55 us so, 40 as whole tiles of 144 -, but a call of both kinds is what
+            // provides a stream's workspace where one is warmed up for a capture.)
+            if (steps <= 16 && few && (tt < 16 || s != (tiles > kMaxCus / 2 ? 0 : 1))) continue;
             const double us = wide_kinds_time(kinds, n_kinds, steps, s, false);
             if (!best || us < together) best = tt, together = us, *split = s;
         }
