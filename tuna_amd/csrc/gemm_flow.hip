@@ -125,15 +125,16 @@ __global__ __launch_bounds__(kFlowThreads, 2) void gemm_flow_kernel(const FlowAr
     // decode table at LDS address 0: entry (byte << 8) | ((lane & 31) << 2) - a copy per 32 lanes, in the lower 128 bytes of
     // every 256; the upper 128 hold the activation stages: row r of the ring of three stages at r * 256 + 128
     {
+        // (as in pair_table.hpp: a thread's entries share their low code, a wave's their high one)
         const int code_bits = (int)(uint32_t)__builtin_bit_cast(uint16_t, (f16)a.code[lane & 15]);
-#pragma unroll 4
-        for (int p = tid; p < 256 * 8; p += kFlowThreads) {
-            const int e = p >> 3;
-            const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute((e >> 4) << 2, code_bits);
-            const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute((e & 15) << 2, code_bits);
-            const uint32_t v = hi | (lo << 16);
-            *reinterpret_cast<u32x4 *>(smem + e * 256 + (p & 7) * 16) = u32x4{v, v, v, v};
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(((tid >> 3) & 15) << 2, code_bits) << 16;
+        const int high = __builtin_amdgcn_readfirstlane(tid >> 7);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t v = lo | (uint32_t)__builtin_amdgcn_readlane(code_bits, high + 2 * i);
+            *reinterpret_cast<u32x4 *>(smem + ((tid >> 3) + 32 * i) * 256 + (tid & 7) * 16) = u32x4{v, v, v, v};
         }
+        static_assert(kFlowThreads == 256, "eight entries of 128 bytes a thread");
     }
     unsigned char *const x_dst = smem + (tid >> 3) * 256 + 128 + (((tid & 7) ^ ((tid >> 3) & 7)) << 4);
     const int swz = (g ^ (i16 & 7)) << 4;

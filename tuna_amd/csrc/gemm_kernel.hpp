@@ -60,7 +60,7 @@
 //   * The store applies the fused epilogue (none / + residual / SiLU(gate) * up on
 //     interleaved rows), see epilogue.hpp.
 #pragma once
-#include "epilogue.hpp"
+#include "pair_table.hpp"
 
 namespace tuna {
 
@@ -478,25 +478,7 @@ __global__ __launch_bounds__(MAXT, MINW) void gemm_kernel(const GemmArgs a)
         if constexpr (DEC == TUNA_DECODE_GEMM) {
             // Lane l holds fp16(code[l % 16]) (kernel.cu:2800 rounds the codebook to fp16);
             // entries are gathered across lanes, no memory traffic.
-            // piece p: 16 bytes of row (p >> 4); all 64 slots of a row hold the same half2
-            const int code_bits = (int)f16_bits((f16)code_lane);
-            // four pieces per thread and round: the eight cross-lane reads of a round are in
-            // flight together instead of one LDS round trip per piece
-            for (int p0 = tid; p0 < kLutBytes / 16; p0 += 4 * nthreads) {
-                uint32_t v[4];
-    #pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const int e = (p0 + b * nthreads) >> 4;
-                    const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute((e >> 4) << 2, code_bits);
-                    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute((e & 15) << 2, code_bits);
-                    v[b] = hi | (lo << 16);
-                }
-    #pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const int p = p0 + b * nthreads;
-                    if (p < kLutBytes / 16) reinterpret_cast<u32x4 *>(lut)[p] = u32x4{v[b], v[b], v[b], v[b]};
-                }
-            }
+            build_pair_table(tid, nthreads, code_lane, [&](int p, const u32x4 &v) { reinterpret_cast<u32x4 *>(lut)[p] = v; });
         } else {
             if (tid < 16) reinterpret_cast<float *>(lut)[tid] = code_lane;
         }

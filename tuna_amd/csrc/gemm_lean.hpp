@@ -131,24 +131,7 @@ __global__ __launch_bounds__(MAXT, MINW) void gemm_lean_kernel(const uint8_t *a_
         wq[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(qp + (size_t)u * (WK * 128) + lb));
     qp += (size_t)U * (WK * 128);
     // ---- decode table (see gemm_kernel.hpp), built while the loads are in flight ------------
-    {
-        const int code_bits = (int)f16_bits((f16)code_lane);
-        for (int p0 = tid; p0 < kLutBytes / 16; p0 += 4 * nthreads) {
-            uint32_t v[4];
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int e = (p0 + b * nthreads) >> 4;
-                const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute((e >> 4) << 2, code_bits);
-                const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute((e & 15) << 2, code_bits);
-                v[b] = hi | (lo << 16);
-            }
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int p = p0 + b * nthreads;
-                if (p < kLutBytes / 16) reinterpret_cast<u32x4 *>(lut)[p] = u32x4{v[b], v[b], v[b], v[b]};
-            }
-        }
-    }
+    build_pair_table(tid, nthreads, code_lane, [&](int p, const u32x4 &v) { reinterpret_cast<u32x4 *>(lut)[p] = v; });
     f16x2 sc16[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {

@@ -262,24 +262,10 @@ __global__ __launch_bounds__(1024, 4) void gemm_multi_kernel(const MultiArgs a)
     }
 
     // ---- decode table (see gemm_kernel.hpp), built while the first loads are in flight --------
-    {
-        const int code_bits = (int)f16_bits((f16)code_lane);
-        for (int p0 = tid; p0 < kLutBytes / 16; p0 += 4 * 1024) {
-            uint32_t v[4];
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int e = (p0 + b * 1024) >> 4;
-                const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute((e >> 4) << 2, code_bits);
-                const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute((e & 15) << 2, code_bits);
-                v[b] = hi | (lo << 16);
-            }
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                if constexpr (LDSW) lds_store16_opaque(lut + (size_t)(p0 + b * 1024) * 16, u32x4{v[b], v[b], v[b], v[b]});
-                else reinterpret_cast<u32x4 *>(lut)[p0 + b * 1024] = u32x4{v[b], v[b], v[b], v[b]};
-            }
-        }
-    }
+    build_pair_table<1024>(tid, code_lane, [&](int p, const u32x4 &v) {
+        if constexpr (LDSW) lds_store16_opaque(lut + (size_t)p * 16, v);
+        else reinterpret_cast<u32x4 *>(lut)[p] = v;
+    });
     // chunk 0 of the first segment into buffer 0; one barrier publishes it and the table
     if constexpr (LDSW) {
         __builtin_amdgcn_s_waitcnt(wait_vmcnt(U));  // chunk 0 and the scales are older than the ring's U loads

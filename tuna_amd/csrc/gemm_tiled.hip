@@ -34,7 +34,7 @@
 //     slot), half as many MFMA instructions for the same bytes read from LDS.  The sums are the
 //     same products added in another order, so results differ from the 16 x 16 variants in the
 //     last bits of the fp32 accumulation only.
-#include "epilogue.hpp"
+#include "pair_table.hpp"
 
 namespace tuna {
 
@@ -168,17 +168,7 @@ __global__ __launch_bounds__(kTiledThreads, 2) void gemm_tiled_kernel(const Tile
     }
 
     // ---- decode table (as in the streaming kernel) ------------------------------------------
-    {
-        const int code_bits = (int)(uint32_t)__builtin_bit_cast(uint16_t, (f16)a.code[lane & 15]);
-#pragma unroll 4
-        for (int p = tid; p < kLutBytes / 16; p += kTiledThreads) {
-            const int e = p >> 4;
-            const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute((e >> 4) << 2, code_bits);
-            const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute((e & 15) << 2, code_bits);
-            const uint32_t v = hi | (lo << 16);
-            reinterpret_cast<u32x4 *>(lut)[p] = u32x4{v, v, v, v};
-        }
-    }
+    build_pair_table<kTiledThreads>(lut, tid, a.code[lane & 15]);
 
     // Accumulators as TM * TN float4 "slots" in both variants.  16 x 16 tiles: slot tm * TN + tn, element
     // v of lane l is weight row 16*tm + 4*(l/16) + v, token 16*tn + l%16.  32 x 32 tiles: tile t holds 16

@@ -1,7 +1,8 @@
 // What the kernels whose lanes hold one packed dword per 16-row tile (gemm_tall.hip, gemm_broad.hip) have in common: how they group
-// those tiles into loads, the decode table, and a tile's end - the exchange between parts of k and the output.
+// those tiles into loads, and a tile's end - the exchange between parts of k and the output.
 #pragma once
 #include "epilogue.hpp"
+#include "pair_table.hpp"
 
 namespace tuna {
 
@@ -16,23 +17,6 @@ struct Pieces {
     static __device__ __forceinline__ int width_at(int r) { return r < 4 * fours ? 4 : r < 4 * fours + 2 * twos ? 2 : 1; }
     static __device__ __forceinline__ int first_at(int r) { return r < 4 * fours ? r & ~3 : r < 4 * fours + 2 * twos ? 4 * fours : RT - 1; }
 };
-
-// The decode table at LDS address 0: each of the 256 pairs of codes for each bank (as in the streaming kernels).  A thread's entries
-// share their low code; the high ones are the same for a whole wave: seven instructions an entry of four banks instead of eighteen,
-// 0.7 -> 0.3 us of a launch's start with eight waves.
-template <int THREADS>
-__device__ __forceinline__ void build_pair_table(unsigned char *smem, int tid, float code_lane)
-{
-    static_assert(THREADS % 256 == 0 && kLutBytes % (16 * THREADS) == 0, "threads");
-    const int code_bits = (int)(uint32_t)__builtin_bit_cast(uint16_t, (f16)code_lane);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(((tid >> 4) & 15) << 2, code_bits) << 16;
-    const int high = __builtin_amdgcn_readfirstlane(tid >> 8);
-#pragma unroll
-    for (int i = 0; i < kLutBytes / (16 * THREADS); ++i) {
-        const uint32_t v = lo | (uint32_t)__builtin_amdgcn_readlane(code_bits, high + i * (THREADS / 256));
-        reinterpret_cast<u32x4 *>(smem)[tid + i * THREADS] = u32x4{v, v, v, v};
-    }
-}
 
 // Sums of a tile between its parts of k: each part's go to its slot of the workspace, and the last workgroup to arrive adds all of
 // them in k order.  Wave w holds the sums of row tiles w, w + WAVES .. of TILES; PB parts' loads are issued before the first is
