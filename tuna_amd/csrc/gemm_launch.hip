@@ -224,11 +224,12 @@ typedef void (*NarrowKernelFn)(const uint8_t *, const void *, const float *, con
                                const void *, int, int, int);
 struct NarrowVariant {
     int rows, wk, u, tt;
-    NarrowKernelFn fn, fn_perm;  // B fragments loaded per lane (up to 4 tokens) / contiguously and permuted
+    NarrowKernelFn fn[3];  // by narrow_fragments(n)
 };
-#define N(LW, WK, U) {16 * LW, WK, U, 1, gemm_narrow_kernel<LW, WK, U, false, 1>, gemm_narrow_kernel<LW, WK, U, true, 1>}
-#define NT(LW, WK, U, TT) {16 * LW, WK, U, TT, gemm_narrow_kernel<LW, WK, U, true, TT>, gemm_narrow_kernel<LW, WK, U, true, TT>}
-#define N24(WK, U) {24, WK, U, 1, gemm_narrow_kernel<2, WK, U, false, 1, false, 24>, gemm_narrow_kernel<2, WK, U, true, 1, false, 24>}
+#define EIGHT(LW) (LW > 1 ? 2 : 1)  // (16 rows: the second cross-lane read costs more than the line saves, 4.8 -> 4.95 us at 4096 x 4096)
+#define N(LW, WK, U) {16 * LW, WK, U, 1, {gemm_narrow_kernel<LW, WK, U, 0, 1>, gemm_narrow_kernel<LW, WK, U, EIGHT(LW), 1>, gemm_narrow_kernel<LW, WK, U, 1, 1>}}
+#define NT(LW, WK, U, TT) {16 * LW, WK, U, TT, {gemm_narrow_kernel<LW, WK, U, 1, TT>, gemm_narrow_kernel<LW, WK, U, 1, TT>, gemm_narrow_kernel<LW, WK, U, 1, TT>}}
+#define N24(WK, U) {24, WK, U, 1, {gemm_narrow_kernel<2, WK, U, 0, 1, false, 24>, gemm_narrow_kernel<2, WK, U, 2, 1, false, 24>, gemm_narrow_kernel<2, WK, U, 1, 1, false, 24>}}
 static const NarrowVariant kNarrow[] = {
     N(1, 4, 2),  N(1, 4, 4),  N(1, 4, 8),  N(1, 8, 2),  N(1, 8, 4),  N(1, 8, 8),  N(1, 16, 2), N(1, 16, 4), N(1, 16, 8),
     N(2, 4, 2),  N(2, 4, 4),  N(2, 4, 8),  N(2, 8, 2),  N(2, 8, 4),  N(2, 8, 8),  N(2, 16, 2), N(2, 16, 4), N(2, 16, 8),
@@ -248,7 +249,7 @@ static const NarrowVariant kNarrow[] = {
 #undef NT
 #undef N24
 static constexpr int kNumNarrow = sizeof(kNarrow) / sizeof(kNarrow[0]);
-static OptInFlag g_narrow_attr_done[16][kNumNarrow][2];
+static OptInFlag g_narrow_attr_done[16][kNumNarrow][3];
 
 static const NarrowVariant *find_narrow(int rows, int wk, int u, int tt)
 {
@@ -265,7 +266,7 @@ bool narrow_variant_exists(int rows, int waves_k, int prefetch, int token_tiles)
 void describe_narrow_launch(int rows, int waves_k, int prefetch, int token_tiles, int n, char *buf, size_t len)
 {
     snprintf(buf, len, "gemm_narrow_kernel<LW=%d,WK=%d,U=%d,PERM=%d,TT=%d%s>", (rows + 15) / 16, waves_k, prefetch,
-             (n > 4 || token_tiles > 1) ? 1 : 0, token_tiles, rows == 24 ? ",ROWS=24" : "");
+             narrow_perm(rows, token_tiles, n), token_tiles, rows == 24 ? ",ROWS=24" : "");
 }
 
 hipError_t launch_gemm_narrow(const NarrowArgs &args, int rows, int waves_k, int prefetch, int token_tiles, hipStream_t stream)
@@ -277,8 +278,8 @@ hipError_t launch_gemm_narrow(const NarrowArgs &args, int rows, int waves_k, int
     if (e != hipSuccess) return e;
     if (dev < 0 || dev >= 16) return hipErrorInvalidDevice;
     const int vi = (int)(v - kNarrow);
-    const int perm = args.n > 4;
-    const NarrowKernelFn fn = perm ? v->fn_perm : v->fn;
+    const int perm = narrow_fragments(args.n);
+    const NarrowKernelFn fn = v->fn[perm];
     if ((e = ensure_lds_opt_in(g_narrow_attr_done[dev][vi][perm], reinterpret_cast<const void *>(fn))) != hipSuccess) return e;
     const size_t lds = (size_t)kLutBytes + (size_t)waves_k * ((rows + 15) / 16) * token_tiles * 1024;
     const dim3 grid((unsigned)(args.m / rows), (unsigned)((args.n + 16 * token_tiles - 1) / (16 * token_tiles)), 1);
@@ -291,10 +292,10 @@ hipError_t launch_gemm_narrow(const NarrowArgs &args, int rows, int waves_k, int
 // through the ring with its weights).  block = 64 << blk_shift weights per scale.
 struct BlockwiseVariant {
     int rows, wk, u, tt;
-    NarrowKernelFn fn, fn_perm;
+    NarrowKernelFn fn[3];
 };
-#define B(LW, WK, U) {16 * LW, WK, U, 1, gemm_narrow_kernel<LW, WK, U, false, 1, true>, gemm_narrow_kernel<LW, WK, U, true, 1, true>}
-#define B2(LW, WK, U) {16 * LW, WK, U, 2, gemm_narrow_kernel<LW, WK, U, true, 2, true>, gemm_narrow_kernel<LW, WK, U, true, 2, true>}
+#define B(LW, WK, U) {16 * LW, WK, U, 1, {gemm_narrow_kernel<LW, WK, U, 0, 1, true>, gemm_narrow_kernel<LW, WK, U, EIGHT(LW), 1, true>, gemm_narrow_kernel<LW, WK, U, 1, 1, true>}}
+#define B2(LW, WK, U) {16 * LW, WK, U, 2, {gemm_narrow_kernel<LW, WK, U, 1, 2, true>, gemm_narrow_kernel<LW, WK, U, 1, 2, true>, gemm_narrow_kernel<LW, WK, U, 1, 2, true>}}
 static const BlockwiseVariant kBlockwise[] = {
     B(1, 4, 2), B(1, 8, 4), B(1, 16, 2), B(2, 8, 2), B(2, 8, 4), B(2, 16, 2), B(4, 4, 4), B(4, 8, 2), B(4, 8, 4), B(4, 16, 2),
     // two token tiles per workgroup: 17..32 tokens in one pass over the weights
@@ -302,6 +303,7 @@ static const BlockwiseVariant kBlockwise[] = {
 };
 #undef B
 #undef B2
+#undef EIGHT
 static constexpr int kNumBlockwise = sizeof(kBlockwise) / sizeof(kBlockwise[0]);
 
 static const BlockwiseVariant *find_blockwise(int rows, int waves_k, int prefetch, int tt)
@@ -374,9 +376,9 @@ hipError_t launch_gemm_blockwise(const NarrowArgs &args, int blk_shift, int rows
     const BlockwiseVariant *v = find_blockwise(rows, waves_k, prefetch, tt);
     if (!v || !blockwise_fits(*v, args.m, args.k)) return hipErrorInvalidConfiguration;
     const int vi = (int)(v - kBlockwise);
-    const int perm = args.n > 4;
-    const NarrowKernelFn fn = perm ? v->fn_perm : v->fn;
-    static OptInFlag done[16][kNumBlockwise][2];
+    const int perm = narrow_fragments(args.n);
+    const NarrowKernelFn fn = v->fn[perm];
+    static OptInFlag done[16][kNumBlockwise][3];
     if ((e = ensure_lds_opt_in(done[dev][vi][perm], reinterpret_cast<const void *>(fn))) != hipSuccess) return e;
     size_t lds = blockwise_base_lds(*v);
     const dim3 grid((unsigned)(args.m / v->rows), (unsigned)((args.n + 16 * v->tt - 1) / (16 * v->tt)), 1);

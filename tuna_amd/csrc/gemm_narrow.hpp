@@ -50,7 +50,7 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 // dwords of a kernel's arguments can be preloaded into scalar registers with the wave (built
 // with -amdgpu-kernarg-preload-count=16), which takes the argument fetch - a round trip to
 // memory - off the start of every wave.  A struct passed by value is not preloaded.
-template <int LW, int WK, int U, bool PERM, int TT, bool BLK = false, int ROWS = 16 * LW, bool ANY = false>
+template <int LW, int WK, int U, int PERM, int TT, bool BLK = false, int ROWS = 16 * LW, bool ANY = false>
 __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q, const void *a_x, const float *a_code,
                                                               const float *a_absmax, int a_k, int a_n, int a_n_it, int a_m,
                                                               void *a_out, int a_epilogue, const void *a_residual,
@@ -115,17 +115,36 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
     // B fragments: the MFMA wants lane (token i16, group g) to hold x[token][32*step + 8g ..], i.e.
     // four consecutive lanes on four different token rows - a wave instruction loading it that
     // way touches 16 rows with no two neighbouring lanes on one line and takes about three times
-    // as long in the address path as a contiguous one.  PERM: lane l LOADS token l / 4, 8-k group
-    // l % 4 (each quad of lanes reads 64 contiguous bytes) and the fragment goes to the lane that
-    // needs it by a cross-lane read (ds_bpermute: no LDS memory, no barrier) when it is consumed:
-    // lane (i16, g) takes the piece lane 4*i16 + g loaded.  Without PERM every lane loads its own
-    // fragment: cheaper for one to four tokens, where the clamped rows coincide anyway.
-    uint32_t xoff[TT];
+    // as long in the address path as a contiguous one.  PERM: neighbouring lanes LOAD neighbouring
+    // pieces and the fragment goes to the lane that needs it by a cross-lane read (ds_bpermute: no
+    // LDS memory, no barrier) when it is consumed.  Without PERM every lane loads its own fragment:
+    // cheaper for one to four tokens, where the clamped rows coincide anyway.
+    // kLines: the two k-steps of a double step load whole lines, 8 lanes each, the even slot tokens 0..7 of the
+    // tile, the odd one 8..15 with the halves of the line exchanged; one select per dword then puts the pieces of
+    // the even k-step into one register and those of the odd one into the other, and the reads across lanes do the
+    // rest.  A wave instruction that takes half a line of 16 tokens looks up twice the lines, and x, which every
+    // workgroup reads whole, is what bounds the loop (without its loads 6144 x 4096 at 16 tokens takes 5.0 us, without
+    // the decode 6.1): 6.4 -> 5.9 us.  A ring of one double step has no room for it - the even k-step waits for the odd
+    // slot's load - and 16-row tiles decode too little per fragment to hide the selects (4096 x 4096 at 16 tokens 5.05 ->
+    // 5.2 us; with a scale per block, whose refills are longer, 6.5 -> 6.35).
+    // kEight: at most eight tokens, one load a double step and no select; the accumulators' other columns repeat them and
+    // are never stored.  6144 x 4096 at 8 tokens 5.8 -> 5.45 us, 8192 x 8192 9.45 -> 8.6.
+    constexpr bool kEight = PERM == 2;
+    static_assert(!kEight || TT == 1, "one tile");
+    constexpr bool kLines = kEight || (PERM && U > 2 && (LW > 1 || BLK));
+    constexpr int kXOff = kLines && !kEight ? 2 : 1;                               // offsets of even and odd slots
+    const int xg[2] = {kLines ? lane & 7 : PERM ? lane & 3 : g, (lane & 7) ^ 4};  // 8-k group of the (double) step
+    uint32_t xoff[kXOff][TT];
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt)
-        xoff[tt] = PERM ? ((uint32_t)min(tt * 16 + (lane >> 2), a.n - 1 - tok0) * (uint32_t)a.k + (uint32_t)(lane & 3) * 8u) * 2u
-                        : ((uint32_t)min(tt * 16 + i16, a.n - 1 - tok0) * (uint32_t)a.k + (uint32_t)g * 8u) * 2u;
-    const int x_src = (i16 * 4 + g) << 2;  // byte address of the source lane for ds_bpermute
+#pragma unroll
+        for (int h = 0; h < kXOff; ++h) {
+            const int row = tt * 16 + (kLines ? 8 * h + (lane >> 3) : PERM ? lane >> 2 : i16);
+            xoff[h][tt] = ((uint32_t)min(row, a.n - 1 - tok0) * (uint32_t)a.k + (uint32_t)xg[h] * 8u) * 2u;
+        }
+    // byte address of the source lane for ds_bpermute (kLines: in even k-steps; in odd ones four lanes over)
+    const int x_src = (kEight ? (i16 & 7) * 8 + g : kLines ? (i16 & 7) * 8 + (i16 >> 3) * 4 + g : i16 * 4 + g) << 2;
+    const bool x_low = (lane & 4) == 0;
     // uniform: this wave's double step 0; one ring turn (U/2 double steps) further per group
     const unsigned char *qp = a.q + (size_t)wk * 256;
     const unsigned char *xp = reinterpret_cast<const unsigned char *>(a.x) + (size_t)tok0 * a.k * 2 + (size_t)wk * 128;
@@ -151,16 +170,16 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
                                                    0, (int)((uint32_t)(a.n - tok0) * (uint32_t)a.k * 2u), 0x00020000);
     }
     uint32_t q_at = lb + (uint32_t)wk * 256u, x_at = (uint32_t)wk * 128u;  // ANY: byte offsets of the turn being loaded
-    const int g8 = g * 8, xg8 = PERM ? (lane & 3) * 8 : g8;
+    const int g8 = g * 8;
 #define TUNA_NARROW_LOAD_ANY(u)                                                                 \
     {                                                                                          \
         const int rem_ = rem - ((u) >> 1) * (WK * 64) - ((u) & 1) * 32;                        \
         const uint32_t qo_ = g8 < rem_ ? q_at + (uint32_t)(((u) >> 1) * (WK * 256) + ((u) & 1) * 128) : kBeyond; \
-        const uint32_t xo_ = x_at + (uint32_t)(((u) >> 1) * (WK * 128) + ((u) & 1) * 64);      \
-        const bool in_ = xg8 < rem_;                                                           \
+        const uint32_t xo_ = x_at + (uint32_t)(((u) >> 1) * (WK * 128) + (kLines ? 0 : ((u) & 1) * 64)); \
+        const bool in_ = xg[(u) & (kXOff - 1)] * 8 < (kLines ? rem - ((u) >> 1) * (WK * 64) : rem_); \
         TUNA_NARROW_SCALES(u)                                                                  \
-        _Pragma("unroll") for (int tt = 0; tt < TT; ++tt) xq[u][tt] = __builtin_bit_cast(u32x4, \
-            __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, (int)(in_ ? xo_ + xoff[tt] : kBeyond), 0, 0)); \
+        if (!kEight || ((u) & 1) == 0) _Pragma("unroll") for (int tt = 0; tt < TT; ++tt) xq[u][tt] = __builtin_bit_cast(u32x4, \
+            __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, (int)(in_ ? xo_ + xoff[(u) & (kXOff - 1)][tt] : kBeyond), 0, 0)); \
         if constexpr (LW == 1) {                                                               \
             wq[u][0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(q_rsrc, (int)qo_, 0, 2); \
         } else if constexpr (LW == 2) {                                                        \
@@ -191,10 +210,10 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
         }
 #define TUNA_NARROW_LOAD(u)                                                                     \
     {                                                                                          \
-        const size_t xo_ = (size_t)((u) >> 1) * (WK * 128) + ((u) & 1) * 64;               \
+        const size_t xo_ = (size_t)((u) >> 1) * (WK * 128) + (kLines ? 0 : ((u) & 1) * 64);      \
         const size_t qo_ = (size_t)((u) >> 1) * (WK * 256) + ((u) & 1) * 128;              \
         TUNA_NARROW_SCALES(u)                                                                  \
-        _Pragma("unroll") for (int tt = 0; tt < TT; ++tt) xq[u][tt] = *reinterpret_cast<const u32x4 *>(xp + xo_ + xoff[tt]); \
+        if (!kEight || ((u) & 1) == 0) _Pragma("unroll") for (int tt = 0; tt < TT; ++tt) xq[u][tt] = *reinterpret_cast<const u32x4 *>(xp + xo_ + xoff[(u) & (kXOff - 1)][tt]); \
         if constexpr (LW == 1) {                                                               \
             wq[u][0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(qp + qo_ + lb)); \
         } else if constexpr (LW == 2) {                                                        \
@@ -224,7 +243,10 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
         }
     };
 #pragma unroll
-    for (int u = 0; u < U; ++u) TUNA_NARROW_REFILL(u)
+    for (int u = 0; u < U; ++u) {
+        TUNA_NARROW_REFILL(u)
+        if constexpr (kLines) __builtin_amdgcn_sched_barrier(0);  // in the order of the refills: waiting for a load is waiting for all before it
+    }
     next_turn();
     // BLK, scales through LDS: the first eight scales per thread of the workgroup's slice are requested here and
     // stored behind the table build; longer slices follow in further rounds
@@ -290,8 +312,22 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
         _Pragma("unroll") for (int tt = 0; tt < TT; ++tt)                                      \
         {                                                                                      \
             u32x4 xb_ = xq[u][tt];                                                             \
-            if constexpr (PERM) {                                                              \
-                _Pragma("unroll") for (int e = 0; e < 4; ++e) xb_[e] = (uint32_t)__builtin_amdgcn_ds_bpermute(x_src, (int)xq[u][tt][e]); \
+            if constexpr (kEight) {                                                            \
+                if (((u) & 1) == 0)                                                            \
+                    _Pragma("unroll") for (int e = 0; e < 4; ++e) {                            \
+                        xq[(u) | 1][tt][e] = (uint32_t)__builtin_amdgcn_ds_bpermute(x_src ^ 16, (int)xq[u][tt][e]); \
+                        xb_[e] = (uint32_t)__builtin_amdgcn_ds_bpermute(x_src, (int)xq[u][tt][e]); \
+                    }                                                                          \
+            } else if constexpr (PERM) {                                                       \
+                if (kLines && ((u) & 1) == 0) {                                                \
+                    const u32x4 xc_ = xq[(u) | 1][tt];                                         \
+                    _Pragma("unroll") for (int e = 0; e < 4; ++e) {                            \
+                        xq[(u) | 1][tt][e] = x_low ? xc_[e] : xb_[e];                          \
+                        xb_[e] = x_low ? xb_[e] : xc_[e];                                      \
+                    }                                                                          \
+                }                                                                              \
+                _Pragma("unroll") for (int e = 0; e < 4; ++e)                                  \
+                    xb_[e] = (uint32_t)__builtin_amdgcn_ds_bpermute(kLines && ((u) & 1) ? x_src ^ 16 : x_src, (int)xb_[e]); \
             }                                                                                  \
             b_[tt] = __builtin_bit_cast(f16x8, xb_);                                           \
         }                                                                                      \

@@ -345,6 +345,13 @@ hipError_t launch_gemm_mid(const GemmPlan &plan, int dev, int cus, hipStream_t s
 bool mid_describe(const GemmPlan &plan, char *buf, size_t len);
 // Name and template arguments of the kernel launch_gemm would start for `plan` on a device of `cus` CUs.
 void describe_gemm_launch(const GemmPlan &plan, int cus, char *buf, size_t len);
+// How the narrow-row kernel gets its B fragments at n tokens, an index of a variant's forms, and the kernel's PERM for each: every lane
+// its own (0), lines of eight tokens (2, one token tile and more than 16 rows), lines or half lines of sixteen (1).
+inline int narrow_fragments(int n) { return n <= 4 ? 0 : n <= 8 ? 1 : 2; }
+inline int narrow_perm(int rows, int token_tiles, int n)
+{
+    return token_tiles > 1 || n > 8 ? 1 : n <= 4 ? 0 : rows > 16 ? 2 : 1;
+}
 void describe_narrow_launch(int rows, int waves_k, int prefetch, int token_tiles, int n, char *buf, size_t len);
 // Narrow-row kernel (gemm_narrow.hpp): 16 or 32 rows per workgroup, all waves along k.
 struct NarrowArgs {
