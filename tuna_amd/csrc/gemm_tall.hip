@@ -67,6 +67,15 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tall_kernel(const uint8_t *a
     constexpr int LR = 2;      // table reads of two turns are on their way
     constexpr int T = 2 * RT;  // turns of a step: a row tile of a half each
     constexpr int ROWS = 16 * RT;
+    // kPairs: the loop goes two steps a turn with the odd one behind it, and the first loads are issued in the order of a step's.
+    // A wait for a load is a wait for all loads before it, and the compiler counts for the worst way into an instruction: with a
+    // branch around the second step (or another order of the first loads) each second step waited for weights requested one step
+    // ago, not two.  4096 x 11008 at 16 tokens 10.4 -> 9.9 us, at 37 13.4 -> 13.0, 4096 x 14336 at 64 19.3 -> 18.3; 8192 x 8192 at
+    // 16 with blocks of 64 13.6 -> 12.4.  Not where the registers don't allow it (the two steps are one block of instructions:
+    // 7 x 4 tiles spill 40 registers, 25 -> 53 us), and not with scale blocks above 64 rows, whose scales take two passes over the
+    // rows: there the loads that the branch lets go ahead of them are worth more (24576 x 4096 at 16 15.5 -> 17.2 us).
+    constexpr bool kPairs = RT * NT <= 20 && (!BLK || RT <= 4);
+    constexpr int XS = kPairs && RT > 6 ? RT - 3 : RT / 2;  // the turn in which the activations' exchange begins
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -198,7 +207,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tall_kernel(const uint8_t *a
         TALL_SCALE(u, tau + 1)                                                                                \
         TALL_LUT(u, tau + 2)                                                                                  \
         _Pragma("unroll") for (int t = 0; t < NT; ++t) if (tau == t * RT / (2 * NT)) TALL_READ_B(1, t)        \
-        _Pragma("unroll") for (int i = 0; i < 2 * NT; ++i) if (tau == RT / 2 + i * RT / (2 * NT)) {           \
+        _Pragma("unroll") for (int i = 0; i < 2 * NT; ++i) if (tau == XS + i * RT / (2 * NT)) {               \
             *reinterpret_cast<u32x4 *>(x_dst + i * 1024) = xr[i];                                             \
             TALL_LOAD_X(i)                                                                                    \
         }                                                                                                     \
@@ -218,43 +227,62 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tall_kernel(const uint8_t *a
     int s_sc = s_first + 8 * (int)turn;
     unsigned char *const scales = work + (size_t)kWaves * NT * 2048;
     const lds_u32 *const sc_lane = reinterpret_cast<const lds_u32 *>((uintptr_t)(uint32_t)(kLutBytes + kWaves * NT * 2048 + i16 * (SD * 4)));
-    if constexpr (BLK) {
-        // Four blocks of a row a lane, 64 rows a wave: the LDS banks of a store are those of 16 lanes and two or four pairs of
-        // row tiles.  (The last four of a row where four from here on would go beyond it: what is in front of the part or
-        // behind it isn't stored.)
-        const int nb = ((s1 - 1) >> a_blk_shift) + 1 - b0, quads = (nb + 3) >> 2;
-        constexpr int RG = (ROWS + 63) / 64, PIECES = 4;  // groups of 64 rows; loads on their way
-        for (int j0 = wave; j0 < RG * quads; j0 += kWaves * PIECES) {
-            u32x4 v[PIECES];
+    // Four blocks of a row a lane, 64 rows a wave: the LDS banks of a store are those of 16 lanes and two or four pairs of
+    // row tiles.  (The last four of a row where four from here on would go beyond it: what is in front of the part or
+    // behind it isn't stored.)
+    constexpr int RG = (ROWS + 63) / 64, PIECES = 4;  // groups of 64 rows; loads on their way
+    const int nb = BLK ? ((s1 - 1) >> a_blk_shift) + 1 - b0 : 0, pieces = RG * ((nb + 3) >> 2);
+    u32x4 sv[BLK ? PIECES : 1];
+    const auto load_scales = [&](int j0) {
 #pragma unroll
-            for (int i = 0; i < PIECES; ++i) {
-                const int j = min(j0 + kWaves * i, RG * quads - 1), rg = RG == 1 ? 0 : j & 1, c = min(b0 + 4 * (RG == 1 ? j : j >> 1), nblk - 4);
-                v[i] = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, ((64 * rg + lane) * nblk + c) * 4, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < PIECES; ++i) {
-                const int j = min(j0 + kWaves * i, RG * quads - 1), rg = RG == 1 ? 0 : j & 1, c = min(b0 + 4 * (RG == 1 ? j : j >> 1), nblk - 4) - b0;
-                const int row = 64 * rg + lane, r16 = row >> 4;
-                const int width = P::width_at(r16), first = P::first_at(r16);
-                const int in = row - 16 * first, lane16 = in / width, r = first + in % width;
-                if (row < ROWS)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const uint32_t bits = v[i][e];  // (a copy: a bit cast of a vector's element would take the first)
-                        if (c + e >= 0 && c + e < nb)
-                            *reinterpret_cast<f16 *>(scales + ((c + e) * 16 + lane16) * (SD * 4) + r * 2) = (f16)__builtin_bit_cast(float, bits);
-                    }
-            }
+        for (int i = 0; i < PIECES; ++i) {
+            const int j = min(j0 + kWaves * i, pieces - 1), rg = RG == 1 ? 0 : j & 1, c = min(b0 + 4 * (RG == 1 ? j : j >> 1), nblk - 4);
+            sv[BLK ? i : 0] = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, ((64 * rg + lane) * nblk + c) * 4, 0, 0);
         }
-    }
+    };
+    const auto store_scales = [&](int j0) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int j = min(j0 + kWaves * i, pieces - 1), rg = RG == 1 ? 0 : j & 1, c = min(b0 + 4 * (RG == 1 ? j : j >> 1), nblk - 4) - b0;
+            const int row = 64 * rg + lane, r16 = row >> 4;
+            const int width = P::width_at(r16), first = P::first_at(r16);
+            const int in = row - 16 * first, lane16 = in / width, r = first + in % width;
+            if (row < ROWS)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t bits = sv[BLK ? i : 0][e];  // (a copy: a bit cast of a vector's element would take the first)
+                    if (c + e >= 0 && c + e < nb)
+                        *reinterpret_cast<f16 *>(scales + ((c + e) * 16 + lane16) * (SD * 4) + r * 2) = (f16)__builtin_bit_cast(float, bits);
+                }
+        }
+    };
+    const auto stage_scales = [&](int j0) {
+        for (; j0 < pieces; j0 += kWaves * PIECES) {
+            load_scales(j0);
+            store_scales(j0);
+        }
+    };
+    if constexpr (BLK && kPairs) load_scales(wave);
+    if constexpr (BLK && !kPairs) stage_scales(wave);
     build_pair_table<kThreads>(smem, tid, code_lane);
     TALL_LOAD_W(1, 0)
-    TALL_LOAD_W(1, 1)
+    if constexpr (BLK && kPairs) {
+        store_scales(wave);
+        stage_scales(wave + kWaves * PIECES);
+    }
+    // (kPairs: the loads in the order of a step's, turn by turn: waiting for one of them is waiting for all before it)
+    if (!kPairs) TALL_LOAD_W(1, 1)
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 2 * NT; ++i) {
-        *reinterpret_cast<u32x4 *>(x_dst + i * 1024) = xr[i];
-        TALL_LOAD_X(i)
+    for (int tau = 0; tau < T; ++tau) {
+        if (kPairs && tau == T - 3) TALL_LOAD_W(1, 1)
+#pragma unroll
+        for (int i = 0; i < 2 * NT; ++i)
+            if (tau == XS + i * RT / (2 * NT)) {
+                *reinterpret_cast<u32x4 *>(x_dst + i * 1024) = xr[i];
+                TALL_LOAD_X(i)
+            }
+        if (kPairs) __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (BLK) {
         const lds_u32 *const from = sc_lane + ((s_sc >> a_blk_shift) - b0) * (16 * SD);
@@ -269,7 +297,15 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tall_kernel(const uint8_t *a
     TALL_LUT(0, 1)
 #pragma unroll
     for (int t = 0; t < NT; ++t) TALL_READ_B(0, t)
-    if (mine > 0) {
+    if constexpr (kPairs) {
+        for (int pairs = mine >> 1; pairs > 0; --pairs) {
+            TALL_STEP(0)
+            TALL_STEP(1)
+        }
+        if (mine & 1) {
+            TALL_STEP(0)
+        }
+    } else if (mine > 0) {
         int left = mine;
         do {
             TALL_STEP(0)
