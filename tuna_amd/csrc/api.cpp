@@ -573,8 +573,8 @@ static int launch_narrow_any(NarrowPlan &np, const void *q, const void *x, const
 
 static int describe_narrow_any(const NarrowPlan &p, int n, char *buf, size_t len, const char *then = "")
 {
-    return snprintf(buf, len, "gemm_narrow_kernel<LW=%d,WK=%d,U=%d,PERM=%d,TT=%d,any k>%s", p.rows / 16, p.waves_k, p.prefetch,
-                    narrow_perm(p.rows, p.token_tiles, n), p.token_tiles, then);
+    return snprintf(buf, len, "gemm_narrow_kernel<LW=%d,WK=%d,U=%d,PERM=%d,TT=%d,any k>%s", p.rows / 16, p.waves_k, p.prefetch, n > 4,
+                    p.token_tiles, then);
 }
 
 // The streaming-kernel branch of the derivation: 64 rows per wave, rings of 2 k-steps (those

@@ -126,12 +126,13 @@ __global__ __launch_bounds__(WK * 64) void gemm_narrow_kernel(const uint8_t *a_q
     // workgroup reads whole, is what bounds the loop (without its loads 6144 x 4096 at 16 tokens takes 5.0 us, without
     // the decode 6.1): 6.4 -> 5.9 us.  A ring of one double step has no room for it - the even k-step waits for the odd
     // slot's load - and 16-row tiles decode too little per fragment to hide the selects (4096 x 4096 at 16 tokens 5.05 ->
-    // 5.2 us; with a scale per block, whose refills are longer, 6.5 -> 6.35).
+    // 5.2 us; with a scale per block, whose refills are longer, 6.5 -> 6.35), nor do ANY's 64-row tiles, whose loads take an
+    // address and a check each (7552 x 1216 at 26 tokens 5.55 -> 5.77; its 32-row tiles: 6144 x 8960 at 14 11.9 -> 10.4).
     // kEight: at most eight tokens, one load a double step and no select; the accumulators' other columns repeat them and
     // are never stored.  6144 x 4096 at 8 tokens 5.8 -> 5.45 us, 8192 x 8192 9.45 -> 8.6.
     constexpr bool kEight = PERM == 2;
     static_assert(!kEight || TT == 1, "one tile");
-    constexpr bool kLines = kEight || (PERM && U > 2 && (LW > 1 || BLK));
+    constexpr bool kLines = kEight || (PERM && U > 2 && (ANY ? LW == 2 : LW > 1 || BLK));
     constexpr int kXOff = kLines && !kEight ? 2 : 1;                               // offsets of even and odd slots
     const int xg[2] = {kLines ? lane & 7 : PERM ? lane & 3 : g, (lane & 7) ^ 4};  // 8-k group of the (double) step
     uint32_t xoff[kXOff][TT];

@@ -11,28 +11,22 @@ namespace tuna {
 
 typedef void (*NarrowKernelFn)(const uint8_t *, const void *, const float *, const float *, int, int, int, int, void *, int,
                                const void *, int, int, int);
-// (fn[3] and on: with a scale per block of a row)
+// (fn[2], fn[3]: with a scale per block of a row)
 #define BLKV(LW, WK, U, TT, P) gemm_narrow_kernel<LW, WK, U, P, TT, true, 16 * LW, true>
-#define ROWV(LW, WK, U, TT, P) gemm_narrow_kernel<LW, WK, U, P, TT, false, 16 * LW, true>
-#define EIGHT(LW) (LW > 1 ? 2 : 1)  // (as the aligned variants)
-#define FORMS(V, LW, WK, U, TT, OWN, EIGHT) V(LW, WK, U, TT, OWN), V(LW, WK, U, TT, EIGHT), V(LW, WK, U, TT, 1)
-#define ANY1(LW, WK, U) {16 * LW, WK, U, 1, {FORMS(ROWV, LW, WK, U, 1, 0, EIGHT(LW)), FORMS(BLKV, LW, WK, U, 1, 0, EIGHT(LW))}}
-#define ANYT(LW, WK, U, TT) {16 * LW, WK, U, TT, {FORMS(ROWV, LW, WK, U, TT, 1, 1), FORMS(BLKV, LW, WK, U, TT, 1, 1)}}
+#define ANY1(LW, WK, U) {16 * LW, WK, U, 1, {gemm_narrow_kernel<LW, WK, U, 0, 1, false, 16 * LW, true>, gemm_narrow_kernel<LW, WK, U, 1, 1, false, 16 * LW, true>, BLKV(LW, WK, U, 1, 0), BLKV(LW, WK, U, 1, 1)}}
+#define ANYT(LW, WK, U, TT) {16 * LW, WK, U, TT, {gemm_narrow_kernel<LW, WK, U, 1, TT, false, 16 * LW, true>, gemm_narrow_kernel<LW, WK, U, 1, TT, false, 16 * LW, true>, BLKV(LW, WK, U, TT, 1), BLKV(LW, WK, U, TT, 1)}}
 static const struct {
     int rows, wk, u, tt;
-    NarrowKernelFn fn[6];  // by narrow_fragments(n)
+    NarrowKernelFn fn[4];  // B fragments loaded per lane (up to 4 tokens) / contiguously and permuted
 } kAny[] = {
     ANY1(1, 16, 4), ANY1(1, 16, 2), ANY1(2, 8, 4), ANY1(2, 8, 8), ANY1(4, 4, 4), ANY1(4, 8, 4),
     ANYT(2, 8, 2, 2), ANYT(2, 8, 4, 2), ANYT(4, 8, 2, 2), ANYT(2, 8, 2, 4), ANYT(4, 4, 2, 4),
 };
 #undef ANY1
 #undef ANYT
-#undef FORMS
-#undef EIGHT
-#undef ROWV
 #undef BLKV
 static constexpr int kNumAny = sizeof(kAny) / sizeof(kAny[0]);
-static OptInFlag g_any_attr_done[16][kNumAny][6];
+static OptInFlag g_any_attr_done[16][kNumAny][4];
 
 static int find_any(int rows, int wk, int u, int tt)
 {
@@ -50,7 +44,7 @@ bool narrow_any_variant_exists(int rows, int waves_k, int prefetch, int token_ti
 hipError_t launch_gemm_narrow_any(const NarrowArgs &args, int blk_shift, int rows, int waves_k, int prefetch, int token_tiles, int dev,
                                   hipStream_t stream)
 {
-    const int vi = find_any(rows, waves_k, prefetch, token_tiles), fi = narrow_fragments(args.n) + (blk_shift >= 0 ? 3 : 0);
+    const int vi = find_any(rows, waves_k, prefetch, token_tiles), fi = (args.n > 4 ? 1 : 0) + (blk_shift >= 0 ? 2 : 0);
     if (vi < 0 || dev < 0 || dev >= 16) return hipErrorInvalidConfiguration;
     const NarrowKernelFn fn = kAny[vi].fn[fi];
     const hipError_t e = ensure_lds_opt_in(g_any_attr_done[dev][vi][fi], reinterpret_cast<const void *>(fn));

@@ -345,7 +345,7 @@ hipError_t launch_gemm_mid(const GemmPlan &plan, int dev, int cus, hipStream_t s
 bool mid_describe(const GemmPlan &plan, char *buf, size_t len);
 // Name and template arguments of the kernel launch_gemm would start for `plan` on a device of `cus` CUs.
 void describe_gemm_launch(const GemmPlan &plan, int cus, char *buf, size_t len);
-// How the narrow-row kernel gets its B fragments at n tokens, an index of a variant's forms, and the kernel's PERM for each: every lane
+// How the narrow-row kernel (the variants for any k apart) gets its B fragments at n tokens, an index of a variant's forms, and the kernel's PERM for each: every lane
 // its own (0), lines of eight tokens (2, one token tile and more than 16 rows), lines or half lines of sixteen (1).
 inline int narrow_fragments(int n) { return n <= 4 ? 0 : n <= 8 ? 1 : 2; }
 inline int narrow_perm(int rows, int token_tiles, int n)
