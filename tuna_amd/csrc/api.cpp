@@ -1531,8 +1531,12 @@ static bool narrow_any_instead(int m, int n, int k, const tuna_gemm_config &c, b
 
 // Up to 64 tokens, after all of these: tall tiles where their model is ahead of the price of what is picked so far - that
 // kernel's model, or straight lines in MB of weights.  Against the picks without it on 1100 random shapes, as far as they
-// differ (465, 1.34 x): decode-batch picks 1.3 x, many-token tiles 1.9 x, general 1.6 x, narrow rows 1.07 x.  Lean and batched launches are
-// left alone, and so is what the table holds for one token tile a workgroup of narrow rows.
+// differ (465, 1.34 x): decode-batch picks 1.3 x, many-token tiles 1.9 x, general 1.6 x, narrow rows 1.07 x.  Lean launches and
+// batched ones with the weights through LDS: prices read off 920 random shapes with such a pick (one row tile more than there are
+// compute units costs a batched launch a second round: 33024 x 7168 at 9 tokens 40.6 -> 27.3 us).  They give way on 45 of 100 shapes;
+// there tall tiles are 1.23 x (up to 16 tokens, batched), 1.24 x (up to 32), 1.7 x (beyond), in place of lean launches 1.2 x; of
+// all 920 one takes more than 3 per cent longer (4.5).  What the table holds of these two goes by the older lines or is left alone, and
+// so is what it holds for one token tile a workgroup of narrow rows.
 static bool tall_instead(int m, int n, int k, const tuna_gemm_config &c, bool from_table, double flow_us, const Room &room, tuna_gemm_config *tall)
 {
     if (n > 64) return false;
@@ -1548,10 +1552,23 @@ static bool tall_instead(int m, int n, int k, const tuna_gemm_config &c, bool fr
         price = 0.95 * (11.5 + 0.65 * mb);
     } else {
         GemmPlan plan;
-        if (plan_gemm(m, n, k, c, TUNA_DECODE_GEMM, &plan) != TUNA_OK || launch_is_lean(plan, kMaxCus) || stream_applies(c, n, TUNA_DECODE_GEMM))
-            return false;
+        if (plan_gemm(m, n, k, c, TUNA_DECODE_GEMM, &plan) != TUNA_OK) return false;
+        if (stream_applies(c, n, TUNA_DECODE_GEMM)) return false;
+        const bool lean = launch_is_lean(plan, kMaxCus);
+        if (lean && from_table) return false;
         static const double kMid[5] = {0, 0.172, 0.22, 0.40, 0.37}, kGeneral[5] = {0, 0.286, 0.40, 0.55, 0.60};
-        if (!mid_applies(plan)) price = 0.95 * (7.0 + 1.5 * nt + kGeneral[nt] * mb);
+        // by token tiles - one, two, more -: launch, MB of weights, thousands of k (lean); launch, a round of row tiles, MB of weights,
+        // thousands of k of the rounds' tiles of 256 rows (batched, the weights through LDS)
+        static const double kLean[3][3] = {{5.526, 0.173, 0.0789}, {6.635, 0.3688, 0.016}, {4.075, 0.4873, 0.3234}};
+        static const double kMidLds[3][4] = {{1.152, 3.797, 0.1433, 3.878}, {4.614, 1.57, 0.1819, 5.2}, {3.927, 1.237, 0.5915, 3.99}};
+        const int at = std::min(nt, 3) - 1;
+        if (lean) {
+            price = kLean[at][0] + kLean[at][1] * mb + kLean[at][2] * 1e-3 * k;
+        } else if (!from_table && !plan.ws_bytes && mid_lds_applies(plan)) {
+            const double rounds = ceil_div(ceil_div(m, 64 * c.waves_m), kMaxCus), *p = kMidLds[at];
+            const double stream = p[2] * mb, tiles = p[3] * rounds * 0.25e-3 * c.waves_m * k;
+            price = p[0] + p[1] * rounds + std::cbrt(stream * stream * stream + tiles * tiles * tiles);
+        } else if (!mid_applies(plan)) price = 0.95 * (7.0 + 1.5 * nt + kGeneral[nt] * mb);
         else if (plan.ws_bytes) price = 0.88 * (9.0 + (nt > 1 ? nt : 0) + kMid[nt] * mb); // (split: with the hand-over of its sums)
         else price = 0.85 * (6.0 + (nt > 1 ? nt : 0) + kMid[nt] * mb);
     }
