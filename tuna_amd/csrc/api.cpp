@@ -2382,9 +2382,9 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
     // tokens) run as dense GEMMs of their own, each with the table's config for its token count - from 128 tokens a
     // group that is the many-token kernel at two to three times the rate, and a launch per group is nothing beside
     // hundreds of microseconds of matrix work.  (With an explicit config every group goes through the grouped kernel.)
-    // Several such groups become ONE launch of 256 x 256 tiles (gemm_wide.hip) where that is predicted to be faster than a
-    // launch each, priced at 6 us and the larger of 0.85 PFLOP/s and 3.5 TB/s: eight experts of 14336 x 4096 on 4096
-    // tokens leave the device half empty at the end of each of eight launches (706 us; 452 in one).
+    // Several such groups become ONE launch of 256-row tiles (gemm_wide.hip, gemm_wide_whole.hip) where that is predicted to be faster than a
+    // launch each, priced at 8 us and the larger of 0.95 PFLOP/s and 1.9 TB/s: eight experts of 14336 x 4096 on 4096
+    // tokens leave the device half empty at the end of each of eight launches (706 us; 406 in one).
     // Before either: one launch of broad tiles over all groups where its model is ahead of these two and of the decode-batch
     // kernel's for the groups of up to 64.
     constexpr int kGroupedPassTokens = 64;

@@ -13,7 +13,7 @@
 //     covers 2*LW block rows x 128 contiguous bytes.
 //   * Every wave has its own k range, so nothing of x is shared inside the workgroup: B fragments
 //     come straight from global memory (L2 hits: x is 128 KB per 16 tokens and read by everyone),
-//     one 16-byte load per lane and k-step, loaded contiguously and moved to the lane that needs
+//     one 16-byte load per lane and k-step, whole lines at a time, moved to the lane that needs
 //     them by cross-lane reads; no staging, no barrier before the main loop.  Token rows past n
 //     are clamped, not zeroed: a B column only feeds its own output column, which is never stored.
 //   * Weights and B fragments travel through one ring of U k-steps per wave.
