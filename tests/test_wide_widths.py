@@ -145,6 +145,26 @@ def test_configs_that_no_kernel_runs_are_refused():
         ops.validate_config(1024, 300, 1024, _cfg(16, 1), _lib.DECODE_DEQUANT)
 
 
+def test_launches_of_any_number_of_steps_are_planned():
+    """Shares are worked out in 32 bits, whole tiles are not: a launch of more steps than that is whole tiles, not refused."""
+    from tuna_amd import ops
+
+    for m, n, k in ((57344, 262144, 28672), (57344, 300000, 28672), (131072, 131072, 28672), (152064, 400000, 8192), (40960, 52000, 204800)):
+        for cfg in (_cfg256(1), _cfg256(2), _cfg(16, 1), _cfg(16, 2), _cfg(13, 1)):
+            ops.validate_config(m, n, k, cfg)
+            sums = ops.config_footprint(m, n, k, cfg)[1]  # (256 x 256 tiles, unsplit: the last ones behind whole rounds may be shared)
+            assert sums == 0 or (cfg.waves_m, cfg.split_k) == (1, 1) and sums < 1 << 28
+            assert ops.describe_launch(m, n, k, cfg).startswith("gemm_wide_kernel")
+        assert ops.describe_launch(m, n, k).startswith("gemm_wide_kernel")
+    for cfg in (_cfg256(1), _cfg256(3), _cfg(16, 1)):
+        ops.validate_config_blockwise(62912, 638681, 30720, 128, cfg)
+        ops.validate_config_blockwise(44800, 933118, 29184, 256, cfg)
+    # the most steps that are still divided, and one tile more
+    tiles, steps = 1024, 0x7fffffff // 21 // 1024
+    assert ops.config_footprint(256, 256 * tiles, 64 * steps, _cfg256(3))[1] > 0
+    assert ops.config_footprint(256, 256 * (tiles + 1), 64 * steps, _cfg256(3))[1] == 0
+
+
 def test_the_static_entry_point_refuses_no_pick_of_many_tokens_for_its_workspace():
     import random
 

@@ -234,20 +234,19 @@ bool plan_gemm_wide(int split, int cus, WidePlan *plan)
     a.row_tiles = ceil_div_i(a.m, kWideRows);
     a.n_shares = 0;
     long long tiles = 0, weight = 0, widest = 0;  // widest: tiles of the first group's kind
-    unsigned total[kMaxGroups];
+    long long total[kMaxGroups];
     for (int e = 0; e < a.n_groups; ++e) {
         a.g.tok_tiles[e] = ceil_div_i(a.g.tok_count[e], a.g.width[e]);
         const int nt = wide_token_tiles(a.g.tok_count[e] < a.g.width[e] ? a.g.tok_count[e] : a.g.width[e]);
         a.g.nt[e] = split == 1 ? nt : wide_divided_token_tiles(nt);
         const long long here = (long long)a.row_tiles * a.g.tok_tiles[e];
         tiles += here;
+        if (tiles > 0x7ffffffe) return false;
         weight += here * a.steps_total * wide_step_weight(a.g.nt[e]);
-        if (tiles > 0x7ffffffe || weight > 0x7fffffff) return false;
-        a.g.tile_end[e] = (int)tiles, total[e] = (unsigned)weight;
+        a.g.tile_end[e] = (int)tiles, total[e] = weight;
         if (a.g.nt[e] == a.g.nt[0]) widest += here;
     }
     if (tiles < 1) return false;
-    const unsigned per_tile = wide_step_weight(a.g.nt[0]) * (unsigned)a.steps_total;
     a.tiles = (int)tiles;
     a.whole = (int)tiles;
     if (split > 1 && tiles * split <= 0xffff) {  // (more shares are no use, and their bounds are worked out in 32 bits)
@@ -256,14 +255,16 @@ bool plan_gemm_wide(int split, int cus, WidePlan *plan)
     } else if (split == 0) {
         wide_balance(tiles, widest, weight, wide_step_weight(a.g.nt[0]), a.steps_total, cus, &a.whole, &a.n_shares);
     }
-    const unsigned skipped = (unsigned)a.whole * per_tile, divided_weight = (unsigned)weight - (a.n_shares ? skipped : 0);
+    const long long skipped = (long long)a.whole * a.steps_total * wide_step_weight(a.g.nt[0]);
+    long long divided_weight = a.n_shares ? weight - skipped : 0;
+    if (divided_weight > 0x7fffffff) a.whole = (int)tiles, a.n_shares = 0, divided_weight = 0;  // (as above: whole tiles have no such bounds)
     // (a share is at least a step of a wide tile, so that every share between a tile's first and last has a part of it)
     const int most = (int)(divided_weight / wide_step_weight(a.g.nt[0]));
     if (a.n_shares > most) a.n_shares = most > 0 ? most : 1;
-    if (a.n_shares) a.share_each = divided_weight / (unsigned)a.n_shares, a.share_rest = divided_weight % (unsigned)a.n_shares;
+    if (a.n_shares) a.share_each = (unsigned)(divided_weight / a.n_shares), a.share_rest = (unsigned)(divided_weight % a.n_shares);
     for (int e = 0; e < kMaxGroups; ++e) {
         if (e >= a.n_groups) a.g.tile_end[e] = 0x7fffffff, a.weight_end[e] = 0xffffffffu;
-        else a.weight_end[e] = a.n_shares && total[e] > skipped ? total[e] - skipped : 0u;
+        else a.weight_end[e] = a.n_shares && total[e] > skipped ? (unsigned)(total[e] - skipped) : 0u;
     }
     plan->grid = (unsigned)(a.n_shares ? a.n_shares : tiles);
     const long long divided = tiles - a.whole;
