@@ -134,6 +134,18 @@ def test_a_call_without_a_config_takes_the_width_that_is_predicted_to_be_fastest
     assert not ops.describe_launch(4096, 64, 14336).startswith("gemm_wide_kernel")
 
 
+# (whole tiles; split ones, of which a launch runs an even number of token tiles; shared last tiles)
+@pytest.mark.parametrize("m,n,k,token_tiles,split,ends", [(4096, 2000, 4096, 8, 1, "128 tokens> split_k=1 (gemm_wide_whole_kernel)"),
+                                                          (7552, 826, 21632, 13, 2, "224 tokens> split_k=2"),
+                                                          (10816, 351, 4032, 8, 0, "128 tokens> split_k=1, last tiles shared")])
+def test_a_pick_is_described_as_its_config_is(m, n, k, token_tiles, split, ends):
+    from tuna_amd import ops
+
+    pick, _, before = ops.describe_launch(m, n, k).partition(" in place of ")
+    assert before and pick == ops.describe_launch(m, n, k, _cfg(token_tiles, split))
+    assert pick.endswith(ends)
+
+
 def test_configs_that_no_kernel_runs_are_refused():
     from tuna_amd import _lib, ops
 

@@ -3588,6 +3588,15 @@ TUNA_EXPORT int tuna_config_table_derived_range(int i, int *from, int *to)
     return TUNA_OK;
 }
 
+// (the token tiles are the launch's: one that divides tiles runs an even number of them)
+static int describe_width(int m, int n, int k, const tuna_gemm_config &c, int decode, char *buf, size_t len, const char *suffix)
+{
+    WidePlan wp;
+    if (plan_width(m, n, k, c, decode, &wp) != TUNA_OK) return -1;
+    return snprintf(buf, len, "gemm_wide_kernel<256 rows x %d tokens> split_k=%d%s%s", 16 * wp.args.g.nt[0], c.split_k ? c.split_k : 1,
+                    !wp.args.n_shares ? " (gemm_wide_whole_kernel)" : c.split_k ? "" : ", last tiles shared", suffix);
+}
+
 TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config *cfg, int decode_mode, char *buf, size_t len)
 {
     if (!buf || len < 16) return fail(TUNA_ERR_INVALID_ARG, "buf is null or shorter than 16 bytes");
@@ -3601,19 +3610,12 @@ TUNA_EXPORT int tuna_describe_launch(int m, int n, int k, const tuna_gemm_config
         const int at = is_narrow_any(w) && plan_narrow_any(m, n, k, w, decode_mode, &np) == TUNA_OK
                            ? describe_narrow_any(np, n, buf, len, " in place of ")
                        : is_flow(w) ? snprintf(buf, len, "gemm_flow_kernel<NT=%d> %d shares in place of ", w.token_tiles, w.split_k)
-                       : is_width(w) ? snprintf(buf, len, "gemm_wide_kernel<256 rows x %d tokens> split_k=%d in place of ", 16 * WidthTiles(n, w.waves_m).nt, w.split_k ? w.split_k : 1)
+                       : is_width(w) ? describe_width(m, n, k, w, decode_mode, buf, len, " in place of ")
                        : is_broad(w) ? snprintf(buf, len, "gemm_broad_kernel<%d rows x %d tokens> split_k=%d in place of ", w.rows_per_wave, 16 * w.token_tiles, w.split_k)
-                       : is_tall(w) ? snprintf(buf, len, "gemm_tall_kernel<%d rows,NT=%d> split_k=%d in place of ", w.rows_per_wave, w.token_tiles, w.split_k)
-                                    : snprintf(buf, len, "gemm_wide_kernel<256 rows x 256 tokens> split_k=%d in place of ", w.split_k);
+                                     : snprintf(buf, len, "gemm_tall_kernel<%d rows,NT=%d> split_k=%d in place of ", w.rows_per_wave, w.token_tiles, w.split_k);
         return at < 0 || (size_t)at + 16 > len ? TUNA_OK : tuna_describe_launch(m, n, k, &c, decode_mode, buf + at, len - (size_t)at);
     }
-    if (is_width(c)) {
-        WidePlan wp;
-        if ((rc = plan_width(m, n, k, c, decode_mode, &wp))) return rc;
-        snprintf(buf, len, "gemm_wide_kernel<256 rows x %d tokens> split_k=%d%s", 16 * wp.args.g.nt[0], c.split_k ? c.split_k : 1,
-                 !c.split_k && wp.args.n_shares ? ", last tiles shared" : "");
-        return TUNA_OK;
-    }
+    if (is_width(c)) return describe_width(m, n, k, c, decode_mode, buf, len, "") < 0 ? validate_for(m, n, k, c, decode_mode) : TUNA_OK;
     if (c.lds_tile_rows > 0) {
         TiledPlan tp;
         if ((rc = plan_tiled(m, n, k, c, decode_mode, &tp))) return rc;
