@@ -94,6 +94,8 @@ def launched(m, n, k):
         r = dict(kind="tall", rows=numbers[0], token_tiles=numbers[1], split=numbers[2])
     elif kernel == "gemm_broad_kernel":
         r = dict(kind="broad", rows=numbers[0], token_tiles=numbers[1] // 16, split=numbers[2])
+    elif kernel == "gemm_wide_kernel" and " in place of" in d:  # (tiles of any width)
+        r = dict(kind="width", token_tiles=numbers[1] // 16, split=0 if "last tiles shared" in d.split(" in place of")[0] else numbers[2])
     elif kernel == "gemm_wide_kernel":
         r = dict(kind="wide", token_tiles=16, split=numbers[2])
     else:

@@ -60,7 +60,7 @@ def test_static_entry_point(kernel, m, n, k):
 
 def _calls():
     """(name, bytes of partial sums of an eager call, call, output, check, whether there is a launch without partial sums)"""
-    for _kernel, m, n, k in SHARED + [("gemm_flow_kernel", 33136, 41, 1088), ("gemm_wide_kernel", 8832, 497, 3456)]:
+    for _kernel, m, n, k in SHARED + [("gemm_flow_kernel", 33136, 41, 1088), ("gemm_wide_kernel", 10816, 351, 4032)]:
         q, s, x, code = _inputs(m, n, k, seed=n)
         out = _out(n, m)
         yield (f"matmul {m} {n} {k}", launched(m, n, k)[1], lambda q=q, s=s, x=x, code=code, out=out, m=m, n=n, k=k:

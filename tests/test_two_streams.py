@@ -9,11 +9,11 @@ pytestmark = pytest.mark.gpu
 
 
 # decode-batch shares that cross tiles (three and one token tile) and equal parts of tiles; tall and broad tiles in parts of k;
-# 256 x 256 tiles with the last ones shared, and split in three
+# 256-row tiles with the last ones shared, and split in three
 @pytest.mark.parametrize("kernel,m,n,k", [("gemm_flow_kernel", 33136, 41, 1088), ("gemm_flow_kernel", 33832, 16, 6336),
                                           ("gemm_flow_kernel", 33056, 35, 1024), ("gemm_tall_kernel", 4096, 64, 14336),
                                           ("gemm_tall_kernel", 5120, 37, 13824), ("gemm_broad_kernel", 8192, 160, 8192),
-                                          ("gemm_wide_kernel", 8448, 1100, 4096), ("gemm_wide_kernel", 8832, 497, 3456)])
+                                          ("gemm_wide_kernel", 10816, 351, 4032), ("gemm_wide_kernel", 10112, 406, 6272)])
 def test_two_streams(kernel, m, n, k):
     import torch
 
