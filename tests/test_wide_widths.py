@@ -177,6 +177,14 @@ def test_launches_of_any_number_of_steps_are_planned():
     assert ops.config_footprint(256, 256 * (tiles + 1), 64 * steps, _cfg256(3))[1] == 0
 
 
+def test_an_unsplit_config_of_up_to_half_a_round_of_tiles_needs_no_workspace():
+    from tuna_amd import ops
+
+    for m, n, k in ((8832, 497, 3456), (20992, 201, 7680), (2816, 2293, 14784), (17920, 4, 5376), (32768, 256, 28672)):
+        assert ops.config_footprint(m, n, k, _cfg256(1))[1] == 0, (m, n, k)
+        assert "shared" not in ops.describe_launch(m, n, k, _cfg256(1))
+
+
 def test_the_static_entry_point_refuses_no_pick_of_many_tokens_for_its_workspace():
     import random
 

@@ -232,7 +232,7 @@ static int planned_cus()
     return kMaxCus;
 }
 
-static bool wide_shares_last(int m, int n, int k);
+static bool wide_balance_pays(int m, int n, int k);
 static bool stream_applies(const tuna_gemm_config &c, int n, int decode);
 static bool plan_wide_dense(int m, int n, int k, int split, WidePlan *plan)
 {
@@ -310,7 +310,7 @@ static int plan_tiled(int m, int n, int k, const tuna_gemm_config &c, int decode
     a.steps_per_split = ceil_div(steps, c.split_k);
     if (wide) {
         plan->wide = true;
-        if (!plan_wide_dense(m, n, k, c.split_k == 1 && wide_shares_last(m, n, k) ? 0 : c.split_k, &plan->wide_plan))
+        if (!plan_wide_dense(m, n, k, c.split_k == 1 && wide_balance_pays(m, n, k) ? 0 : c.split_k, &plan->wide_plan))
             return fail(TUNA_ERR_UNSUPPORTED, "m=%d n=%d k=%d has too many 256 x 256 tiles for one launch", m, n, k);
         plan->ws_bytes = plan->wide_plan.ws_bytes;
         plan->n_counters = plan->wide_plan.n_counters;
@@ -865,14 +865,6 @@ static double wide_width_time(int m, int n, int k, int split_k, int nblk)
     if (t.large > 0) kinds[n_kinds++] = {(long long)t.large, wide_token_tiles(n < 256 ? n : 256)};
     if (t.small > 0) kinds[n_kinds++] = {(long long)t.small, 8};
     return wide_kinds_time(kinds, n_kinds, (int)t.steps, split_k, nblk > 0);
-}
-// Whether an unsplit config's 256 x 256 tiles are shared between the compute units in the end: as above, and from a quarter of a round on
-// by the model of any width (8832 x 3456 at 497 tokens, 70 tiles: 63 us whole, 59.5).
-static bool wide_shares_last(int m, int n, int k)
-{
-    const WideTiles t(m, n, k);
-    return wide_balance_pays(m, n, k) || (t.large + t.small > kMaxCus / 4 && t.large + t.small <= kMaxCus / 2 &&
-                                          wide_width_time(m, n, k, 0, 0) < wide_width_time(m, n, k, 1, 0));
 }
 static double width_time(int m, int n, int k, int token_tiles, int split, int nblk)
 {
@@ -1689,7 +1681,7 @@ static bool width_instead(int m, int n, int k, const tuna_gemm_config &c, bool f
     if (n <= 64) return false;
     const bool wide = c.lds_tile_rows == 256 && c.token_tiles == 16 && c.rows_per_wave != 32;
     double price;
-    if (wide) price = 0.97 * wide_width_time(m, n, k, c.split_k == 1 && wide_shares_last(m, n, k) ? 0 : c.split_k, 0);
+    if (wide) price = 0.97 * wide_width_time(m, n, k, c.split_k == 1 && wide_balance_pays(m, n, k) ? 0 : c.split_k, 0);
     else if (is_broad(c)) price = 0.96 * broad_time(m, n, k, c.rows_per_wave, c.token_tiles, c.split_k);
     else if (is_narrow(c) || is_narrow_any(c)) price = from_table ? 0.0 : 0.96 * narrow_time(m, n, k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles);
     else price = 0.96 * many_token_price(m, n, k, c);
@@ -3202,7 +3194,7 @@ static bool blockwise_width_instead(const BlockwiseCall &b, const tuna_gemm_conf
     const int nblk = b.k / b.block_size;
     const bool wide = blockwise_family(c) == kBlkTiled && c.lds_tile_rows == 256 && c.token_tiles == 16;
     double price = 0.0;
-    if (wide) price = 0.97 * wide_width_time(b.m, b.n, b.k, c.split_k == 1 && wide_shares_last(b.m, b.n, b.k) ? 0 : c.split_k, nblk);
+    if (wide) price = 0.97 * wide_width_time(b.m, b.n, b.k, c.split_k == 1 && wide_balance_pays(b.m, b.n, b.k) ? 0 : c.split_k, nblk);
     else if (is_broad(c)) price = 0.96 * broad_time(b.m, b.n, b.k, c.rows_per_wave, c.token_tiles, c.split_k, nblk);
     else if (blockwise_family(c) == kBlkNarrow) price = 0.96 * narrow_time(b.m, b.n, b.k, c.rows_per_wave, c.waves_k, c.prefetch, c.token_tiles, nblk);
     else if (blockwise_family(c) == kBlkTiled) price = 0.96 * blockwise_tiled_price(b, c);
