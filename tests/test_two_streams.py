@@ -77,3 +77,24 @@ def test_groups_on_two_streams(m, k, counts):
     for want, out in zip(alone, outs):
         for o in out:
             assert torch.equal(o, want)
+
+
+# (k of a few steps: whole tiles of the groups' own widths are ahead of shared ones of 256 tokens, and need no partial sums)
+def test_a_call_of_few_and_many_tokens_leaves_the_least_workspace():
+    import numpy as np
+    import torch
+
+    from tuna_amd import _lib, ops
+
+    m, k, counts = 5120, 1024, (157, 232, 14, 1207, 1494, 4)
+    offs = np.concatenate([[0], np.cumsum(counts)]).tolist()
+    q, s, x, code = _inputs(m * len(counts), offs[-1], k, seed=k)
+    out = _out(offs[-1], m)
+    ops.matmul_grouped(x, q, s, code, out, m, len(counts), k, offs)
+    torch.cuda.synchronize()
+    assert _lib.lib().tuna_release_workspaces() == _lib.OK
+    free = torch.cuda.mem_get_info()[0]
+    for _ in range(2):
+        ops.matmul_grouped(x, q, s, code, out, m, len(counts), k, offs)
+        torch.cuda.synchronize()
+        assert 8 << 20 <= free - torch.cuda.mem_get_info()[0] <= 16 << 20

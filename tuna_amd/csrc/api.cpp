@@ -2238,12 +2238,10 @@ static int grouped_flow_shares(int m_group, int n_active, int nt, int k)
 static double grouped_many_time(int m_group, int n_groups, int k, const int32_t *offsets, int pass, WideArgs *a, int *split)
 {
     int many = 0;
-    bool few = false;
     double apart = 0.0, together = 0.0;
     *split = -1;
     for (int e = 0; e < n_groups; ++e) {
         const int cnt = offsets[e + 1] - offsets[e];
-        few = few || (cnt > 0 && cnt <= pass);
         if (cnt <= pass) continue;
         const double flops = 2.0 * m_group * cnt * k, bytes = 0.5 * m_group * k + 2.0 * cnt * ((double)m_group + k);
         const double t_flops = flops / 0.95e9, t_bytes = bytes / 1.9e6;
@@ -2267,10 +2265,6 @@ static double grouped_many_time(int m_group, int n_groups, int k, const int32_t 
             if (of[nt]) kinds[n_kinds++] = {of[nt], nt};
         for (const int s : kWidthSplits) {
             if (!width_split_sensible(tiles, steps, s)) continue;
-            // (up to 16 steps, with groups of up to `pass` tokens beside these: the last tiles of 256 tokens shared, as ever.  Not for
-            // speed - 5120 x 1024 on 157 to 1494 tokens takes 55 us so, 40 as whole tiles of 144 -, but a call of both kinds is what
-            // provides a stream's workspace where one is warmed up for a capture.)
-            if (steps <= 16 && few && (tt < 16 || s != (tiles > kMaxCus / 2 ? 0 : 1))) continue;
             const double us = wide_kinds_time(kinds, n_kinds, steps, s, false);
             if (!best || us < together) best = tt, together = us, *split = s;
         }
@@ -2339,6 +2333,8 @@ static bool grouped_broad_pays(int m_group, int n_groups, int k, const int32_t *
     return plan_gemm_broad_groups(best_rows, best_nt, plan, groups);
 }
 
+constexpr int kGroupedPassTokens = 64;  // of a group in one pass of the grouped kernels
+
 // Grouped GEMM: n_groups stacked weight matrices of m_group rows, group e applied to the
 // activation rows offsets[e] .. offsets[e+1]-1 only.  The offsets are a host array: they are
 // validated here and travel to the kernel as launch arguments (no device buffer, no copy).
@@ -2379,7 +2375,6 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
     // tokens leave the device half empty at the end of each of eight launches (706 us; 406 in one).
     // Before either: one launch of broad tiles over all groups where its model is ahead of these two and of the decode-batch
     // kernel's for the groups of up to 64.
-    constexpr int kGroupedPassTokens = 64;
     if (!cfg && decode == TUNA_DECODE_GEMM) {
         BroadPlan plan;
         BroadGroups groups;
@@ -2504,6 +2499,19 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
     hipError_t e = launch_gemm(plan, stream);
     if (e != hipSuccess) return hip_fail(e, "grouped gemm launch");
     return TUNA_OK;
+}
+
+// A call with groups of up to 64 tokens and of more leaves its stream a workspace, the least one where its own launches need none: tokens
+// are routed differently in every call, and one that is captured behind this one finds some room for its partial sums.
+static void leave_workspace(int n_groups, const int32_t *offsets, hipStream_t stream)
+{
+    bool few = false, many = false;
+    for (int e = 0; e < n_groups; ++e) {
+        const int cnt = offsets[e + 1] - offsets[e];
+        (cnt > kGroupedPassTokens ? many : few) |= cnt > 0;
+    }
+    Workspace w;
+    if (few && many && !workspace_room(stream).bytes) (void)get_workspace(stream, 1, 1, &w);  // (a capturing stream keeps what it has)
 }
 
 extern "C" int tuna_matmul_blockwise(const void *q, const void *x, const void *code, const void *absmax, void *out, int m, int n,
@@ -2720,8 +2728,9 @@ TUNA_EXPORT int tuna_matmul_grouped(const void *q, const void *x, const void *co
                                     int m_group, int n_groups, int k, const int32_t *token_offsets,
                                     const tuna_gemm_config *cfg, int decode_mode, void *stream)
 {
-    return matmul_grouped_impl(q, x, code, absmax, out, m_group, n_groups, k, token_offsets, cfg, decode_mode,
-                               static_cast<hipStream_t>(stream));
+    const int rc = matmul_grouped_impl(q, x, code, absmax, out, m_group, n_groups, k, token_offsets, cfg, decode_mode, static_cast<hipStream_t>(stream));
+    if (!rc && !cfg && decode_mode == TUNA_DECODE_GEMM) leave_workspace(n_groups, token_offsets, static_cast<hipStream_t>(stream));
+    return rc;
 }
 
 TUNA_EXPORT int tuna_dequant(const void *q, const void *absmax, const void *code, void *out, int m, int k, void *stream)
