@@ -124,10 +124,11 @@ def test_the_stated_errors_are_those_of_the_kept_launches(kind, off):
     assert 100 * lm.errors(rows, *lm.MODELS[kind])[0] == pytest.approx(off, abs=0.06)
 
 
-# (one row tile of a batched launch more than compute units; lean launches; two and three token tiles)
+# (one row tile of a batched launch more than compute units; lean launches; two and three token tiles; narrow rows with two)
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k,before", [(33024, 9, 1536, "weights through LDS"), (20480, 20, 8192, "weights through LDS"), (18944, 4, 3584, "gemm_lean_kernel"),
-                                          (13824, 17, 5120, ""), (24576, 40, 3072, "")])
+                                          (24576, 40, 3072, "weights through LDS"), (9728, 33, 3072, "gemm_lean_kernel"),
+                                          (13824, 17, 5120, "gemm_narrow_kernel<LW=4")])
 @pytest.mark.parametrize("epilogue", [0, 1, 2])
 def test_picks_in_place_of_lean_and_batched_launches(m, n, k, before, epilogue):
     """What the library picks by itself against the general kernel: the same products, summed in another order."""
@@ -135,8 +136,8 @@ def test_picks_in_place_of_lean_and_batched_launches(m, n, k, before, epilogue):
 
     from tuna_amd import _lib, ops
 
-    name = ops.describe_launch(m, n, k)
-    assert "gemm_tall_kernel" in name and before in name.split("in place of")[-1]
+    pick, _, instead = ops.describe_launch(m, n, k).partition(" in place of ")
+    assert pick.startswith("gemm_tall_kernel") and before in instead
     general = ops.GemmConfig.from_dict(dict(rows_per_wave=64, waves_m=1, waves_k=8, split_k=1, prefetch=2, x_chunk=512, token_tiles=1,
                                             xcd_swizzle=0, lds_tile_rows=0))
     q, s, x, code = _inputs(m, n, k, seed=m + n)

@@ -40,10 +40,11 @@ def test_two_streams(kernel, m, n, k):
             assert torch.equal(o, want)
 
 
-# decode-batch shares that are equal parts of tiles, and that cross them; 256 x 256 tiles split in two and with shared last
-# tiles, with decode-batch shares that need partial sums behind theirs
+# decode-batch shares that are equal parts of tiles, and that cross them; 256-row tiles of groups, whole with decode-batch shares behind
+# them, split in two, and with shared last tiles and decode-batch shares whose partial sums lie behind theirs
 @pytest.mark.parametrize("m,k,counts", [(2816, 2048, (3, 0, 17, 32, 1, 16, 8, 2)), (4096, 4096, (3, 0, 17, 32, 1, 16, 8, 2)),
-                                        (4608, 2688, (5, 1250, 0, 420, 30)), (5120, 1024, (157, 232, 14, 1207, 1494, 4))])
+                                        (4608, 2688, (5, 1250, 0, 420, 30)), (5120, 1024, (157, 232, 14, 1207, 1494, 4)),
+                                        (2048, 3712, (538, 0, 1544)), (6656, 4096, (503, 16, 1981, 42))])
 def test_groups_on_two_streams(m, k, counts):
     import numpy as np
     import torch
