@@ -828,19 +828,20 @@ static double wide_kinds_time(const WideKind *kinds, int n_kinds, int steps, int
         // in rounds of a tile per compute unit, each as long as its widest tile
         double us = 0.0;
         long long first = 0, seen = 0;
+        const double u = busy((double)tiles);
         for (int i = 0; i < n_kinds; ++i) {
             seen += kinds[i].tiles;
             const long long rounds = seen > first ? (seen - first + kMaxCus - 1) / kMaxCus : 0;
-            us += rounds * (steps * step_us(run(i), busy((double)tiles)) + c.end * run(i));
+            us += rounds * (steps * step_us(run(i), u) + c.end * run(i));
             first += rounds * kMaxCus;
         }
         return us;
     }
     auto over = [&](double parts, double wgs) { return c.over + c.parts * widest * (parts > 2 ? parts - 2 : 0) + c.sums * widest * (wgs < cus ? wgs : cus) / cus; };
     if (split > 1) {
-        const double wgs = (double)tiles * split;
+        const double wgs = (double)tiles * split, u = busy(wgs);
         double work = 0.0;
-        for (int i = 0; i < n_kinds; ++i) work += kinds[i].tiles * (steps * step_us(run(i), busy(wgs)) / split + c.end * run(i));
+        for (int i = 0; i < n_kinds; ++i) work += kinds[i].tiles * (steps * step_us(run(i), u) / split + c.end * run(i));
         if (n_kinds > 1) return 1.09 * (ceil(wgs / cus) * work / tiles * c.ragged + c.end * widest * c.cross + over(split + 1, wgs));  // (shares cross tiles)
         return ceil(wgs / cus) * work / tiles + over(split, wgs);
     }
@@ -881,19 +882,24 @@ static bool width_split_sensible(long long tiles, int steps, int split)
 // The launch of such tiles that takes least time, below *us, with partial sums that `room` holds.
 static bool best_width(int m, int n, int k, int nblk, const Room &room, tuna_gemm_config *width, double *us)
 {
+    const int row_tiles = ceil_div(m, 256), steps = ceil_div(k, 64);
     bool found = false;
     for (int tt = 16; tt >= 8; --tt) {
         const WidthTiles t(n, tt);
         if (t.nt != tt) continue;  // (that many token tiles, evenly divided, are narrower ones)
+        const WideKind kind = {(long long)row_tiles * t.count, t.nt};
+        if (kind.tiles > kWideMostTiles) continue;
         for (const int split : kWidthSplits) {
-            if (!width_split_sensible((long long)ceil_div(m, 256) * t.count, ceil_div(k, 64), split)) continue;
-            const double time = width_time(m, n, k, tt, split, nblk);
+            if (!width_split_sensible(kind.tiles, steps, split)) continue;
+            const double time = wide_kinds_time(&kind, 1, steps, split, nblk > 0);
             if (time >= *us) continue;
             tuna_gemm_config c;
             memset(&c, 0, sizeof(c));
             c.rows_per_wave = 64, c.waves_m = tt, c.waves_k = 1, c.prefetch = 2, c.x_chunk = 64, c.token_tiles = 16, c.split_k = split, c.lds_tile_rows = 256;
-            WidePlan plan;
-            if (plan_width(m, n, k, c, TUNA_DECODE_GEMM, &plan) != TUNA_OK || !room.holds(plan.ws_bytes, plan.n_counters)) continue;
+            if (room.bytes != kRoomToGrow.bytes) {
+                WidePlan plan;
+                if (plan_width(m, n, k, c, TUNA_DECODE_GEMM, &plan) != TUNA_OK || !room.holds(plan.ws_bytes, plan.n_counters)) continue;
+            }
             *width = c, *us = time, found = true;
         }
     }
@@ -2290,7 +2296,7 @@ static double grouped_many_time(int m_group, int n_groups, int k, const int32_t 
 // group each, k unsplit - is ahead of the launches below: eight experts of 14336 x 4096 on 512 tokens, some of them with more than
 // 64, 147 -> 98 us, of 4096 x 14336 131 -> 84; 64 experts of 1536 x 4096 on 6144 tokens 135 -> 120.  On 120 random launches of 16 to
 // 400 tokens per group 1.18 x, up to 3.3 x for small experts, which launched one by one before; worst 0.92.
-static bool grouped_broad_pays(int m_group, int n_groups, int k, const int32_t *offsets, int max_tok, BroadPlan *plan, BroadGroups *groups)
+static bool grouped_broad_pays(int m_group, int n_groups, int k, const int32_t *offsets, int max_tok, double many_us, BroadPlan *plan, BroadGroups *groups)
 {
     if (max_tok <= 32) return false;
     memset(groups, 0, sizeof(*groups));
@@ -2306,12 +2312,7 @@ static bool grouped_broad_pays(int m_group, int n_groups, int k, const int32_t *
     // (less than 4 MB of weights: as before, a large group by the launch that a dense call takes; none of the measured ones is
     // that small)
     if (groups->n < 2 || 0.5 * m_group * groups->n * k < 4e6) return false;
-    double price = 0.0, us = 0.0;
-    if (groups->n > few) {
-        WideArgs wide;
-        int split;
-        price += grouped_many_time(m_group, n_groups, k, offsets, 64, &wide, &split);
-    }
+    double price = many_us, us = 0.0;  // (of the launches below)
     if (few) {
         if (!flow_best_shares((long long)ceil_div(m_group, 256) * few, ceil_div(ceil_div(k, 64), 4), ceil_div(few_tok, 16), kRoomToGrow, &us)) return false;
         price += us;
@@ -2375,10 +2376,17 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
     // tokens leave the device half empty at the end of each of eight launches (706 us; 406 in one).
     // Before either: one launch of broad tiles over all groups where its model is ahead of these two and of the decode-batch
     // kernel's for the groups of up to 64.
+    WidePlan many;
+    int many_split = -1;
+    double many_us = 0.0;
+    if (!cfg && decode == TUNA_DECODE_GEMM && max_tok > kGroupedPassTokens) {
+        memset(&many, 0, sizeof(many));
+        many_us = grouped_many_time(m_group, n_groups, k, offsets, kGroupedPassTokens, &many.args, &many_split);
+    }
     if (!cfg && decode == TUNA_DECODE_GEMM) {
         BroadPlan plan;
         BroadGroups groups;
-        if (grouped_broad_pays(m_group, n_groups, k, offsets, max_tok, &plan, &groups)) {
+        if (grouped_broad_pays(m_group, n_groups, k, offsets, max_tok, many_us, &plan, &groups)) {
             BroadArgs &a = plan.args;
             a.q = static_cast<const uint8_t *>(q);
             a.x = x;
@@ -2392,28 +2400,22 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
     const size_t group_q_bytes = (size_t)m_group * (size_t)k / 2;
     bool many_done = false;
     size_t many_ws = 0;  // bytes of its partial sums
-    if (!cfg && decode == TUNA_DECODE_GEMM && max_tok > kGroupedPassTokens) {
-        WidePlan plan;
-        memset(&plan, 0, sizeof(plan));
-        WideArgs &a = plan.args;
-        int split;
-        grouped_many_time(m_group, n_groups, k, offsets, kGroupedPassTokens, &a, &split);
-        if (split >= 0) {
-            a.q = static_cast<const uint8_t *>(q);
-            a.x = x;
-            a.code = static_cast<const float *>(code);
-            a.absmax = static_cast<const float *>(absmax);
-            a.out = out;
-            rc = plan_gemm_wide(split, planned_cus(), &plan) ? TUNA_OK : TUNA_ERR_UNSUPPORTED;
-            if (!rc && plan.ws_bytes) rc = provide_workspace(false, stream, plan.ws_bytes, plan.n_counters, &a.ws, &a.counters);
-            if (rc && split != 1)  // (a stream that is capturing, with too small a workspace: whole tiles)
-                rc = plan_gemm_wide(1, planned_cus(), &plan) ? TUNA_OK : TUNA_ERR_UNSUPPORTED;
-            if (!rc) {
-                const hipError_t e = launch_gemm_wide(plan, false, stream);
-                if (e != hipSuccess) return hip_fail(e, "grouped many-token gemm launch");
-                many_done = true;
-                many_ws = plan.ws_bytes;
-            }
+    if (many_split >= 0) {
+        WideArgs &a = many.args;
+        a.q = static_cast<const uint8_t *>(q);
+        a.x = x;
+        a.code = static_cast<const float *>(code);
+        a.absmax = static_cast<const float *>(absmax);
+        a.out = out;
+        rc = plan_gemm_wide(many_split, planned_cus(), &many) ? TUNA_OK : TUNA_ERR_UNSUPPORTED;
+        if (!rc && many.ws_bytes) rc = provide_workspace(false, stream, many.ws_bytes, many.n_counters, &a.ws, &a.counters);
+        if (rc && many_split != 1)  // (a stream that is capturing, with too small a workspace: whole tiles)
+            rc = plan_gemm_wide(1, planned_cus(), &many) ? TUNA_OK : TUNA_ERR_UNSUPPORTED;
+        if (!rc) {
+            const hipError_t e = launch_gemm_wide(many, false, stream);
+            if (e != hipSuccess) return hip_fail(e, "grouped many-token gemm launch");
+            many_done = true;
+            many_ws = many.ws_bytes;
         }
     }
     if (!cfg && !many_done) {

@@ -241,7 +241,7 @@ bool plan_gemm_wide(int split, int cus, WidePlan *plan)
         a.g.nt[e] = split == 1 ? nt : wide_divided_token_tiles(nt);
         const long long here = (long long)a.row_tiles * a.g.tok_tiles[e];
         tiles += here;
-        if (tiles > 0x7ffffffe) return false;
+        if (tiles > kWideMostTiles) return false;
         weight += here * a.steps_total * wide_step_weight(a.g.nt[e]);
         a.g.tile_end[e] = (int)tiles, total[e] = weight;
         if (a.g.nt[e] == a.g.nt[0]) widest += here;

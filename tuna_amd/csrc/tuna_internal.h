@@ -202,6 +202,8 @@ inline void wide_balance(long long tiles, long long widest, long long weight, un
     *n_shares = tiles > *whole ? (int)shares : 0;
 }
 
+constexpr long long kWideMostTiles = 0x7ffffffe;  // of a launch
+
 // Bytes between the partial-sum slots: a tile's 256 KB and 4352 more.
 constexpr size_t kWideSlot = (size_t)256 * 256 * 4 + 4352;
 
