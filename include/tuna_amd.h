@@ -223,7 +223,8 @@ int tuna_matmul_multi_blockwise(const tuna_gemm_problem *problems, int count, in
  * cannot grow -, and the groups of more than 64 tokens (prefill sizes) leave the grouped launch, which would stream their weights once per 64 tokens: each runs
  * as a dense GEMM of its own on the same stream - tuna_matmul on its slices of q, absmax, x and
  * out, bit-identical to that call - or, several of them where that is predicted to be faster, all
- * in one launch of 256-row tiles, within the GEMM's tolerance of it.  No counterpart in the reference, whose 8-expert
+ * in one launch of 256-row tiles, within the GEMM's tolerance of it.  A call with groups of both
+ * kinds leaves its stream a workspace of at least 8 MB.  No counterpart in the reference, whose 8-expert
  * benchmark applies every expert to every token (README.md:16-18); this is the op a
  * router-driven Mixtral layer needs. */
 int tuna_matmul_grouped(const void *q, const void *x, const void *code, const void *absmax,
@@ -291,9 +292,10 @@ int tuna_blockwise_table_entry(int i, int *m, int *n_lo, int *n_hi, int *k, int 
 /* Shape -> config.  Replaces the if-chain of kernel.cu:3018-3156 over the constants of
  * configs.cu:56-3331 by a table lookup on (m, n-bucket, k) with a derived fallback.
  * Runs on the host only (no device needed).  Returns 1 in *from_table when the shape
- * hit a tuned entry.  A call without a config runs it, except that the decode-batch kernel or the
- * narrow-row kernel's variants for any k (up to 64 tokens) or 256-row tiles (from 65) take its place where they are predicted to be faster
- * (tuna_describe_launch says so). */
+ * hit a tuned entry.  A call without a config runs it, except that the decode-batch kernel, the
+ * narrow-row kernel's variants for any k or tall tiles (up to 64 tokens), broad tiles (from 49) or
+ * 256-row tiles (from 65) take its place where they are predicted to be faster (tuna_describe_launch
+ * says so). */
 int tuna_select_config(int m, int n, int k, tuna_gemm_config *cfg, int *from_table);
 /* The config tuna_matmul_ex(cfg = NULL, decode_mode) runs: the table lookup above for
  * TUNA_DECODE_GEMM; for TUNA_DECODE_DEQUANT, whose kernel variants the table is not tuned for,

@@ -2373,7 +2373,7 @@ static int matmul_grouped_impl(const void *q, const void *x, const void *code, c
     // hundreds of microseconds of matrix work.  (With an explicit config every group goes through the grouped kernel.)
     // Several such groups become ONE launch of 256-row tiles (gemm_wide.hip, gemm_wide_whole.hip) where that is predicted to be faster than a
     // launch each, priced at 8 us and the larger of 0.95 PFLOP/s and 1.9 TB/s: eight experts of 14336 x 4096 on 4096
-    // tokens leave the device half empty at the end of each of eight launches (706 us; 406 in one).
+    // tokens leave the device half empty at the end of each of eight launches (706 us; 424 in one, 458 with tiles of 256 and 128 only).
     // Before either: one launch of broad tiles over all groups where its model is ahead of these two and of the decode-batch
     // kernel's for the groups of up to 64.
     WidePlan many;

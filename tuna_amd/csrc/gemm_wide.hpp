@@ -13,11 +13,13 @@
 //     reads, addresses and scalings; the loads behind the step's one barrier.
 //
 // What bounds it: the power limit.  With all compute units at work a step of 256 tokens takes 1.4 us, with half of them 1.08 (0.85 at 2.4 GHz
-// would be the matrix pipes alone), and what is left out of it saves what it draws: table reads 10 per cent, the way of the
-// activations into LDS 9, their fragments 5; an fp16 product of torch takes the same time per k.  So what pays is no work for
+// would be the matrix pipes alone, which are busy for 75 per cent of the cycles over 128 steps, 68 over 64, 52 with tiles of 128 tokens), and
+// what is left out of it saves what it draws: table reads 10 per cent, the way of the activations into LDS 9, their fragments 5.  torch's fp16
+// product, which decodes nothing, takes as long on the same card (8192 x 8192 at 2048 tokens 182 us, here 190; at 2000 tokens 28672 x 4096 347
+// and 350, 4096 x 14336 190 and 185, 6144 x 4096 82 and 81, 4096 x 4096 60 and 62).  So what pays is no work for
 // tokens that are not there: NT for every number of token tiles (of 8 and 16 only, 4096 x 14336 at 777 tokens with blocks of 128 took
-// 119 us in the smaller tiles that were picked then and takes 95; 4096 x 4096 at 2000 tokens 80 -> 62, 6144 x 4096 91 -> 84).  A step decodes as
-// much whatever NT is: 0.33 us of it, beside 0.06 per token tile.  Around the loop (stamps at 4096 x 4096 x 4096): 3.2 us to the
+// 119 us in the smaller tiles that were picked then and takes 93; 4096 x 4096 at 2000 tokens 74 -> 62, 6144 x 4096 88 -> 81.5).  A step decodes as
+// much whatever NT is: 0.36 us of it, beside 0.04 to 0.065 per token tile.  Around the loop (stamps at 4096 x 4096 x 4096): 3.2 us to the
 // first step (4.9 with the table made before the first loads) and 3.1 for the outputs (6.9 as 16-byte pieces of 64 rows, a lane its own).
 //
 // KTAIL: k is any multiple of 8 - the slots of the last k-step beyond k load the last slot inside k (no access leaves a row), and their
